@@ -32,15 +32,14 @@ FP64_PEAK_TFLOPS = 78.6
 
 def alg_bytes(N):
     """Compulsory FP64 traffic of the two-sweep DGSEM+BR1 stage (bytes):
-    per node  - gradient sweep: Q(5) Ja(9) 1/J(1) in, grad(15) out  = 240 B
-              - flux sweep (volume kernel): Q(5) grad(15) Ja(9) J(1) G(5) in, G(5) Q(5) out = 360 B
+    per node  - gradient sweep: Q(5) Ja(9) J(1) in, the viscous flux tensor(9) out  = 192 B
+              - flux sweep: Q(5) tensor(9) Ja(9) J(1) G(5) in, G(5) Q(5) out = 312 B
     per face node - gradient sweep: both traces of Q (10), n and |Ja| (4) = 112 B
-                  - flux sweep (face kernel): both traces of Q and grad (40), n t1 |Ja| (7) = 376 B
+                  - flux sweep: both traces of Q and the tensor (28), n t1 |Ja| (7) = 280 B
                     (the second tangent is n x t1, formed in the kernel)
     with 3/(N+1) face nodes per node on a conforming hexahedral mesh."""
     fpn = 3.0 / (N + 1)
-    return dict(grad=240.0 + 112.0 * fpn, face=376.0 * fpn, volume=360.0,
-                stage=600.0 + 488.0 * fpn)
+    return dict(grad=192.0 + 112.0 * fpn, volume=312.0 + 280.0 * fpn, stage=504.0 + 392.0 * fpn)
 
 
 def host_cpu():
@@ -447,13 +446,11 @@ def main():
     # per-kernel HIP-event timing over a second pass of the same steps
     eng.set_timing(True)
     eng.advance(args.steps, 0.4, 0.4)
-    kt = eng.kernel_times()   # ms per launch: grad, face, volume, stage
+    kt = eng.kernel_times()   # ms per launch: grad, face (no launch of its own here), volume, stage
     eng.set_timing(False)
     B = alg_bytes(args.order)
-    FS = case["F"] * (args.order + 1) ** 2
     kern = {
         "grad": dict(ms=kt[0], bytes=B["grad"] * nd),
-        "face": dict(ms=kt[1], bytes=376.0 * FS),
         "volume": dict(ms=kt[2], bytes=B["volume"] * nd),
     }
     for k in kern.values():

@@ -1,28 +1,29 @@
 // hx3d engine: MI355X (gfx950) HIP kernels for one explicit RK3 step of HORSES3D's
 // compressible Navier-Stokes DGSEM on Gauss-Lobatto nodes, and the C ABI of include/hx3d.h.
 //
-// One stage (ComputeTimeDerivative, SpatialDiscretization.f90:227-320) is three launches:
+// One stage (ComputeTimeDerivative, SpatialDiscretization.f90:227-320) is two launches:
 //   k_grad    per element: local gradient (HexElement_ComputeLocalGradient,
 //             HexElementClass.f90:427-531) + BR1 lifting (BR1_LiftGradients,
-//             EllipticBR1.f90:168-397).  With GL nodes the face trace is the boundary node
-//             itself (ProlongSolutionToFaces is a copy) and the lifting only touches
-//             boundary nodes, so the neighbour's boundary state is gathered directly.
-//   k_face    per face node: Riemann flux (Roe/LxF) + BR1 viscous average
-//             (computeElementInterfaceFlux, SD.f90:1710-1799), written once per face.
-//   k_volume  per element: viscosity (Sutherland + LES), inviscid/viscous contravariant
-//             fluxes, the standard or split-form volume integral
+//             EllipticBR1.f90:168-397), viscosity (Sutherland + LES) and the viscous flux
+//             tensor.  With GL nodes the face trace is the
+//             boundary node itself (ProlongSolutionToFaces is a copy) and the lifting only
+//             touches boundary nodes, so the neighbour's boundary state is gathered directly.
+//   k_volume  per element: the face fluxes of its faces, Riemann flux (Roe/LxF) + BR1 viscous
+//             average (computeElementInterfaceFlux, SD.f90:1710-1799); inviscid/viscous
+//             contravariant fluxes, the standard or split-form volume integral
 //             (TimeDerivative_VolumetricContribution, SD.f90:1602-1682), the surface
 //             integral of the face fluxes, 1/J (SD.f90:483-494), and the Williamson RK3
 //             register update (TakeRK3Step, ExplicitMethods.f90:748-775), fused.
+// The state is kept twice: k_volume reads one copy and writes the other, which the host then swaps.
 // Device layout: structure of arrays, one contiguous array per variable:
 //   per node g = e*(N+1)^3 + i + (N+1)(j + (N+1)k), S the padded node count:
-//     Q[v*S + g], G[v*S + g], vgrad[c*S + g] (velocity gradients, grad T), Ja[(3d + c)*S + g],
-//     J[g], invJ[g]
+//     Q[v*S + g], G[v*S + g], visc[c*S + g] (viscous values), Ja[(3d + c)*S + g], J[g]
 //   per element face node x = (6e + slot)(N+1)^2 + a + (N+1)b, ES the padded count:
-//     fe[v*ES + x] (face flux times 1/w_0, negated on the right side), egeo[c*ES + x]
-//     (normal, |Ja|), nbr[x] (2 * neighbour node + side)
-//   per face node q = f(N+1)^2 + i + (N+1)j (left element's face coordinates), FS the count:
-//     fgeo[c*FS + q] (n, t1, t2, |Ja|), fnode[q] (left node, right node, left x, right x)
+//     egeo[c*ES + x] (normal, |Ja|, with
+//     Lax-Friedrichs t1, and t2 where it is not n x t1), nbr[x] (2 * neighbour node + side),
+//     nbx[x] (2 * neighbour's element face node + side)
+// Gauss nodes add per face node q = f(N+1)^2 + i + (N+1)j (left element's face coordinates), FS
+// the count: fgeo[c*FS + q] (n, t1, t2, |Ja|), fnode[q] (left node, right node, left x, right x)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -87,10 +88,12 @@ __device__ __forceinline__ double wave_sum(double x)
 }
 
 // MaxTimeStep (DGSEMClass.f90:870-1035): per-node convective and viscous limits, block
-// minima to part, reduced by k_dt_reduce (the minimum is exact and independent of order).
+// minima to part, reduced by k_dt_reduce (the minimum is exact and independent of order), or to
+// the dt slots the volume kernel reads (slots, see hxk::DtLimits).
 __global__ void __launch_bounds__(256)
 k_maxdt(const double *__restrict__ Q, const double *__restrict__ Ja, const double *__restrict__ Jac,
-        long nodes, long S, double dcsi, double cfl, double dcfl, Phys ph, double *__restrict__ part)
+        long nodes, long S, double dcsi, double cfl, double dcfl, Phys ph, double *__restrict__ part,
+        unsigned long long *__restrict__ slots)
 {
     const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
     double tc = INFINITY, tv = INFINITY;
@@ -103,7 +106,8 @@ k_maxdt(const double *__restrict__ Q, const double *__restrict__ Ja, const doubl
         for (int c = 0; c < 9; ++c) ja[c] = Ja[c * S + g];
         hx::dt_limits(ph, q, ja, Jac[g], dcsi, dcsi, dcsi, cfl, dcfl, tc, tv);
     }
-    hxk::block_min_pair(tc, tv, part, threadIdx.x, blockIdx.x);
+    if (slots) hxk::block_min_slot(tc, tv, slots, threadIdx.x, 0, blockIdx.x);
+    else hxk::block_min_pair(tc, tv, part, threadIdx.x, blockIdx.x);
 }
 
 // The minima of n (convective, viscous) pairs as the bit patterns of a dt slot.
@@ -263,11 +267,12 @@ k_kinetic(const double *__restrict__ Q, const double *__restrict__ Jac, const do
 //        4 internal energy      rho e
 //        5 entropy              log p - gamma log rho
 //        6 math entropy         -rho (log p - gamma log rho) / (gamma - 1)
-// The velocity gradients are the gradient kernel's viscous state (uniform orders) or formed from
-// the lifted state gradients U_x, U_y, U_z as getVelocityGradients_State does (mixed orders).
+// |curl u|^2 as the volume kernel left it (Gauss-Lobatto nodes of one order), or from the velocity
+// gradients: the gradient kernel's viscous state (Gauss nodes of one order), or formed from the
+// lifted state gradients U_x, U_y, U_z as getVelocityGradients_State does (mixed orders).
 __global__ void __launch_bounds__(256)
-k_monitor(int kind, const double *__restrict__ Q, const double *__restrict__ QD, const double *__restrict__ vgrad,
-          const double *__restrict__ U, const double *__restrict__ Jac, const double *__restrict__ wq, long nodes,
+k_monitor(int kind, const double *__restrict__ Q, const double *__restrict__ QD, const double *__restrict__ curl2,
+          const double *__restrict__ vgrad, const double *__restrict__ U, const double *__restrict__ Jac, const double *__restrict__ wq, long nodes,
           long S, Phys ph, double *__restrict__ part)
 {
     __shared__ double sk[4], sv[4];
@@ -286,6 +291,8 @@ k_monitor(int kind, const double *__restrict__ Q, const double *__restrict__ QD,
             f = f + u * QD[2 * S + g] - 0.5 * (u * u) * QD[g];
             u = q[3] / q[0];
             f = f + u * QD[3 * S + g] - 0.5 * (u * u) * QD[g];
+        } else if (kind == 2 && curl2) {
+            f = curl2[g];
         } else if (kind == 2) {
             double ux[3], uy[3], uz[3];   // d(u, v, w)/dx, /dy, /dz
             if (vgrad) {
@@ -458,6 +465,11 @@ struct hx3d_engine {
     double dcsi = 0;
     hipStream_t stream = nullptr;
     double *dQ = nullptr, *dG = nullptr, *dVgrad = nullptr, *dJa = nullptr;
+    // Gauss-Lobatto nodes, one order: the state's second copy (swapped with dQ by every update), the
+    // viscous values at the nodes (hxk::viscous_values), |curl u|^2 where a stage leaves its derivative (the
+    // enstrophy monitor's), the filter widths of the element faces, the slots of the dt limits
+    double *dQn = nullptr, *dVisc = nullptr, *dCurl = nullptr, *dEfdelta = nullptr;
+    unsigned long long *dSlots = nullptr;
     double *dFe = nullptr, *dQDot = nullptr, *dEdelta = nullptr, *dFdelta = nullptr, *dWq = nullptr;
     // Gauss nodes, one order: Q and gradient traces in element-face order, the neighbour table
     double *dQtr = nullptr, *dGtr = nullptr;
@@ -470,7 +482,7 @@ struct hx3d_engine {
     int4 *dFnode = nullptr;
     // mixed orders (p-anisotropic elements, mortar faces)
     bool mixed = false;
-    bool t2x = false;     // uniform orders: the face kernel forms t2 = n x t1 (see tangent2_is_cross)
+    bool t2x = false;     // uniform orders: the volume kernel forms t2 = n x t1 (see tangent2_is_cross)
     bool gauss = false;   // Gauss nodes (one order: hxg kernels; per-element orders: the mixed path's)
     long FSm = 0;
     int *dN3 = nullptr, *dEfoff = nullptr, *dEofn = nullptr;
@@ -509,7 +521,7 @@ struct hx3d_engine {
     hxk::Multi mc{};
     int4 *dBlocks = nullptr;
     hxk::CaseConst *dCC = nullptr;
-    int *dActive = nullptr, *dFcase = nullptr, *dPfirst = nullptr;
+    int *dActive = nullptr;
     double *dTimeM = nullptr;
     double *dTime = nullptr;   // [ncases] the time of each case
     long dev_bytes = 0;   // device memory the engine holds
@@ -518,6 +530,7 @@ struct hx3d_engine {
     bool use_graph = false;
     hipGraphExec_t step_graph = nullptr;
     double graph_cfl = 0, graph_dcfl = 0;
+    double *graph_Q = nullptr;   // the copy of the state the captured steps start from
     double ktime[4] = {0, 0, 0, 0};
     std::vector<hipEvent_t> evpool;   // timing: 4 events per stage of the last hx3d_advance
     std::string err;
@@ -537,7 +550,18 @@ int dalloc(hx3d_engine *eng, T **p, size_t n)
     return 0;
 }
 
-// elements per block for the element kernels
+// The dt limits' slots of ncases cases (hxk::DtLimits), emptied by init_slots on the engine's stream
+int alloc_slots(hx3d_engine *eng, int ncases)
+{
+    return dalloc(eng, &eng->dSlots, (size_t)ncases * hxk::DT_FAN * hxk::DT_LINE);
+}
+void init_slots(hx3d_engine *eng, int ncases)
+{
+    const long n = (long)ncases * hxk::DT_FAN * hxk::DT_LINE;
+    hipLaunchKernelGGL(k_fill, dim3((n + 255) / 256), dim3(256), 0, eng->stream, reinterpret_cast<double *>(eng->dSlots), n,
+                       (double)INFINITY);
+}
+
 // The stage kernels address every array plane through a 32-bit byte offset (hxk::ldg), and the
 // neighbour table stores 2 * node + side in an int: each plane must hold fewer than 2^29
 // elements.
@@ -547,10 +571,12 @@ inline bool offsets_fit(long S, long ES, long FS)
     return S < lim && ES < lim && FS < lim;
 }
 
-#ifndef HX3D_EPB4
-#define HX3D_EPB4 2
-#endif
-constexpr int epb_for(int N) { return N == 1 ? 16 : N == 2 ? 8 : N == 3 ? 4 : N == 4 ? HX3D_EPB4 : 1; }
+// Elements per block of the Gauss-Lobatto kernels.  Up to N = 3 as many as fill one wave (64, 54 and
+// 64 of its lanes): its barriers are free, small meshes make more blocks, and large ones measure the
+// same (4^3 x N=3: 14.0 us a stage against 16.5 us with four elements per block; 64 such boxes in
+// one engine 42.9 against 42.6; 15^3 x N=2 23.1 against 23.4 with eight).  N = 4: two elements, 250
+// of 256 lanes (one element, 125 of 128, measured 1% slower).  Larger elements: one.
+constexpr int epb_for(int N) { return N == 1 ? 8 : N == 2 ? 2 : N == 4 ? 2 : 1; }
 
 // blocks of the uniform-order element kernels (a multiple of 8, see xcd_block): EPB elements per
 // block, or the block table of several cases
@@ -583,27 +609,13 @@ void refresh_traces(hx3d_engine *eng)
 }
 
 template <int N>
-void launch_grad(hx3d_engine *eng, const hxk::DtLimits &dtl)
+void launch_grad(hx3d_engine *eng, const hxk::DtLimits &dtl, double *curl)
 {
     constexpr int EPB = epb_for(N), ne = (N + 1) * (N + 1) * (N + 1);
     constexpr int TPB = ((EPB * ne + 63) / 64) * 64;
     hipLaunchKernelGGL((hxk::k_grad<N, EPB>), dim3(elem_grid(eng, EPB)), dim3(TPB), 0, eng->stream, eng->dQ, eng->dJa,
-                       eng->dJ, eng->dNbr, eng->dEgeo, eng->dVgrad, eng->K, eng->S, eng->ES,
-                       eng->ops, eng->ph, dtl, eng->mc);
-}
-
-template <int N>
-void launch_face(hx3d_engine *eng, const hxk::DtReduce &dtr)
-{
-    const int nb = grid_for((int)((eng->FS + hxk::FACE_TPB - 1) / hxk::FACE_TPB));
-    auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(nb), dim3(hxk::FACE_TPB), 0, eng->stream, eng->dQ, eng->dVgrad, eng->dFgeo,
-                           eng->dFnode, eng->dFdelta, eng->dFe, eng->FS, eng->S, eng->ES, 1.0 / eng->ops.w[0],
-                           eng->ph, dtr, eng->mc);
-    };
-    if (eng->ph.riemann != 1) go(hxk::k_face<N, false, false>);   // Roe: no tangents
-    else if (eng->t2x) go(hxk::k_face<N, true, true>);
-    else go(hxk::k_face<N, false, true>);
+                       eng->dJ, eng->dNbr, eng->dEgeo, eng->dVisc, curl, eng->K, eng->S, eng->ES, eng->ops, eng->ph, dtl,
+                       eng->mc);
 }
 
 template <int N, int FORM, int EPB>
@@ -611,9 +623,17 @@ void launch_volume_e(hx3d_engine *eng, double a_k, double c_k, int update, const
 {
     constexpr int ne = (N + 1) * (N + 1) * (N + 1);
     constexpr int TPB = ((EPB * ne + 63) / 64) * 64;
-    hipLaunchKernelGGL((hxk::k_volume<N, EPB, FORM>), dim3(elem_grid(eng, EPB)), dim3(TPB), 0, eng->stream, eng->dQ,
-                       eng->dVgrad, eng->dJa, eng->dJ, eng->dEdelta, eng->dFe, eng->dG,
-                       qdot, a_k, c_k, update, dta, eng->K, eng->S, eng->ES, eng->ops, eng->ph, eng->mc);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(elem_grid(eng, EPB)), dim3(TPB), 0, eng->stream, eng->dQ, eng->dQn, eng->dVisc,
+                           eng->dEdelta, eng->dEfdelta, eng->dNbx, eng->dEgeo, eng->t2x ? 1 : 0, eng->dJa, eng->dJ, eng->dG, qdot, a_k, c_k,
+                           update, dta, eng->K, eng->S, eng->ES, eng->ops, eng->ph, eng->mc);
+    };
+    const bool lxf = eng->ph.riemann == HX3D_RIEMANN_LXF, les = eng->ph.les != 0;
+    if (lxf && les) go(hxk::k_volume<N, EPB, FORM, true, true>);
+    else if (lxf) go(hxk::k_volume<N, EPB, FORM, true, false>);
+    else if (les) go(hxk::k_volume<N, EPB, FORM, false, true>);
+    else go(hxk::k_volume<N, EPB, FORM, false, false>);
+    if (update) std::swap(eng->dQ, eng->dQn);
 }
 
 template <int N, int FORM>
@@ -635,7 +655,10 @@ void launch_volume(hx3d_engine *eng, double a_k, double c_k, int update, const D
     }
 }
 
-// One stage on the engine stream.  ev: NULL, or 4 events recorded around the three launches
+// Whether the stage kernels are k_grad and k_volume (one order, Gauss-Lobatto nodes)
+bool two_launch(const hx3d_engine *eng) { return !eng->mixed && !eng->gauss; }
+
+// One stage on the engine stream.  ev: NULL, or 4 events recorded around the launches
 // (timing only); like a failed launch, a failed record surfaces through hipGetLastError, which
 // the calling entry point checks after its launches.
 template <int N>
@@ -663,10 +686,11 @@ void stage_n(hx3d_engine *eng, double a_k, double c_k, int update, const DtArgs 
         return;
     }
     if (ev) (void)hipEventRecord(ev[0], eng->stream);
-    if (!eng->ph.euler) launch_grad<N>(eng, dta.lim);
-    if (ev) (void)hipEventRecord(ev[1], eng->stream);
-    launch_face<N>(eng, dta.red);
-    if (ev) (void)hipEventRecord(ev[2], eng->stream);
+    if (!eng->ph.euler) launch_grad<N>(eng, dta.lim, qdot ? eng->dCurl : nullptr);
+    if (ev) {   // no face kernel of its own
+        (void)hipEventRecord(ev[1], eng->stream);
+        (void)hipEventRecord(ev[2], eng->stream);
+    }
     launch_volume<N>(eng, a_k, c_k, update, dta, qdot);
     if (ev) (void)hipEventRecord(ev[3], eng->stream);
 }
@@ -799,7 +823,7 @@ void launch_maxdt_bits(hx3d_engine *eng, double cfl, double dcfl, unsigned long 
                            eng->dN3, eng->dOpsAll, eng->nodes, eng->S, cfl, dcfl, eng->ph, eng->dDtPart);
     else
         hipLaunchKernelGGL(k_maxdt, dim3(nb), dim3(256), 0, eng->stream, eng->dQ, eng->dJa, eng->dJ, eng->nodes,
-                           eng->S, eng->dcsi, cfl, dcfl, eng->ph, eng->dDtPart);
+                           eng->S, eng->dcsi, cfl, dcfl, eng->ph, eng->dDtPart, (unsigned long long *)nullptr);
     hipLaunchKernelGGL(k_dt_reduce, dim3(1), dim3(1024), 0, eng->stream, eng->dDtPart, (int)nb, bits);
 }
 
@@ -843,6 +867,7 @@ void set_physics(hx3d_engine *eng, const hx3d_case_desc *d)
     ph.les_c = d->les_c;
     ph.riemann = d->riemann;
     ph.cp = ph.gamma * (1.0 / (1.4 - 1.0));
+    ph.g_gm1 = ph.gamma / (ph.gamma - 1.0);
     ph.averaging = d->averaging;
     ph.les = d->euler ? 0 : d->les;
     eng->inviscid = d->inviscid;
@@ -1023,20 +1048,13 @@ int set_tiles(hx3d_engine *eng, int policy)
     return HX3D_OK;
 }
 
-// Whether the stored second face tangent is n x t1 with vCross's arithmetic
-// (MappedGeometry.f90:745, :807-817) at every face node, bit for bit (fgeo[c*FS + q]: n at c = 0..2,
-// t1 at 3..5, t2 at 6..8).  The reference's geometry and the mesh front end's are; a descriptor
-// with other tangents keeps them, read by the face kernel.
-bool tangent2_is_cross(const std::vector<double> &fgeo, long FS)
+// Whether a face node's second tangent t2 is n x t1 with vCross's arithmetic (MappedGeometry.f90:745,
+// :807-817), bit for bit.  The reference's geometry and the mesh front end's are at every face node;
+// a descriptor with other tangents keeps them, read by the volume kernel.
+bool tangent2_is_cross(const double n[3], const double u[3], const double t2[3])
 {
-    for (long q = 0; q < FS; ++q) {
-        const double *n0 = &fgeo[q], *t = &fgeo[3 * FS + q], *t2 = &fgeo[6 * FS + q];
-        const double n[3] = {n0[0], n0[FS], n0[2 * FS]}, u[3] = {t[0], t[FS], t[2 * FS]};
-        const double x[3] = {n[1] * u[2] - u[1] * n[2], n[2] * u[0] - u[2] * n[0], n[0] * u[1] - u[0] * n[1]};
-        for (int c = 0; c < 3; ++c)
-            if (std::memcmp(&x[c], &t2[c * FS], sizeof(double)) != 0) return false;
-    }
-    return true;
+    const double x[3] = {n[1] * u[2] - u[1] * n[2], n[2] * u[0] - u[2] * n[0], n[0] * u[1] - u[0] * n[1]};
+    return std::memcmp(x, t2, sizeof(x)) == 0;
 }
 
 // The waves of the mortar face kernels (hxm::face_lane): a face of more than 32 nodes alone, a
@@ -1376,20 +1394,17 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
     }
     for (size_t x = 0; x < nbr.size(); ++x)
         if (nbr[x] < 0) return bail(eng->fail(HX3D_EINVAL, "an element face node has no neighbour"));
-    // Gauss nodes: 2 * (the neighbour's matching element face node) + (1 on the face's right side)
-    std::vector<int> nbx;
-    if (eng->gauss) {
-        nbx.assign(nbr.size(), 0);
-        for (long q = 0; q < FS; ++q) {
-            nbx[fnode[q].z] = 2 * fnode[q].w;
-            nbx[fnode[q].w] = 2 * fnode[q].z + 1;
-        }
+    // 2 * (the neighbour's matching element face node) + (1 on the face's right side)
+    std::vector<int> nbx(nbr.size(), 0);
+    for (long q = 0; q < FS; ++q) {
+        nbx[fnode[q].z] = 2 * fnode[q].w;
+        nbx[fnode[q].w] = 2 * fnode[q].z + 1;
     }
     if (!offsets_fit(S, ES, FS))
         return bail(eng->fail(HX3D_EUNSUPPORTED, "mesh too large: more than 2^29 - 1 nodes (or face nodes) per array"));
     // geometry SoA, J, 1/J, quadrature weights, LES filter widths, face frames
     std::vector<double> ja((size_t)9 * S, 0.0), jj((size_t)S, 1.0), wq((size_t)S, 0.0),
-        edelta(K), fdelta(F), fgeo((size_t)10 * FS, 0.0), egeo((size_t)4 * ES, 0.0);
+        edelta(K), fdelta(F), fgeo, egeo, efdelta((size_t)6 * K);
     double xg[8], wg[8];
     hxs::nodes_of(eng->gauss, N, xg, wg);
     for (long g = 0; g < nodes; ++g) {
@@ -1407,6 +1422,13 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
     // dS = +-Ja^d of the left element at the face node, |Ja| = |dS|, n = dS/|Ja|
     // (ConstructMappedGeometryFace, MappedGeometry.f90:482-760) and a fixed orthonormal
     // completion t1, t2 of n (the Riemann fluxes do not depend on the tangent choice).
+    // Stored in element-face order, the left element's frame on both sides: n and |Ja|, for the
+    // volume kernel with Lax-Friedrichs t1, and t2 unless it is formed as n x t1 (tangent2_is_cross);
+    // Gauss nodes also per face node.
+    const bool lxf = d->riemann == HX3D_RIEMANN_LXF && !eng->gauss;
+    eng->t2x = lxf;
+    egeo.resize((size_t)(lxf ? 10 : 4) * ES, 0.0);
+    if (eng->gauss) fgeo.resize((size_t)10 * FS);
     const bool have_fg = d->fNormal && d->fT1 && d->fT2 && d->fJac;
     if (!have_fg && (d->fNormal || d->fT1 || d->fT2 || d->fJac))
         return bail(eng->fail(HX3D_EINVAL, "descriptor: give all four face geometry arrays or none"));
@@ -1437,51 +1459,56 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
                     t2[1] = nr[2] * t1[0] - nr[0] * t1[2];
                     t2[2] = nr[0] * t1[1] - nr[1] * t1[0];
                 }
-                for (int c = 0; c < 3; ++c) {
-                    fgeo[(size_t)c * FS + q] = nr[c];
-                    fgeo[(size_t)(3 + c) * FS + q] = t1[c];
-                    fgeo[(size_t)(6 + c) * FS + q] = t2[c];
+                const double frame[10] = {nr[0], nr[1], nr[2], jac, t1[0], t1[1], t1[2], t2[0], t2[1], t2[2]};
+                for (int c = 0; c < (lxf ? 10 : 4); ++c)
+                    egeo[(size_t)c * ES + fnode[q].z] = egeo[(size_t)c * ES + fnode[q].w] = frame[c];
+                if (lxf && eng->t2x) eng->t2x = tangent2_is_cross(nr, t1, t2);
+                if (eng->gauss) {
+                    for (int c = 0; c < 3; ++c) {
+                        fgeo[(size_t)c * FS + q] = nr[c];
+                        fgeo[(size_t)(3 + c) * FS + q] = t1[c];
+                        fgeo[(size_t)(6 + c) * FS + q] = t2[c];
+                    }
+                    fgeo[(size_t)9 * FS + q] = jac;
                 }
-                fgeo[(size_t)9 * FS + q] = jac;
-                for (int c = 0; c < 3; ++c) {
-                    egeo[(size_t)c * ES + fnode[q].z] = nr[c];
-                    egeo[(size_t)c * ES + fnode[q].w] = nr[c];
-                }
-                egeo[(size_t)3 * ES + fnode[q].z] = jac;
-                egeo[(size_t)3 * ES + fnode[q].w] = jac;
                 surf += wg[i] * wg[j] * jac;
             }
         fdelta[f] = std::sqrt(surf / nf);   // SD.f90:1378
     }
-    eng->t2x = tangent2_is_cross(fgeo, FS);
+    if (eng->t2x) egeo.resize((size_t)7 * ES);
+    for (long x = 0; x < 6L * K; ++x) efdelta[x] = fdelta[d->faceID[x]];
     // ---- device -------------------------------------------------------------------
     int rc;
     if ((rc = dalloc(eng, &eng->dQ, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dG, (size_t)NV * S)) ||
-        (rc = dalloc(eng, &eng->dVgrad, (size_t)(eng->ph.les ? 13 : 12) * S)) || (rc = dalloc(eng, &eng->dJa, (size_t)9 * S)) ||
-        (rc = dalloc(eng, &eng->dWq, (size_t)S)) ||
-        (rc = dalloc(eng, &eng->dJ, (size_t)S)) || (rc = dalloc(eng, &eng->dFgeo, (size_t)10 * FS)) ||
-        (rc = dalloc(eng, &eng->dFe, (size_t)NV * ES)) || (rc = dalloc(eng, &eng->dEgeo, (size_t)4 * ES)) || (rc = dalloc(eng, &eng->dQDot, (size_t)NV * S)) ||
-        (rc = dalloc(eng, &eng->dEdelta, (size_t)K)) || (rc = dalloc(eng, &eng->dFdelta, (size_t)F)) ||
+        (rc = dalloc(eng, &eng->dJa, (size_t)9 * S)) || (rc = dalloc(eng, &eng->dWq, (size_t)S)) ||
+        (rc = dalloc(eng, &eng->dJ, (size_t)S)) || (rc = dalloc(eng, &eng->dEgeo, egeo.size())) ||
+        (rc = dalloc(eng, &eng->dQDot, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dEdelta, (size_t)K)) ||
         (rc = dalloc(eng, &eng->dScal, 4)) || (rc = dalloc(eng, &eng->dPart, (size_t)NV * ((S + 255) / 256 + 1))) ||
         (rc = dalloc(eng, &eng->dDtPart, (size_t)2 * (std::max((long)K, (S + 255) / 256) + 64))) ||
         (rc = dalloc(eng, &eng->dStage, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dBits, 2 * DT_SLOTS)) ||
-        (rc = dalloc(eng, &eng->dNbr, nbr.size())) ||
-        (rc = dalloc(eng, &eng->dFlag, 2)) || (rc = dalloc(eng, &eng->dFnode, fnode.size())))
+        (rc = dalloc(eng, &eng->dFlag, 2)) || (rc = dalloc(eng, &eng->dNbx, nbx.size())))
         return bail(rc);
-    if (eng->gauss && ((rc = dalloc(eng, &eng->dQtr, (size_t)NV * ES)) || (rc = dalloc(eng, &eng->dGtr, (size_t)15 * ES)) ||
-                       (rc = dalloc(eng, &eng->dNbx, nbx.size()))))
+    if (eng->gauss) {
+        if ((rc = dalloc(eng, &eng->dVgrad, (size_t)(eng->ph.les ? 13 : 12) * S)) ||
+            (rc = dalloc(eng, &eng->dFe, (size_t)NV * ES)) || (rc = dalloc(eng, &eng->dFgeo, (size_t)10 * FS)) ||
+            (rc = dalloc(eng, &eng->dFdelta, (size_t)F)) || (rc = dalloc(eng, &eng->dFnode, fnode.size())) ||
+            (rc = dalloc(eng, &eng->dQtr, (size_t)NV * ES)) || (rc = dalloc(eng, &eng->dGtr, (size_t)15 * ES)))
+            return bail(rc);
+    } else if ((rc = dalloc(eng, &eng->dQn, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dVisc, (size_t)hxk::viscous_values(eng->ph.les) * S)) ||
+               (rc = dalloc(eng, &eng->dCurl, (size_t)S)) || (rc = dalloc(eng, &eng->dEfdelta, efdelta.size())) ||
+               (rc = dalloc(eng, &eng->dNbr, nbr.size())) || (rc = alloc_slots(eng, 1)))
         return bail(rc);
     if (hipStreamCreateWithFlags(&eng->stream, hipStreamNonBlocking) != hipSuccess)
         return bail(eng->fail(HX3D_EDEVICE, "hipStreamCreate failed"));
     auto up = [&](void *dst, const void *src, size_t bytes) {
         return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) == hipSuccess;
     };
-    if (!up(eng->dJa, ja.data(), ja.size() * 8) ||
-        !up(eng->dJ, jj.data(), jj.size() * 8) || !up(eng->dFgeo, fgeo.data(), fgeo.size() * 8) ||
+    if (!up(eng->dJa, ja.data(), ja.size() * 8) || !up(eng->dJ, jj.data(), jj.size() * 8) ||
         !up(eng->dWq, wq.data(), wq.size() * 8) || !up(eng->dEdelta, edelta.data(), edelta.size() * 8) ||
-        !up(eng->dFdelta, fdelta.data(), fdelta.size() * 8) || !up(eng->dNbr, nbr.data(), nbr.size() * 4) ||
-        !up(eng->dEgeo, egeo.data(), egeo.size() * 8) || !up(eng->dFnode, fnode.data(), fnode.size() * 16) ||
-        (eng->gauss && !up(eng->dNbx, nbx.data(), nbx.size() * 4)))
+        !up(eng->dEgeo, egeo.data(), egeo.size() * 8) || !up(eng->dNbx, nbx.data(), nbx.size() * 4) ||
+        (eng->gauss && (!up(eng->dFgeo, fgeo.data(), fgeo.size() * 8) || !up(eng->dFdelta, fdelta.data(), fdelta.size() * 8) ||
+                        !up(eng->dFnode, fnode.data(), fnode.size() * 16))) ||
+        (!eng->gauss && (!up(eng->dNbr, nbr.data(), nbr.size() * 4) || !up(eng->dEfdelta, efdelta.data(), efdelta.size() * 8))))
         return bail(eng->fail(HX3D_EDEVICE, "upload failed"));
     // zero state, RK register and time
     const long nb = (NV * S + 255) / 256;
@@ -1491,6 +1518,9 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
     if (eng->gauss) {
         hipLaunchKernelGGL(k_fill, dim3((15 * ES + 255) / 256), dim3(256), 0, eng->stream, eng->dGtr, 15L * ES, 0.0);
         refresh_traces(eng);
+    } else {
+        hipLaunchKernelGGL(k_fill, dim3(nb), dim3(256), 0, eng->stream, eng->dQn, (long)NV * S, 0.0);
+        init_slots(eng, 1);
     }
     if (int rc2 = init_flags(eng)) return bail(rc2);
     if (hipStreamSynchronize(eng->stream) != hipSuccess)
@@ -1540,7 +1570,7 @@ int hx3d_engine_create_multi(const hx3d_case_desc *descs, int ncases, hx3d_engin
     }
     if (K >= (1L << 31) / 8) return reject(HX3D_EUNSUPPORTED, "too many elements");
     const int n1 = d0.N[0] + 1, nf = n1 * n1;
-    std::vector<int> N(3 * K), faceID(6 * K), faceSide(6 * K), fElem(2 * F), fESide(2 * F), fRot(F), fcase(F);
+    std::vector<int> N(3 * K), faceID(6 * K), faceSide(6 * K), fElem(2 * F), fESide(2 * F), fRot(F);
     std::vector<double> Ja(9 * nodes), J(nodes), fN, fT1, fT2, fJ;
     if (fg) { fN.resize(3 * fnodes); fT1.resize(3 * fnodes); fT2.resize(3 * fnodes); fJ.resize(fnodes); }
     long k0 = 0, f0 = 0, g0 = 0, q0 = 0;
@@ -1549,7 +1579,7 @@ int hx3d_engine_create_multi(const hx3d_case_desc *descs, int ncases, hx3d_engin
         for (long x = 0; x < 3 * Kc[c]; ++x) N[3 * k0 + x] = d.N[x];
         for (long x = 0; x < 6 * Kc[c]; ++x) { faceID[6 * k0 + x] = d.faceID[x] + (int)f0; faceSide[6 * k0 + x] = d.faceSide[x]; }
         for (long x = 0; x < 2 * Fc[c]; ++x) { fElem[2 * f0 + x] = d.fElem[x] + (int)k0; fESide[2 * f0 + x] = d.fESide[x]; }
-        for (long x = 0; x < Fc[c]; ++x) { fRot[f0 + x] = d.fRot[x]; fcase[f0 + x] = c; }
+        for (long x = 0; x < Fc[c]; ++x) fRot[f0 + x] = d.fRot[x];
         std::memcpy(&Ja[9 * g0], d.Ja, sizeof(double) * 9 * nc[c]);
         std::memcpy(&J[g0], d.J, sizeof(double) * nc[c]);
         if (fg) {
@@ -1575,15 +1605,12 @@ int hx3d_engine_create_multi(const hx3d_case_desc *descs, int ncases, hx3d_engin
     // block table: EPB elements per block within each case
     const int epb = epb_for(eng->N);
     std::vector<int4> blocks;
-    std::vector<int> pfirst(ncases + 1, 0);
     k0 = 0;
     for (int c = 0; c < ncases; ++c) {
-        pfirst[c] = (int)blocks.size();
         for (long e = 0; e < Kc[c]; e += epb)
             blocks.push_back(make_int4((int)(k0 + e), (int)std::min<long>(epb, Kc[c] - e), c, e == 0 ? 1 : 0));
         k0 += Kc[c];
     }
-    pfirst[ncases] = (int)blocks.size();
     eng->nblocks_multi = (int)blocks.size();
     while ((long)blocks.size() < grid_for(eng->nblocks_multi)) blocks.push_back(make_int4(0, 0, 0, 0));
     std::vector<hxk::CaseConst> cc(ncases);
@@ -1596,30 +1623,32 @@ int hx3d_engine_create_multi(const hx3d_case_desc *descs, int ncases, hx3d_engin
         cc[c].les_c = d.les_c;
     }
     if ((long)eng->F * nf / hxk::FACE_TPB + 1 < ncases)
-        return eng->fail(HX3D_EUNSUPPORTED, "more cases than face blocks to reduce their dt");
+        return eng->fail(HX3D_EUNSUPPORTED, "too many cases of too few face nodes");
     // per-case replacements of the one-case dt slots, flags and time
     (void)hipStreamSynchronize(eng->stream);
     (void)hipFree(eng->dBits);
     (void)hipFree(eng->dFlag);
+    (void)hipFree(eng->dSlots);
+    eng->dSlots = nullptr;
     (void)hipHostFree(eng->hFlag);
     eng->dBits = nullptr; eng->dFlag = nullptr; eng->hFlag = nullptr;
     eng->ncases = ncases;
     const std::vector<int> ones(ncases, 1);
     if ((rc = dalloc(eng, &eng->dBits, (size_t)2 * DT_SLOTS * ncases)) || (rc = dalloc(eng, &eng->dFlag, (size_t)1 + ncases)) ||
         (rc = dalloc(eng, &eng->dBlocks, blocks.size())) || (rc = dalloc(eng, &eng->dCC, cc.size())) ||
-        (rc = dalloc(eng, &eng->dActive, (size_t)ncases)) || (rc = dalloc(eng, &eng->dFcase, fcase.size())) ||
-        (rc = dalloc(eng, &eng->dPfirst, pfirst.size())) || (rc = dalloc(eng, &eng->dTimeM, (size_t)ncases)))
+        (rc = dalloc(eng, &eng->dActive, (size_t)ncases)) || (rc = dalloc(eng, &eng->dTimeM, (size_t)ncases)) ||
+        (rc = alloc_slots(eng, ncases)))
         return rc;
     auto up = [&](void *dst, const void *src, size_t bytes) {
         return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) == hipSuccess;
     };
     if (!up(eng->dBlocks, blocks.data(), blocks.size() * sizeof(int4)) || !up(eng->dCC, cc.data(), cc.size() * sizeof(hxk::CaseConst)) ||
-        !up(eng->dActive, ones.data(), ones.size() * 4) || !up(eng->dFcase, fcase.data(), fcase.size() * 4) ||
-        !up(eng->dPfirst, pfirst.data(), pfirst.size() * 4))
+        !up(eng->dActive, ones.data(), ones.size() * 4))
         return eng->fail(HX3D_EDEVICE, "upload failed");
     hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, eng->stream, eng->dTimeM, (long)ncases, 0.0);
     eng->dTime = eng->dTimeM;
-    eng->mc = hxk::Multi{eng->dBlocks, eng->dCC, eng->dActive, eng->dFcase, eng->dPfirst, ncases};
+    eng->mc = hxk::Multi{eng->dBlocks, eng->dCC, eng->dActive, ncases};
+    init_slots(eng, ncases);
     if ((rc = init_flags(eng))) return rc;
     if (hipStreamSynchronize(eng->stream) != hipSuccess) return eng->fail(HX3D_EDEVICE, "initialisation failed");
     return HX3D_OK;
@@ -1651,8 +1680,8 @@ int hx3d_engine_destroy(hx3d_engine *eng)
                     eng->dQDot, eng->dEdelta, eng->dFdelta, eng->dWq, eng->dScal, eng->dPart, eng->dStage,
                     eng->dBits, eng->dNbr, eng->dFlag, eng->dFnode, eng->dN3, eng->dEfoff,
                     eng->dEofn, eng->dOff, eng->dFaces, eng->dSched, eng->dOpsAll, eng->dU, eng->dLift, eng->dDtPart, eng->dTmap,
-                    eng->dBlocks, eng->dCC, eng->dActive, eng->dFcase, eng->dPfirst, eng->dTimeM,
-                    eng->dQtr, eng->dGtr, eng->dNbx};
+                    eng->dBlocks, eng->dCC, eng->dActive, eng->dTimeM,
+                    eng->dQtr, eng->dGtr, eng->dNbx, eng->dQn, eng->dVisc, eng->dCurl, eng->dEfdelta, eng->dSlots};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     for (auto &e : eng->evpool) (void)hipEventDestroy(e);
@@ -1851,9 +1880,10 @@ int hx3d_advance(hx3d_engine *eng, int nsteps, double cfl, double dcfl, double *
     }
     // dt of step s (slot 0): MaxTimeStep of the state the step starts from.  The first stage's
     // gradient kernel leaves block minima of the limits (an Euler case has no gradient kernel:
-    // a standalone pass writes them), which block 0 of the first stage's face kernel reduces into
-    // the slot before any volume kernel of the step reads dt.  Every step issues the same
-    // launches with the same arguments: ev, when given, holds 12 events for the step.
+    // a standalone pass writes them), which block 0 of the first stage's face kernel (Gauss-Lobatto
+    // nodes of one order: every block of its volume kernel) reduces before the step's volume
+    // kernels use dt.  Every step issues the same launches, with the same arguments up to the two
+    // copies of the state: ev, when given, holds 12 events for the step.
     auto issue_step = [eng, cfl, dcfl](hipEvent_t *ev, double *qdot) {
         unsigned long long *slot = dt_slot(eng, 0);
         int nparts;
@@ -1865,7 +1895,8 @@ int hx3d_advance(hx3d_engine *eng, int nsteps, double cfl, double dcfl, double *
                                    eng->dDtPart);
             else
                 hipLaunchKernelGGL(k_maxdt, dim3(nb), dim3(256), 0, eng->stream, eng->dQ, eng->dJa, eng->dJ,
-                                   eng->nodes, eng->S, eng->dcsi, cfl, dcfl, eng->ph, eng->dDtPart);
+                                   eng->nodes, eng->S, eng->dcsi, cfl, dcfl, eng->ph, eng->dDtPart,
+                                   two_launch(eng) ? eng->dSlots : nullptr);
             nparts = (int)nb;
         } else {
             nparts = eng->mixed ? eng->grid_mgrad_s + eng->grid_mgrad_b : grad_grid(eng);
@@ -1873,8 +1904,15 @@ int hx3d_advance(hx3d_engine *eng, int nsteps, double cfl, double dcfl, double *
         for (int k = 0; k < 3; ++k) {
             DtArgs a{};
             a.in = slot;
-            if (k == 0) {
-                if (!eng->ph.euler) a.lim = hxk::DtLimits{eng->dDtPart, cfl, dcfl, eng->dcsi};
+            if (two_launch(eng)) {   // dt through the slots: filled before, read by, emptied after stage 0
+                if (k == 0) {
+                    if (!eng->ph.euler) a.lim = hxk::DtLimits{nullptr, cfl, dcfl, eng->dcsi, eng->dSlots};
+                    a.slots = eng->dSlots;
+                    a.fin = slot;
+                }
+                if (k == 1) a.empty = eng->dSlots;
+            } else if (k == 0) {
+                if (!eng->ph.euler) a.lim = hxk::DtLimits{eng->dDtPart, cfl, dcfl, eng->dcsi, nullptr};
                 a.red = hxk::DtReduce{eng->dDtPart, nparts, slot};
             }
             if (k == 2) a.time = eng->dTime;
@@ -1886,7 +1924,10 @@ int hx3d_advance(hx3d_engine *eng, int nsteps, double cfl, double dcfl, double *
         for (int s = 0; s < nsteps; ++s)
             issue_step(eng->timing ? &eng->evpool[(size_t)12 * s] : nullptr, s == nsteps - 1 ? eng->dQDot : nullptr);
     } else if (nsteps > 0) {
-        // capture the step once per (cfl, dcfl); the graph holds kernel launches only
+        // Capture the step once per (cfl, dcfl); the graph holds kernel launches only.  With two
+        // copies of the state (two_launch) a step of three stages ends in the other copy: the graph
+        // holds two steps then, from the copy graph_Q.
+        const int per = two_launch(eng) ? 2 : 1;
         if (!eng->step_graph || eng->graph_cfl != cfl || eng->graph_dcfl != dcfl) {
             if (eng->step_graph) {
                 HIPCHK(hipGraphExecDestroy(eng->step_graph));
@@ -1895,7 +1936,8 @@ int hx3d_advance(hx3d_engine *eng, int nsteps, double cfl, double dcfl, double *
             hipGraph_t g = nullptr;
             HIPCHK(hipStreamBeginCapture(eng->stream, hipStreamCaptureModeThreadLocal));
             eng->capturing = true;
-            issue_step(nullptr, nullptr);
+            eng->graph_Q = eng->dQ;
+            for (int s = 0; s < per; ++s) issue_step(nullptr, nullptr);
             eng->capturing = false;
             const hipError_t ce = hipStreamEndCapture(eng->stream, &g);
             if (ce != hipSuccess || !g) return eng->fail(HX3D_EDEVICE, std::string("step capture: ") + hipGetErrorString(ce));
@@ -1908,8 +1950,15 @@ int hx3d_advance(hx3d_engine *eng, int nsteps, double cfl, double dcfl, double *
             eng->graph_cfl = cfl;
             eng->graph_dcfl = dcfl;
         }
-        // the last step is issued directly: it also leaves its last stage's time derivative
-        for (int s = 0; s + 1 < nsteps; ++s) HIPCHK(hipGraphLaunch(eng->step_graph, eng->stream));
+        // the last step is issued directly: it also leaves its last stage's time derivative; before
+        // it the replays, from the copy of the state they start from, and what is left over
+        int left = nsteps - 1;
+        if (left >= 1 + per && eng->dQ != eng->graph_Q) {
+            issue_step(nullptr, nullptr);
+            --left;
+        }
+        for (; left >= per && eng->dQ == eng->graph_Q; left -= per) HIPCHK(hipGraphLaunch(eng->step_graph, eng->stream));
+        for (; left > 0; --left) issue_step(nullptr, nullptr);
         issue_step(nullptr, eng->dQDot);
     }
     HIPCHK(hipGetLastError());
@@ -2001,7 +2050,7 @@ int hx3d_volume_monitor(hx3d_engine *eng, int kind, double *value)
     }
     const int nb = (int)((eng->nodes + 255) / 256);
     hipLaunchKernelGGL(k_monitor, dim3(nb), dim3(256), 0, eng->stream, kind, eng->dQ, eng->dQDot,
-                       eng->mixed ? nullptr : eng->dVgrad, eng->dU, eng->dJ, eng->dWq, eng->nodes, eng->S, eng->ph,
+                       two_launch(eng) ? eng->dCurl : nullptr, eng->mixed ? nullptr : eng->dVgrad, eng->dU, eng->dJ, eng->dWq, eng->nodes, eng->S, eng->ph,
                        eng->dPart);
     hipLaunchKernelGGL(k_finish_sum2, dim3(1), dim3(64), 0, eng->stream, eng->dPart, nb, eng->dStage);
     double r[2];

@@ -15,15 +15,26 @@ constexpr int NV = 5;
 
 struct Phys {
     double gamma, gm1, gammaM2, mu, mu_to_kappa, S_div_T, Trenorm, lambda_stab, les_c, cp;
+    double g_gm1;   // gamma / (gamma - 1)
     int riemann, averaging, les, euler;
 };
 
+// a / b with y = 1 / b in hand, the bits of the division: q = a y, the exact remainder a - b q by a
+// fused multiply-add, and one correction (Markstein, IBM J. Res. Dev. 34(1), 1990).  Three
+// instructions instead of the division's eleven, for the many quotients by one density.
+HX_HD double quot(double a, double b, double y)
+{
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+
 // navierstokes/VariableConversion_NS.f90:64 Pressure, :99-112 Temperature,
 // :146-186 get_laminar_mu_kappa + SutherlandsLaw
-HX_HD double pressure(const Phys &ph, const double q[NV])
+HX_HD double pressure(const Phys &ph, const double q[NV], double ir)   // ir = 1 / rho
 {
-    return ph.gm1 * (q[4] - 0.5 * (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]) / q[0]);
+    return ph.gm1 * (q[4] - quot(0.5 * (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]), q[0], ir));
 }
+HX_HD double pressure(const Phys &ph, const double q[NV]) { return pressure(ph, q, 1.0 / q[0]); }
 
 HX_HD double sutherland(const Phys &ph, double T)
 {
@@ -33,7 +44,8 @@ HX_HD double sutherland(const Phys &ph, double T)
 
 HX_HD void laminar_mu_kappa(const Phys &ph, const double q[NV], double &mu, double &kappa)
 {
-    const double T = ph.gammaM2 * pressure(ph, q) / q[0];
+    const double ir = 1.0 / q[0];
+    const double T = quot(ph.gammaM2 * pressure(ph, q, ir), q[0], ir);
     mu = ph.mu * sutherland(ph, T);
     kappa = mu * ph.mu_to_kappa;
 }
@@ -45,9 +57,10 @@ HX_HD void laminar_mu_kappa(const Phys &ph, const double q[NV], double &mu, doub
 HX_HD void dt_limits(const Phys &ph, const double q[NV], const double ja[9], double jg, double dc, double de,
                      double dz, double cfl, double dcfl, double &tc, double &tv)
 {
-    const double u = fabs(q[1] / q[0]), v = fabs(q[2] / q[0]), w = fabs(q[3] / q[0]);
-    const double p = pressure(ph, q);
-    const double a = sqrt(ph.gamma * p / q[0]);
+    const double ir = 1.0 / q[0];
+    const double u = fabs(quot(q[1], q[0], ir)), v = fabs(quot(q[2], q[0], ir)), w = fabs(quot(q[3], q[0], ir));
+    const double p = pressure(ph, q, ir);
+    const double a = sqrt(quot(ph.gamma * p, q[0], ir));
     const double e0 = u + a, e1 = v + a, e2 = w + a;
     const double lx = fabs(ja[0] * e0 + ja[1] * e1 + ja[2] * e2) * dc;
     const double ly = fabs(ja[3] * e0 + ja[4] * e1 + ja[5] * e2) * de;
@@ -55,7 +68,7 @@ HX_HD void dt_limits(const Phys &ph, const double q[NV], const double ja[9], dou
     tc = cfl * fabs(jg) / (lx + ly + lz);
     tv = INFINITY;
     if (!ph.euler) {
-        const double mu = sutherland(ph, ph.gammaM2 * p / q[0]);
+        const double mu = sutherland(ph, quot(ph.gammaM2 * p, q[0], ir));
         const double vx = mu * (dc * dc) * fabs(ja[0] + ja[1] + ja[2]);
         const double vy = mu * (de * de) * fabs(ja[3] + ja[4] + ja[5]);
         const double vz = mu * (dz * dz) * fabs(ja[6] + ja[7] + ja[8]);
@@ -68,7 +81,7 @@ HX_HD void dt_limits(const Phys &ph, const double q[NV], const double ja[9], dou
 // out[d][v] = F_x[v] Ja^d_x + F_y[v] Ja^d_y + F_z[v] Ja^d_z
 HX_HD void euler_contravariant(const Phys &ph, const double q[NV], const double ja[9], double out[3][NV])
 {
-    const double u = q[1] / q[0], v = q[2] / q[0], w = q[3] / q[0];
+    const double ir = 1.0 / q[0], u = quot(q[1], q[0], ir), v = quot(q[2], q[0], ir), w = quot(q[3], q[0], ir);
     const double p = ph.gm1 * (q[4] - 0.5 * (q[1] * u + q[2] * v + q[3] * w));
     double F[NV][3];
     F[0][0] = q[1]; F[1][0] = q[1] * u + p; F[2][0] = q[1] * v; F[3][0] = q[1] * w; F[4][0] = (q[4] + p) * u;
@@ -85,7 +98,8 @@ HX_HD void euler_contravariant(const Phys &ph, const double q[NV], const double 
 //   viscous_state   the velocity gradients u_x, u_y, u_z and grad T it forms from Q and the
 //                   lifted state gradients: vg[0..2] = u_x, vg[3..5] = u_y, vg[6..8] = u_z,
 //                   vg[9..11] = grad T;
-//   viscous_flux    the stress / heat-flux tail F[v][c] from mu, kappa, the velocity and vg.
+//   viscous_flux    the stress / heat-flux tail F[v][c] from mu, kappa, the velocity and vg, itself
+//                   the viscous_tensor of the stress_shape.
 // Together they perform the reference's operations in its order.
 HX_HD void viscous_state(const Phys &ph, const double q[NV], const double gx[NV], const double gy[NV],
                          const double gz[NV], double vg[12])
@@ -105,26 +119,48 @@ HX_HD void viscous_state(const Phys &ph, const double q[NV], const double gx[NV]
     vg[11] = g * (ir * gz[4] - q[4] * ir * ir * gz[0] - u * vg[6] - v * vg[7] - w * vg[8]);
 }
 
-HX_HD void viscous_flux(double mu, double kappa, double u, double v, double w, const double vg[12],
-                        double F[NV][3])
+// The stress without its viscosity, s = (xx, xy, xz, yy, yz, zz).
+HX_HD void stress_shape(const double vg[12], double s[6])
 {
     const double *ux = vg, *uy = vg + 3, *uz = vg + 6;
     const double divV = ux[0] + uy[1] + uz[2];
-    F[0][0] = 0.0;
-    F[1][0] = mu * (2.0 * ux[0] - 2.0 / 3.0 * divV);
-    F[2][0] = mu * (ux[1] + uy[0]);
-    F[3][0] = mu * (ux[2] + uz[0]);
-    F[4][0] = F[1][0] * u + F[2][0] * v + F[3][0] * w + kappa * vg[9];
-    F[0][1] = 0.0;
-    F[1][1] = F[2][0];
-    F[2][1] = mu * (2.0 * uy[1] - 2.0 / 3.0 * divV);
-    F[3][1] = mu * (uy[2] + uz[1]);
-    F[4][1] = F[1][1] * u + F[2][1] * v + F[3][1] * w + kappa * vg[10];
-    F[0][2] = 0.0;
-    F[1][2] = F[3][0];
-    F[2][2] = F[3][1];
-    F[3][2] = mu * (2.0 * uz[2] - 2.0 / 3.0 * divV);
-    F[4][2] = F[1][2] * u + F[2][2] * v + F[3][2] * w + kappa * vg[11];
+    s[0] = 2.0 * ux[0] - 2.0 / 3.0 * divV;
+    s[1] = ux[1] + uy[0];
+    s[2] = ux[2] + uz[0];
+    s[3] = 2.0 * uy[1] - 2.0 / 3.0 * divV;
+    s[4] = uy[2] + uz[1];
+    s[5] = 2.0 * uz[2] - 2.0 / 3.0 * divV;
+}
+
+// The nine entries of the viscous flux tensor F[v][c], v = 1..4: the symmetric stress f[0..5] =
+// (xx, xy, xz, yy, yz, zz), then the energy flux f[6..8]; gT = grad T.
+HX_HD void viscous_tensor(double mu, double kappa, double u, double v, double w, const double s[6], const double gT[3],
+                          double f[9])
+{
+#pragma unroll
+    for (int c = 0; c < 6; ++c) f[c] = mu * s[c];
+    f[6] = f[0] * u + f[1] * v + f[2] * w + kappa * gT[0];
+    f[7] = f[1] * u + f[3] * v + f[4] * w + kappa * gT[1];
+    f[8] = f[2] * u + f[4] * v + f[5] * w + kappa * gT[2];
+}
+// index of F[v][c], v = 1..4, in the nine entries
+constexpr int viscous_entry(int v, int c)
+{
+    return v == 4 ? 6 + c : v == 1 ? c : v == 2 ? (c == 0 ? 1 : 2 + c) : (c == 0 ? 2 : 3 + c);
+}
+
+HX_HD void viscous_flux(double mu, double kappa, double u, double v, double w, const double vg[12],
+                        double F[NV][3])
+{
+    double s[6], f[9];
+    stress_shape(vg, s);
+    viscous_tensor(mu, kappa, u, v, w, s, vg + 9, f);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        F[0][c] = 0.0;
+#pragma unroll
+        for (int q = 1; q < NV; ++q) F[q][c] = f[viscous_entry(q, c)];
+    }
 }
 
 // common/LESModels.f90:256-307 Smagorinsky and :358-~440 WALE eddy viscosity (no wall model),
@@ -191,7 +227,10 @@ HX_HD double les_factor(const Phys &ph, const double q[NV], const double gx[NV],
 #pragma unroll
             for (int i = 0; i < 3; ++i) normSd += Sd[i][j] * Sd[i][j];
         if (normS < 1.0e-8 && normSd < 1.0e-8) return 0.0;   // mu = 0
-        return pow(normSd, 1.5) / (pow(normS, 2.5) + pow(normSd, 1.25));
+        // normSd^1.5 / (normS^2.5 + normSd^1.25), the powers by square roots (three of about 15
+        // instructions each against three general powers of over 100)
+        const double rs = sqrt(normSd);
+        return normSd * rs / (normS * normS * sqrt(normS) + normSd * sqrt(rs));
     }
     return 0.0;
 }
@@ -204,19 +243,21 @@ HX_HD double les_mu(const Phys &ph, double delta, double rho, double X)
 
 // navierstokes/RiemannSolvers_NS.f90:1541-1656 RoeRiemannSolver: the one-sided Roe flux with
 // the entropy fix of the one wave that can change sign, the reference's operation order.
-HX_HD void roe_flux(const Phys &ph, const double L[NV], const double R[NV], const double n[3], double f[NV])
+// iL, iR: 1 / rho of the two sides
+HX_HD void roe_flux(const Phys &ph, const double L[NV], const double R[NV], double iL, double iR, const double n[3],
+                    double f[NV])
 {
     const double g = ph.gamma;
     const double rL = L[0], mxL = L[1], myL = L[2], mzL = L[3], EL = L[4];
     const double rR = R[0], mxR = R[1], myR = R[2], mzR = R[3], ER = R[4];
-    const double uL = mxL / rL, vL = myL / rL, wL = mzL / rL;
-    const double pL = (g - 1.0) * (EL - 0.5 / rL * (mxL * mxL + myL * myL + mzL * mzL));
-    const double uR = mxR / rR, vR = myR / rR, wR = mzR / rR;
-    const double pR = (g - 1.0) * (ER - 0.5 / rR * (mxR * mxR + myR * myR + mzR * mzR));
+    const double uL = quot(mxL, rL, iL), vL = quot(myL, rL, iL), wL = quot(mzL, rL, iL);
+    const double pL = (g - 1.0) * (EL - 0.5 * iL * (mxL * mxL + myL * myL + mzL * mzL));   // 0.5 / rho = 0.5 (1 / rho)
+    const double uR = quot(mxR, rR, iR), vR = quot(myR, rR, iR), wR = quot(mzR, rR, iR);
+    const double pR = (g - 1.0) * (ER - 0.5 * iR * (mxR * mxR + myR * myR + mzR * mzR));
     const double unL = n[0] * uL + n[1] * vL + n[2] * wL;
     const double unR = n[0] * uR + n[1] * vR + n[2] * wR;
-    const double HL = 0.5 * (uL * uL + vL * vL + wL * wL) + g / (g - 1.0) * pL / rL;
-    const double HR = 0.5 * (uR * uR + vR * vR + wR * wR) + g / (g - 1.0) * pR / rR;
+    const double HL = 0.5 * (uL * uL + vL * vL + wL * wL) + quot(ph.g_gm1 * pL, rL, iL);
+    const double HR = 0.5 * (uR * uR + vR * vR + wR * wR) + quot(ph.g_gm1 * pR, rR, iR);
     // Roe averages: weights sqrt(rho) of each side
     const double srr = sqrt(rL * rR);
     const double wtL = rL / (rL + srr), wtR = 1.0 - wtL;
@@ -256,6 +297,11 @@ HX_HD void roe_flux(const Phys &ph, const double L[NV], const double R[NV], cons
         f[3] = mn * wR + pR * n[2] - s4 * (wa + ca * n[2]);
         f[4] = mn * HR - s4 * (Ha + una * ca);
     }
+}
+
+HX_HD void roe_flux(const Phys &ph, const double L[NV], const double R[NV], const double n[3], double f[NV])
+{
+    roe_flux(ph, L, R, 1.0 / L[0], 1.0 / R[0], n, f);
 }
 
 // AveragedStates (RiemannSolvers_NS.f90:1784-2077) of rotated states (rho, rho u_n, rho u_t1,
@@ -309,11 +355,11 @@ HX_HD void averaged_states(const Phys &ph, const double QL[NV], const double QR[
 }
 
 // navierstokes/RiemannSolvers_NS.f90:1251-1334 LxFRiemannSolver (rotated face frame)
-HX_HD void lxf_flux(const Phys &ph, const double QL[NV], const double QR[NV], const double n[3],
+// iL, iR: 1 / rho of the two sides
+HX_HD void lxf_flux(const Phys &ph, const double QL[NV], const double QR[NV], double iL, double iR, const double n[3],
                     const double t1[3], const double t2[3], double f[NV])
 {
     const double rhoL = QL[0], rhoR = QR[0];
-    const double iL = 1.0 / rhoL, iR = 1.0 / rhoR;
     const double ruL = QL[1] * n[0] + QL[2] * n[1] + QL[3] * n[2];
     const double ruR = QR[1] * n[0] + QR[2] * n[1] + QR[3] * n[2];
     const double rvL = QL[1] * t1[0] + QL[2] * t1[1] + QL[3] * t1[2];
@@ -333,6 +379,12 @@ HX_HD void lxf_flux(const Phys &ph, const double QL[NV], const double QR[NV], co
     const double f1 = f[1], f2 = f[2], f3 = f[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) f[1 + d] = n[d] * f1 + t1[d] * f2 + t2[d] * f3;
+}
+
+HX_HD void lxf_flux(const Phys &ph, const double QL[NV], const double QR[NV], const double n[3],
+                    const double t1[3], const double t2[3], double f[NV])
+{
+    lxf_flux(ph, QL, QR, 1.0 / QL[0], 1.0 / QR[0], n, t1, t2, f);
 }
 
 // Two-point volume fluxes, RiemannSolvers_NS.f90:2085-2438 (Standard, Ducros, Kennedy-Gruber,
@@ -463,9 +515,10 @@ HX_HD void two_point(const double *a, const double *ja, const double *b, const d
 // The velocity and pressure euler_contravariant forms (the same operations).
 HX_HD void euler_primitives(const Phys &ph, const double q[NV], double &u, double &v, double &w, double &p)
 {
-    u = q[1] / q[0];
-    v = q[2] / q[0];
-    w = q[3] / q[0];
+    const double ir = 1.0 / q[0];
+    u = quot(q[1], q[0], ir);
+    v = quot(q[2], q[0], ir);
+    w = quot(q[3], q[0], ir);
     p = ph.gm1 * (q[4] - 0.5 * (q[1] * u + q[2] * v + q[3] * w));
 }
 

@@ -1,4 +1,5 @@
-// Stage kernels of the hx3d engine (one explicit RK3 stage = k_grad, k_face, k_volume).
+// Stage kernels of the hx3d engine on Gauss-Lobatto nodes of one order (one explicit RK3 stage =
+// k_grad, k_volume).
 // Included by hx3d_engine.hip.  See that file for the device data layout.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -67,6 +68,14 @@ __device__ __forceinline__ void stg(T *x, unsigned i, T v)
     *(HX_GLOBAL T *)((HX_GLOBAL char *)sbase(x) + i * (unsigned)sizeof(T)) = v;
 }
 
+// Instructions are not moved across this point (no instruction is emitted).
+__device__ __forceinline__ void sched_fence()
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+
 // Entry t of an (N+1) x (N+1) operator (row stride 8 in Ops); threads t >= (N+1)^2 get 0.
 // Loaded before the node data and stored to LDS after it has been issued, so the wait for it
 // does not hold back the other loads.
@@ -78,6 +87,7 @@ __device__ __forceinline__ double operator_entry(const double *src, int t)
 }
 
 __device__ __forceinline__ void block_min_pair(double a, double b, double *part, int t, int slot);
+__device__ __forceinline__ void block_min_slot(double a, double b, unsigned long long *slots, int t, int cs, int lb);
 
 // Several independent cases of one order in one engine (batching): each case has its own
 // physics constants, dt, time, divergence flag and active mask; element blocks never straddle
@@ -88,9 +98,7 @@ struct CaseConst {
 struct Multi {
     const int4 *blocks;     // per logical block: first element, element count, case, first block of its case
     const CaseConst *cc;    // [cases]
-    const int *active;      // [cases]: 0 = finished, its blocks and faces do no work
-    const int *fcase;       // [faces]: the case of each face
-    const int *pfirst;      // [cases + 1]: each case's range of logical blocks (its dt partials)
+    const int *active;      // [cases]: 0 = finished, its blocks do no work
     int cases;
 };
 
@@ -103,16 +111,20 @@ __device__ __forceinline__ void case_physics(Phys &ph, const CaseConst &c)
 }
 
 // The elements of logical block lb: first element e0, count cnt (0: nothing to do), case cs,
-// and whether the block is its case's first.  One case: EPB elements per block.
+// and whether the block is its case's first; idle: the count of a finished case's block, whose
+// cnt is 0.  One case: EPB elements per block.
 template <int EPB>
 __device__ __forceinline__ void block_elements(const Multi &mc, int lb, int K, int &e0, int &cnt, int &cs, bool &first,
-                                               Phys &ph)
+                                               int &idle, Phys &ph)
 {
+    idle = 0;
     if (mc.blocks) {
         const int4 b = mc.blocks[lb];
+        const bool on = mc.active[b.z] != 0;
         e0 = b.x;
         cs = b.z;
-        cnt = mc.active[cs] ? b.y : 0;
+        cnt = on ? b.y : 0;
+        idle = on ? 0 : b.y;
         first = b.w != 0;
         case_physics(ph, mc.cc[cs]);
     } else {
@@ -123,13 +135,21 @@ __device__ __forceinline__ void block_elements(const Multi &mc, int lb, int K, i
     }
 }
 
-// MaxTimeStep of the state a stage starts from, accumulated by the stage's gradient kernel
-// (part == null: not this stage): block minima of the convective and viscous limits to
-// part[2*block + 0/1], reduced by the face kernel that follows (DtReduce).
+// MaxTimeStep of the state a stage starts from, accumulated by the stage's gradient kernel.
+// Mixed orders and Gauss nodes (part; null: not this stage): block minima of the convective and
+// viscous limits to part[2*block + 0/1], reduced by the face kernel that follows (DtReduce).
+// Gauss-Lobatto nodes of one order (slots; null: not this stage): each block's minima by atomicMin
+// into one of the case's DT_FAN slots, from which every block of the volume kernel that follows
+// takes the minimum.  The minimum of doubles does not depend on the order, and the limits are
+// positive or NaN, whose bit patterns order like the numbers (NaN above +inf, so it is passed over
+// as fmin passes it over).  DT_FAN slots on lines of their own: one slot alone serialises (16k
+// atomics on one address cost 150 us), 32 leave at most a few hundred per line at 24^3 elements.
 struct DtLimits {
     double *part;
     double cfl, dcfl, dcsi;
+    unsigned long long *slots;
 };
+constexpr int DT_FAN = 32, DT_LINE = 16;   // slots per case; slot stride in 8-byte words (128 B)
 
 // Averaging selectors of the templated split-form kernel (RiemannSolvers_NS.f90:229-285)
 enum { AVG_STANDARD = 0, AVG_DUCROS = 1, AVG_KG = 2, AVG_PIROZZOLI = 3, AVG_MORINISHI = 4, FORM_STANDARD = -1 };
@@ -145,47 +165,111 @@ __device__ __forceinline__ unsigned efx(int e, int slot, int a, int b)
 
 // ------------------------------------------------------------------------------------
 // k_grad: per element, local gradient (HexElement_ComputeLocalGradient,
-// HexElementClass.f90:427-531) + BR1 lifting (EllipticBR1.f90:168-397), then the viscous
-// state of ViscousFlux_STATE (velocity gradients, grad T) at every node.
-//   nbr[x]        2 * (neighbour's node) + (1 if this element is the face's right side)
-//   egeo[c*ES+x]  face normal (c = 0..2) and surface Jacobian |Ja| (c = 3) of the face
+// HexElementClass.f90:427-531) + BR1 lifting (EllipticBR1.f90:168-397), then the viscous flux
+// tensor at every node (nine values, against twelve of the gradients it is formed from; the volume
+// kernel's faces and nodes read it, and neither forms a viscosity), or with LES what it is formed
+// from (viscous_values).
+//   nbr[x]         2 * (neighbour's node) + (1 if this element is the face's right side)
+//   egeo[c*ES+x]   face normal (c = 0..2) and surface Jacobian |Ja| (c = 3) of the face
+//   visc[c*S+g]    out: the viscous flux tensor or the LES values
 // ------------------------------------------------------------------------------------
 #ifndef HX3D_GRAD_WAVES
 #define HX3D_GRAD_WAVES 1
 #endif
+
+// The gradient at node (i, j, k) of the element whose state is sQ[v*ne + m] (LDS), in the
+// reference's order: with u_d = sum_l D(own, l) q(l) along reference direction d,
+// gr[c][v] = (sum_d u_d Ja^d_c) / J + gr[c][v] / J, the lifting sums given in gr.  One variable at a
+// time, its results pinned (hold), so that the sums of a variable, not of all five, hold registers
+// (k_volume at N = 4: 255 registers with all in flight).
+template <int n1>
+__device__ __forceinline__ void element_gradient(const double *sQ, const double *sD, int i, int j, int k,
+                                                 const double *ja, double iJ, double (*gr)[NV])
+{
+    constexpr int nf = n1 * n1, ne = nf * n1;
+    double dx[n1], dy[n1], dz[n1];
+#pragma unroll
+    for (int l = 0; l < n1; ++l) { dx[l] = sD[i * n1 + l]; dy[l] = sD[j * n1 + l]; dz[l] = sD[k * n1 + l]; }
+    const double *lx = sQ + n1 * (j + n1 * k), *ly = sQ + i + nf * k, *lz = sQ + i + n1 * j;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        double u0 = 0.0, u1 = 0.0, u2 = 0.0;
+#pragma unroll
+        for (int l = 0; l < n1; ++l) {
+            u0 = u0 + lx[v * ne + l] * dx[l];
+            u1 = u1 + ly[v * ne + n1 * l] * dy[l];
+            u2 = u2 + lz[v * ne + nf * l] * dz[l];
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            gr[c][v] = (u0 * ja[c] + u1 * ja[3 + c] + u2 * ja[6 + c]) * iJ + gr[c][v] * iJ;
+            hold(gr[c][v]);
+        }
+        sched_fence();
+    }
+}
+
+// BR1 lifting of one face (BR1_ComputeElementInterfaceAverage, EllipticBR1.f90:571-627, and
+// BR1_GradientFaceLoop, :531-569): unStar = 1/2 (U_R - U_L) |Ja| n with the face frame of the left
+// element, the same value for both sides; the GL surface integral weights it by b = 1/w_0.  qn: the
+// neighbour's state; jac: |Ja|, negated on the face's right side (so that 1/2 (qn - q) jac is the
+// jump's product on both sides, bit for bit).
+__device__ __forceinline__ void lift_face(const double *q, const double *qn, const double *n, double jac, double b0,
+                                          double (*gr)[NV])
+{
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        const double uS = 0.5 * (qn[v] - q[v]) * jac;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) gr[c][v] = gr[c][v] + (uS * n[c]) * b0;
+    }
+}
+
+// What the gradient kernel leaves per node: the viscous flux tensor (NVF values); with LES, whose
+// eddy viscosity takes the element's filter width at the nodes and the face's on the faces, what
+// the tensor is formed from: the stress without its viscosity (6), grad T (3), mu, and the
+// filter-width-free factor X of the eddy viscosity.
+constexpr int NVF = 9, NVL = 11;
+constexpr int viscous_values(bool les) { return les ? NVL : NVF; }
+
+// The tensor of a node's LES values with filter width d (mu, kappa of SD.f90:403-436 and :1345-1398)
+__device__ __forceinline__ void les_tensor(const Phys &ph, const double *q, double ir, const double *x, double d,
+                                           double *f)
+{
+    const double mt = hx::les_mu(ph, d, q[0], x[10]);
+    const double mu = x[9] + mt, kappa = x[9] * ph.mu_to_kappa + mt * ph.mu_to_kappa;
+    hx::viscous_tensor(mu, kappa, q[1] * ir, q[2] * ir, q[3] * ir, x, x + 6, f);
+}
+
 template <int N, int EPB>
 __global__ void __launch_bounds__(((EPB * (N + 1) * (N + 1) * (N + 1) + 63) / 64) * 64)
 __attribute__((amdgpu_waves_per_eu(HX3D_GRAD_WAVES)))
 k_grad(const double *__restrict__ Q, const double *__restrict__ Ja, const double *__restrict__ Jac,
-       const int *__restrict__ nbr, const double *__restrict__ egeo, double *__restrict__ vgrad,
-       int K, long S, long ES, Ops ops, Phys ph, DtLimits dtl, Multi mc)
+       const int *__restrict__ nbr, const double *__restrict__ egeo,
+       double *__restrict__ visc, double *__restrict__ curl_out, int K, long S, long ES, Ops ops, Phys ph, DtLimits dtl, Multi mc)
 {
     constexpr int n1 = N + 1, nf = n1 * n1, ne = nf * n1;
     __shared__ double sQ[EPB][NV][ne];
     __shared__ double sD[n1 * n1];
     const int lb = xcd_block(blockIdx.x, gridDim.x);
     const int t = threadIdx.x;
-    int e0, cnt, cs;
+    int e0, cnt, cs, idle;
     bool first;
-    block_elements<EPB>(mc, lb, K, e0, cnt, cs, first, ph);
-    if (cnt == 0) {   // uniform: a padding block or a finished case
-        if (dtl.part && t == 0) { dtl.part[2 * lb] = INFINITY; dtl.part[2 * lb + 1] = INFINITY; }
-        return;
-    }
+    block_elements<EPB>(mc, lb, K, e0, cnt, cs, first, idle, ph);
+    if (cnt == 0) return;   // uniform: a padding block or a finished case
     const int el = t / ne, n = t - el * ne;
     const int e = e0 + el;
     const bool active = el < cnt;
-    const unsigned g = (unsigned)e * ne + n;
     const int i = n % n1, j = (n / n1) % n1, k = n / nf;
     // Every load is unconditional (padding threads read a clamped element and discard it; see
     // k_volume).  The node's (at most three) faces: x-face slot 5 / 3, y-face 0 / 1, z-face
     // 2 / 4; faces the node is not on get zero traces and zero geometry, so their lifting term
     // is an exact zero and the accumulation below is branch-free.
     const int ec = active ? e : e0 + cnt - 1;
-    const unsigned gc = (unsigned)ec * ne + n;
+    const unsigned gc = (unsigned)ec * ne + n, g = (unsigned)e * ne + n;
     const bool onx = i == 0 || i == N, ony = j == 0 || j == N, onz = k == 0 || k == N;
-    const unsigned fx = efx<N>(ec, i == 0 ? 5 : 3, j, k), fy = efx<N>(ec, j == 0 ? 0 : 1, i, k),
-                   fz = efx<N>(ec, k == 0 ? 2 : 4, i, j);
+    const int sx = i == 0 ? 5 : 3, sy = j == 0 ? 0 : 1, sz = k == 0 ? 2 : 4;
+    const unsigned fx = efx<N>(ec, sx, j, k), fy = efx<N>(ec, sy, i, k), fz = efx<N>(ec, sz, i, j);
     const double dop = operator_entry<n1>(ops.D, t);
     const int cx = ldg(nbr, fx), cy = ldg(nbr, fy), cz = ldg(nbr, fz);
     double q[NV], ja[9], gx[4], gy[4], gz[4];
@@ -220,207 +304,73 @@ k_grad(const double *__restrict__ Q, const double *__restrict__ Ja, const double
     __syncthreads();
     double tc = INFINITY, tv = INFINITY;   // MaxTimeStep limits of this node (stage 1)
     if (active) {
-    double uxi[NV], ueta[NV], uzeta[NV];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) { uxi[v] = 0.0; ueta[v] = 0.0; uzeta[v] = 0.0; }
-#pragma unroll
-    for (int l = 0; l < n1; ++l) {
-        const double di = sD[i * n1 + l];
-#pragma unroll
-        for (int v = 0; v < NV; ++v) uxi[v] = uxi[v] + sQ[el][v][l + n1 * (j + n1 * k)] * di;
-    }
-#pragma unroll
-    for (int l = 0; l < n1; ++l) {
-        const double dj = sD[j * n1 + l];
-#pragma unroll
-        for (int v = 0; v < NV; ++v) ueta[v] = ueta[v] + sQ[el][v][i + n1 * (l + n1 * k)] * dj;
-    }
-#pragma unroll
-    for (int l = 0; l < n1; ++l) {
-        const double dk = sD[k * n1 + l];
-#pragma unroll
-        for (int v = 0; v < NV; ++v) uzeta[v] = uzeta[v] + sQ[el][v][i + n1 * (j + n1 * l)] * dk;
-    }
-    double gr[3][NV];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        gr[0][v] = (uxi[v] * ja[0] + ueta[v] * ja[3] + uzeta[v] * ja[6]) * iJ;
-        gr[1][v] = (uxi[v] * ja[1] + ueta[v] * ja[4] + uzeta[v] * ja[7]) * iJ;
-        gr[2][v] = (uxi[v] * ja[2] + ueta[v] * ja[5] + uzeta[v] * ja[8]) * iJ;
-    }
-    // BR1 lifting (BR1_ComputeElementInterfaceAverage, EllipticBR1.f90:571-627, and
-    // BR1_GradientFaceLoop, :531-569): on each face the node lies on,
-    // unStar = 1/2 (U_R - U_L) |Ja| n with the face frame of the left element, the same value
-    // for both sides; the GL surface integral weights it by b = 1/w_0.  Faces in slot order
-    // 5, 3, 0, 1, 2, 4 (ELEFT/ERIGHT, EFRONT/EBACK, EBOTTOM/ETOP).
-    {
+        double gr[3][NV];
+        // Faces in slot order 5, 3, 0, 1, 2, 4 (ELEFT/ERIGHT, EFRONT/EBACK, EBOTTOM/ETOP)
         const double b0 = 1.0 / ops.w[0];
-        double fi[3][NV];
 #pragma unroll
         for (int d = 0; d < 3; ++d)
 #pragma unroll
-            for (int v = 0; v < NV; ++v) fi[d][v] = 0.0;
-        auto lift = [&](const double *fg, int code, const double *qn) {
-            const bool right = code & 1;
-#pragma unroll
-            for (int v = 0; v < NV; ++v) {
-                const double uS = 0.5 * (right ? q[v] - qn[v] : qn[v] - q[v]) * fg[3];
-                fi[0][v] = fi[0][v] + (uS * fg[0]) * b0;
-                fi[1][v] = fi[1][v] + (uS * fg[1]) * b0;
-                fi[2][v] = fi[2][v] + (uS * fg[2]) * b0;
-            }
-        };
-        lift(gx, cx, qx);
-        lift(gy, cy, qy);
-        lift(gz, cz, qz);
-        if (onx || ony || onz) {
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-#pragma unroll
-                for (int v = 0; v < NV; ++v) gr[d][v] = gr[d][v] + fi[d][v] * iJ;
+            for (int v = 0; v < NV; ++v) gr[d][v] = 0.0;
+        lift_face(q, qx, gx, cx & 1 ? -gx[3] : gx[3], b0, gr);
+        lift_face(q, qy, gy, cy & 1 ? -gy[3] : gy[3], b0, gr);
+        lift_face(q, qz, gz, cz & 1 ? -gz[3] : gz[3], b0, gr);
+        element_gradient<n1>(&sQ[el][0][0], sD, i, j, k, ja, iJ, gr);
+        double vg[12], sh[6], mu, kappa, X = 0.0;
+        if (ph.les) X = hx::les_factor(ph, q, gr[0], gr[1], gr[2]);
+        hx::viscous_state(ph, q, gr[0], gr[1], gr[2], vg);
+        if (curl_out) {   // |curl u|^2 of the enstrophy monitor
+            const double a = vg[5] - vg[7], b = vg[6] - vg[2], c = vg[1] - vg[3];
+            stg(curl_out, g, a * a + b * b + c * c);
         }
-    }
-    double vg[12];
-    hx::viscous_state(ph, q, gr[0], gr[1], gr[2], vg);
+        hx::laminar_mu_kappa(ph, q, mu, kappa);
+        hx::stress_shape(vg, sh);
+        if (ph.les) {
 #pragma unroll
-    for (int c = 0; c < 12; ++c) stg(vgrad + c * S, g, vg[c]);
-    // LES: the filter-width-free factor of the eddy viscosity, from the conservative gradients
-    // (the face and volume kernels apply their own filter widths)
-    if (ph.les) stg(vgrad + 12 * S, g, hx::les_factor(ph, q, gr[0], gr[1], gr[2]));
-    if (dtl.part) hx::dt_limits(ph, q, ja, jg, dtl.dcsi, dtl.dcsi, dtl.dcsi, dtl.cfl, dtl.dcfl, tc, tv);
+            for (int c = 0; c < 6; ++c) stg(visc + c * S, g, sh[c]);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) stg(visc + (6 + c) * S, g, vg[9 + c]);
+            stg(visc + 9 * S, g, mu);
+            stg(visc + 10 * S, g, X);
+        } else {
+            double f[NVF];
+            const double ir = 1.0 / q[0];
+            hx::viscous_tensor(mu, kappa, q[1] * ir, q[2] * ir, q[3] * ir, sh, vg + 9, f);
+#pragma unroll
+            for (int c = 0; c < NVF; ++c) stg(visc + c * S, g, f[c]);
+        }
+        if (dtl.slots) hx::dt_limits(ph, q, ja, jg, dtl.dcsi, dtl.dcsi, dtl.dcsi, dtl.cfl, dtl.dcfl, tc, tv);
     }
-    if (dtl.part) block_min_pair(tc, tv, dtl.part, t, lb);
+    if (dtl.slots) block_min_slot(tc, tv, dtl.slots, t, cs, lb);
 }
 
-// ------------------------------------------------------------------------------------
-// k_face: one thread per face node (computeElementInterfaceFlux, SD.f90:1710-1799).
-// fnode[q] = (left node, right node, left element face node, right element face node).
-// The flux times the surface weight b = 1/w_0 is stored for both sides in element face order,
-// negated for the right side (TimeDerivative_FacesContribution, SD.f90:1686-1701).
-// ------------------------------------------------------------------------------------
+// dtred: (partials, count, slot) of the step's dt limits, reduced by block 0 of the mixed-order and
+// Gauss face kernels
 __device__ __forceinline__ void reduce_dt_partials(const double *part, int n, unsigned long long *bits, int t);
-
-// dtred: (partials, count, slot) of the step's dt limits, reduced by block 0 first (or null);
-// with several cases, logical block c < cases reduces case c's partials into slot c
 struct DtReduce {
     const double *part;
     int n;
     unsigned long long *bits;
 };
 
-#ifndef HX3D_FACE_WAVES
-#define HX3D_FACE_WAVES 1
-#endif
-// threads (face nodes) per block of k_face (128 and 512 measured 12% and 18% slower at 16^3 x N=4)
+// threads (face nodes) per block of the Gauss face kernel
 constexpr int FACE_TPB = 256;
-// T2X: the stored second tangent is n x t1 (vCross, MappedGeometry.f90:745, :807-817) bit for
-// bit at every face node (checked on the host), so it is formed here instead of read.  LXF: the
-// engine's Riemann solver is Lax-Friedrichs, the one that reads the tangents (Roe does not).
-template <int N, bool T2X, bool LXF>
-__global__ void __launch_bounds__(FACE_TPB)
-__attribute__((amdgpu_waves_per_eu(HX3D_FACE_WAVES)))
-k_face(const double *__restrict__ Q, const double *__restrict__ vgrad, const double *__restrict__ fgeo,
-       const int4 *__restrict__ fnode, const double *__restrict__ fdelta, double *__restrict__ fe,
-       long FS, long S, long ES, double b0, Phys ph, DtReduce dtr, Multi mc)
-{
-    constexpr int n1 = N + 1, nf = n1 * n1;
-    const int lb = xcd_block(blockIdx.x, gridDim.x);
-    if (dtr.bits) {
-        if (!mc.blocks) {
-            if (blockIdx.x == 0) reduce_dt_partials(dtr.part, dtr.n, dtr.bits, threadIdx.x);
-        } else if (lb < mc.cases) {   // case lb's dt (its blocks' partials)
-            const int p0 = mc.pfirst[lb];
-            reduce_dt_partials(dtr.part + 2 * p0, mc.pfirst[lb + 1] - p0, dtr.bits + 2 * lb, threadIdx.x);
-        }
-    }
-    const unsigned fq = (unsigned)lb * blockDim.x + threadIdx.x;
-    if (fq >= FS) return;
-    if (mc.blocks) {
-        const int cs = mc.fcase[fq / nf];
-        if (!mc.active[cs]) return;
-        case_physics(ph, mc.cc[cs]);
-    }
-    const int4 gi = ldg(fnode, fq);
-    const unsigned gx = gi.x, gy = gi.y, gz = gi.z, gw = gi.w;
-    // face frame: fgeo[c*FS + fq], c = n (0..2), t1 (3..5), t2 (6..8), |Ja| (9)
-    double nrm[3], t1[3], t2[3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) nrm[c] = ldg(fgeo + c * FS, fq);
-    const double jac = ldg(fgeo + 9 * FS, fq);
-    // all loads unconditional (see k_volume)
-    double qL[NV], qR[NV], vgL[12], vgR[12];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) { qL[v] = ldg(Q + v * S, gx); qR[v] = ldg(Q + v * S, gy); }
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        t1[c] = LXF ? ldg(fgeo + (3 + c) * FS, fq) : 0.0;
-        t2[c] = (LXF && !T2X) ? ldg(fgeo + (6 + c) * FS, fq) : 0.0;
-    }
-#pragma unroll
-    for (int c = 0; c < 12; ++c) { vgL[c] = ldg(vgrad + c * S, gx); vgR[c] = ldg(vgrad + c * S, gy); }
-    const double fd = ldg(fdelta, fq / nf);
-    double xL = 0.0, xR = 0.0;   // LES factors of the two sides (the gradient kernel's plane 12)
-    if (ph.les) { xL = ldg(vgrad + 12 * S, gx); xR = ldg(vgrad + 12 * S, gy); }
-    double visc[NV] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    if (!ph.euler) {
-        // BR1_RiemannSolver (EllipticBR1.f90:816-868) with the face viscosities of
-        // compute_viscosity_at_faces (SpatialDiscretization.f90:1345-1398)
-        double FL[NV][3], FR[NV][3];
-        {
-            double mu, kappa;
-            hx::laminar_mu_kappa(ph, qL, mu, kappa);
-            if (ph.les) {
-                const double mt = hx::les_mu(ph, fd, qL[0], xL);
-                mu = mu + mt; kappa = kappa + mt * ph.mu_to_kappa;
-            }
-            const double ir = 1.0 / qL[0];
-            hx::viscous_flux(mu, kappa, qL[1] * ir, qL[2] * ir, qL[3] * ir, vgL, FL);
-        }
-        {
-            double mu, kappa;
-            hx::laminar_mu_kappa(ph, qR, mu, kappa);
-            if (ph.les) {
-                const double mt = hx::les_mu(ph, fd, qR[0], xR);
-                mu = mu + mt; kappa = kappa + mt * ph.mu_to_kappa;
-            }
-            const double ir = 1.0 / qR[0];
-            hx::viscous_flux(mu, kappa, qR[1] * ir, qR[2] * ir, qR[3] * ir, vgR, FR);
-        }
-#pragma unroll
-        for (int v = 0; v < NV; ++v)
-            visc[v] = 0.5 * (FL[v][0] + FR[v][0]) * nrm[0] + 0.5 * (FL[v][1] + FR[v][1]) * nrm[1] +
-                      0.5 * (FL[v][2] + FR[v][2]) * nrm[2];
-    }
-    double inv[NV];
-    if (LXF) {
-        if (T2X) {
-            t2[0] = nrm[1] * t1[2] - t1[1] * nrm[2];
-            t2[1] = nrm[2] * t1[0] - t1[2] * nrm[0];
-            t2[2] = nrm[0] * t1[1] - t1[0] * nrm[1];
-        }
-        hx::lxf_flux(ph, qL, qR, nrm, t1, t2, inv);
-    } else {
-        hx::roe_flux(ph, qL, qR, nrm, inv);
-    }
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        const double fb = ((inv[v] - visc[v]) * jac) * b0;
-        stg(fe + v * ES, gz, fb);
-        stg(fe + v * ES, gw, -fb);
-    }
-}
 
 // ------------------------------------------------------------------------------------
-// k_volume: per element, the volume integral (standard or split form), the surface integral
-// of the stored face fluxes, 1/J, the Williamson RK3 register update, and (last stage) the
-// MaxTimeStep reduction of the updated state for the next step.
+// k_volume: per element, the face fluxes of its six faces (computeElementInterfaceFlux,
+// SD.f90:1710-1799), the volume integral (standard or split form), the surface integral, 1/J and
+// the Williamson RK3 register update.
 // ------------------------------------------------------------------------------------
 struct DtArgs {
     const unsigned long long *in;   // [2]: convective, viscous limit bit patterns of this step's dt
     double *time;                   // t += dt by one thread (or null)
     int *nan;                       // set to 1 when an updated state value is NaN (or null)
     DtLimits lim;                   // consumed by the stage's gradient kernel
-    DtReduce red;                   // consumed by the stage's face kernel
+    DtReduce red;                   // consumed by the stage's face kernel (mixed orders, Gauss nodes)
+    // Gauss-Lobatto nodes of one order: the first stage takes dt from the limits' slots (not from
+    // `in`) and leaves it in `in`'s place, fin, for the later stages; the second stage empties the
+    // slots for the next step (each null in the other stages)
+    const unsigned long long *slots;
+    unsigned long long *fin, *empty;
 };
 
 __device__ __forceinline__ double bits_to_double(unsigned long long b) { return __longlong_as_double((long long)b); }
@@ -443,6 +393,25 @@ __device__ __forceinline__ void block_min_pair(double a, double b, double *part,
         for (int w = 1; w < nw; ++w) { a = fmin(a, sm[0][w]); b = fmin(b, sm[1][w]); }
         part[2 * slot] = a;
         part[2 * slot + 1] = b;
+    }
+}
+
+// Block minimum of (a, b) by atomicMin into slot lb mod DT_FAN of case cs (see DtLimits)
+__device__ __forceinline__ void block_min_slot(double a, double b, unsigned long long *slots, int t, int cs, int lb)
+{
+    __shared__ double sm[2][16];
+    for (int o = 32; o > 0; o >>= 1) {
+        a = fmin(a, __shfl_xor(a, o, 64));
+        b = fmin(b, __shfl_xor(b, o, 64));
+    }
+    if ((t & 63) == 0) { sm[0][t >> 6] = a; sm[1][t >> 6] = b; }
+    __syncthreads();
+    if (t == 0) {
+        const int nw = (blockDim.x + 63) >> 6;
+        for (int w = 1; w < nw; ++w) { a = fmin(a, sm[0][w]); b = fmin(b, sm[1][w]); }
+        unsigned long long *s = slots + (long)(cs * DT_FAN + lb % DT_FAN) * DT_LINE;
+        atomicMin(s, (unsigned long long)__double_as_longlong(a));
+        atomicMin(s + 1, (unsigned long long)__double_as_longlong(b));
     }
 }
 
@@ -477,7 +446,8 @@ __host__ __device__ constexpr int pair_slot(int n1, int lo, int hi)
     return lo * n1 - (lo * (lo + 1)) / 2 + (hi - lo - 1);
 }
 
-// One thread per node, EPB elements per block.  The contravariant fluxes of all three
+// One thread per node, EPB elements per block.  First the face fluxes, one thread per element face
+// node, through LDS.  Then the contravariant fluxes of all three
 // directions (split form: the viscous ones, whose mass entry is zero; standard form: inviscid
 // minus viscous) go to LDS once.  Per direction each node accumulates, in l order,
 // qd = (qd + sharpD F#) + hatD Fv (DGIntegrals.f90:92-129) or qd = qd + hatD F (:56-87).
@@ -505,105 +475,307 @@ constexpr int volume_waves(int n, int form)
     return form == -1 ? 3 : (form == 2 || form == 3) && n <= 5 ? HX3D_VOL_WAVES : 1;
 }
 
-template <int N, int EPB, int FORM>
+// Element face node x of an element (x = slot nf + a + (N+1) b) as the element's node index
+template <int N>
+__device__ __forceinline__ int face_element_node(int x)
+{
+    constexpr int n1 = N + 1, nf = n1 * n1;
+    const int s = x / nf, r = x - s * nf, a = r % n1, b = r / n1;
+    if (s == 3 || s == 5) return n1 * a + nf * b + (s == 3 ? N : 0);   // x faces: (a, b) = (j, k)
+    if (s < 2) return a + nf * b + (s == 1 ? n1 * N : 0);              // y faces: (i, k)
+    return r + (s == 4 ? nf * N : 0);                                  // z faces: (i, j)
+}
+
+// Doubles of k_volume's LDS pool per block: first the elements' state [NV][ne] and viscous
+// values [9 or 11][ne] and the face fluxes [NV] per element face node; then the contravariant fluxes and
+// the direction loop's space.
+constexpr int vol_max(int a, int b) { return a > b ? a : b; }
+template <int N, int EPB, int FORM, bool LES>
+struct VolumeLds {
+    static constexpr int n1 = N + 1, nf = n1 * n1, ne = nf * n1, NI = 6 * nf;
+    static constexpr bool SPLIT = FORM >= 0;
+    static constexpr int ND = hx::node_data_size(SPLIT ? FORM : 0);
+    static constexpr int NF = SPLIT ? 4 : 5;
+    // split form: node data [ND][ne] and metric rows [3][ne], then the pair fluxes
+    // [pair][NV][line] of the current direction, in one space per element; at N = 5 each node
+    // evaluates its own row of pair fluxes (ROW), without the pair table
+    static constexpr bool ROW = SPLIT && N == 5 && HX3D_ROW5;
+    static constexpr int RN = (ND + 3) * ne, RP = ROW ? 0 : n1 * (n1 - 1) / 2 * NV * nf;
+    static constexpr int RSZ = SPLIT ? vol_max(RN, RP) : 0;
+    static constexpr int FSZ = 3 * NF * ne;
+    static constexpr int FACES = EPB * NI;
+    static constexpr int SIZE = vol_max(EPB * (NV + viscous_values(LES)) * ne + NV * FACES, EPB * (FSZ + RSZ));
+};
+
+// What bounds it: bytes first.  Per node 312 B (Q, Ja, J, G, viscous tensor in; G, Q out; 328 B with
+// LES), per element face node 172 B with Lax-Friedrichs, 148 B with Roe (the neighbour's state and
+// viscous values, 16 B more with LES, the face frame, the neighbour index).  The face fluxes are formed by both elements
+// of a face, from the same values in the same order, hence with the same bits: that costs 1.2
+// instead of 0.6 Riemann fluxes per node at N = 4, and saves the launch, the 80 B per face node
+// of stored fluxes each way and the second read of both traces.  Measured per stage (k_grad and
+// k_volume; before, with a face kernel between them and the gradients stored): 16^3 x N=4 Pirozzoli
+// 88 us (97), 24^3 x N=5 Kennedy-Gruber + WALE 592 (690), 4^3 x N=3 14 (18), 9^3 x N=6 62 (62).
+// At 16^3 x N=4 the kernel moves 265 MB in 59 us; without the direction loop it takes 40 us, the
+// rate of a large copy, and the loop's LDS traffic (97 accesses per node and direction) adds the
+// rest.  Forming the gradient again here instead of reading the viscous values measured 76 us.
+// New state to Qn, not in place: the neighbours of later blocks still read Q.
+// LXF: the engine's Riemann solver is Lax-Friedrichs, the one that reads the tangents (Roe does not).
+template <int N, int EPB, int FORM, bool LXF, bool LES>
 __global__ void __launch_bounds__(((EPB * (N + 1) * (N + 1) * (N + 1) + 63) / 64) * 64)
 __attribute__((amdgpu_waves_per_eu(volume_waves(N, FORM))))
-k_volume(double *__restrict__ Q, const double *__restrict__ vgrad, const double *__restrict__ Ja,
-         const double *__restrict__ Jac, const double *__restrict__ edelta, const double *__restrict__ fe,
-         double *__restrict__ G, double *__restrict__ qdot_out, double a_k, double c_k, int update,
+k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__restrict__ visc,
+         const double *__restrict__ edelta, const double *__restrict__ efdelta, const int *__restrict__ nbx,
+         const double *__restrict__ egeo, int t2x, const double *__restrict__ Ja,
+         const double *__restrict__ Jac, double *__restrict__ G, double *__restrict__ qdot_out, double a_k, double c_k, int update,
          DtArgs dta, int K, long S, long ES, Ops ops, Phys ph, Multi mc)
 {
-    constexpr int n1 = N + 1, nf = n1 * n1, ne = nf * n1;
-    constexpr bool SPLIT = FORM >= 0;
-    constexpr int AVG = SPLIT ? FORM : 0;
-    constexpr int ND = hx::node_data_size(AVG);
+    using L = VolumeLds<N, EPB, FORM, LES>;
+    constexpr int NVT = viscous_values(LES);
+    constexpr int n1 = L::n1, nf = L::nf, ne = L::ne, NI = L::NI, ND = L::ND, NF = L::NF, FACES = L::FACES;
+    constexpr bool SPLIT = L::SPLIT, ROW = L::ROW;
+    constexpr int AVG = SPLIT ? FORM : 0, V0 = SPLIT ? 1 : 0, NP = n1 / 2;
     constexpr bool SYM = hx::two_point_symmetric(AVG);
-    constexpr int NF = SPLIT ? 4 : 5, V0 = SPLIT ? 1 : 0;
-    // split form: node data [ND][ne] and metric rows [3][ne], then the pair fluxes
-    // [pair][NV][line] of the current direction, in one space per element
-    constexpr int NPAIR = n1 * (n1 - 1) / 2, NP = n1 / 2;
-    // split form at N = 5: each node evaluates its own row of pair fluxes (ROW), without the
-    // pair table
-    constexpr bool ROW = SPLIT && N == 5 && HX3D_ROW5;
-    constexpr int RN = (ND + 3) * ne, RP = ROW ? 0 : NPAIR * NV * nf;
-    constexpr int RSZ = SPLIT ? (RN > RP ? RN : RP) : 1;
-    __shared__ double sF[EPB][3][NF][ne];
-    __shared__ double sR[EPB][RSZ];
-    __shared__ double sHat[n1 * n1], sSharp[n1 * n1];
+    constexpr int TPB = ((EPB * ne + 63) / 64) * 64, P = (FACES + TPB - 1) / TPB;
+    __shared__ double pool[L::SIZE];
+    __shared__ double sHat[n1 * n1], sSharp[n1 * n1], sDt;
     __shared__ int sSlot[n1 * n1];   // pair table offset of (own, l); 0 on the diagonal
+    double *const sQ = pool;                       // [EPB][NV][ne]
+    double *const sT = sQ + EPB * NV * ne;         // [EPB][NVT][ne]
+    double *const sFb = sT + EPB * NVT * ne;       // [NV][FACES]
     const int lb = xcd_block(blockIdx.x, gridDim.x);
     const int t = threadIdx.x;
-    int e0, cnt, cs;
+    int e0, cnt, cs, idle;
     bool first;
-    block_elements<EPB>(mc, lb, K, e0, cnt, cs, first, ph);
-    if (cnt == 0) return;   // uniform: a padding block or a finished case
+    if (SPLIT) ph.averaging = FORM;   // the Lax-Friedrichs flux averages as the volume fluxes do
+    block_elements<EPB>(mc, lb, K, e0, cnt, cs, first, idle, ph);
     const int el = t / ne, n = t - el * ne;
     const int e = e0 + el;
+    if (cnt == 0) {   // uniform: a padding block, or a finished case, whose state moves to Qn as it is
+        if (update && el < idle) {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) stg(Qn + v * S, (unsigned)e * ne + n, ldg(Q + v * S, (unsigned)e * ne + n));
+        }
+        return;
+    }
     const bool active = el < cnt;
     const int i = n % n1, j = (n / n1) % n1, k = n / nf;
     const bool onx = i == 0 || i == N, ony = j == 0 || j == N, onz = k == 0 || k == N;
     // ---- Loads are unconditional (padding threads read a clamped element and discard it): a
     // load inside a branch makes the compiler wait for the whole memory queue at the first use
-    // of any earlier load.  The face values are issued first and summed once the node's own
-    // data has arrived (loads complete in order); G and dt are issued at the last direction
-    // and consumed after it.
+    // of any earlier load.
     const int ec = active ? e : e0 + cnt - 1;
     const unsigned gc = (unsigned)ec * ne + n, gw = (unsigned)e * ne + n;
-    const double hop = operator_entry<n1>(ops.hatD, t), sop = operator_entry<n1>(ops.sharpD, t);
-    double sx[NV], sy[NV], sz[NV];
-    {
-        const unsigned xx = efx<N>(ec, i == 0 ? 5 : 3, j, k), xy = efx<N>(ec, j == 0 ? 0 : 1, i, k),
-                       xz = efx<N>(ec, k == 0 ? 2 : 4, i, j);
+    int code[P];
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            const double fx = ldg(fe + v * ES, xx), fy = ldg(fe + v * ES, xy), fz = ldg(fe + v * ES, xz);
-            sx[v] = onx ? fx : 0.0;   // faces the node is not on add an exact zero
-            sy[v] = ony ? fy : 0.0;
-            sz[v] = onz ? fz : 0.0;
-        }
+    for (int p = 0; p < P; ++p) {
+        const int it = t + p * TPB;
+        code[p] = ldg(nbx, (unsigned)e0 * NI + (it < cnt * NI ? it : 0));
     }
-    double q[NV], ja[9], vg[12];
+    const double hop = operator_entry<n1>(ops.hatD, t),
+                 sop = operator_entry<n1>(ops.sharpD, t);
+    double q[NV], ja[9], vt[NVT];
 #pragma unroll
     for (int v = 0; v < NV; ++v) q[v] = ldg(Q + v * S, gc);
+    if (!ph.euler) {   // uniform
+#pragma unroll
+        for (int c = 0; c < NVT; ++c) vt[c] = ldg(visc + c * S, gc);
+    }
+    double dtl0 = INFINITY, dtl1 = INFINITY;   // this step's dt limits (first wave)
+    if (update && t < 64) {
+        if (dta.slots) {
+            const unsigned long long *sl = dta.slots + (long)(cs * DT_FAN + t % DT_FAN) * DT_LINE;
+            dtl0 = bits_to_double(sl[0]);
+            dtl1 = bits_to_double(sl[1]);
+        } else {
+            dtl0 = bits_to_double(dta.in[2 * cs]);
+            dtl1 = bits_to_double(dta.in[2 * cs + 1]);
+        }
+    }
+    if (t < n1 * n1) {
+        sHat[t] = hop;
+        sSharp[t] = sop;
+        const int a = t / n1, b = t - a * n1;
+        sSlot[t] = a == b ? 0 : pair_slot(n1, a < b ? a : b, a < b ? b : a) * NV * nf;
+    }
 #pragma unroll
     for (int c = 0; c < 9; ++c) ja[c] = ldg(Ja + c * S, gc);
+    const double jg = ldg(Jac, gc), dl = LES ? ldg(edelta, (unsigned)ec) : 0.0;
+    const double b0 = 1.0 / ops.w[0];
+    // What round p's face flux reads from memory; round 0's is asked for before the barrier, to
+    // arrive with the element's own data.
+    double qR[NV], nrm[3], jac, t1[3], fn[NVT], fd = 0.0;
+    auto load_face = [&](int p) {
+        const int it = t + p * TPB;
+        const unsigned x = (unsigned)e0 * NI + (it < cnt * NI ? it : 0), xn = (unsigned)code[p] >> 1;
+        const unsigned en = xn / NI, gn = en * ne + face_element_node<N>(xn - en * NI);
 #pragma unroll
-    for (int c = 0; c < 12; ++c) vg[c] = ldg(vgrad + c * S, gc);
-    const double dl = ldg(edelta, (unsigned)ec);
-    double lx = 0.0;   // LES factor (the gradient kernel's plane 12)
-    if (ph.les) lx = ldg(vgrad + 12 * S, gc);
-    const double jg = ldg(Jac, gc);
-    double own[ND] = {};   // this node's two-point data (split form)
-    if (active) {
-        double Fvc[3][NV];
+        for (int v = 0; v < NV; ++v) qR[v] = ldg(Q + v * S, gn);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) nrm[c] = ldg(egeo + c * ES, x);
+        jac = ldg(egeo + 3 * ES, x);
         if (!ph.euler) {
-            // BR1_ComputeInnerFluxes (EllipticBR1.f90:740-814) with mu, kappa of SD.f90:403-436
-            double mu, kappa;
-            hx::laminar_mu_kappa(ph, q, mu, kappa);
-            if (ph.les) {
-                const double mt = hx::les_mu(ph, dl, q[0], lx);
-                mu = mu + mt;
-                kappa = kappa + mt * ph.mu_to_kappa;
+#pragma unroll
+            for (int c = 0; c < NVT; ++c) fn[c] = ldg(visc + c * S, gn);
+        }
+        if (LES) fd = ldg(efdelta, x / nf);
+        if (LXF) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) t1[c] = ldg(egeo + (4 + c) * ES, x);
+        }
+    };
+    load_face(0);
+    if (active) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) sQ[(el * NV + v) * ne + n] = q[v];
+        if (!ph.euler) {
+#pragma unroll
+            for (int c = 0; c < NVT; ++c) sT[(el * NVT + c) * ne + n] = vt[c];
+        }
+    }
+    __syncthreads();
+    const int fx = el * NI + (i == 0 ? 5 : 3) * nf + j + n1 * k, fy = el * NI + (j == 0 ? 0 : 1) * nf + i + n1 * k,
+              fz = el * NI + (k == 0 ? 2 : 4) * nf + i + n1 * j;
+    // ---- the face fluxes, one thread per element face node, P rounds
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int it = t + p * TPB;
+        if (p) load_face(p);
+        if (it < cnt * NI) {
+            const bool right = code[p] & 1;
+            const int eo = it / NI, no = face_element_node<N>(it - eo * NI);
+            double qL[NV], vn[NV];
+            const double io = 1.0 / sQ[eo * NV * ne + no], in = 1.0 / qR[0];
+            vn[0] = 0.0;
+            if (!ph.euler) {
+                // BR1_RiemannSolver (EllipticBR1.f90:816-868): the average of both sides' tensors,
+                // summed in either order with the same bits, and its product with the normal
+                double f[NVF];
+                if (LES) {
+                    double qo[NV], vo[NVT], fo[NVF];
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) qo[v] = sQ[(eo * NV + v) * ne + no];
+#pragma unroll
+                    for (int c = 0; c < NVT; ++c) vo[c] = sT[(eo * NVT + c) * ne + no];
+                    les_tensor(ph, qo, io, vo, fd, fo);
+                    les_tensor(ph, qR, in, fn, fd, f);
+#pragma unroll
+                    for (int c = 0; c < NVF; ++c) f[c] = 0.5 * (f[c] + fo[c]);
+                } else {
+#pragma unroll
+                    for (int c = 0; c < NVF; ++c) f[c] = 0.5 * (fn[c] + sT[(eo * NVT + c) * ne + no]);
+                }
+#pragma unroll
+                for (int v = 1; v < NV; ++v) {
+                    vn[v] = f[hx::viscous_entry(v, 0)] * nrm[0] + f[hx::viscous_entry(v, 1)] * nrm[1] +
+                            f[hx::viscous_entry(v, 2)] * nrm[2];
+                    hold(vn[v]);
+                }
+            } else {
+#pragma unroll
+                for (int v = 1; v < NV; ++v) vn[v] = 0.0;
             }
-            const double ir = 1.0 / q[0];
-            double Fv[NV][3];
-            hx::viscous_flux(mu, kappa, q[1] * ir, q[2] * ir, q[3] * ir, vg, Fv);
 #pragma unroll
-            for (int d = 0; d < 3; ++d)
+            for (int v = 0; v < NV; ++v) {
+                const double o = sQ[(eo * NV + v) * ne + no], a = qR[v];
+                qL[v] = right ? a : o;
+                qR[v] = right ? o : a;
+            }
+            double inv[NV];
+            if (LXF) {
+                // t2x: the stored second tangent is n x t1 (vCross, MappedGeometry.f90:745, :807-817)
+                // bit for bit at every face node (checked on the host), so it is formed here
+                double t2[3];
+                if (!t2x) {
+                    const unsigned x = (unsigned)e0 * NI + it;
 #pragma unroll
-                for (int v = 0; v < NV; ++v)
-                    Fvc[d][v] = Fv[v][0] * ja[3 * d] + Fv[v][1] * ja[3 * d + 1] + Fv[v][2] * ja[3 * d + 2];
+                    for (int c = 0; c < 3; ++c) t2[c] = ldg(egeo + (7 + c) * ES, x);
+                } else {
+                    t2[0] = nrm[1] * t1[2] - t1[1] * nrm[2];
+                    t2[1] = nrm[2] * t1[0] - t1[2] * nrm[0];
+                    t2[2] = nrm[0] * t1[1] - t1[0] * nrm[1];
+                }
+                hx::lxf_flux(ph, qL, qR, right ? in : io, right ? io : in, nrm, t1, t2, inv);
+            } else {
+                hx::roe_flux(ph, qL, qR, right ? in : io, right ? io : in, nrm, inv);
+            }
+            // the right side negated (TimeDerivative_FacesContribution, SD.f90:1686-1701)
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                const double fb = ((inv[v] - vn[v]) * jac) * b0;
+                sFb[v * FACES + it] = right ? -fb : fb;
+            }
+        }
+    }
+    if (update && t < 64) {
+        for (int o = 32; o > 0; o >>= 1) {
+            dtl0 = fmin(dtl0, __shfl_xor(dtl0, o, 64));
+            dtl1 = fmin(dtl1, __shfl_xor(dtl1, o, 64));
+        }
+        if (t == 0) {
+            sDt = fmin(dtl0, dtl1);
+            if (first && dta.slots) {
+                dta.fin[2 * cs] = (unsigned long long)__double_as_longlong(dtl0);
+                dta.fin[2 * cs + 1] = (unsigned long long)__double_as_longlong(dtl1);
+            }
+        }
+        if (first && dta.empty && t < DT_FAN) {
+            unsigned long long *sl = dta.empty + (long)(cs * DT_FAN + t) * DT_LINE;
+            sl[0] = sl[1] = (unsigned long long)__double_as_longlong(INFINITY);
+        }
+    }
+    __syncthreads();
+    // The RK register.  The first RK stage (a_k = 0) does not read it: the reference's 0 G + QDot is
+    // QDot up to the sign of an exact zero, which no state value sees (Q + c dt (+-0) = Q); every
+    // later stage does.  Asked for here in the standard form, whose contractions are short, and at
+    // the last direction in the split form, where it would hold registers through two of them.
+    double gk[NV];
+    auto load_register = [&]() {
+        if (a_k != 0.0) {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) gk[v] = ldg(G + v * S, gc);
         } else {
 #pragma unroll
+            for (int v = 0; v < NV; ++v) gk[v] = 0.0;
+        }
+    };
+    if (!SPLIT) load_register();
+    double own[ND] = {};   // this node's two-point data (split form)
+    double xs[NV];         // the surface integral at this node
+    double Fvc[3][NV];     // contravariant viscous fluxes; standard form: inviscid minus viscous
+    if (active) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) q[v] = sQ[(el * NV + v) * ne + n];   // held no longer than needed
+        // Surface integral (SD.f90:1686-1701) of the node's faces in slot order; faces the node is
+        // not on add an exact zero
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const double a = sFb[v * FACES + fx], b = sFb[v * FACES + fy], c = sFb[v * FACES + fz];
+            xs[v] = ((0.0 + (onx ? a : 0.0)) + (ony ? b : 0.0)) + (onz ? c : 0.0);
+            hold(xs[v]);   // summed here, not at its use: one register pair instead of three
+        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+            for (int v = 0; v < NV; ++v) Fvc[d][v] = 0.0;
+        if (!ph.euler) {
+            // BR1_ComputeInnerFluxes (EllipticBR1.f90:740-814)
+            double f[NVF];
+#pragma unroll
+            for (int c = 0; c < NVT; ++c) vt[c] = sT[(el * NVT + c) * ne + n];   // held no longer than needed
+            if (LES) {
+                les_tensor(ph, q, 1.0 / q[0], vt, dl, f);
+            } else {
+#pragma unroll
+                for (int c = 0; c < NVF; ++c) f[c] = vt[c];
+            }
+#pragma unroll
             for (int d = 0; d < 3; ++d)
 #pragma unroll
-                for (int v = 0; v < NV; ++v) Fvc[d][v] = 0.0;
+                for (int v = 1; v < NV; ++v)
+                    Fvc[d][v] = f[hx::viscous_entry(v, 0)] * ja[3 * d] + f[hx::viscous_entry(v, 1)] * ja[3 * d + 1] +
+                                f[hx::viscous_entry(v, 2)] * ja[3 * d + 2];
         }
         if (SPLIT) {
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-#pragma unroll
-                for (int v = 1; v < NV; ++v) sF[el][d][v - V0][n] = Fvc[d][v];
             hx::node_data<AVG>(ph, q, own);
         } else {
             double Fi[3][NV];
@@ -611,21 +783,19 @@ k_volume(double *__restrict__ Q, const double *__restrict__ vgrad, const double 
 #pragma unroll
             for (int d = 0; d < 3; ++d)
 #pragma unroll
-                for (int v = 0; v < NV; ++v) sF[el][d][v - V0][n] = Fi[d][v] - Fvc[d][v];
+                for (int v = 0; v < NV; ++v) Fvc[d][v] = Fi[d][v] - Fvc[d][v];
         }
     }
-    // Surface integral (TimeDerivative_FacesContribution, SD.f90:1686-1701): the stored face
-    // values already carry b = 1/w_0 and the side's sign; faces in slot order 5, 3, 0, 1, 2, 4
-    double xs[NV];
+    __syncthreads();   // the state and the face values are read: the pool takes the fluxes
+    double *const sF = pool + el * (L::FSZ + L::RSZ);   // [3][NF][ne]
+    double *const sR = sF + L::FSZ;                     // [RSZ]
+    if (active) {
 #pragma unroll
-    for (int v = 0; v < NV; ++v) xs[v] = ((0.0 + sx[v]) + sy[v]) + sz[v];
-    if (t < n1 * n1) {
-        sHat[t] = hop;
-        sSharp[t] = sop;
-        const int a = t / n1, b = t - a * n1;
-        sSlot[t] = a == b ? 0 : pair_slot(n1, a < b ? a : b, a < b ? b : a) * NV * nf;
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+            for (int v = V0; v < NV; ++v) sF[(d * NF + v - V0) * ne + n] = Fvc[d][v];
     }
-    double qd[NV], gk[NV], dt0 = 0.0, dt1 = 0.0;
+    double qd[NV];
 #pragma unroll
     for (int v = 0; v < NV; ++v) qd[v] = 0.0;
     double pu, pv, pw, pp;   // the diagonal's primitives, formed once for the three directions
@@ -645,26 +815,13 @@ k_volume(double *__restrict__ Q, const double *__restrict__ vgrad, const double 
             if (d) __syncthreads();     // the previous direction's pair fluxes are read
             if (active) {
 #pragma unroll
-                for (int c = 0; c < ND; ++c) sR[el][c * ne + n] = own[c];
+                for (int c = 0; c < ND; ++c) sR[c * ne + n] = own[c];
 #pragma unroll
-                for (int c = 0; c < 3; ++c) sR[el][(ND + c) * ne + n] = jh[c];
+                for (int c = 0; c < 3; ++c) sR[(ND + c) * ne + n] = jh[c];
             }
         }
         if (SPLIT || d == 0) __syncthreads();
-        if (d == 2) {
-            // The first RK stage (a_k = 0) does not read the register: the reference's
-            // 0 G + QDot is QDot up to the sign of an exact zero, which no state value sees
-            // (Q + c dt (+-0) = Q); every later stage reads it.
-            if (a_k != 0.0) {
-#pragma unroll
-                for (int v = 0; v < NV; ++v) gk[v] = ldg(G + v * S, gc);
-            } else {
-#pragma unroll
-                for (int v = 0; v < NV; ++v) gk[v] = 0.0;
-            }
-            dt0 = bits_to_double(dta.in[2 * cs]);
-            dt1 = bits_to_double(dta.in[2 * cs + 1]);
-        }
+        if (SPLIT && d == 2) load_register();
         if (!SPLIT) {
             if (active) {
 #pragma unroll
@@ -672,7 +829,7 @@ k_volume(double *__restrict__ Q, const double *__restrict__ vgrad, const double 
                     const double hh = sHat[own_i * n1 + l];
                     const int m = base + l * stride;
 #pragma unroll
-                    for (int v = 0; v < NV; ++v) qd[v] = qd[v] + hh * sF[el][d][v][m];
+                    for (int v = 0; v < NV; ++v) qd[v] = qd[v] + hh * sF[(d * NF + v) * ne + m];
                 }
             }
             continue;
@@ -690,9 +847,9 @@ k_volume(double *__restrict__ Q, const double *__restrict__ vgrad, const double 
                     const int m = base + l * stride;
                     double b[ND], jb[3], tp[NV];
 #pragma unroll
-                    for (int c = 0; c < ND; ++c) b[c] = sR[el][c * ne + m];
+                    for (int c = 0; c < ND; ++c) b[c] = sR[c * ne + m];
 #pragma unroll
-                    for (int c = 0; c < 3; ++c) jb[c] = sR[el][(ND + c) * ne + m];
+                    for (int c = 0; c < 3; ++c) jb[c] = sR[(ND + c) * ne + m];
                     if (SYM) {
                         hx::two_point<AVG>(own, jh, b, jb, tp);
                     } else {
@@ -707,7 +864,7 @@ k_volume(double *__restrict__ Q, const double *__restrict__ vgrad, const double 
                     qd[0] = qd[0] + sh * (l == own_i ? fi[0] : tp[0]);
 #pragma unroll
                     for (int v = 1; v < NV; ++v)
-                        qd[v] = qd[v] + sh * (l == own_i ? fi[v] : tp[v]) + hh * sF[el][d][v - V0][m];
+                        qd[v] = qd[v] + sh * (l == own_i ? fi[v] : tp[v]) + hh * sF[(d * NF + v - V0) * ne + m];
                 }
             }
             continue;
@@ -721,9 +878,9 @@ k_volume(double *__restrict__ Q, const double *__restrict__ vgrad, const double 
                 const int m = base + l * stride;
                 double b[ND], jb[3];
 #pragma unroll
-                for (int c = 0; c < ND; ++c) b[c] = sR[el][c * ne + m];
+                for (int c = 0; c < ND; ++c) b[c] = sR[c * ne + m];
 #pragma unroll
-                for (int c = 0; c < 3; ++c) jb[c] = sR[el][(ND + c) * ne + m];
+                for (int c = 0; c < 3; ++c) jb[c] = sR[(ND + c) * ne + m];
                 if (SYM) {
                     hx::two_point<AVG>(own, jh, b, jb, pf[s - 1]);
                 } else {
@@ -745,7 +902,7 @@ k_volume(double *__restrict__ Q, const double *__restrict__ vgrad, const double 
                 const int l = own_i + s < n1 ? own_i + s : own_i + s - n1;
                 const int po = sSlot[own_i * n1 + l] + line;
 #pragma unroll
-                for (int v = 0; v < NV; ++v) sR[el][po + v * nf] = pf[s - 1][v];
+                for (int v = 0; v < NV; ++v) sR[po + v * nf] = pf[s - 1][v];
             }
         }
         __syncthreads();
@@ -760,10 +917,10 @@ k_volume(double *__restrict__ Q, const double *__restrict__ vgrad, const double 
                 const double sh = sSharp[own_i * n1 + l], hh = sHat[own_i * n1 + l];
                 const int m = base + l * stride;
                 const int po = sSlot[own_i * n1 + l] + line;
-                qd[0] = qd[0] + sh * (l == own_i ? fi[0] : sR[el][po]);
+                qd[0] = qd[0] + sh * (l == own_i ? fi[0] : sR[po]);
 #pragma unroll
                 for (int v = 1; v < NV; ++v)
-                    qd[v] = qd[v] + sh * (l == own_i ? fi[v] : sR[el][po + v * nf]) + hh * sF[el][d][v - V0][m];
+                    qd[v] = qd[v] + sh * (l == own_i ? fi[v] : sR[po + v * nf]) + hh * sF[(d * NF + v - V0) * ne + m];
             }
         }
     }
@@ -771,7 +928,6 @@ k_volume(double *__restrict__ Q, const double *__restrict__ vgrad, const double 
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             if (SPLIT) qd[v] = -qd[v];
-            hold(xs[v]);
             qd[v] = qd[v] - xs[v];
         }
         // QDot / J (SD.f90:490) as a product with 1/J: the rounding difference is one ulp of the
@@ -784,9 +940,7 @@ k_volume(double *__restrict__ Q, const double *__restrict__ vgrad, const double 
             for (int v = 0; v < NV; ++v) stg(qdot_out + v * S, gw, qd[v]);
         }
         if (update) {
-            hold(dt0);
-            hold(dt1);
-            const double dt = fmin(dt0, dt1);
+            const double dt = sDt;
             if (dta.time && first && t == 0) dta.time[cs] += dt;
             const double cdt = c_k * dt;
 #pragma unroll
@@ -795,7 +949,7 @@ k_volume(double *__restrict__ Q, const double *__restrict__ vgrad, const double 
                 const double gv = a_k * gk[v] + qd[v];
                 stg(G + v * S, gw, gv);
                 q[v] = q[v] + cdt * gv;
-                stg(Q + v * S, gw, q[v]);
+                stg(Qn + v * S, gw, q[v]);
             }
             // checkForNan (ExplicitMethods.f90:1856-1905) of the updated state: a sticky flag,
             // written only where a NaN appears
