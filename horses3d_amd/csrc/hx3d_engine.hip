@@ -175,19 +175,10 @@ k_absmax(const double *__restrict__ X, long nodes, long S, double *__restrict__ 
     }
 }
 
-__global__ void k_finish_max(const double *part, int nparts, double *out)
-{
-    if (threadIdx.x < NV) {
-        double r = 0.0;
-        for (int b = 0; b < nparts; ++b) r = fmax(r, part[(long)b * NV + threadIdx.x]);
-        out[threadIdx.x] = r;
-    }
-}
-
 // The allocation-free residuals (hx3d_residuals_noalloc): max |X| per variable over all nodes
 // by at most NOALLOC_BLOCKS blocks, each striding over the nodes, partial maxima to part[b*NV + v];
 // then one block reduces the nparts partials into out[0..NV-1].  The maximum of doubles is exact
-// and independent of order, so the result has the bits of k_absmax + k_finish_max.
+// and independent of order, so the result has the bits of k_absmax + k_finish_max_block.
 constexpr int NOALLOC_BLOCKS = 2048;
 
 __global__ void __launch_bounds__(256)
@@ -339,11 +330,22 @@ k_monitor(int kind, const double *__restrict__ Q, const double *__restrict__ QD,
     }
 }
 
-__global__ void k_finish_sum2(const double *part, int nparts, double *out)
+// The (value, volume) partials summed by one block, in a fixed order: thread t takes the partials
+// t, t + 1024, ..., then a tree over the threads.  A chain of dependent loads and additions bounds
+// this kernel, so the chain is split over the block: one thread over all partials took 71 us at
+// 12^3 x N=4 (844 partials), this takes 3.
+constexpr int FINISH_TPB = 1024;
+__global__ void __launch_bounds__(FINISH_TPB) k_finish_sum2(const double *__restrict__ part, int nparts, double *out)
 {
+    __shared__ double sa[FINISH_TPB / 64], sb[FINISH_TPB / 64];
+    double a = 0.0, b = 0.0;
+    for (int x = threadIdx.x; x < nparts; x += FINISH_TPB) { a += part[2 * x]; b += part[2 * x + 1]; }
+    a = wave_sum(a);
+    b = wave_sum(b);
+    if ((threadIdx.x & 63) == 0) { sa[threadIdx.x >> 6] = a; sb[threadIdx.x >> 6] = b; }
+    __syncthreads();
     if (threadIdx.x == 0) {
-        double a = 0.0, b = 0.0;
-        for (int x = 0; x < nparts; ++x) { a += part[2 * x]; b += part[2 * x + 1]; }
+        for (int w = 1; w < FINISH_TPB / 64; ++w) { a += sa[w]; b += sb[w]; }
         out[0] = a;
         out[1] = b;
     }
@@ -1988,7 +1990,7 @@ int hx3d_residuals(hx3d_engine *eng, double res[5])
     }
     const int nb = (int)((eng->nodes + 255) / 256);
     hipLaunchKernelGGL(k_absmax, dim3(nb), dim3(256), 0, eng->stream, eng->dQDot, eng->nodes, eng->S, eng->dPart);
-    hipLaunchKernelGGL(k_finish_max, dim3(1), dim3(64), 0, eng->stream, eng->dPart, nb, eng->dStage);
+    hipLaunchKernelGGL(k_finish_max_block, dim3(1), dim3(256), 0, eng->stream, eng->dPart, nb, eng->dStage);
     HIPCHK(hipMemcpyAsync(res, eng->dStage, sizeof(double) * NV, hipMemcpyDeviceToHost, eng->stream));
     HIPCHK(hipStreamSynchronize(eng->stream));
     return HX3D_OK;
@@ -2025,7 +2027,7 @@ int hx3d_kinetic_energy(hx3d_engine *eng, double *ke)
     if (!eng || !ke) return HX3D_EINVAL;
     const int nb = (int)((eng->nodes + 255) / 256);
     hipLaunchKernelGGL(k_kinetic, dim3(nb), dim3(256), 0, eng->stream, eng->dQ, eng->dJ, eng->dWq, eng->nodes, eng->S, eng->dPart);
-    hipLaunchKernelGGL(k_finish_sum2, dim3(1), dim3(64), 0, eng->stream, eng->dPart, nb, eng->dStage);
+    hipLaunchKernelGGL(k_finish_sum2, dim3(1), dim3(FINISH_TPB), 0, eng->stream, eng->dPart, nb, eng->dStage);
     double r[2];
     HIPCHK(hipMemcpyAsync(r, eng->dStage, sizeof(r), hipMemcpyDeviceToHost, eng->stream));
     HIPCHK(hipStreamSynchronize(eng->stream));
@@ -2052,7 +2054,7 @@ int hx3d_volume_monitor(hx3d_engine *eng, int kind, double *value)
     hipLaunchKernelGGL(k_monitor, dim3(nb), dim3(256), 0, eng->stream, kind, eng->dQ, eng->dQDot,
                        two_launch(eng) ? eng->dCurl : nullptr, eng->mixed ? nullptr : eng->dVgrad, eng->dU, eng->dJ, eng->dWq, eng->nodes, eng->S, eng->ph,
                        eng->dPart);
-    hipLaunchKernelGGL(k_finish_sum2, dim3(1), dim3(64), 0, eng->stream, eng->dPart, nb, eng->dStage);
+    hipLaunchKernelGGL(k_finish_sum2, dim3(1), dim3(FINISH_TPB), 0, eng->stream, eng->dPart, nb, eng->dStage);
     double r[2];
     HIPCHK(hipMemcpyAsync(r, eng->dStage, sizeof(r), hipMemcpyDeviceToHost, eng->stream));
     HIPCHK(hipStreamSynchronize(eng->stream));
