@@ -22,8 +22,8 @@
 //     egeo[c*ES + x] (normal, |Ja|, with
 //     Lax-Friedrichs t1, and t2 where it is not n x t1), nbr[x] (2 * neighbour node + side),
 //     nbx[x] (2 * neighbour's element face node + side)
-// Gauss nodes add per face node q = f(N+1)^2 + i + (N+1)j (left element's face coordinates), FS
-// the count: fgeo[c*FS + q] (n, t1, t2, |Ja|), fnode[q] (left node, right node, left x, right x)
+// Gauss nodes add the state's traces Qtr[v*ES + x] (twice) and the tensors at the face nodes
+// fvis[c*ES + x], and keep one copy of the state.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -32,6 +32,7 @@
 #include <cstdlib>
 #include <climits>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <type_traits>
@@ -258,12 +259,11 @@ k_kinetic(const double *__restrict__ Q, const double *__restrict__ Jac, const do
 //        4 internal energy      rho e
 //        5 entropy              log p - gamma log rho
 //        6 math entropy         -rho (log p - gamma log rho) / (gamma - 1)
-// |curl u|^2 as the volume kernel left it (Gauss-Lobatto nodes of one order), or from the velocity
-// gradients: the gradient kernel's viscous state (Gauss nodes of one order), or formed from the
-// lifted state gradients U_x, U_y, U_z as getVelocityGradients_State does (mixed orders).
+// |curl u|^2 as the gradient kernel left it (one order), or from the lifted state gradients U_x,
+// U_y, U_z as getVelocityGradients_State forms the velocity gradients (mixed orders).
 __global__ void __launch_bounds__(256)
 k_monitor(int kind, const double *__restrict__ Q, const double *__restrict__ QD, const double *__restrict__ curl2,
-          const double *__restrict__ vgrad, const double *__restrict__ U, const double *__restrict__ Jac, const double *__restrict__ wq, long nodes,
+          const double *__restrict__ U, const double *__restrict__ Jac, const double *__restrict__ wq, long nodes,
           long S, Phys ph, double *__restrict__ part)
 {
     __shared__ double sk[4], sv[4];
@@ -286,22 +286,13 @@ k_monitor(int kind, const double *__restrict__ Q, const double *__restrict__ QD,
             f = curl2[g];
         } else if (kind == 2) {
             double ux[3], uy[3], uz[3];   // d(u, v, w)/dx, /dy, /dz
-            if (vgrad) {
+            const double ir = 1.0 / q[0], ir2 = ir * ir;
 #pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    ux[c] = vgrad[c * S + g];
-                    uy[c] = vgrad[(3 + c) * S + g];
-                    uz[c] = vgrad[(6 + c) * S + g];
-                }
-            } else {
-                const double ir = 1.0 / q[0], ir2 = ir * ir;
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    const double ud = q[1 + c] * ir2;
-                    ux[c] = ir * U[(0 * NV + 1 + c) * S + g] - ud * U[(0 * NV) * S + g];
-                    uy[c] = ir * U[(1 * NV + 1 + c) * S + g] - ud * U[(1 * NV) * S + g];
-                    uz[c] = ir * U[(2 * NV + 1 + c) * S + g] - ud * U[(2 * NV) * S + g];
-                }
+            for (int c = 0; c < 3; ++c) {
+                const double ud = q[1 + c] * ir2;
+                ux[c] = ir * U[(0 * NV + 1 + c) * S + g] - ud * U[(0 * NV) * S + g];
+                uy[c] = ir * U[(1 * NV + 1 + c) * S + g] - ud * U[(1 * NV) * S + g];
+                uz[c] = ir * U[(2 * NV + 1 + c) * S + g] - ud * U[(2 * NV) * S + g];
             }
             const double a = uy[2] - uz[1], b = uz[0] - ux[2], c = ux[1] - uy[0];
             f = a * a + b * b + c * c;
@@ -466,22 +457,22 @@ struct hx3d_engine {
     int inviscid = 0;
     double dcsi = 0;
     hipStream_t stream = nullptr;
-    double *dQ = nullptr, *dG = nullptr, *dVgrad = nullptr, *dJa = nullptr;
-    // Gauss-Lobatto nodes, one order: the state's second copy (swapped with dQ by every update), the
+    double *dQ = nullptr, *dG = nullptr, *dJa = nullptr;
+    // One order: the state's second copy (Gauss-Lobatto nodes; swapped with dQ by every update), the
     // viscous values at the nodes (hxk::viscous_values), |curl u|^2 where a stage leaves its derivative (the
     // enstrophy monitor's), the filter widths of the element faces, the slots of the dt limits
     double *dQn = nullptr, *dVisc = nullptr, *dCurl = nullptr, *dEfdelta = nullptr;
     unsigned long long *dSlots = nullptr;
     double *dFe = nullptr, *dQDot = nullptr, *dEdelta = nullptr, *dFdelta = nullptr, *dWq = nullptr;
-    // Gauss nodes, one order: Q and gradient traces in element-face order, the neighbour table
-    double *dQtr = nullptr, *dGtr = nullptr;
+    // Gauss nodes, one order: the state's traces in element-face order, their second copy (swapped
+    // by every update), the viscous flux tensors at the element face nodes
+    double *dQtr = nullptr, *dQtn = nullptr, *dFvis = nullptr;
     int *dNbx = nullptr;
     hxg::GaussOps gops{};
     double *dJ = nullptr, *dFgeo = nullptr, *dEgeo = nullptr;
     double *dScal = nullptr, *dPart = nullptr, *dStage = nullptr, *dDtPart = nullptr;
     unsigned long long *dBits = nullptr;
     int *dNbr = nullptr, *dFlag = nullptr;
-    int4 *dFnode = nullptr;
     // mixed orders (p-anisotropic elements, mortar faces)
     bool mixed = false;
     bool t2x = false;     // uniform orders: the volume kernel forms t2 = n x t1 (see tangent2_is_cross)
@@ -532,7 +523,7 @@ struct hx3d_engine {
     bool use_graph = false;
     hipGraphExec_t step_graph = nullptr;
     double graph_cfl = 0, graph_dcfl = 0;
-    double *graph_Q = nullptr;   // the copy of the state the captured steps start from
+    double *graph_Q = nullptr;   // the copy of the state (Gauss: of its traces) the captured steps start from
     double ktime[4] = {0, 0, 0, 0};
     std::vector<hipEvent_t> evpool;   // timing: 4 events per stage of the last hx3d_advance
     std::string err;
@@ -657,8 +648,11 @@ void launch_volume(hx3d_engine *eng, double a_k, double c_k, int update, const D
     }
 }
 
-// Whether the stage kernels are k_grad and k_volume (one order, Gauss-Lobatto nodes)
-bool two_launch(const hx3d_engine *eng) { return !eng->mixed && !eng->gauss; }
+// Whether a stage is two launches (one order): the gradient kernel, then the volume kernel, which
+// forms the face fluxes, takes dt from the slots and swaps the two copies of the state (Gauss: of
+// its traces), current_copy
+bool two_launch(const hx3d_engine *eng) { return !eng->mixed; }
+double *current_copy(const hx3d_engine *eng) { return eng->gauss ? eng->dQtr : eng->dQ; }
 
 // One stage on the engine stream.  ev: NULL, or 4 events recorded around the launches
 // (timing only); like a failed launch, a failed record surfaces through hipGetLastError, which
@@ -667,6 +661,11 @@ template <int N>
 void stage_n(hx3d_engine *eng, double a_k, double c_k, int update, const DtArgs &dta, double *qdot,
              hipEvent_t *ev)
 {
+    auto face_events = [&]() {   // no face kernel of its own
+        if (!ev) return;
+        (void)hipEventRecord(ev[1], eng->stream);
+        (void)hipEventRecord(ev[2], eng->stream);
+    };
     if (eng->gauss) {
         // Gauss nodes: traces in element-face order (hxg)
         constexpr int TPB = hxg::gauss_tpb<N>();
@@ -674,25 +673,24 @@ void stage_n(hx3d_engine *eng, double a_k, double c_k, int update, const DtArgs 
         if (ev) (void)hipEventRecord(ev[0], eng->stream);
         if (!eng->ph.euler)
             hipLaunchKernelGGL((hxg::kg_grad<N>), dim3(nb), dim3(TPB), 0, eng->stream, eng->dQ, eng->dQtr, eng->dJa,
-                               eng->dJ, eng->dNbx, eng->dEgeo, eng->dGtr, eng->dVgrad, eng->K, eng->S, eng->ES,
-                               eng->ops, eng->gops, eng->ph, dta.lim);
-        if (ev) (void)hipEventRecord(ev[1], eng->stream);
-        const int nbf = grid_for((int)((eng->FS + hxk::FACE_TPB - 1) / hxk::FACE_TPB));
-        hipLaunchKernelGGL((hxg::kg_face<N>), dim3(nbf), dim3(hxk::FACE_TPB), 0, eng->stream, eng->dQtr, eng->dGtr,
-                           eng->dFgeo, eng->dFnode, eng->dFdelta, eng->dFe, eng->FS, eng->ES, eng->ph, dta.red);
-        if (ev) (void)hipEventRecord(ev[2], eng->stream);
-        hipLaunchKernelGGL((hxg::kg_volume<N>), dim3(nb), dim3(TPB), 0, eng->stream, eng->dQ, eng->dQtr, eng->dVgrad,
-                           eng->dJa, eng->dJ, eng->dEdelta, eng->dFe, eng->dG, qdot, a_k, c_k, update, dta, eng->K,
-                           eng->S, eng->ES, eng->ops, eng->gops, eng->ph);
+                               eng->dJ, eng->dNbx, eng->dEgeo, eng->dEdelta, eng->dEfdelta, eng->dVisc, eng->dFvis,
+                               qdot ? eng->dCurl : nullptr, eng->K, eng->S, eng->ES, eng->ops, eng->gops, eng->ph,
+                               dta.lim);
+        face_events();
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(nb), dim3(TPB), 0, eng->stream, eng->dQ, eng->dQtr, eng->dQtn, eng->dVisc,
+                               eng->dFvis, eng->dNbx, eng->dEgeo, eng->t2x ? 1 : 0, eng->dJa, eng->dJ, eng->dG, qdot, a_k,
+                               c_k, update, dta, eng->K, eng->S, eng->ES, eng->ops, eng->gops, eng->ph);
+        };
+        if (eng->ph.riemann == HX3D_RIEMANN_LXF) go(hxg::kg_volume<N, true>);
+        else go(hxg::kg_volume<N, false>);
+        if (update) std::swap(eng->dQtr, eng->dQtn);
         if (ev) (void)hipEventRecord(ev[3], eng->stream);
         return;
     }
     if (ev) (void)hipEventRecord(ev[0], eng->stream);
     if (!eng->ph.euler) launch_grad<N>(eng, dta.lim, qdot ? eng->dCurl : nullptr);
-    if (ev) {   // no face kernel of its own
-        (void)hipEventRecord(ev[1], eng->stream);
-        (void)hipEventRecord(ev[2], eng->stream);
-    }
+    face_events();
     launch_volume<N>(eng, a_k, c_k, update, dta, qdot);
     if (ev) (void)hipEventRecord(ev[3], eng->stream);
 }
@@ -1367,11 +1365,20 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
         idx[SLOT_V[slot]] = b;
         return (long)e * ne + idx[0] + n1 * (idx[1] + n1 * idx[2]);
     };
-    // per element face node x = (6e + slot) nf + a + (N+1) b: nbr[x] = 2 * (neighbour node) +
-    // (1 on the face's right side); per face node: (left node, right node, left x, right x)
-    std::vector<int> nbr((size_t)K * 6 * nf, -1);
-    std::vector<int4> fnode((size_t)FS);
-    std::vector<unsigned char> fslot(F);
+    // per element face node x = (6e + slot) nf + a + (N+1) b: nbr[x] = 2 * (neighbour's node) and
+    // nbx[x] = 2 * (neighbour's element face node), each + 1 on the face's right side; per face, the
+    // right side's element face nodes in the left side's order (permuted by the rotation)
+    std::vector<int> nbr(eng->gauss ? 0 : (size_t)K * 6 * nf), nbx((size_t)K * 6 * nf, -1);
+    auto right_nodes = [&](int f, long *xR, long *gR) {
+        const int eR = d->fElem[2 * f + 1], sR = d->fESide[2 * f + 1] - 1, rot = d->fRot[f];
+        for (int j = 0; j <= N; ++j)
+            for (int i = 0; i <= N; ++i) {
+                int ii, jj;
+                left_to_right(i, j, N, N, rot, ii, jj);
+                xR[i + n1 * j] = ((long)eR * 6 + sR) * nf + ii + n1 * jj;
+                if (gR) gR[i + n1 * j] = node_of(eR, sR, ii, jj);
+            }
+    };
     for (int f = 0; f < F; ++f) {
         const int eL = d->fElem[2 * f], eR = d->fElem[2 * f + 1];
         const int sL = d->fESide[2 * f] - 1, sR = d->fESide[2 * f + 1] - 1, rot = d->fRot[f];
@@ -1380,33 +1387,25 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
         if (d->faceID[6 * eL + sL] != f || d->faceSide[6 * eL + sL] != 1 || d->faceID[6 * eR + sR] != f ||
             d->faceSide[6 * eR + sR] != 2)
             return bail(eng->fail(HX3D_EINVAL, "face " + std::to_string(f) + ": inconsistent with element faceID/faceSide"));
-        fslot[f] = (unsigned char)sL;
-        for (int j = 0; j <= N; ++j)
-            for (int i = 0; i <= N; ++i) {
-                int ii, jj;
-                left_to_right(i, j, N, N, rot, ii, jj);
-                const long gL = node_of(eL, sL, i, j), gR = node_of(eR, sR, ii, jj);
-                const long q = (long)f * nf + i + n1 * j;
-                const long xL = ((long)eL * 6 + sL) * nf + i + n1 * j;
-                const long xR = ((long)eR * 6 + sR) * nf + ii + n1 * jj;
-                fnode[q] = make_int4((int)gL, (int)gR, (int)xL, (int)xR);
-                nbr[xL] = (int)(2 * gR);
-                nbr[xR] = (int)(2 * gL + 1);
+        long xR[64], gR[64];
+        right_nodes(f, xR, gR);
+        const long xL0 = ((long)eL * 6 + sL) * nf;
+        for (int x = 0; x < nf; ++x) {
+            nbx[xL0 + x] = (int)(2 * xR[x]);
+            nbx[xR[x]] = (int)(2 * (xL0 + x) + 1);
+            if (!eng->gauss) {
+                nbr[xL0 + x] = (int)(2 * gR[x]);
+                nbr[xR[x]] = (int)(2 * node_of(eL, sL, x % n1, x / n1) + 1);
             }
+        }
     }
-    for (size_t x = 0; x < nbr.size(); ++x)
-        if (nbr[x] < 0) return bail(eng->fail(HX3D_EINVAL, "an element face node has no neighbour"));
-    // 2 * (the neighbour's matching element face node) + (1 on the face's right side)
-    std::vector<int> nbx(nbr.size(), 0);
-    for (long q = 0; q < FS; ++q) {
-        nbx[fnode[q].z] = 2 * fnode[q].w;
-        nbx[fnode[q].w] = 2 * fnode[q].z + 1;
-    }
+    for (size_t x = 0; x < nbx.size(); ++x)
+        if (nbx[x] < 0) return bail(eng->fail(HX3D_EINVAL, "an element face node has no neighbour"));
     if (!offsets_fit(S, ES, FS))
         return bail(eng->fail(HX3D_EUNSUPPORTED, "mesh too large: more than 2^29 - 1 nodes (or face nodes) per array"));
     // geometry SoA, J, 1/J, quadrature weights, LES filter widths, face frames
     std::vector<double> ja((size_t)9 * S, 0.0), jj((size_t)S, 1.0), wq((size_t)S, 0.0),
-        edelta(K), fdelta(F), fgeo, egeo, efdelta((size_t)6 * K);
+        edelta(K), efdelta((size_t)6 * K);
     double xg[8], wg[8];
     hxs::nodes_of(eng->gauss, N, xg, wg);
     for (long g = 0; g < nodes; ++g) {
@@ -1425,81 +1424,96 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
     // (ConstructMappedGeometryFace, MappedGeometry.f90:482-760) and a fixed orthonormal
     // completion t1, t2 of n (the Riemann fluxes do not depend on the tangent choice).
     // Stored in element-face order, the left element's frame on both sides: n and |Ja|, for the
-    // volume kernel with Lax-Friedrichs t1, and t2 unless it is formed as n x t1 (tangent2_is_cross);
-    // Gauss nodes also per face node.
-    const bool lxf = d->riemann == HX3D_RIEMANN_LXF && !eng->gauss;
-    eng->t2x = lxf;
-    egeo.resize((size_t)(lxf ? 10 : 4) * ES, 0.0);
-    if (eng->gauss) fgeo.resize((size_t)10 * FS);
+    // volume kernel with Lax-Friedrichs t1, and t2 unless it is formed as n x t1 (tangent2_is_cross,
+    // looked at face by face: t2's planes are filled in a second sweep where one is not).
+    const bool lxf = d->riemann == HX3D_RIEMANN_LXF;
     const bool have_fg = d->fNormal && d->fT1 && d->fT2 && d->fJac;
     if (!have_fg && (d->fNormal || d->fT1 || d->fT2 || d->fJac))
         return bail(eng->fail(HX3D_EINVAL, "descriptor: give all four face geometry arrays or none"));
-    for (int f = 0; f < F; ++f) {
-        const int sL = fslot[f];
-        const int dax = SLOT_AXIS[sL];
+    // the frame of face f, planes n (0-2), |Ja| (3), t1 (4-6), t2 (7-9) of nf nodes
+    auto face_frame = [&](int f, double (*fr)[64]) {
+        const int eL = d->fElem[2 * f], sL = d->fESide[2 * f] - 1, dax = SLOT_AXIS[sL];
         const double sg = SLOT_PLUS[sL] ? 1.0 : -1.0;
-        double surf = 0.0;
-        for (int j = 0; j <= N; ++j)
-            for (int i = 0; i <= N; ++i) {
-                const long q = (long)f * nf + i + n1 * j;
-                double nr[3], t1[3], t2[3], jac;
-                if (have_fg) {
-                    for (int c = 0; c < 3; ++c) { nr[c] = d->fNormal[3 * q + c]; t1[c] = d->fT1[3 * q + c]; t2[c] = d->fT2[3 * q + c]; }
-                    jac = d->fJac[q];
-                } else {
-                    const long g = fnode[q].x;
-                    for (int c = 0; c < 3; ++c) nr[c] = sg * d->Ja[9 * g + 3 * dax + c];
-                    jac = std::sqrt(nr[0] * nr[0] + nr[1] * nr[1] + nr[2] * nr[2]);
-                    for (int c = 0; c < 3; ++c) nr[c] /= jac;
-                    // t1 = e_m - (e_m . n) n for the axis e_m least aligned with n, normalised
-                    int m = 0;
-                    for (int c = 1; c < 3; ++c) if (std::fabs(nr[c]) < std::fabs(nr[m])) m = c;
-                    for (int c = 0; c < 3; ++c) t1[c] = (c == m ? 1.0 : 0.0) - nr[m] * nr[c];
-                    const double tn = std::sqrt(t1[0] * t1[0] + t1[1] * t1[1] + t1[2] * t1[2]);
-                    for (int c = 0; c < 3; ++c) t1[c] /= tn;
-                    t2[0] = nr[1] * t1[2] - nr[2] * t1[1];
-                    t2[1] = nr[2] * t1[0] - nr[0] * t1[2];
-                    t2[2] = nr[0] * t1[1] - nr[1] * t1[0];
-                }
-                const double frame[10] = {nr[0], nr[1], nr[2], jac, t1[0], t1[1], t1[2], t2[0], t2[1], t2[2]};
-                for (int c = 0; c < (lxf ? 10 : 4); ++c)
-                    egeo[(size_t)c * ES + fnode[q].z] = egeo[(size_t)c * ES + fnode[q].w] = frame[c];
-                if (lxf && eng->t2x) eng->t2x = tangent2_is_cross(nr, t1, t2);
-                if (eng->gauss) {
-                    for (int c = 0; c < 3; ++c) {
-                        fgeo[(size_t)c * FS + q] = nr[c];
-                        fgeo[(size_t)(3 + c) * FS + q] = t1[c];
-                        fgeo[(size_t)(6 + c) * FS + q] = t2[c];
-                    }
-                    fgeo[(size_t)9 * FS + q] = jac;
-                }
-                surf += wg[i] * wg[j] * jac;
+        for (int x = 0; x < nf; ++x) {
+            const long q = (long)f * nf + x;
+            double nr[3], t1[3], t2[3], jac;
+            if (have_fg) {
+                for (int c = 0; c < 3; ++c) { nr[c] = d->fNormal[3 * q + c]; t1[c] = d->fT1[3 * q + c]; t2[c] = d->fT2[3 * q + c]; }
+                jac = d->fJac[q];
+            } else {
+                const long g = node_of(eL, sL, x % n1, x / n1);
+                for (int c = 0; c < 3; ++c) nr[c] = sg * d->Ja[9 * g + 3 * dax + c];
+                jac = std::sqrt(nr[0] * nr[0] + nr[1] * nr[1] + nr[2] * nr[2]);
+                for (int c = 0; c < 3; ++c) nr[c] /= jac;
+                // t1 = e_m - (e_m . n) n for the axis e_m least aligned with n, normalised
+                int m = 0;
+                for (int c = 1; c < 3; ++c) if (std::fabs(nr[c]) < std::fabs(nr[m])) m = c;
+                for (int c = 0; c < 3; ++c) t1[c] = (c == m ? 1.0 : 0.0) - nr[m] * nr[c];
+                const double tn = std::sqrt(t1[0] * t1[0] + t1[1] * t1[1] + t1[2] * t1[2]);
+                for (int c = 0; c < 3; ++c) t1[c] /= tn;
+                t2[0] = nr[1] * t1[2] - nr[2] * t1[1];
+                t2[1] = nr[2] * t1[0] - nr[0] * t1[2];
+                t2[2] = nr[0] * t1[1] - nr[1] * t1[0];
             }
-        fdelta[f] = std::sqrt(surf / nf);   // SD.f90:1378
+            for (int c = 0; c < 3; ++c) { fr[c][x] = nr[c]; fr[4 + c][x] = t1[c]; fr[7 + c][x] = t2[c]; }
+            fr[3][x] = jac;
+            if (lxf && eng->t2x) eng->t2x = tangent2_is_cross(nr, t1, t2);
+        }
+    };
+    // planes c0..c1-1 of a face's frame to both sides, a run of nodes at a time
+    std::unique_ptr<double[]> egeo(new double[(size_t)(lxf ? 10 : 4) * ES]);   // pages touched as planes are filled
+    auto put_frame = [&](int f, const double (*fr)[64], int c0, int c1) {
+        long xR[64];
+        right_nodes(f, xR, nullptr);
+        const long xL0 = ((long)d->fElem[2 * f] * 6 + d->fESide[2 * f] - 1) * nf;
+        for (int c = c0; c < c1; ++c) {
+            double *eg = egeo.get() + (size_t)c * ES;
+            for (int x = 0; x < nf; ++x) eg[xL0 + x] = fr[c][x];
+            for (int x = 0; x < nf; ++x) eg[xR[x]] = fr[c][x];
+        }
+    };
+    eng->t2x = lxf;
+    double fr[10][64];
+    for (int f = 0; f < F; ++f) {
+        face_frame(f, fr);
+        put_frame(f, fr, 0, lxf ? 7 : 4);
+        double surf = 0.0;
+        for (int x = 0; x < nf; ++x) surf += wg[x % n1] * wg[x / n1] * fr[3][x];
+        // SD.f90:1378, at both elements' slots of the face
+        const double fd = std::sqrt(surf / nf);
+        efdelta[6 * (long)d->fElem[2 * f] + d->fESide[2 * f] - 1] = fd;
+        efdelta[6 * (long)d->fElem[2 * f + 1] + d->fESide[2 * f + 1] - 1] = fd;
     }
-    if (eng->t2x) egeo.resize((size_t)7 * ES);
-    for (long x = 0; x < 6L * K; ++x) efdelta[x] = fdelta[d->faceID[x]];
+    const int gplanes = !lxf ? 4 : eng->t2x ? 7 : 10;
+    if (gplanes == 10)
+        for (int f = 0; f < F; ++f) {
+            face_frame(f, fr);
+            put_frame(f, fr, 7, 10);
+        }
+    for (int c = 0; c < gplanes; ++c)   // the padding past the last face node
+        for (long x = (long)K * 6 * nf; x < ES; ++x) egeo[(size_t)c * ES + x] = 0.0;
     // ---- device -------------------------------------------------------------------
     int rc;
     if ((rc = dalloc(eng, &eng->dQ, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dG, (size_t)NV * S)) ||
         (rc = dalloc(eng, &eng->dJa, (size_t)9 * S)) || (rc = dalloc(eng, &eng->dWq, (size_t)S)) ||
-        (rc = dalloc(eng, &eng->dJ, (size_t)S)) || (rc = dalloc(eng, &eng->dEgeo, egeo.size())) ||
+        (rc = dalloc(eng, &eng->dJ, (size_t)S)) || (rc = dalloc(eng, &eng->dEgeo, (size_t)gplanes * ES)) ||
         (rc = dalloc(eng, &eng->dQDot, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dEdelta, (size_t)K)) ||
         (rc = dalloc(eng, &eng->dScal, 4)) || (rc = dalloc(eng, &eng->dPart, (size_t)NV * ((S + 255) / 256 + 1))) ||
         (rc = dalloc(eng, &eng->dDtPart, (size_t)2 * (std::max((long)K, (S + 255) / 256) + 64))) ||
         (rc = dalloc(eng, &eng->dStage, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dBits, 2 * DT_SLOTS)) ||
         (rc = dalloc(eng, &eng->dFlag, 2)) || (rc = dalloc(eng, &eng->dNbx, nbx.size())))
         return bail(rc);
-    if (eng->gauss) {
-        if ((rc = dalloc(eng, &eng->dVgrad, (size_t)(eng->ph.les ? 13 : 12) * S)) ||
-            (rc = dalloc(eng, &eng->dFe, (size_t)NV * ES)) || (rc = dalloc(eng, &eng->dFgeo, (size_t)10 * FS)) ||
-            (rc = dalloc(eng, &eng->dFdelta, (size_t)F)) || (rc = dalloc(eng, &eng->dFnode, fnode.size())) ||
-            (rc = dalloc(eng, &eng->dQtr, (size_t)NV * ES)) || (rc = dalloc(eng, &eng->dGtr, (size_t)15 * ES)))
-            return bail(rc);
-    } else if ((rc = dalloc(eng, &eng->dQn, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dVisc, (size_t)hxk::viscous_values(eng->ph.les) * S)) ||
-               (rc = dalloc(eng, &eng->dCurl, (size_t)S)) || (rc = dalloc(eng, &eng->dEfdelta, efdelta.size())) ||
-               (rc = dalloc(eng, &eng->dNbr, nbr.size())) || (rc = alloc_slots(eng, 1)))
+    if ((rc = dalloc(eng, &eng->dVisc, (size_t)(eng->gauss ? hxk::NVF : hxk::viscous_values(eng->ph.les)) * S)) ||
+        (rc = dalloc(eng, &eng->dCurl, (size_t)S)) || (rc = dalloc(eng, &eng->dEfdelta, efdelta.size())) ||
+        (rc = alloc_slots(eng, 1)))
         return bail(rc);
+    if (eng->gauss) {
+        if ((rc = dalloc(eng, &eng->dQtr, (size_t)NV * ES)) || (rc = dalloc(eng, &eng->dQtn, (size_t)NV * ES)) ||
+            (rc = dalloc(eng, &eng->dFvis, (size_t)hxk::NVF * ES)))
+            return bail(rc);
+    } else if ((rc = dalloc(eng, &eng->dQn, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dNbr, nbr.size()))) {
+        return bail(rc);
+    }
     if (hipStreamCreateWithFlags(&eng->stream, hipStreamNonBlocking) != hipSuccess)
         return bail(eng->fail(HX3D_EDEVICE, "hipStreamCreate failed"));
     auto up = [&](void *dst, const void *src, size_t bytes) {
@@ -1507,23 +1521,18 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
     };
     if (!up(eng->dJa, ja.data(), ja.size() * 8) || !up(eng->dJ, jj.data(), jj.size() * 8) ||
         !up(eng->dWq, wq.data(), wq.size() * 8) || !up(eng->dEdelta, edelta.data(), edelta.size() * 8) ||
-        !up(eng->dEgeo, egeo.data(), egeo.size() * 8) || !up(eng->dNbx, nbx.data(), nbx.size() * 4) ||
-        (eng->gauss && (!up(eng->dFgeo, fgeo.data(), fgeo.size() * 8) || !up(eng->dFdelta, fdelta.data(), fdelta.size() * 8) ||
-                        !up(eng->dFnode, fnode.data(), fnode.size() * 16))) ||
-        (!eng->gauss && (!up(eng->dNbr, nbr.data(), nbr.size() * 4) || !up(eng->dEfdelta, efdelta.data(), efdelta.size() * 8))))
+        !up(eng->dEgeo, egeo.get(), (size_t)gplanes * ES * 8) || !up(eng->dNbx, nbx.data(), nbx.size() * 4) ||
+        !up(eng->dEfdelta, efdelta.data(), efdelta.size() * 8) ||
+        (!eng->gauss && !up(eng->dNbr, nbr.data(), nbr.size() * 4)))
         return bail(eng->fail(HX3D_EDEVICE, "upload failed"));
     // zero state, RK register and time
     const long nb = (NV * S + 255) / 256;
     hipLaunchKernelGGL(k_fill, dim3(nb), dim3(256), 0, eng->stream, eng->dQ, (long)NV * S, 0.0);
     hipLaunchKernelGGL(k_fill, dim3(nb), dim3(256), 0, eng->stream, eng->dG, (long)NV * S, 0.0);
     hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, eng->stream, eng->dScal, 4L, 0.0);
-    if (eng->gauss) {
-        hipLaunchKernelGGL(k_fill, dim3((15 * ES + 255) / 256), dim3(256), 0, eng->stream, eng->dGtr, 15L * ES, 0.0);
-        refresh_traces(eng);
-    } else {
-        hipLaunchKernelGGL(k_fill, dim3(nb), dim3(256), 0, eng->stream, eng->dQn, (long)NV * S, 0.0);
-        init_slots(eng, 1);
-    }
+    if (eng->gauss) refresh_traces(eng);
+    else hipLaunchKernelGGL(k_fill, dim3(nb), dim3(256), 0, eng->stream, eng->dQn, (long)NV * S, 0.0);
+    init_slots(eng, 1);
     if (int rc2 = init_flags(eng)) return bail(rc2);
     if (hipStreamSynchronize(eng->stream) != hipSuccess)
         return bail(eng->fail(HX3D_EDEVICE, "initialisation failed"));
@@ -1624,7 +1633,7 @@ int hx3d_engine_create_multi(const hx3d_case_desc *descs, int ncases, hx3d_engin
         cc[c].mu_to_kappa = 1.0 / (eng->ph.gm1 * M2 * d.prandtl);
         cc[c].les_c = d.les_c;
     }
-    if ((long)eng->F * nf / hxk::FACE_TPB + 1 < ncases)
+    if ((long)eng->F * nf / 256 + 1 < ncases)
         return eng->fail(HX3D_EUNSUPPORTED, "too many cases of too few face nodes");
     // per-case replacements of the one-case dt slots, flags and time
     (void)hipStreamSynchronize(eng->stream);
@@ -1678,12 +1687,12 @@ int hx3d_engine_destroy(hx3d_engine *eng)
     if (!eng) return HX3D_OK;
     // teardown: nothing is left to report an error to, so the calls' statuses are not checked
     if (eng->stream) (void)hipStreamSynchronize(eng->stream);
-    void *ptrs[] = {eng->dQ, eng->dG, eng->dVgrad, eng->dJa, eng->dJ, eng->dFgeo, eng->dEgeo, eng->dFe,
+    void *ptrs[] = {eng->dQ, eng->dG, eng->dJa, eng->dJ, eng->dFgeo, eng->dEgeo, eng->dFe,
                     eng->dQDot, eng->dEdelta, eng->dFdelta, eng->dWq, eng->dScal, eng->dPart, eng->dStage,
-                    eng->dBits, eng->dNbr, eng->dFlag, eng->dFnode, eng->dN3, eng->dEfoff,
+                    eng->dBits, eng->dNbr, eng->dFlag, eng->dN3, eng->dEfoff,
                     eng->dEofn, eng->dOff, eng->dFaces, eng->dSched, eng->dOpsAll, eng->dU, eng->dLift, eng->dDtPart, eng->dTmap,
                     eng->dBlocks, eng->dCC, eng->dActive, eng->dTimeM,
-                    eng->dQtr, eng->dGtr, eng->dNbx, eng->dQn, eng->dVisc, eng->dCurl, eng->dEfdelta, eng->dSlots};
+                    eng->dQtr, eng->dQtn, eng->dFvis, eng->dNbx, eng->dQn, eng->dVisc, eng->dCurl, eng->dEfdelta, eng->dSlots};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     for (auto &e : eng->evpool) (void)hipEventDestroy(e);
@@ -1938,7 +1947,7 @@ int hx3d_advance(hx3d_engine *eng, int nsteps, double cfl, double dcfl, double *
             hipGraph_t g = nullptr;
             HIPCHK(hipStreamBeginCapture(eng->stream, hipStreamCaptureModeThreadLocal));
             eng->capturing = true;
-            eng->graph_Q = eng->dQ;
+            eng->graph_Q = current_copy(eng);
             for (int s = 0; s < per; ++s) issue_step(nullptr, nullptr);
             eng->capturing = false;
             const hipError_t ce = hipStreamEndCapture(eng->stream, &g);
@@ -1955,11 +1964,11 @@ int hx3d_advance(hx3d_engine *eng, int nsteps, double cfl, double dcfl, double *
         // the last step is issued directly: it also leaves its last stage's time derivative; before
         // it the replays, from the copy of the state they start from, and what is left over
         int left = nsteps - 1;
-        if (left >= 1 + per && eng->dQ != eng->graph_Q) {
+        if (left >= 1 + per && per == 2 && current_copy(eng) != eng->graph_Q) {
             issue_step(nullptr, nullptr);
             --left;
         }
-        for (; left >= per && eng->dQ == eng->graph_Q; left -= per) HIPCHK(hipGraphLaunch(eng->step_graph, eng->stream));
+        for (; left >= per && (per == 1 || current_copy(eng) == eng->graph_Q); left -= per) HIPCHK(hipGraphLaunch(eng->step_graph, eng->stream));
         for (; left > 0; --left) issue_step(nullptr, nullptr);
         issue_step(nullptr, eng->dQDot);
     }
@@ -2052,7 +2061,7 @@ int hx3d_volume_monitor(hx3d_engine *eng, int kind, double *value)
     }
     const int nb = (int)((eng->nodes + 255) / 256);
     hipLaunchKernelGGL(k_monitor, dim3(nb), dim3(256), 0, eng->stream, kind, eng->dQ, eng->dQDot,
-                       two_launch(eng) ? eng->dCurl : nullptr, eng->mixed ? nullptr : eng->dVgrad, eng->dU, eng->dJ, eng->dWq, eng->nodes, eng->S, eng->ph,
+                       eng->mixed ? nullptr : eng->dCurl, eng->dU, eng->dJ, eng->dWq, eng->nodes, eng->S, eng->ph,
                        eng->dPart);
     hipLaunchKernelGGL(k_finish_sum2, dim3(1), dim3(FINISH_TPB), 0, eng->stream, eng->dPart, nb, eng->dStage);
     double r[2];

@@ -136,9 +136,8 @@ __device__ __forceinline__ void block_elements(const Multi &mc, int lb, int K, i
 }
 
 // MaxTimeStep of the state a stage starts from, accumulated by the stage's gradient kernel.
-// Mixed orders and Gauss nodes (part; null: not this stage): block minima of the convective and
-// viscous limits to part[2*block + 0/1], reduced by the face kernel that follows (DtReduce).
-// Gauss-Lobatto nodes of one order (slots; null: not this stage): each block's minima by atomicMin
+// Mixed orders (part; null: not this stage): block minima of the convective and viscous limits to
+// part[2*block + 0/1], reduced by the face kernel that follows (DtReduce).  One order (slots; null: not this stage): each block's minima by atomicMin
 // into one of the case's DT_FAN slots, from which every block of the volume kernel that follows
 // takes the minimum.  The minimum of doubles does not depend on the order, and the limits are
 // positive or NaN, whose bit patterns order like the numbers (NaN above +inf, so it is passed over
@@ -343,17 +342,14 @@ k_grad(const double *__restrict__ Q, const double *__restrict__ Ja, const double
     if (dtl.slots) block_min_slot(tc, tv, dtl.slots, t, cs, lb);
 }
 
-// dtred: (partials, count, slot) of the step's dt limits, reduced by block 0 of the mixed-order and
-// Gauss face kernels
+// dtred: (partials, count, slot) of the step's dt limits, reduced by block 0 of the mixed-order face
+// kernels
 __device__ __forceinline__ void reduce_dt_partials(const double *part, int n, unsigned long long *bits, int t);
 struct DtReduce {
     const double *part;
     int n;
     unsigned long long *bits;
 };
-
-// threads (face nodes) per block of the Gauss face kernel
-constexpr int FACE_TPB = 256;
 
 // ------------------------------------------------------------------------------------
 // k_volume: per element, the face fluxes of its six faces (computeElementInterfaceFlux,
@@ -365,8 +361,8 @@ struct DtArgs {
     double *time;                   // t += dt by one thread (or null)
     int *nan;                       // set to 1 when an updated state value is NaN (or null)
     DtLimits lim;                   // consumed by the stage's gradient kernel
-    DtReduce red;                   // consumed by the stage's face kernel (mixed orders, Gauss nodes)
-    // Gauss-Lobatto nodes of one order: the first stage takes dt from the limits' slots (not from
+    DtReduce red;                   // consumed by the stage's face kernel (mixed orders)
+    // One order: the first stage takes dt from the limits' slots (not from
     // `in`) and leaves it in `in`'s place, fin, for the later stages; the second stage empties the
     // slots for the next step (each null in the other stages)
     const unsigned long long *slots;
@@ -436,6 +432,35 @@ __device__ __forceinline__ void reduce_dt_partials(const double *part, int n, un
         for (int w = 1; w < nw; ++w) { a = fmin(a, sm[0][w]); b = fmin(b, sm[1][w]); }
         bits[0] = (unsigned long long)__double_as_longlong(a);
         bits[1] = (unsigned long long)__double_as_longlong(b);
+    }
+}
+
+// This step's dt limits in a block of a volume kernel, by its first wave: load_dt asks for the
+// case's slots (or the reduced pair), reduce_dt takes their minimum to sDt (visible after the next
+// barrier); the case's first block leaves the reduced pair for the later stages, or empties the
+// slots (see DtArgs).
+__device__ __forceinline__ void load_dt(const DtArgs &dta, int cs, int t, double &a, double &b)
+{
+    const unsigned long long *s = dta.slots ? dta.slots + (long)(cs * DT_FAN + t % DT_FAN) * DT_LINE : dta.in + 2 * cs;
+    a = bits_to_double(s[0]);
+    b = bits_to_double(s[1]);
+}
+__device__ __forceinline__ void reduce_dt(const DtArgs &dta, int cs, bool first, int t, double a, double b, double &sDt)
+{
+    for (int o = 32; o > 0; o >>= 1) {
+        a = fmin(a, __shfl_xor(a, o, 64));
+        b = fmin(b, __shfl_xor(b, o, 64));
+    }
+    if (t == 0) {
+        sDt = fmin(a, b);
+        if (first && dta.slots) {
+            dta.fin[2 * cs] = (unsigned long long)__double_as_longlong(a);
+            dta.fin[2 * cs + 1] = (unsigned long long)__double_as_longlong(b);
+        }
+    }
+    if (first && dta.empty && t < DT_FAN) {
+        unsigned long long *sl = dta.empty + (long)(cs * DT_FAN + t) * DT_LINE;
+        sl[0] = sl[1] = (unsigned long long)__double_as_longlong(INFINITY);
     }
 }
 
@@ -580,17 +605,8 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
 #pragma unroll
         for (int c = 0; c < NVT; ++c) vt[c] = ldg(visc + c * S, gc);
     }
-    double dtl0 = INFINITY, dtl1 = INFINITY;   // this step's dt limits (first wave)
-    if (update && t < 64) {
-        if (dta.slots) {
-            const unsigned long long *sl = dta.slots + (long)(cs * DT_FAN + t % DT_FAN) * DT_LINE;
-            dtl0 = bits_to_double(sl[0]);
-            dtl1 = bits_to_double(sl[1]);
-        } else {
-            dtl0 = bits_to_double(dta.in[2 * cs]);
-            dtl1 = bits_to_double(dta.in[2 * cs + 1]);
-        }
-    }
+    double dtl0, dtl1;   // this step's dt limits (first wave)
+    if (update && t < 64) load_dt(dta, cs, t, dtl0, dtl1);
     if (t < n1 * n1) {
         sHat[t] = hop;
         sSharp[t] = sop;
@@ -706,23 +722,7 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
             }
         }
     }
-    if (update && t < 64) {
-        for (int o = 32; o > 0; o >>= 1) {
-            dtl0 = fmin(dtl0, __shfl_xor(dtl0, o, 64));
-            dtl1 = fmin(dtl1, __shfl_xor(dtl1, o, 64));
-        }
-        if (t == 0) {
-            sDt = fmin(dtl0, dtl1);
-            if (first && dta.slots) {
-                dta.fin[2 * cs] = (unsigned long long)__double_as_longlong(dtl0);
-                dta.fin[2 * cs + 1] = (unsigned long long)__double_as_longlong(dtl1);
-            }
-        }
-        if (first && dta.empty && t < DT_FAN) {
-            unsigned long long *sl = dta.empty + (long)(cs * DT_FAN + t) * DT_LINE;
-            sl[0] = sl[1] = (unsigned long long)__double_as_longlong(INFINITY);
-        }
-    }
+    if (update && t < 64) reduce_dt(dta, cs, first, t, dtl0, dtl1, sDt);
     __syncthreads();
     // The RK register.  The first RK stage (a_k = 0) does not read it: the reference's 0 G + QDot is
     // QDot up to the sign of an exact zero, which no state value sees (Q + c dt (+-0) = Q); every

@@ -1,11 +1,12 @@
-"""The two-launch stage of Gauss-Lobatto cases of one order: every pairing of Riemann solver and
-LES model (the volume kernel's template flags) at orders with whole and remainder element blocks,
-against the oracle; and the two copies of the state through odd and even step counts."""
+"""The two-launch stage of cases of one order: every pairing of Riemann solver and LES model (the
+volume kernel's template flags) at orders with whole and remainder element blocks, and Gauss nodes
+with Lax-Friedrichs, against the oracle; and the two copies of the state through odd and even step
+counts."""
 import numpy as np
 import pytest
 
 import pyoracle as po
-from horses3d_amd import mesh
+from horses3d_amd import mesh, specmesh
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-12   # the parity bar: normwise per variable
@@ -38,14 +39,47 @@ def test_volume_kernel_variants_match_oracle(N, inviscid, averaging, riemann, le
     eng.close()
 
 
-@pytest.mark.parametrize("euler", [False, True])
-def test_state_copies_through_odd_and_even_steps(euler):
-    """A step of three stages ends in the other copy of the state: any split of the steps, with
-    host reads, derivatives and captured steps between, gives the same bits."""
+def gauss_box(n, N, tmp_path):
+    """An n^3 curvilinear box from the front end on Gauss nodes, with the oracle's face tables."""
+    path = str(tmp_path / "box.mesh")
+    specmesh.write_specmesh(path, n, 0.1, mesh.box_phases(30 + N), bface_order=max(4, N))
+    from horses3d_amd.engine import read_specmesh
+    case = read_specmesh(path, N=N, periodic=dict(specmesh.PERIODIC_PAIRS), nodes="gauss")
+    case["fNf"] = np.full((case["F"], 2), N, np.int32)
+    case["foff"] = np.arange(case["F"] + 1, dtype=np.int64) * (N + 1) ** 2
+    return case
+
+
+@pytest.mark.parametrize("tangents", ["cross product", "turned"])
+@pytest.mark.parametrize("N,les", [(1, None), (3, "wale"), (4, None), (6, "smagorinsky")])
+def test_gauss_lax_friedrichs_matches_oracle(N, les, tangents, tmp_path):
+    """Gauss nodes with Lax-Friedrichs face fluxes (one to three rounds of face nodes per thread),
+    the second tangent formed in the kernel or, where it is not n x t1, read."""
     from horses3d_amd.engine import Engine
-    case = mesh.periodic_box(3, 3, amplitude=0.1, phase_seed=4)
+    case = gauss_box(2, N, tmp_path)
+    if tangents == "turned":   # the opposite second tangent: another frame, the same flux
+        case["t2"] = -case["t2"]
+    kw = dict(mach=0.3, reynolds=700.0, riemann="lxf", les=les, nodes="gauss")
+    Q0 = mesh.taylor_green(case, 0.3, noise=1e-2, seed=N)
+    ora = po.Oracle(case, po.make_params(0.3, 700.0, riemann="lxf", les=les, nodes="gauss"))
+    eng = Engine(case, **kw)
+    eng.set_state(Q0)
+    err = po.normwise_error(eng.qdot(), ora.qdot(Q0))
+    print(N, les, tangents, err, flush=True)
+    assert err.max() <= TOL
+    eng.close()
+
+
+@pytest.mark.parametrize("kind", ["gauss-lobatto", "euler", "gauss"])
+def test_state_copies_through_odd_and_even_steps(kind, tmp_path):
+    """A step of three stages ends in the other copy of the state (Gauss nodes: of its traces): any
+    split of the steps, with host reads, derivatives and captured steps between, gives the same
+    bits."""
+    from horses3d_amd.engine import Engine
+    case = gauss_box(3, 3, tmp_path) if kind == "gauss" else mesh.periodic_box(3, 3, amplitude=0.1, phase_seed=4)
     Q0 = mesh.taylor_green(case, 0.2, noise=1e-3, seed=9)
-    kw = dict(mach=0.2, reynolds=800.0, riemann="roe", euler=euler)
+    kw = dict(mach=0.2, reynolds=800.0, riemann="roe", euler=kind == "euler",
+              nodes="gauss" if kind == "gauss" else "gauss-lobatto")
     ref = Engine(case, **kw)
     ref.set_state(Q0)
     t = ref.advance(17, 0.4, 0.4, t=0.0)
