@@ -478,10 +478,10 @@ struct hx3d_engine {
     bool t2x = false;     // uniform orders: the volume kernel forms t2 = n x t1 (see tangent2_is_cross)
     bool gauss = false;   // Gauss nodes (one order: hxg kernels; per-element orders: the mixed path's)
     long FSm = 0;
-    int *dN3 = nullptr, *dEfoff = nullptr, *dEofn = nullptr;
+    int *dN3 = nullptr, *dEofn = nullptr;
     long *dOff = nullptr;
     hxm::FaceRec *dFaces = nullptr;
-    int2 *dSched = nullptr;   // the face kernels' waves (hxm::face_lane): one face, or two of one shape
+    int4 *dSched = nullptr;   // the face kernels' waves (hxm::face_lane): one face, or two of one shape
     int nwaves = 0;
     hxm::OpsAll *dOpsAll = nullptr;
     double *dU = nullptr, *dLift = nullptr;
@@ -756,14 +756,14 @@ void launch_mvolume(hx3d_engine *eng, double a_k, double c_k, int update, const 
     if (eng->ntiles_s)
         hipLaunchKernelGGL((hxm::km_volume<FORM, GAUSS, hxm::TILE_SMALL>), dim3(eng->grid_mvol_s), dim3(hxm::TILE_SMALL),
                            mvolume_lds<FORM>(hxm::TILE_SMALL), eng->stream, eng->dTmap, eng->ntiles_s, eng->dQ, eng->dU,
-                           eng->dEfoff, eng->dJa, eng->dJ, eng->dEdelta, eng->dFe, eng->dOpsAll, eng->dG, qdot, a_k, c_k,
+                           eng->dJa, eng->dJ, eng->dEdelta, eng->dFe, eng->dOpsAll, eng->dG, qdot, a_k, c_k,
                            update, dta, eng->S, eng->ES, eng->ph);
     if (eng->ntiles_b) {
         DtArgs db = dta;   // the time advances once per stage: in the first launch
         if (eng->ntiles_s) db.time = nullptr;
         hipLaunchKernelGGL((hxm::km_volume<FORM, GAUSS, hxm::TILE>), dim3(eng->grid_mvol_b), dim3(hxm::TILE),
                            mvolume_lds<FORM>(hxm::TILE), eng->stream, eng->dTmap + eng->map_big, eng->ntiles_b, eng->dQ,
-                           eng->dU, eng->dEfoff, eng->dJa, eng->dJ, eng->dEdelta, eng->dFe, eng->dOpsAll, eng->dG, qdot,
+                           eng->dU, eng->dJa, eng->dJ, eng->dEdelta, eng->dFe, eng->dOpsAll, eng->dG, qdot,
                            a_k, c_k, update, db, eng->S, eng->ES, eng->ph);
     }
 }
@@ -777,23 +777,23 @@ void stage_mixed_nodes(hx3d_engine *eng, double a_k, double c_k, int update, con
     hxk::DtLimits lim = dta.lim;
     if (!eng->ph.euler) {
         hipLaunchKernelGGL(hxm::km_face_grad<GAUSS>, dim3(grid_for(eng->nwaves)), dim3(64), 0, eng->stream, eng->dQ,
-                           eng->dN3, eng->dOff, eng->dEfoff, eng->dFaces, eng->dSched, eng->dFgeo, eng->dOpsAll,
-                           eng->dLift, eng->nwaves, eng->S, eng->ES, eng->FSm);
+                           eng->dFaces, eng->dSched, eng->dFgeo, eng->dOpsAll, eng->dLift, eng->nwaves, eng->S, eng->ES, eng->FSm);
         // dt partials: the small tiles' blocks first, then the large tiles'
         if (eng->ntiles_s)
             hipLaunchKernelGGL((hxm::km_grad<GAUSS, hxm::TILE_SMALL>), dim3(eng->grid_mgrad_s), dim3(hxm::TILE_SMALL),
-                               mgrad_lds(hxm::TILE_SMALL), eng->stream, eng->dTmap, eng->ntiles_s, eng->dQ, eng->dEfoff,
+                               mgrad_lds(hxm::TILE_SMALL), eng->stream, eng->dTmap, eng->ntiles_s, eng->dQ,
                                eng->dJa, eng->dJ, eng->dLift, eng->dOpsAll, eng->dU, eng->S, eng->ES, eng->ph, lim, 0);
         if (eng->ntiles_b)
             hipLaunchKernelGGL((hxm::km_grad<GAUSS, hxm::TILE>), dim3(eng->grid_mgrad_b), dim3(hxm::TILE),
                                mgrad_lds(hxm::TILE), eng->stream, eng->dTmap + eng->map_big, eng->ntiles_b, eng->dQ,
-                               eng->dEfoff, eng->dJa, eng->dJ, eng->dLift, eng->dOpsAll, eng->dU, eng->S, eng->ES,
+                               eng->dJa, eng->dJ, eng->dLift, eng->dOpsAll, eng->dU, eng->S, eng->ES,
                                eng->ph, lim, eng->grid_mgrad_s);
     }
     if (ev) (void)hipEventRecord(ev[1], eng->stream);
-    hipLaunchKernelGGL(hxm::km_face<GAUSS>, dim3(grid_for(eng->nwaves)), dim3(64), 0, eng->stream, eng->dQ, eng->dU,
-                       eng->dN3, eng->dOff, eng->dEfoff, eng->dFaces, eng->dSched, eng->dFgeo, eng->dFdelta,
-                       eng->dOpsAll, eng->dFe, eng->nwaves, eng->S, eng->ES, eng->FSm, eng->ph, dta.red);
+    auto *face = eng->ph.les ? &hxm::km_face<GAUSS, true> : &hxm::km_face<GAUSS, false>;
+    hipLaunchKernelGGL(face, dim3(grid_for(eng->nwaves)), dim3(64), 0, eng->stream, eng->dQ, eng->dU, eng->dFaces,
+                       eng->dSched, eng->dFgeo, eng->dFdelta, eng->dOpsAll, eng->dFe, eng->nwaves, eng->S, eng->ES,
+                       eng->FSm, eng->ph, dta.red);
     if (ev) (void)hipEventRecord(ev[2], eng->stream);
     if (GAUSS) launch_mvolume<hxk::FORM_STANDARD, true>(eng, a_k, c_k, update, dta, qdot);
     else if (eng->inviscid != HX3D_INVISCID_SPLIT) launch_mvolume<hxk::FORM_STANDARD>(eng, a_k, c_k, update, dta, qdot);
@@ -967,7 +967,12 @@ int set_tiles(hx3d_engine *eng, int policy)
     // the threads' node map (hxm::NodeMap): node offsets as the device's element offsets; the
     // small tiles' entries, then the large tiles'
     std::vector<long> eoff(K + 1, 0);
-    for (int e = 0; e < K; ++e) eoff[e + 1] = eoff[e] + ne[e];
+    std::vector<int> ef0(K + 1, 0);   // element face nodes (offsets_fit, create_mixed)
+    for (int e = 0; e < K; ++e) {
+        const int nx = N3[3 * e] + 1, ny = N3[3 * e + 1] + 1, nz = N3[3 * e + 2] + 1;
+        eoff[e + 1] = eoff[e] + ne[e];
+        ef0[e + 1] = ef0[e] + 2 * (nx * ny + ny * nz + nz * nx);
+    }
     if (eoff[K] > INT_MAX) return eng->fail(HX3D_EUNSUPPORTED, "mixed orders: more than 2^31 - 1 nodes");
     const size_t map_big = ts.size() * (size_t)hxm::TILE_SMALL;
     std::vector<hxm::NodeMap> map(map_big + tb.size() * (size_t)hxm::TILE);
@@ -985,6 +990,7 @@ int set_tiles(hx3d_engine *eng, int policy)
                 hxm::NodeMap &m = map[base + ti * cap + t];
                 m.g = (int)(eoff[e] + n);
                 m.e = e;
+                m.ef0 = ef0[e];
                 m.code = i | j << 3 | k << 6 | N3[3 * e] << 9 | N3[3 * e + 1] << 12 | N3[3 * e + 2] << 15 |
                          (active ? T.off[s] : 0) << 18 | (active ? 1 : 0) << 27;
             }
@@ -1066,24 +1072,20 @@ bool tangent2_is_cross(const double n[3], const double u[3], const double t2[3])
 #ifndef HX3D_FACE_PAIRS
 #define HX3D_FACE_PAIRS 1
 #endif
-std::vector<int2> face_waves(const std::vector<hxm::FaceRec> &faces)
+std::vector<int4> face_waves(const std::vector<int> &shapes)
 {
-    const int F = (int)faces.size();
-    std::vector<int2> w;
+    const int F = (int)shapes.size();
+    std::vector<int4> w;
     w.reserve(F);
     std::vector<int> pending(1 << 18, -1);   // by shape: six orders of 3 bits
     for (int f = 0; f < F; ++f) {
-        const hxm::FaceRec &r = faces[f];
-        if (!HX3D_FACE_PAIRS || (r.Nf[0] + 1) * (r.Nf[1] + 1) > 32) {
-            w.push_back(make_int2(f, -1));
-            continue;
-        }
-        const int key = r.Nf[0] | r.Nf[1] << 3 | r.Nfs[0][0] << 6 | r.Nfs[0][1] << 9 | r.Nfs[1][0] << 12 |
-                        r.Nfs[1][1] << 15;
-        if (pending[key] < 0) {
+        const int key = shapes[f];
+        if (!HX3D_FACE_PAIRS || ((key & 7) + 1) * ((key >> 3 & 7) + 1) > 32) {
+            w.push_back(make_int4(f, -1, key, 0));
+        } else if (pending[key] < 0) {
             pending[key] = f;
         } else {
-            w.push_back(make_int2(pending[key], f));
+            w.push_back(make_int4(pending[key], f, key, 0));
             pending[key] = -1;
         }
     }
@@ -1091,7 +1093,7 @@ std::vector<int2> face_waves(const std::vector<hxm::FaceRec> &faces)
     for (int p : pending)
         if (p >= 0) rest.push_back(p);
     std::sort(rest.begin(), rest.end());
-    for (int f : rest) w.push_back(make_int2(f, -1));
+    for (int f : rest) w.push_back(make_int4(f, -1, shapes[f], 0));
     return w;
 }
 
@@ -1119,38 +1121,52 @@ int create_mixed(hx3d_engine *eng, const hx3d_case_desc *d)
     const long ES = eng->ES;
     if (!offsets_fit(eng->S, ES, 0))
         return eng->fail(HX3D_EUNSUPPORTED, "mesh too large: more than 2^29 - 1 nodes (or face nodes) per array");
-    // faces
+    // faces: shapes (both sides' orders in the face orientation) and the affine index maps
     std::vector<hxm::FaceRec> faces(F);
+    std::vector<int> shapes(F);
     long fsm = 0;
     for (int f = 0; f < F; ++f) {
         hxm::FaceRec &r = faces[f];
         const int rot = d->fRot[f];
+        int No[2][2], Ns[2][2];   // each side's orders in its own and in the face orientation
+        r.na = 0;
         for (int sd = 0; sd < 2; ++sd) {
             const int e = d->fElem[2 * f + sd], s = d->fESide[2 * f + sd] - 1;
             if (e < 0 || e >= K || s < 0 || s > 5 || rot < 0 || rot > 7)
                 return eng->fail(HX3D_EINVAL, "face " + std::to_string(f) + ": bad element/side/rotation");
             if (d->faceID[6 * e + s] != f || d->faceSide[6 * e + s] != sd + 1)
                 return eng->fail(HX3D_EINVAL, "face " + std::to_string(f) + ": inconsistent with element faceID/faceSide");
-            r.e[sd] = e; r.slot[sd] = s;
-            r.Nel[sd][0] = N3[3 * e + SLOT_U[s]];
-            r.Nel[sd][1] = N3[3 * e + SLOT_V[s]];
+            No[sd][0] = N3[3 * e + SLOT_U[s]];
+            No[sd][1] = N3[3 * e + SLOT_V[s]];
+            const bool keep = sd == 0 || rot == 0 || rot == 2 || rot == 5 || rot == 7;
+            Ns[sd][0] = No[sd][keep ? 0 : 1];
+            Ns[sd][1] = No[sd][keep ? 1 : 0];
+            const int ax = 3 - SLOT_U[s] - SLOT_V[s], step[3] = {1, N3[3 * e] + 1, (N3[3 * e] + 1) * (N3[3 * e + 1] + 1)};
+            const bool plus = SLOT_PLUS[s];
+            auto map = [&](int i, int j, int &g, int &x) {
+                int a = i, b = j;
+                if (sd == 1) hxs::left_to_right(i, j, Ns[1][0], Ns[1][1], rot, a, b);
+                g = (int)off[e] + a * step[SLOT_U[s]] + b * step[SLOT_V[s]] + (plus ? N3[3 * e + ax] * step[ax] : 0);
+                x = efoff[6 * e + s] + a + (No[sd][0] + 1) * b;
+            };
+            int g, x;
+            map(0, 0, r.g0[sd], r.x0[sd]);
+            map(1, 0, g, x);
+            r.gi[sd] = g - r.g0[sd];
+            r.xi[sd] = x - r.x0[sd];
+            map(0, 1, g, x);
+            r.gj[sd] = g - r.g0[sd];
+            r.xj[sd] = x - r.x0[sd];
+            r.gn[sd] = plus ? -step[ax] : step[ax];
+            r.na |= N3[3 * e + ax] << (8 * sd) | (plus ? 1 : 0) << (16 + sd);
         }
-        r.rot = rot;
-        r.Nfs[0][0] = r.Nel[0][0]; r.Nfs[0][1] = r.Nel[0][1];
-        const bool keep = rot == 0 || rot == 2 || rot == 5 || rot == 7;
-        r.Nfs[1][0] = keep ? r.Nel[1][0] : r.Nel[1][1];
-        r.Nfs[1][1] = keep ? r.Nel[1][1] : r.Nel[1][0];
-        r.Nf[0] = std::max(r.Nfs[0][0], r.Nfs[1][0]);
-        r.Nf[1] = std::max(r.Nfs[0][1], r.Nfs[1][1]);
-        for (int sd = 0; sd < 2; ++sd) {
-            const bool a = r.Nfs[sd][0] != r.Nf[0], b = r.Nfs[sd][1] != r.Nf[1];
-            r.proj[sd] = (!a && !b) ? 0 : (a && !b) ? 1 : (!a && b) ? 2 : 3;
-        }
+        const int Nf0 = std::max(Ns[0][0], Ns[1][0]), Nf1 = std::max(Ns[0][1], Ns[1][1]);
+        shapes[f] = hxm::pack_shape(Nf0, Nf1, Ns[0][0], Ns[0][1], Ns[1][0], Ns[1][1]);
         r.foff = (int)fsm;
-        fsm += (long)(r.Nf[0] + 1) * (r.Nf[1] + 1);
+        fsm += (long)(Nf0 + 1) * (Nf1 + 1);
     }
     eng->FSm = fsm;
-    const std::vector<int2> sched = face_waves(faces);
+    const std::vector<int4> sched = face_waves(shapes);
     eng->nwaves = (int)sched.size();
     // operators of every order
     hxm::OpsAll oa;
@@ -1198,20 +1214,20 @@ int create_mixed(hx3d_engine *eng, const hx3d_case_desc *d)
         edelta[e] = std::pow(vol / (nx * ny * nz), 1.0 / 3.0);
     }
     for (int f = 0; f < F; ++f) {
-        const hxm::FaceRec &r = faces[f];
+        const int Nf0 = shapes[f] & 7, Nf1 = shapes[f] >> 3 & 7;
         double surf = 0.0;
-        for (int j = 0; j <= r.Nf[1]; ++j)
-            for (int i = 0; i <= r.Nf[0]; ++i) {
-                const long q = r.foff + i + (r.Nf[0] + 1) * j;
+        for (int j = 0; j <= Nf1; ++j)
+            for (int i = 0; i <= Nf0; ++i) {
+                const long q = faces[f].foff + i + (Nf0 + 1) * j;
                 for (int c = 0; c < 3; ++c) {
                     fgeo[(size_t)c * fsm + q] = d->fNormal[3 * q + c];
                     fgeo[(size_t)(3 + c) * fsm + q] = d->fT1[3 * q + c];
                     fgeo[(size_t)(6 + c) * fsm + q] = d->fT2[3 * q + c];
                 }
                 fgeo[(size_t)9 * fsm + q] = d->fJac[q];
-                surf += wn[r.Nf[0]][i] * wn[r.Nf[1]][j] * d->fJac[q];
+                surf += wn[Nf0][i] * wn[Nf1][j] * d->fJac[q];
             }
-        fdelta[f] = std::sqrt(surf / ((r.Nf[0] + 1) * (r.Nf[1] + 1)));
+        fdelta[f] = std::sqrt(surf / ((Nf0 + 1) * (Nf1 + 1)));
     }
     {
         // the volume kernel keeps three directions of fluxes (+ two-point node data and a metric
@@ -1238,8 +1254,7 @@ int create_mixed(hx3d_engine *eng, const hx3d_case_desc *d)
         (rc = dalloc(eng, &eng->dDtPart, (size_t)2 * (std::max((long)K, (S + 255) / 256) + 64))) ||
         (rc = dalloc(eng, &eng->dStage, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dBits, 2 * DT_SLOTS)) ||
         (rc = dalloc(eng, &eng->dFlag, 2)) || (rc = dalloc(eng, &eng->dN3, N3.size())) ||
-        (rc = dalloc(eng, &eng->dOff, off.size())) || (rc = dalloc(eng, &eng->dEfoff, efoff.size())) ||
-        (rc = dalloc(eng, &eng->dEofn, eofn.size())) ||
+        (rc = dalloc(eng, &eng->dOff, off.size())) || (rc = dalloc(eng, &eng->dEofn, eofn.size())) ||
         (rc = dalloc(eng, &eng->dFaces, faces.size())) || (rc = dalloc(eng, &eng->dSched, sched.size())) ||
         (rc = dalloc(eng, &eng->dOpsAll, 1)))
         return rc;
@@ -1252,10 +1267,10 @@ int create_mixed(hx3d_engine *eng, const hx3d_case_desc *d)
         !up(eng->dJ, jj.data(), jj.size() * 8) || !up(eng->dFgeo, fgeo.data(), fgeo.size() * 8) ||
         !up(eng->dWq, wq.data(), wq.size() * 8) || !up(eng->dEdelta, edelta.data(), edelta.size() * 8) ||
         !up(eng->dFdelta, fdelta.data(), fdelta.size() * 8) || !up(eng->dN3, N3.data(), N3.size() * 4) ||
-        !up(eng->dOff, off.data(), off.size() * 8) || !up(eng->dEfoff, efoff.data(), efoff.size() * 4) ||
+        !up(eng->dOff, off.data(), off.size() * 8) ||
         !up(eng->dEofn, eofn.data(), eofn.size() * 4) ||
         !up(eng->dFaces, faces.data(), faces.size() * sizeof(hxm::FaceRec)) ||
-        !up(eng->dSched, sched.data(), sched.size() * sizeof(int2)) || !up(eng->dOpsAll, &oa, sizeof(oa)))
+        !up(eng->dSched, sched.data(), sched.size() * sizeof(int4)) || !up(eng->dOpsAll, &oa, sizeof(oa)))
         return eng->fail(HX3D_EDEVICE, "upload failed");
     const long nb = (NV * S + 255) / 256;
     hipLaunchKernelGGL(k_fill, dim3(nb), dim3(256), 0, eng->stream, eng->dQ, (long)NV * S, 0.0);
@@ -1689,7 +1704,7 @@ int hx3d_engine_destroy(hx3d_engine *eng)
     if (eng->stream) (void)hipStreamSynchronize(eng->stream);
     void *ptrs[] = {eng->dQ, eng->dG, eng->dJa, eng->dJ, eng->dFgeo, eng->dEgeo, eng->dFe,
                     eng->dQDot, eng->dEdelta, eng->dFdelta, eng->dWq, eng->dScal, eng->dPart, eng->dStage,
-                    eng->dBits, eng->dNbr, eng->dFlag, eng->dN3, eng->dEfoff,
+                    eng->dBits, eng->dNbr, eng->dFlag, eng->dN3,
                     eng->dEofn, eng->dOff, eng->dFaces, eng->dSched, eng->dOpsAll, eng->dU, eng->dLift, eng->dDtPart, eng->dTmap,
                     eng->dBlocks, eng->dCC, eng->dActive, eng->dTimeM,
                     eng->dQtr, eng->dQtn, eng->dFvis, eng->dNbx, eng->dQn, eng->dVisc, eng->dCurl, eng->dEfdelta, eng->dSlots};

@@ -46,15 +46,46 @@ struct OpsAll {
     double vL[MAXN1][8], vR[MAXN1][8], bL[MAXN1][8], bR[MAXN1][8];
 };
 
-// Face record: elements, slots, orders, rotation and projection types (Face_LinkWithElements,
-// FaceClass.f90:187-278).  NfL/NfR are each side's orders in the face orientation, Nf their max.
-struct FaceRec {
-    int e[2], slot[2];          // left, right element and element face slot (0..5)
-    int Nel[2][2];              // element face orders (element face orientation)
-    int Nfs[2][2];              // the same in the face orientation
-    int Nf[2], rot, proj[2];    // proj: 0 none, 1 first index, 2 second, 3 both
-    int foff;                   // first face node (face order) of this face
+// Face record (Face_LinkWithElements, FaceClass.f90:187-278), with every index the kernels form of a
+// face laid out on the host as an affine map of the face coordinates (i, j), the right side's
+// rotation (leftIndexes2Right, MeshTypes.f90:70-108) included.  The face kernels are bound by latency
+// (one wave per face, three or four waves per SIMD): their traces start after two dependent loads
+// (wave, record) instead of five through element, order and offset tables, the shape's loops count
+// in scalar registers and the node arrays are addressed in 32 bits.  20^3 elements, orders 2..7:
+// km_face_grad 104.7 -> 79.5 us, km_face 176.4 -> 129.7 us; 10^3 Gauss, orders 2..5: 20.1 -> 16.2 us and
+// 39.9 -> 34.5 us.
+struct __align__(16) FaceRec {
+    int g0[2], gi[2], gj[2];   // side s's node at (i, j), at the face's end of the normal axis
+    int x0[2], xi[2], xj[2];   // side s's element face node at (i, j)
+    int gn[2];                 // node step along side s's normal axis, from the face inwards
+    int foff;                  // first face node (face order) of this face
+    int na;                    // order along the normal axis, side s in bits 8s..; bit 16 + s: the plus end
 };
+// What the faces of a wave share: the face orders Nf and each side's orders Ns in the face
+// orientation (three bits each), from which the projection types follow.
+struct Shape {
+    int Nf0, Nf1, N0[2], N1[2];
+};
+__host__ __device__ inline int pack_shape(int Nf0, int Nf1, int L0, int L1, int R0, int R1)
+{
+    return Nf0 | Nf1 << 3 | L0 << 6 | L1 << 9 | R0 << 12 | R1 << 15;
+}
+__device__ __forceinline__ Shape unpack_shape(int c)
+{
+    return Shape{c & 7, (c >> 3) & 7, {(c >> 6) & 7, (c >> 12) & 7}, {(c >> 9) & 7, (c >> 15) & 7}};
+}
+// 0 no projection, 1 along the first face index, 2 along the second, 3 along both
+__device__ __forceinline__ int projection(const Shape &r, int side)
+{
+    return (r.N0[side] != r.Nf0 ? 1 : 0) + (r.N1[side] != r.Nf1 ? 2 : 0);
+}
+// node (i, j) of a grid of rows of d nodes, 2 <= d <= 8, from q < 64: (q + 1/2)/d lies at least 1/16
+// from a whole number, far more than the reciprocal's error
+__device__ __forceinline__ void grid_ij(int q, int d, int &i, int &j)
+{
+    j = (int)(((float)q + 0.5f) * __builtin_amdgcn_rcpf((float)d));
+    i = q - j * d;
+}
 
 // A tile of elements for the persistent element kernels (host side): up to TILE_MAXE elements
 // whose nodes, one thread each, fill at most TILE threads; thread t works on node t - off[s] of
@@ -78,8 +109,9 @@ struct Tile {
 // give through three dependent ones; the element kernels load the next tile's entry while
 // they work on the current one.  Idle threads (active = 0) carry node 0 of the tile's last
 // element, so that their unconditional loads stay in bounds.
-struct NodeMap {
+struct __align__(16) NodeMap {
     int g, e, code;
+    int ef0;   // the element's first element face node
 };
 template <int T>
 __device__ __forceinline__ NodeMap load_map(const NodeMap *__restrict__ map, int tile, int t)
@@ -87,37 +119,16 @@ __device__ __forceinline__ NodeMap load_map(const NodeMap *__restrict__ map, int
     return map[(long)tile * T + t];
 }
 
-// element face slot 0..5 = EFRONT, EBACK, EBOTTOM, ERIGHT, ETOP, ELEFT: the fixed axis, its end,
-// and the axes of the slot's face coordinates (a, b)
-__device__ __constant__ int M_SLOT_AXIS[6] = {1, 1, 2, 0, 2, 0};
-__device__ __constant__ int M_SLOT_PLUS[6] = {0, 1, 0, 1, 1, 0};
-__device__ __constant__ int M_SLOT_U[6] = {0, 0, 0, 1, 0, 1};
-__device__ __constant__ int M_SLOT_V[6] = {2, 2, 1, 2, 1, 2};
-
-__device__ __forceinline__ void left_to_right_d(int i, int j, int Nx, int Ny, int rot, int &ii, int &jj)
+// Element face node of the element's node (i, j, k) on the face of slot s: the element's six faces
+// follow one another in slot order 0..5 = EFRONT, EBACK, EBOTTOM, ERIGHT, ETOP, ELEFT (axes y, y, z,
+// x, z, x), each (first coordinate fastest) at the element's orders.
+struct ElemFaces {
+    int s[6];
+};
+__device__ __forceinline__ ElemFaces elem_faces(int ef0, int nx, int ny, int nz)
 {
-    // leftIndexes2Right (MeshTypes.f90:70-108)
-    switch (rot) {
-    case 0: ii = i; jj = j; break;
-    case 1: ii = Ny - j; jj = i; break;
-    case 2: ii = Nx - i; jj = Ny - j; break;
-    case 3: ii = j; jj = Nx - i; break;
-    case 4: ii = j; jj = i; break;
-    case 5: ii = Nx - i; jj = j; break;
-    case 6: ii = Ny - j; jj = Nx - i; break;
-    default: ii = i; jj = Ny - j; break;
-    }
-}
-
-// node of element e at element face coordinates (a, b) of slot s
-__device__ __forceinline__ long slot_node(const int *N3, const long *off, int e, int s, int a, int b)
-{
-    const int *Ne = &N3[3 * e];
-    int idx[3];
-    idx[M_SLOT_AXIS[s]] = M_SLOT_PLUS[s] ? Ne[M_SLOT_AXIS[s]] : 0;
-    idx[M_SLOT_U[s]] = a;
-    idx[M_SLOT_V[s]] = b;
-    return off[e] + idx[0] + (Ne[0] + 1) * (idx[1] + (Ne[1] + 1) * idx[2]);
+    const int xz = nx * nz, xy = nx * ny, yz = ny * nz;
+    return ElemFaces{{ef0, ef0 + xz, ef0 + 2 * xz, ef0 + 2 * xz + xy, ef0 + 2 * xz + xy + yz, ef0 + 2 * xz + 2 * xy + yz}};
 }
 
 // Face_AdaptSolutionToFace (side trace -> face order Nf) and Face_ProjectFluxToElements (face ->
@@ -136,11 +147,12 @@ struct Mort {
 };
 __device__ __forceinline__ Mort mort_lds(const double (*m)[64]) { return Mort{m[0], m[1], m[2], m[3]}; }
 
-__device__ __forceinline__ void stage_mortar(const OpsAll &ops, const FaceRec &r, double (*m)[64], int lane)
+__device__ __forceinline__ void stage_mortar(const OpsAll &ops, const Shape &r, double (*m)[64], int lane)
 {
 #pragma unroll
     for (int d = 0; d < 2; ++d) {
-        const int n = r.Nf[d], Ns = r.Nfs[0][d] < n ? r.Nfs[0][d] : r.Nfs[1][d];
+        const int n = d ? r.Nf1 : r.Nf0;
+        const int a = d ? r.N1[0] : r.N0[0], b = d ? r.N1[1] : r.N0[1], Ns = a < n ? a : b;
         if (Ns < n) {
             m[d][lane] = ops.T[Ns][n][lane];
             m[2 + d][lane] = ops.T[n][Ns][lane];
@@ -153,11 +165,11 @@ __device__ __forceinline__ void stage_mortar(const OpsAll &ops, const FaceRec &r
 // source node's weight is formed once, and every value accumulates in the reference's order
 // with the reference's products.
 template <int K>
-__device__ __forceinline__ void adapt_k(const Mort &m, const FaceRec &r, int side, const double *tr,
+__device__ __forceinline__ void adapt_k(const Mort &m, const Shape &r, int side, const double *tr,
                                         int i, int j, double *out)
 {
-    const int N0 = r.Nfs[side][0], N1 = r.Nfs[side][1], n0 = r.Nf[0];
-    const int pt = r.proj[side];
+    const int N0 = r.N0[side], N1 = r.N1[side], n0 = r.Nf0;
+    const int pt = projection(r, side);
     if (pt == 0) {
 #pragma unroll
         for (int k = 0; k < K; ++k) out[k] = tr[k * 64 + i + (n0 + 1) * j];
@@ -193,11 +205,11 @@ __device__ __forceinline__ void adapt_k(const Mort &m, const FaceRec &r, int sid
 
 // Face_ProjectFluxToElements for K values at once (values k at fl[k*64 + q], q = m + (Nf0+1) l)
 template <int K>
-__device__ __forceinline__ void project_k(const Mort &m, const FaceRec &r, int side, const double *fl,
+__device__ __forceinline__ void project_k(const Mort &m, const Shape &r, int side, const double *fl,
                                           int i, int j, double *out)
 {
-    const int n0 = r.Nf[0], n1 = r.Nf[1];
-    const int pt = r.proj[side];
+    const int n0 = r.Nf0, n1 = r.Nf1;
+    const int pt = projection(r, side);
     if (pt == 0) {
 #pragma unroll
         for (int k = 0; k < K; ++k) out[k] = fl[k * 64 + i + (n0 + 1) * j];
@@ -245,7 +257,8 @@ __device__ __forceinline__ void interp2_k(const double *T0, const double *T1, in
                                           double *out)
 {
     if (lane < (D0 + 1) * (S1 + 1)) {
-        const int a = lane % (D0 + 1), l = lane / (D0 + 1);
+        int a, l;
+        grid_ij(lane, D0 + 1, a, l);
         double acc[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) acc[k] = 0.0;
@@ -281,11 +294,11 @@ __device__ __forceinline__ void interp2_k(const double *T0, const double *T1, in
 // volume integral, and factorising those measured 1.7e-12 on the 20^3 p-anisotropic case.
 // Uniform per face: every lane of the wave calls it.
 template <int K, bool FACT>
-__device__ __forceinline__ void adapt_face(const Mort &m, const FaceRec &r, int side, const double *tr,
+__device__ __forceinline__ void adapt_face(const Mort &m, const Shape &r, int side, const double *tr,
                                            double *tmp, int lane, int i, int j, bool on, double *out)
 {
-    if (FACT && r.proj[side] == 3) {
-        interp2_k<K>(m.a0, m.a1, r.Nfs[side][0], r.Nfs[side][1], r.Nf[0], r.Nf[1], tr, tmp, lane, i, j, on, out);
+    if (FACT && projection(r, side) == 3) {
+        interp2_k<K>(m.a0, m.a1, r.N0[side], r.N1[side], r.Nf0, r.Nf1, tr, tmp, lane, i, j, on, out);
     } else if (on) {
         adapt_k<K>(m, r, side, tr, i, j, out);
     } else {
@@ -295,11 +308,11 @@ __device__ __forceinline__ void adapt_face(const Mort &m, const FaceRec &r, int 
 }
 
 template <int K, bool FACT>
-__device__ __forceinline__ void project_face(const Mort &m, const FaceRec &r, int side, const double *fl,
+__device__ __forceinline__ void project_face(const Mort &m, const Shape &r, int side, const double *fl,
                                              double *tmp, int lane, int i, int j, bool on, double *out)
 {
-    if (FACT && r.proj[side] == 3) {
-        interp2_k<K>(m.p0, m.p1, r.Nf[0], r.Nf[1], r.Nfs[side][0], r.Nfs[side][1], fl, tmp, lane, i, j, on, out);
+    if (FACT && projection(r, side) == 3) {
+        interp2_k<K>(m.p0, m.p1, r.Nf0, r.Nf1, r.N0[side], r.N1[side], fl, tmp, lane, i, j, on, out);
     } else if (on) {
         project_k<K>(m, r, side, fl, i, j, out);
     } else {
@@ -308,81 +321,88 @@ __device__ __forceinline__ void project_face(const Mort &m, const FaceRec &r, in
     }
 }
 
-// Stage the side's element trace of K node arrays src[c*S + g] into tr[c*64 + q] in the face
-// orientation (the right side is rotated, Face_AdaptSolutionToFace).  Lane q of the face.  On
-// Gauss-Lobatto nodes the trace is the face's row of nodes; on Gauss nodes (GAUSS) it is the
-// Lagrange basis at the face's end of the normal direction applied along it,
-// acc = acc + value * v(l) for l = 0..N (HexElement_ProlongSolutionToFaces,
-// HexElementClass.f90:233-302, and _ProlongGradientsToFaces, :304-372).
-template <int K, bool GAUSS = false>
-__device__ __forceinline__ void gather_trace_k(const FaceRec &r, int side, const int *N3, const long *off,
-                                               const double *src, long S, double *tr, int lane,
-                                               const OpsAll *ops = nullptr)
+// A lane's part of a side's element trace: its node of the trace (at the side's orders, in the face
+// orientation) and whether it has one; lanes without read the side's first node and discard it, so
+// that every load is unconditional.
+struct TraceLane {
+    bool on;
+    unsigned g;
+};
+__device__ __forceinline__ TraceLane trace_lane(const FaceRec &f, const Shape &r, int side, int ql)
 {
-    const int N0 = r.Nfs[side][0], N1 = r.Nfs[side][1];
-    const int nq = (N0 + 1) * (N1 + 1);
-    if (lane < nq) {
-        const int i = lane % (N0 + 1), j = lane / (N0 + 1);
-        int a = i, b = j;
-        if (side == 1) left_to_right_d(i, j, N0, N1, r.rot, a, b);
-        const long g = slot_node(N3, off, r.e[side], r.slot[side], a, b);
-        if (!GAUSS) {
+    int i, j;
+    grid_ij(ql, r.N0[side] + 1, i, j);
+    const bool on = j <= r.N1[side];
+    return TraceLane{on, (unsigned)(f.g0[side] + (on ? i * f.gi[side] + j * f.gj[side] : 0))};
+}
+
+// Gauss-Lobatto nodes: the trace is the face's row of nodes, K values of the node arrays src[c*S + g]
+// in registers; put_trace stores them.
+template <int K>
+__device__ __forceinline__ void load_trace(const TraceLane &tl, const double *src, long S, double *v)
+{
 #pragma unroll
-            for (int c = 0; c < K; ++c) tr[c * 64 + lane] = src[c * S + g];
-        } else {
-            // g is the node at the face's end of the normal axis (index 0 or N); walk the axis
-            const int s = r.slot[side], ax = M_SLOT_AXIS[s];
-            const int *Ne = &N3[3 * r.e[side]];
-            const int Na = Ne[ax];
-            const long stride = ax == 0 ? 1 : (ax == 1 ? (Ne[0] + 1) : (long)(Ne[0] + 1) * (Ne[1] + 1));
-            const long g0 = M_SLOT_PLUS[s] ? g - (long)Na * stride : g;
-            const double *vv = M_SLOT_PLUS[s] ? ops->vR[Na] : ops->vL[Na];
-            double w[MAXN1];
+    for (int c = 0; c < K; ++c) v[c] = hxk::ldg(src + c * S, tl.g);
+}
+template <int K>
+__device__ __forceinline__ void put_trace(const TraceLane &tl, const double *v, double *tr, int ql)
+{
+    if (tl.on) {
 #pragma unroll
-            for (int l = 0; l < MAXN1; ++l) w[l] = l <= Na ? vv[l] : 0.0;
-            // the line's loads all issued before the sum (a loop to Na would wait for each load in
-            // turn); lanes past the line's end load nothing and add nothing
+        for (int c = 0; c < K; ++c) tr[c * 64 + ql] = v[c];
+    }
+}
+
+// Gauss nodes: the trace is the Lagrange basis at the face's end of the normal direction applied along
+// it, acc = acc + value * v(l) for l = 0..N (HexElement_ProlongSolutionToFaces,
+// HexElementClass.f90:233-302, and _ProlongGradientsToFaces, :304-372), into tr.  The line's loads are
+// all in flight before the sum; past a short line's end the load repeats the last node and adds
+// nothing.
+template <int K>
+__device__ __forceinline__ void prolong_trace(const FaceRec &f, int side, const TraceLane &tl, const double *src,
+                                              long S, const OpsAll &ops, double *tr, int ql)
+{
+    const int Na = (f.na >> (8 * side)) & 7;
+    const bool plus = (f.na >> (16 + side)) & 1;
+    const double *vv = plus ? ops.vR[Na] : ops.vL[Na];
+    const int step = plus ? -f.gn[side] : f.gn[side];   // towards larger l
+    const unsigned g0 = tl.g - (plus ? Na * step : 0);
+    if (tl.on) {
+        double w[MAXN1];
 #pragma unroll
-            for (int c = 0; c < K; ++c) {
-                double x[MAXN1];
+        for (int l = 0; l < MAXN1; ++l) w[l] = l <= Na ? vv[l] : 0.0;
 #pragma unroll
-                for (int l = 0; l < MAXN1; ++l) x[l] = l <= Na ? src[c * S + g0 + l * stride] : 0.0;
-                double acc = 0.0;
+        for (int c = 0; c < K; ++c) {
+            double x[MAXN1];
 #pragma unroll
-                for (int l = 0; l < MAXN1; ++l)
-                    if (l <= Na) acc = acc + x[l] * w[l];
-                tr[c * 64 + lane] = acc;
-            }
+            for (int l = 0; l < MAXN1; ++l) x[l] = l <= Na ? hxk::ldg(src + c * S, g0 + l * step) : 0.0;
+            double acc = 0.0;
+#pragma unroll
+            for (int l = 0; l < MAXN1; ++l)
+                if (l <= Na) acc = acc + x[l] * w[l];
+            tr[c * 64 + ql] = acc;
         }
     }
 }
 
-// The faces of one wave of the face kernels: sched[w] = (face, -1) puts one face on all 64
-// lanes; (face a, face b) puts two faces of one shape (the same orders on both sides, so the same
-// projection types and mortar matrices, at most 32 face nodes) on the two half-waves, so that
+// The faces of one wave of the face kernels: sched[w] = (face, -1, shape) puts one face on all 64
+// lanes; (face a, face b, shape) puts two faces of one shape (the same orders on both sides, so the
+// same projection types and mortar matrices, at most 32 face nodes) on the two half-waves, so that
 // small faces do not leave most of a wave idle.  Each half works in its own 32 columns of the
 // per-face LDS rows (every grid of such a face, and every half-interpolated grid, has at most
 // 32 nodes); the mortar matrices are shared.  Both halves take the same branches at every
-// barrier.
+// barrier: the shape comes with the schedule, in scalar registers, so that the interpolation loops
+// count there.
 struct FaceLane {
     int f;     // the lane's face
     int q;     // the lane's index within its face
     int col;   // first LDS column of its face
 };
-__device__ __forceinline__ FaceLane face_lane(const int2 *sched, int w, int lane)
+__device__ __forceinline__ FaceLane face_lane(const int4 s, int lane)
 {
-    const int2 s = sched[w];
     const bool two = s.y >= 0;
     const int h = two ? lane >> 5 : 0;
     return FaceLane{h ? s.y : s.x, two ? (lane & 31) : lane, 32 * h};
-}
-
-// element face node of the side's face-orientation node (i, j)
-__device__ __forceinline__ long elem_face_node(const FaceRec &r, int side, const int *efoff, int i, int j)
-{
-    int a = i, b = j;
-    if (side == 1) left_to_right_d(i, j, r.Nfs[1][0], r.Nfs[1][1], r.rot, a, b);
-    return (long)efoff[6 * r.e[side] + r.slot[side]] + a + (r.Nel[side][0] + 1) * b;
 }
 
 // ------------------------------------------------------------------------------------
@@ -392,8 +412,7 @@ __device__ __forceinline__ long elem_face_node(const FaceRec &r, int side, const
 // ------------------------------------------------------------------------------------
 template <bool GAUSS>
 __global__ void __launch_bounds__(64)
-km_face_grad(const double *__restrict__ Q, const int *__restrict__ N3, const long *__restrict__ off,
-             const int *__restrict__ efoff, const FaceRec *__restrict__ faces, const int2 *__restrict__ sched,
+km_face_grad(const double *__restrict__ Q, const FaceRec *__restrict__ faces, const int4 *__restrict__ sched,
              const double *__restrict__ fgeo, const OpsAll *__restrict__ opsp, double *__restrict__ lift, int W,
              long S, long ES, long FSm)
 {
@@ -406,31 +425,58 @@ km_face_grad(const double *__restrict__ Q, const int *__restrict__ N3, const lon
     // mostly run on one XCD and find the elements' traces in its L2
     const int w = hxk::xcd_block(blockIdx.x, gridDim.x), lane = threadIdx.x;
     if (w >= W) return;   // uniform per block
-    const FaceLane fl = face_lane(sched, w, lane);
+    const int4 sc = sched[w];
+    const Shape r = unpack_shape(sc.z);
+    const FaceLane fl = face_lane(sc, lane);
     const int ql = fl.q;
     double *const tL = sT[0] + fl.col, *const tR = sT[1] + fl.col, *const tmp = sTmp + fl.col;
     double *const sU = tL;   // [NV][64], once both traces are at the face order
-    const FaceRec r = faces[fl.f];
-    stage_mortar(*opsp, r, sM, lane);
+    const FaceRec f = faces[fl.f];
+    double qL[NV], qR[NV];
+    {
+        const TraceLane a = trace_lane(f, r, 0, ql), b = trace_lane(f, r, 1, ql);
+        if (GAUSS) {
+            stage_mortar(*opsp, r, sM, lane);
+            prolong_trace<NV>(f, 0, a, Q, S, *opsp, tL, ql);
+            prolong_trace<NV>(f, 1, b, Q, S, *opsp, tR, ql);
+        } else {
+            load_trace<NV>(a, Q, S, qL);
+            load_trace<NV>(b, Q, S, qR);
+            stage_mortar(*opsp, r, sM, lane);
+            put_trace<NV>(a, qL, tL, ql);
+            put_trace<NV>(b, qR, tR, ql);
+        }
+    }
     const Mort M = mort_lds(sM);
-    gather_trace_k<NV, GAUSS>(r, 0, N3, off, Q, S, tL, ql, opsp);
-    gather_trace_k<NV, GAUSS>(r, 1, N3, off, Q, S, tR, ql, opsp);
-    const int n0 = r.Nf[0], n1 = r.Nf[1], nq = (n0 + 1) * (n1 + 1);
-    const bool on = ql < nq;
-    const int i = on ? ql % (n0 + 1) : 0, j = on ? ql / (n0 + 1) : 0;
-    const long fq = r.foff + (on ? ql : 0);
+    int i, j;
+    grid_ij(ql, r.Nf0 + 1, i, j);
+    const bool on = j <= r.Nf1;
+    if (!on) { i = 0; j = 0; }
+    const long fq = f.foff + (on ? ql : 0);
     double nrm[3];
     nrm[0] = fgeo[fq];
     nrm[1] = fgeo[FSm + fq];
     nrm[2] = fgeo[2 * FSm + fq];
     const double jac = fgeo[9 * FSm + fq];
     __syncthreads();
-    double uS[NV], qL[NV], qR[NV];
+    double uS[NV];
     adapt_face<NV, true>(M, r, 0, tL, tmp, ql, i, j, on, qL);
     adapt_face<NV, true>(M, r, 1, tR, tmp, ql, i, j, on, qR);
 #pragma unroll
     for (int v = 0; v < NV; ++v) uS[v] = 0.5 * (qR[v] - qL[v]) * jac;
+    // each side's node of this lane in the projection
+    bool son[2];
+    int si[2], sj[2];
+    unsigned sx[2];
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+        grid_ij(ql, r.N0[side] + 1, si[side], sj[side]);
+        son[side] = sj[side] <= r.N1[side];
+        if (!son[side]) { si[side] = 0; sj[side] = 0; }
+        sx[side] = (unsigned)(f.x0[side] + si[side] * f.xi[side] + sj[side] * f.xj[side]);
+    }
     // unStar(v) n_d, one direction at a time, projected onto both sides: lift[(5d + v)*ES + x]
+#pragma unroll
     for (int d = 0; d < 3; ++d) {
         __syncthreads();   // the traces (d = 0), the previous direction's unStar (d > 0) have been read
         if (on) {
@@ -438,16 +484,13 @@ km_face_grad(const double *__restrict__ Q, const int *__restrict__ N3, const lon
             for (int v = 0; v < NV; ++v) sU[v * 64 + ql] = uS[v] * nrm[d];
         }
         __syncthreads();
-        for (int side = 0; side < 2; ++side) {
-            const int N0 = r.Nfs[side][0], N1 = r.Nfs[side][1];
-            const bool son = ql < (N0 + 1) * (N1 + 1);
-            const int si = son ? ql % (N0 + 1) : 0, sj = son ? ql / (N0 + 1) : 0;
-            double lv[NV];
-            project_face<NV, true>(M, r, side, sU, tmp, ql, si, sj, son, lv);
-            if (son) {
-                const long x = elem_face_node(r, side, efoff, si, sj);
 #pragma unroll
-                for (int v = 0; v < NV; ++v) lift[(d * NV + v) * ES + x] = lv[v];
+        for (int side = 0; side < 2; ++side) {
+            double lv[NV];
+            project_face<NV, true>(M, r, side, sU, tmp, ql, si[side], sj[side], son[side], lv);
+            if (son[side]) {
+#pragma unroll
+                for (int v = 0; v < NV; ++v) hxk::stg(lift + (d * NV + v) * ES, sx[side], lv[v]);
             }
         }
     }
@@ -460,8 +503,7 @@ km_face_grad(const double *__restrict__ Q, const int *__restrict__ N3, const lon
 // ------------------------------------------------------------------------------------
 template <bool GAUSS, int T>
 __global__ void __launch_bounds__(T)
-km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__ Q,
-        const int *__restrict__ efoff, const double *__restrict__ Ja,
+km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__ Q, const double *__restrict__ Ja,
         const double *__restrict__ Jac, const double *__restrict__ lift, const OpsAll *__restrict__ opsp,
         double *__restrict__ U, long S, long ES, Phys ph, hxk::DtLimits dtl, int pbase)
 {
@@ -474,8 +516,8 @@ km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__
     double tc = INFINITY, tv = INFINITY;   // MaxTimeStep limits of this thread's nodes (stage 1)
     NodeMap nm = load_map<T>(tmap, blockIdx.x < ntiles ? blockIdx.x : 0, t);
     for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int e = nm.e, code = nm.code;
-    const long g = nm.g;   // loads are unconditional (see k_volume)
+    const int code = nm.code, ef0 = nm.ef0;
+    const unsigned g = nm.g;   // loads are unconditional (see k_volume)
     const int i = code & 7, j = (code >> 3) & 7, k = (code >> 6) & 7;
     const int Nx = (code >> 9) & 7, Ny = (code >> 12) & 7, Nz = (code >> 15) & 7;
     const int nx = Nx + 1, ny = Ny + 1, nz = Nz + 1, ne = nx * ny * nz;
@@ -484,16 +526,16 @@ km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__
     const int n = i + nx * (j + ny * k);
     double q[NV], ja[9];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) q[v] = Q[v * S + g];
+    for (int v = 0; v < NV; ++v) q[v] = hxk::ldg(Q + v * S, g);
 #pragma unroll
-    for (int c = 0; c < 9; ++c) ja[c] = Ja[c * S + g];
-    const double jg = Jac[g];
+    for (int c = 0; c < 9; ++c) ja[c] = hxk::ldg(Ja + c * S, g);
+    const double jg = hxk::ldg(Jac, g);
     if (tile + (int)gridDim.x < ntiles) nm = load_map<T>(tmap, tile + gridDim.x, t);   // the next tile's
     const double iJ = 1.0 / jg;   // the same bits as a stored 1/J
     const bool onx = i == 0 || i == Nx, ony = j == 0 || j == Ny, onz = k == 0 || k == Nz;
-    const long xx = efoff[6 * e + (i == 0 ? 5 : 3)] + j + ny * k;
-    const long xy = efoff[6 * e + (j == 0 ? 0 : 1)] + i + nx * k;
-    const long xz = efoff[6 * e + (k == 0 ? 2 : 4)] + i + nx * j;
+    const ElemFaces ef = elem_faces(ef0, nx, ny, nz);
+    const unsigned xx = (i == 0 ? ef.s[5] : ef.s[3]) + j + ny * k, xy = (j == 0 ? ef.s[0] : ef.s[1]) + i + nx * k,
+                   xz = (k == 0 ? ef.s[2] : ef.s[4]) + i + nx * j;
     double *sQ = sQall + NV * first;   // [NV][ne]
     if (active) {
 #pragma unroll
@@ -524,10 +566,9 @@ km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__
         // every node takes the lifting values of all six faces with its surface weights b,
         // in the order L, R (xi), FR, BK (eta), BOT, T (zeta) of VectorWeakIntegrals_StdFace
         // (DGIntegrals.f90:365-443); slots 5, 3, 0, 1, 2, 4
-        const int *ef = &efoff[6 * e];
-        const long xl = ef[5] + j + ny * k, xr = ef[3] + j + ny * k;
-        const long xf = ef[0] + i + nx * k, xb = ef[1] + i + nx * k;
-        const long xo = ef[2] + i + nx * j, xt = ef[4] + i + nx * j;
+        const unsigned xl = ef.s[5] + j + ny * k, xr = ef.s[3] + j + ny * k;
+        const unsigned xf = ef.s[0] + i + nx * k, xb = ef.s[1] + i + nx * k;
+        const unsigned xo = ef.s[2] + i + nx * j, xt = ef.s[4] + i + nx * j;
         const double bl = ops.bL[Nx][i], br = ops.bR[Nx][i], bf = ops.bL[Ny][j], bb = ops.bR[Ny][j];
         const double bo = ops.bL[Nz][k], bt = ops.bR[Nz][k];
 #pragma unroll
@@ -539,13 +580,13 @@ km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
                 const double *lc = lift + (long)(d * NV + v) * ES;
-                double fi = lc[xl] * bl;
-                fi = fi + lc[xr] * br;
-                fi = fi + lc[xf] * bf;
-                fi = fi + lc[xb] * bb;
-                fi = fi + lc[xo] * bo;
-                fi = fi + lc[xt] * bt;
-                U[(d * NV + v) * S + g] = gr[d] + fi * iJ;
+                double fi = hxk::ldg(lc, xl) * bl;
+                fi = fi + hxk::ldg(lc, xr) * br;
+                fi = fi + hxk::ldg(lc, xf) * bf;
+                fi = fi + hxk::ldg(lc, xb) * bb;
+                fi = fi + hxk::ldg(lc, xo) * bo;
+                fi = fi + hxk::ldg(lc, xt) * bt;
+                hxk::stg(U + (d * NV + v) * S, g, gr[d] + fi * iJ);
             }
         }
     } else {
@@ -555,7 +596,7 @@ km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__
         double hx_[3 * NV], hy_[3 * NV], hz_[3 * NV];
 #pragma unroll
         for (int c = 0; c < 3 * NV; ++c) {
-            const double a = lift[c * ES + xx], b = lift[c * ES + xy], d = lift[c * ES + xz];
+            const double a = hxk::ldg(lift + c * ES, xx), b = hxk::ldg(lift + c * ES, xy), d = hxk::ldg(lift + c * ES, xz);
             hx_[c] = onx ? a : 0.0;
             hy_[c] = ony ? b : 0.0;
             hz_[c] = onz ? d : 0.0;
@@ -572,7 +613,7 @@ km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__
                 const double ay = ony ? hy_[d * NV + v] * by : 0.0;
                 const double az = onz ? hz_[d * NV + v] * bz : 0.0;
                 const double fi = ((0.0 + ax) + ay) + az;
-                U[(d * NV + v) * S + g] = (onx || ony || onz) ? gr[d] + fi * iJ : gr[d];
+                hxk::stg(U + (d * NV + v) * S, g, (onx || ony || onz) ? gr[d] + fi * iJ : gr[d]);
             }
         }
     }
@@ -594,11 +635,10 @@ km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__
 // (FaceClass.f90:597-700) and scaled by the receiving element's surface weight:
 // fe[v*ES + x] = (+/-) projected flux * b.
 // ------------------------------------------------------------------------------------
-template <bool GAUSS>
+template <bool GAUSS, bool LES>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
-km_face(const double *__restrict__ Q, const double *__restrict__ U, const int *__restrict__ N3,
-        const long *__restrict__ off, const int *__restrict__ efoff, const FaceRec *__restrict__ faces,
-        const int2 *__restrict__ sched, const double *__restrict__ fgeo, const double *__restrict__ fdelta,
+km_face(const double *__restrict__ Q, const double *__restrict__ U, const FaceRec *__restrict__ faces,
+        const int4 *__restrict__ sched, const double *__restrict__ fgeo, const double *__restrict__ fdelta,
         const OpsAll *__restrict__ opsp, double *__restrict__ fe, int W, long S, long ES, long FSm, Phys ph,
         hxk::DtReduce dtr)
 {
@@ -613,27 +653,46 @@ km_face(const double *__restrict__ Q, const double *__restrict__ U, const int *_
     const int w = hxk::xcd_block(blockIdx.x, gridDim.x), lane = threadIdx.x;
     if (dtr.bits && w == 0) hxk::reduce_dt_partials(dtr.part, dtr.n, dtr.bits, lane);
     if (w >= W) return;   // uniform per block
-    const FaceLane fl = face_lane(sched, w, lane);
-    const int f = fl.f, ql = fl.q;
+    const int4 sc = sched[w];
+    const Shape r = unpack_shape(sc.z);
+    const FaceLane fl = face_lane(sc, lane);
+    const int ql = fl.q;
     double *const qLt = sR + fl.col, *const qRt = sR + NV * 64 + fl.col, *const gT = sR + fl.col,
                   *const tmp = sTmp + fl.col;
-    const FaceRec r = faces[f];
+    const FaceRec f = faces[fl.f];
+    const TraceLane tl[2] = {trace_lane(f, r, 0, ql), trace_lane(f, r, 1, ql)};
+    double qs[2][NV];
+    // Gauss-Lobatto: the left side's gradients are asked for with the state traces, the right side's
+    // while the left's are interpolated.  (Without the LES model as a template flag these 30 registers
+    // would spill at three waves per SIMD.)
+    double gv[3 * NV];
+    if (!GAUSS) {
+        load_trace<NV>(tl[0], Q, S, qs[0]);
+        load_trace<NV>(tl[1], Q, S, qs[1]);
+        if (!ph.euler) load_trace<3 * NV>(tl[0], U, S, gv);
+    }
     stage_mortar(*opsp, r, sM, lane);
     const Mort M = mort_lds(sM);
-    gather_trace_k<NV, GAUSS>(r, 0, N3, off, Q, S, qLt, ql, opsp);
-    gather_trace_k<NV, GAUSS>(r, 1, N3, off, Q, S, qRt, ql, opsp);
-    __syncthreads();
-    const int n0 = r.Nf[0], n1 = r.Nf[1], nq = (n0 + 1) * (n1 + 1);
+    if (GAUSS) {
+        prolong_trace<NV>(f, 0, tl[0], Q, S, *opsp, qLt, ql);
+        prolong_trace<NV>(f, 1, tl[1], Q, S, *opsp, qRt, ql);
+    } else {
+        put_trace<NV>(tl[0], qs[0], qLt, ql);
+        put_trace<NV>(tl[1], qs[1], qRt, ql);
+    }
     // lanes past the face's nodes work on node (0, 0) and discard the result (every index stays
     // inside the face's arrays)
-    const bool on = ql < nq;
-    const int i = on ? ql % (n0 + 1) : 0, j = on ? ql / (n0 + 1) : 0;
-    const long fq = r.foff + (on ? ql : 0);
+    int i, j;
+    grid_ij(ql, r.Nf0 + 1, i, j);
+    const bool on = j <= r.Nf1;
+    if (!on) { i = 0; j = 0; }
+    const long fq = f.foff + (on ? ql : 0);
     double nrm[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) nrm[c] = fgeo[c * FSm + fq];
     const double jac = fgeo[9 * FSm + fq];
-    double qs[2][NV];
+    const double fd = LES ? fdelta[fl.f] : 0.0;
+    __syncthreads();
     adapt_face<NV, false>(M, r, 0, qLt, tmp, ql, i, j, on, qs[0]);
     adapt_face<NV, false>(M, r, 1, qRt, tmp, ql, i, j, on, qs[1]);
     __syncthreads();   // the Q traces are read: the space takes a grad Q trace or the face flux
@@ -646,34 +705,42 @@ km_face(const double *__restrict__ Q, const double *__restrict__ U, const int *_
 #pragma unroll
             for (int c = 0; c < 3; ++c) adapt_face<NV, true>(M, r, s, gT + c * NV * 64, tmp, ql, i, j, on, g + c * NV);
         };
-        auto side_flux = [&](int s, const double *g, double (*Fs)[3]) {
-            double vg[12];
+        auto side_flux = [&](int s, const double *g, double *ft) {
+            double vg[12], sh[6], mu, kappa;
             hx::viscous_state(ph, qs[s], g, g + NV, g + 2 * NV, vg);
-            double mu, kappa;
             hx::laminar_mu_kappa(ph, qs[s], mu, kappa);
-            if (ph.les) {
-                const double mt = hx::les_mu(ph, fdelta[f], qs[s][0], hx::les_factor(ph, qs[s], g, g + NV, g + 2 * NV));
+            if (LES) {
+                const double mt = hx::les_mu(ph, fd, qs[s][0], hx::les_factor(ph, qs[s], g, g + NV, g + 2 * NV));
                 mu = mu + mt;
                 kappa = kappa + mt * ph.mu_to_kappa;
             }
             const double ir = 1.0 / qs[s][0];
-            hx::viscous_flux(mu, kappa, qs[s][1] * ir, qs[s][2] * ir, qs[s][3] * ir, vg, Fs);
+            hx::stress_shape(vg, sh);
+            hx::viscous_tensor(mu, kappa, qs[s][1] * ir, qs[s][2] * ir, qs[s][3] * ir, sh, vg + 9, ft);
         };
-        double Fs[2][NV][3], g[3 * NV];
-        gather_trace_k<3 * NV, GAUSS>(r, 0, N3, off, U, S, gT, ql, opsp);
+        double fa[9], fb[9], g[3 * NV];
+        if (GAUSS) {
+            prolong_trace<3 * NV>(f, 0, tl[0], U, S, *opsp, gT, ql);
+        } else {
+            put_trace<3 * NV>(tl[0], gv, gT, ql);
+            load_trace<3 * NV>(tl[1], U, S, gv);
+        }
         __syncthreads();
         side_grad(0, g);
-        if (on) side_flux(0, g, Fs[0]);
+        if (on) side_flux(0, g, fa);
         __syncthreads();   // side 0's gradients consumed
-        gather_trace_k<3 * NV, GAUSS>(r, 1, N3, off, U, S, gT, ql, opsp);
+        if (GAUSS) prolong_trace<3 * NV>(f, 1, tl[1], U, S, *opsp, gT, ql);
+        else put_trace<3 * NV>(tl[1], gv, gT, ql);
         __syncthreads();
         side_grad(1, g);
         if (on) {
-            side_flux(1, g, Fs[1]);
+            side_flux(1, g, fb);
 #pragma unroll
-            for (int v = 0; v < NV; ++v)
-                visc[v] = 0.5 * (Fs[0][v][0] + Fs[1][v][0]) * nrm[0] + 0.5 * (Fs[0][v][1] + Fs[1][v][1]) * nrm[1] +
-                          0.5 * (Fs[0][v][2] + Fs[1][v][2]) * nrm[2];
+            for (int c = 0; c < 9; ++c) fa[c] = 0.5 * (fa[c] + fb[c]);
+#pragma unroll
+            for (int v = 1; v < NV; ++v)
+                visc[v] = fa[hx::viscous_entry(v, 0)] * nrm[0] + fa[hx::viscous_entry(v, 1)] * nrm[1] +
+                          fa[hx::viscous_entry(v, 2)] * nrm[2];
         }
         __syncthreads();   // the space takes the face flux next
     }
@@ -695,23 +762,22 @@ km_face(const double *__restrict__ Q, const double *__restrict__ U, const int *_
         for (int v = 0; v < NV; ++v) sF[v * 64 + ql] = (inv[v] - visc[v]) * jac;
     }
     __syncthreads();
+#pragma unroll
     for (int side = 0; side < 2; ++side) {
-        const int N0 = r.Nfs[side][0], N1 = r.Nfs[side][1];
-        const bool son = ql < (N0 + 1) * (N1 + 1);
-        const int si = son ? ql % (N0 + 1) : 0, sj = son ? ql / (N0 + 1) : 0;
+        int si, sj;
+        grid_ij(ql, r.N0[side] + 1, si, sj);
+        const bool son = sj <= r.N1[side];
+        if (!son) { si = 0; sj = 0; }
         double a[NV];
         project_face<NV, false>(M, r, side, sF, tmp, ql, si, sj, son, a);
         if (son) {
-            const long x = elem_face_node(r, side, efoff, si, sj);
-            if (GAUSS) {
-                // the surface weights b(i) of every node are applied by the volume kernel
+            const unsigned x = (unsigned)(f.x0[side] + si * f.xi[side] + sj * f.xj[side]);
+            // Gauss nodes: the surface weights b(i) of every node are applied by the volume kernel
+            const double b = GAUSS ? 1.0 : opsp->b0[(f.na >> (8 * side)) & 7];
 #pragma unroll
-                for (int v = 0; v < NV; ++v) fe[v * ES + x] = side == 0 ? a[v] : -1.0 * a[v];
-            } else {
-                const int e = r.e[side], s = r.slot[side];
-                const double b = opsp->b0[N3[3 * e + M_SLOT_AXIS[s]]];
-#pragma unroll
-                for (int v = 0; v < NV; ++v) fe[v * ES + x] = (side == 0 ? a[v] : -1.0 * a[v]) * b;
+            for (int v = 0; v < NV; ++v) {
+                const double x0 = side == 0 ? a[v] : -1.0 * a[v];
+                hxk::stg(fe + v * ES, x, GAUSS ? x0 : x0 * b);
             }
         }
     }
@@ -732,7 +798,6 @@ constexpr int mvolume_per_node()
 template <int FORM, bool GAUSS, int T>
 __global__ void __launch_bounds__(T)
 km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, const double *__restrict__ U,
-          const int *__restrict__ efoff,
           const double *__restrict__ Ja, const double *__restrict__ Jac, const double *__restrict__ edelta,
           const double *__restrict__ fe, const OpsAll *__restrict__ opsp, double *__restrict__ G,
           double *__restrict__ qdot_out, double a_k, double c_k, int update, DtArgs dta, long S, long ES,
@@ -756,7 +821,7 @@ km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, 
     NodeMap nm = load_map<T>(tmap, blockIdx.x < ntiles ? blockIdx.x : 0, t);
     for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     const int e = nm.e, code = nm.code;
-    const long g = nm.g;
+    const unsigned g = nm.g;
     const int i = code & 7, j = (code >> 3) & 7, k = (code >> 6) & 7;
     const int Nx = (code >> 9) & 7, Ny = (code >> 12) & 7, Nz = (code >> 15) & 7;
     const int nx = Nx + 1, ny = Ny + 1, nz = Nz + 1, ne = nx * ny * nz;
@@ -769,36 +834,35 @@ km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, 
     double *sJ = sN + (SPLIT ? ND * ne : 0);        // [3][ne]
     // loads, unconditional (see hxk::k_volume)
     double sx[NV], sy[NV], sz[NV];
+    const ElemFaces ef = elem_faces(nm.ef0, nx, ny, nz);
     if (GAUSS) {
         // surface integral on every node: the face fluxes of all six faces with the node's
         // surface weights, L, R, FR, BK, BOT, T (ScalarWeakIntegrals_StdFace, DGIntegrals.f90:
         // 214-273), accumulated in sx (sy, sz unused)
-        const int *ef = &efoff[6 * e];
-        const long xl = ef[5] + j + ny * k, xr = ef[3] + j + ny * k;
-        const long xf = ef[0] + i + nx * k, xb = ef[1] + i + nx * k;
-        const long xo = ef[2] + i + nx * j, xt = ef[4] + i + nx * j;
+        const unsigned xl = ef.s[5] + j + ny * k, xr = ef.s[3] + j + ny * k;
+        const unsigned xf = ef.s[0] + i + nx * k, xb = ef.s[1] + i + nx * k;
+        const unsigned xo = ef.s[2] + i + nx * j, xt = ef.s[4] + i + nx * j;
         const double bl = ops.bL[Nx][i], br = ops.bR[Nx][i], bf = ops.bL[Ny][j], bb = ops.bR[Ny][j];
         const double bo = ops.bL[Nz][k], bt = ops.bR[Nz][k];
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const double *fv = fe + (long)v * ES;
-            double x = fv[xl] * bl;
-            x = x + fv[xr] * br;
-            x = x + fv[xf] * bf;
-            x = x + fv[xb] * bb;
-            x = x + fv[xo] * bo;
-            x = x + fv[xt] * bt;
+            double x = hxk::ldg(fv, xl) * bl;
+            x = x + hxk::ldg(fv, xr) * br;
+            x = x + hxk::ldg(fv, xf) * bf;
+            x = x + hxk::ldg(fv, xb) * bb;
+            x = x + hxk::ldg(fv, xo) * bo;
+            x = x + hxk::ldg(fv, xt) * bt;
             sx[v] = x;
             sy[v] = 0.0;
             sz[v] = 0.0;
         }
     } else {
-        const long xx = efoff[6 * e + (i == 0 ? 5 : 3)] + j + ny * k;
-        const long xy = efoff[6 * e + (j == 0 ? 0 : 1)] + i + nx * k;
-        const long xz = efoff[6 * e + (k == 0 ? 2 : 4)] + i + nx * j;
+        const unsigned xx = (i == 0 ? ef.s[5] : ef.s[3]) + j + ny * k, xy = (j == 0 ? ef.s[0] : ef.s[1]) + i + nx * k,
+                       xz = (k == 0 ? ef.s[2] : ef.s[4]) + i + nx * j;
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            const double a = fe[v * ES + xx], b = fe[v * ES + xy], c = fe[v * ES + xz];
+            const double a = hxk::ldg(fe + v * ES, xx), b = hxk::ldg(fe + v * ES, xy), c = hxk::ldg(fe + v * ES, xz);
             sx[v] = onx ? a : 0.0;
             sy[v] = ony ? b : 0.0;
             sz[v] = onz ? c : 0.0;
@@ -806,15 +870,15 @@ km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, 
     }
     double q[NV], ja[9], gq[3][NV];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) q[v] = Q[v * S + g];
+    for (int v = 0; v < NV; ++v) q[v] = hxk::ldg(Q + v * S, g);
 #pragma unroll
-    for (int c = 0; c < 9; ++c) ja[c] = Ja[c * S + g];
+    for (int c = 0; c < 9; ++c) ja[c] = hxk::ldg(Ja + c * S, g);
 #pragma unroll
     for (int d = 0; d < 3; ++d)
 #pragma unroll
-        for (int v = 0; v < NV; ++v) gq[d][v] = U[(d * NV + v) * S + g];
-    const double dl = edelta[e];
-    const double jg = Jac[g];
+        for (int v = 0; v < NV; ++v) gq[d][v] = hxk::ldg(U + (d * NV + v) * S, g);
+    const double dl = hxk::ldg(edelta, (unsigned)e);
+    const double jg = hxk::ldg(Jac, g);
     if (tile + (int)gridDim.x < ntiles) nm = load_map<T>(tmap, tile + gridDim.x, t);   // the next tile's
     if (active) {
         double Fvc[3][NV];
@@ -880,7 +944,7 @@ km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, 
         if (SPLIT || d == 0) __syncthreads();
         if (d == 2) {
 #pragma unroll
-            for (int v = 0; v < NV; ++v) gk[v] = G[v * S + g];
+            for (int v = 0; v < NV; ++v) gk[v] = hxk::ldg(G + v * S, g);
             dt0 = hxk::bits_to_double(dta.in[0]);
             dt1 = hxk::bits_to_double(dta.in[1]);
         }
@@ -939,7 +1003,7 @@ km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, 
         for (int v = 0; v < NV; ++v) qd[v] = qd[v] * ijg;
         if (qdot_out) {
 #pragma unroll
-            for (int v = 0; v < NV; ++v) qdot_out[v * S + g] = qd[v];
+            for (int v = 0; v < NV; ++v) hxk::stg(qdot_out + v * S, g, qd[v]);
         }
         if (update) {
             hxk::hold(dt0);
@@ -951,9 +1015,9 @@ km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, 
             for (int v = 0; v < NV; ++v) {
                 hxk::hold(gk[v]);
                 const double gv = a_k * gk[v] + qd[v];
-                G[v * S + g] = gv;
+                hxk::stg(G + v * S, g, gv);
                 q[v] = q[v] + cdt * gv;
-                Q[v * S + g] = q[v];
+                hxk::stg(Q + v * S, g, q[v]);
             }
             if (dta.nan && (isnan(q[0]) || isnan(q[1]) || isnan(q[2]) || isnan(q[3]) || isnan(q[4])))
                 atomicOr(dta.nan, 1);

@@ -96,3 +96,37 @@ def test_state_copies_through_odd_and_even_steps(kind, tmp_path):
         assert np.array_equal(eng.get_state(), ref.get_state()), graph
     eng.close()
     ref.close()
+
+
+@pytest.mark.parametrize("nodes", ["gauss-lobatto", "gauss"])
+@pytest.mark.parametrize("orders,les", [("cubes", None), ("bricks", "smagorinsky")])
+def test_rotated_mortar_faces_match_oracle(orders, les, nodes, tmp_path):
+    """Every rotation of the right side on faces between elements of unlike orders 1..7: elements of
+    equal orders along their axes with all eight rotations, anisotropic ones with the four that keep
+    the face axes.  The rotations are drawn, so neighbouring nodes do not meet: a face flux is as well
+    defined for the engine and the oracle as on a mesh that turns its elements."""
+    from horses3d_amd.engine import Engine, read_specmesh
+    rng = np.random.default_rng(5)
+    K = 27
+    N3 = np.repeat(rng.integers(1, 8, (K, 1)), 3, axis=1) if orders == "cubes" else rng.integers(1, 8, (K, 3))
+    if nodes == "gauss":
+        path = str(tmp_path / "box.mesh")
+        specmesh.write_specmesh(path, 3, 0.1, mesh.box_phases(8), bface_order=7)
+        case = read_specmesh(path, N=4, orders=N3.astype(np.int32), periodic=dict(specmesh.PERIODIC_PAIRS), nodes="gauss")
+        uv = {1: (0, 2), 2: (0, 2), 3: (0, 1), 4: (1, 2), 5: (0, 1), 6: (1, 2)}
+        case["fNf"] = np.array([[max(N3[e][uv[s][d]] for e, s in zip(case["fElem"][f], case["fESide"][f]))
+                                 for d in range(2)] for f in range(case["F"])], np.int32)
+        case["foff"] = np.concatenate([[0], np.cumsum(np.prod(case["fNf"] + 1, axis=1))]).astype(np.int64)
+    else:
+        case = mesh.periodic_box_mixed(3, N3.astype(np.int32))
+    assert not np.any(case["fRot"])   # the box turns no element
+    case["fRot"] = rng.choice(np.arange(8) if orders == "cubes" else [0, 2, 5, 7], case["F"]).astype(np.int32)
+    Q0 = mesh.taylor_green(case, 0.3, noise=1e-3, seed=9)
+    kw = dict(mach=0.3, reynolds=700.0, riemann="roe", inviscid="standard", averaging="standard", les=les)
+    ora = po.Oracle(case, po.make_params(kw["mach"], kw["reynolds"], riemann="roe", les=les, nodes=nodes))
+    eng = Engine(case, nodes=nodes, **kw)
+    eng.set_state(Q0)
+    err = po.normwise_error(eng.qdot(), ora.qdot(Q0))
+    print(orders, les, nodes, err, flush=True)
+    assert err.max() <= TOL
+    eng.close()
