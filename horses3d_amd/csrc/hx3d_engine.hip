@@ -753,18 +753,19 @@ size_t mgrad_lds(int T) { return sizeof(double) * (hxm::MAXN1 * 64 + (size_t)NV 
 template <int FORM, bool GAUSS = false>
 void launch_mvolume(hx3d_engine *eng, double a_k, double c_k, int update, const DtArgs &dta, double *qdot)
 {
-    if (eng->ntiles_s)
-        hipLaunchKernelGGL((hxm::km_volume<FORM, GAUSS, hxm::TILE_SMALL>), dim3(eng->grid_mvol_s), dim3(hxm::TILE_SMALL),
-                           mvolume_lds<FORM>(hxm::TILE_SMALL), eng->stream, eng->dTmap, eng->ntiles_s, eng->dQ, eng->dU,
-                           eng->dJa, eng->dJ, eng->dEdelta, eng->dFe, eng->dOpsAll, eng->dG, qdot, a_k, c_k,
-                           update, dta, eng->S, eng->ES, eng->ph);
+    if (eng->ntiles_s) {
+        auto *k = eng->ph.les ? &hxm::km_volume<FORM, GAUSS, true, hxm::TILE_SMALL> : &hxm::km_volume<FORM, GAUSS, false, hxm::TILE_SMALL>;
+        hipLaunchKernelGGL(k, dim3(eng->grid_mvol_s), dim3(hxm::TILE_SMALL), mvolume_lds<FORM>(hxm::TILE_SMALL), eng->stream,
+                           eng->dTmap, eng->ntiles_s, eng->dQ, eng->dU, eng->dJa, eng->dJ, eng->dEdelta, eng->dFe,
+                           eng->dOpsAll, eng->dG, qdot, a_k, c_k, update, dta, eng->S, eng->ES, eng->ph);
+    }
     if (eng->ntiles_b) {
         DtArgs db = dta;   // the time advances once per stage: in the first launch
         if (eng->ntiles_s) db.time = nullptr;
-        hipLaunchKernelGGL((hxm::km_volume<FORM, GAUSS, hxm::TILE>), dim3(eng->grid_mvol_b), dim3(hxm::TILE),
-                           mvolume_lds<FORM>(hxm::TILE), eng->stream, eng->dTmap + eng->map_big, eng->ntiles_b, eng->dQ,
-                           eng->dU, eng->dJa, eng->dJ, eng->dEdelta, eng->dFe, eng->dOpsAll, eng->dG, qdot,
-                           a_k, c_k, update, db, eng->S, eng->ES, eng->ph);
+        auto *k = eng->ph.les ? &hxm::km_volume<FORM, GAUSS, true, hxm::TILE> : &hxm::km_volume<FORM, GAUSS, false, hxm::TILE>;
+        hipLaunchKernelGGL(k, dim3(eng->grid_mvol_b), dim3(hxm::TILE), mvolume_lds<FORM>(hxm::TILE), eng->stream,
+                           eng->dTmap + eng->map_big, eng->ntiles_b, eng->dQ, eng->dU, eng->dJa, eng->dJ, eng->dEdelta,
+                           eng->dFe, eng->dOpsAll, eng->dG, qdot, a_k, c_k, update, db, eng->S, eng->ES, eng->ph);
     }
 }
 
@@ -1031,10 +1032,10 @@ int set_tiles(hx3d_engine *eng, int policy)
     auto vol = [&](auto form_tag, auto gauss_tag) {
         constexpr int FORM = decltype(form_tag)::value;
         constexpr bool GAUSS = decltype(gauss_tag)::value;
-        const int a = occ(reinterpret_cast<const void *>(&hxm::km_volume<FORM, GAUSS, hxm::TILE_SMALL>), hxm::TILE_SMALL,
-                          mvolume_lds<FORM>(hxm::TILE_SMALL));
-        const int b = occ(reinterpret_cast<const void *>(&hxm::km_volume<FORM, GAUSS, hxm::TILE>), hxm::TILE,
-                          mvolume_lds<FORM>(hxm::TILE));
+        auto *ks = eng->ph.les ? &hxm::km_volume<FORM, GAUSS, true, hxm::TILE_SMALL> : &hxm::km_volume<FORM, GAUSS, false, hxm::TILE_SMALL>;
+        auto *kb = eng->ph.les ? &hxm::km_volume<FORM, GAUSS, true, hxm::TILE> : &hxm::km_volume<FORM, GAUSS, false, hxm::TILE>;
+        const int a = occ(reinterpret_cast<const void *>(ks), hxm::TILE_SMALL, mvolume_lds<FORM>(hxm::TILE_SMALL));
+        const int b = occ(reinterpret_cast<const void *>(kb), hxm::TILE, mvolume_lds<FORM>(hxm::TILE));
         return std::make_pair(a, b);
     };
     using F = std::false_type;
@@ -1233,7 +1234,7 @@ int create_mixed(hx3d_engine *eng, const hx3d_case_desc *d)
         // the volume kernel keeps three directions of fluxes (+ two-point node data and a metric
         // row for the split form) of a tile's elements in LDS
         const bool split = d->inviscid == HX3D_INVISCID_SPLIT;
-        const long per_node = 3 * (split ? 4 : 5) + (split ? hx::node_data_size(d->averaging) + 3 : 0);
+        const long per_node = (3 * (split ? 4 : 5) + (split ? hx::node_data_size(d->averaging) + 3 : 0)) | 1;
         int dev = 0, maxlds = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)

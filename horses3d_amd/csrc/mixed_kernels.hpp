@@ -500,6 +500,11 @@ km_face_grad(const double *__restrict__ Q, const FaceRec *__restrict__ faces, co
 // km_grad: local gradient (HexElement_ComputeLocalGradient, HexElementClass.f90:427-531) and
 // BR1 lifting (BR1_GradientFaceLoop, EllipticBR1.f90:531-569, with the weights b of
 // VectorWeakIntegrals_StdFace): grad Q at every node, U[(5d + v)*S + g].
+// Bound by memory: 256 bytes a node and 120 an element face node (515 MB on 20^3 elements of orders
+// 2..7, 154.9 -> 133.3 us, 3.9 TB/s).  What keeps the registers under 128 and two large tiles on a CU:
+// the nodes of a tile lie together in LDS (one address per node with constant offsets, instead of one
+// per value; the odd stride keeps a line's nodes in distinct banks), derivative loops that are
+// not unrolled, and the lifting a direction at a time.  10^3 Gauss elements of orders 2..5: 29.6 -> 13.3 us.
 // ------------------------------------------------------------------------------------
 template <bool GAUSS, int T>
 __global__ void __launch_bounds__(T)
@@ -511,7 +516,7 @@ km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__
     const OpsAll &ops = *opsp;
     const int t = threadIdx.x;
     double *sD = smem;                   // D of every order, [MAXN1][64] (visible after the first barrier)
-    double *sQall = smem + MAXN1 * 64;   // per element [NV][ne], at NV * off[slot]
+    double *sQall = smem + MAXN1 * 64;   // [node of the tile][NV]
     for (int x = t; x < MAXN1 * 64; x += blockDim.x) sD[x] = ops.D[x / 64][x % 64];
     double tc = INFINITY, tv = INFINITY;   // MaxTimeStep limits of this thread's nodes (stage 1)
     NodeMap nm = load_map<T>(tmap, blockIdx.x < ntiles ? blockIdx.x : 0, t);
@@ -520,7 +525,7 @@ km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__
     const unsigned g = nm.g;   // loads are unconditional (see k_volume)
     const int i = code & 7, j = (code >> 3) & 7, k = (code >> 6) & 7;
     const int Nx = (code >> 9) & 7, Ny = (code >> 12) & 7, Nz = (code >> 15) & 7;
-    const int nx = Nx + 1, ny = Ny + 1, nz = Nz + 1, ne = nx * ny * nz;
+    const int nx = Nx + 1, ny = Ny + 1, nz = Nz + 1;
     const int first = (code >> 18) & 511;
     const bool active = (code >> 27) & 1;
     const int n = i + nx * (j + ny * k);
@@ -536,32 +541,42 @@ km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__
     const ElemFaces ef = elem_faces(ef0, nx, ny, nz);
     const unsigned xx = (i == 0 ? ef.s[5] : ef.s[3]) + j + ny * k, xy = (j == 0 ? ef.s[0] : ef.s[1]) + i + nx * k,
                    xz = (k == 0 ? ef.s[2] : ef.s[4]) + i + nx * j;
-    double *sQ = sQall + NV * first;   // [NV][ne]
+    double *sQ = sQall + NV * first;   // [ne][NV]
     if (active) {
 #pragma unroll
-        for (int v = 0; v < NV; ++v) sQ[v * ne + n] = q[v];
+        for (int v = 0; v < NV; ++v) sQ[NV * n + v] = q[v];
     }
     __syncthreads();
     if (active) {
+    // Gauss-Lobatto: the lifting values of the node's faces (slots 5/3, 0/1, 2/4), a direction of the
+    // gradient at a time (all at once they took 60 registers more); the first direction's are asked
+    // for ahead of the derivatives
+    double h[3][NV];
+    auto ask = [&](int d) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const double *lc = lift + (long)(d * NV + v) * ES;
+            h[0][v] = hxk::ldg(lc, xx);
+            h[1][v] = hxk::ldg(lc, xy);
+            h[2][v] = hxk::ldg(lc, xz);
+        }
+        hxk::sched_fence();
+    };
+    if (!GAUSS) ask(0);
     const double *Dx = sD + 64 * Nx, *Dy = sD + 64 * Ny, *Dz = sD + 64 * Nz;
     double uxi[NV], ueta[NV], uzeta[NV];
+    auto line = [](const double *a, int step, const double *w, int len, double *u) {
 #pragma unroll
-    for (int v = 0; v < NV; ++v) { uxi[v] = 0.0; ueta[v] = 0.0; uzeta[v] = 0.0; }
-    for (int l = 0; l < nx; ++l) {
-        const double di = Dx[i * 8 + l];
+        for (int v = 0; v < NV; ++v) u[v] = 0.0;
+#pragma unroll 1
+        for (int l = 0; l < len; ++l) {
 #pragma unroll
-        for (int v = 0; v < NV; ++v) uxi[v] = uxi[v] + sQ[v * ne + l + nx * (j + ny * k)] * di;
-    }
-    for (int l = 0; l < ny; ++l) {
-        const double dj = Dy[j * 8 + l];
-#pragma unroll
-        for (int v = 0; v < NV; ++v) ueta[v] = ueta[v] + sQ[v * ne + i + nx * (l + ny * k)] * dj;
-    }
-    for (int l = 0; l < nz; ++l) {
-        const double dk = Dz[k * 8 + l];
-#pragma unroll
-        for (int v = 0; v < NV; ++v) uzeta[v] = uzeta[v] + sQ[v * ne + i + nx * (j + ny * l)] * dk;
-    }
+            for (int v = 0; v < NV; ++v) u[v] = u[v] + a[l * step + v] * w[l];
+        }
+    };
+    line(sQ + NV * (nx * (j + ny * k)), NV, Dx + i * 8, nx, uxi);
+    line(sQ + NV * (i + nx * ny * k), NV * nx, Dy + j * 8, ny, ueta);
+    line(sQ + NV * (i + nx * j), NV * nx * ny, Dz + k * 8, nz, uzeta);
     if (GAUSS) {
         // every node takes the lifting values of all six faces with its surface weights b,
         // in the order L, R (xi), FR, BK (eta), BOT, T (zeta) of VectorWeakIntegrals_StdFace
@@ -591,34 +606,26 @@ km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__
         }
     } else {
         const double bx = ops.b0[Nx], by = ops.b0[Ny], bz = ops.b0[Nz];
-        // lifting values of the node's faces (slot order 5/3, 0/1, 2/4); absent faces give 0.
-        // Loaded after the derivatives, so that they do not hold registers through them.
-        double hx_[3 * NV], hy_[3 * NV], hz_[3 * NV];
 #pragma unroll
-        for (int c = 0; c < 3 * NV; ++c) {
-            const double a = hxk::ldg(lift + c * ES, xx), b = hxk::ldg(lift + c * ES, xy), d = hxk::ldg(lift + c * ES, xz);
-            hx_[c] = onx ? a : 0.0;
-            hy_[c] = ony ? b : 0.0;
-            hz_[c] = onz ? d : 0.0;
-        }
+        for (int d = 0; d < 3; ++d) {
+            if (d) ask(d);
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            double gr[3];
-            gr[0] = (uxi[v] * ja[0] + ueta[v] * ja[3] + uzeta[v] * ja[6]) * iJ;
-            gr[1] = (uxi[v] * ja[1] + ueta[v] * ja[4] + uzeta[v] * ja[7]) * iJ;
-            gr[2] = (uxi[v] * ja[2] + ueta[v] * ja[5] + uzeta[v] * ja[8]) * iJ;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                const double ax = onx ? hx_[d * NV + v] * bx : 0.0;
-                const double ay = ony ? hy_[d * NV + v] * by : 0.0;
-                const double az = onz ? hz_[d * NV + v] * bz : 0.0;
+            for (int v = 0; v < NV; ++v) {
+                const double gr = (uxi[v] * ja[d] + ueta[v] * ja[3 + d] + uzeta[v] * ja[6 + d]) * iJ;
+                // absent faces give 0
+                const double ax = onx ? h[0][v] * bx : 0.0;
+                const double ay = ony ? h[1][v] * by : 0.0;
+                const double az = onz ? h[2][v] * bz : 0.0;
                 const double fi = ((0.0 + ax) + ay) + az;
-                hxk::stg(U + (d * NV + v) * S, g, (onx || ony || onz) ? gr[d] + fi * iJ : gr[d]);
+                hxk::stg(U + (d * NV + v) * S, g, (onx || ony || onz) ? gr + fi * iJ : gr);
             }
+            hxk::sched_fence();
         }
     }
     if (dtl.part) {
         double c0, c1;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) q[v] = sQ[NV * n + v];   // again: not held through the derivatives
         hx::dt_limits(ph, q, ja, jg, ops.dcsi[Nx], ops.dcsi[Ny], ops.dcsi[Nz], dtl.cfl, dtl.dcfl, c0, c1);
         tc = fmin(tc, c0);
         tv = fmin(tv, c1);
@@ -786,17 +793,24 @@ km_face(const double *__restrict__ Q, const double *__restrict__ U, const FaceRe
 // ------------------------------------------------------------------------------------
 // km_volume: as hxk::k_volume with the element's own orders per direction, the viscous
 // state formed from grad Q (ViscousFlux_STATE), and MaxTimeStep's 1/|x_1 - x_0| per direction.
-// LDS (dynamic): hatD and sharpD of every order [2][MAXN1][64], then per element of the tile,
-// at per_node * off[slot]: sF[3][NF][ne], sN[ND][ne], sJ[3][ne].
+// LDS (dynamic): hatD and sharpD of every order [2][MAXN1][64], then each node's fluxes and data
+// together (see km_grad).
+// Bound by memory: 376 bytes a node and 40 an element face node (558 MB on 20^3 elements of orders
+// 2..7, standard form, 158.3 -> 123.3 us, 4.5 TB/s).  That takes two large tiles per CU (four waves per SIMD,
+// 128 registers): the surface integral is summed as its loads arrive, the fluxes go to LDS a direction
+// at a time.  The split form's LDS admits one large tile, and Gauss nodes, with six faces' loads in
+// flight per node, are faster with the registers (10^3 elements of orders 2..5: 12.7 us against 18.5 at
+// four waves).
 // ------------------------------------------------------------------------------------
 template <int FORM>
 constexpr int mvolume_per_node()
 {
-    return 3 * (FORM >= 0 ? 4 : 5) + (FORM >= 0 ? hx::node_data_size(FORM) + 3 : 0);
+    // odd: the nodes of a wave's line lie in distinct banks
+    return (3 * (FORM >= 0 ? 4 : 5) + (FORM >= 0 ? hx::node_data_size(FORM) + 3 : 0)) | 1;
 }
 
-template <int FORM, bool GAUSS, int T>
-__global__ void __launch_bounds__(T)
+template <int FORM, bool GAUSS, bool LES, int T>
+__global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(FORM < 0 && !GAUSS && !LES ? 4 : 2)))
 km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, const double *__restrict__ U,
           const double *__restrict__ Ja, const double *__restrict__ Jac, const double *__restrict__ edelta,
           const double *__restrict__ fe, const OpsAll *__restrict__ opsp, double *__restrict__ G,
@@ -820,25 +834,38 @@ km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, 
     double *chunk0 = smem + 2 * MAXN1 * 64;
     NodeMap nm = load_map<T>(tmap, blockIdx.x < ntiles ? blockIdx.x : 0, t);
     for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int e = nm.e, code = nm.code;
+    const int e = nm.e, code = nm.code, ef0 = nm.ef0;
     const unsigned g = nm.g;
     const int i = code & 7, j = (code >> 3) & 7, k = (code >> 6) & 7;
     const int Nx = (code >> 9) & 7, Ny = (code >> 12) & 7, Nz = (code >> 15) & 7;
-    const int nx = Nx + 1, ny = Ny + 1, nz = Nz + 1, ne = nx * ny * nz;
+    const int nx = Nx + 1, ny = Ny + 1, nz = Nz + 1;
     const int first = (code >> 18) & 511;
     const bool active = (code >> 27) & 1;
     const int n = i + nx * (j + ny * k);
     const bool onx = i == 0 || i == Nx, ony = j == 0 || j == Ny, onz = k == 0 || k == Nz;
-    double *sF = chunk0 + PER_NODE * first;   // [3][NF][ne]
-    double *sN = sF + 3 * NF * ne;                  // [ND][ne]
-    double *sJ = sN + (SPLIT ? ND * ne : 0);        // [3][ne]
+    // this node's values: the fluxes [3][NF] (the split form: viscous fluxes), the two-point data
+    // [ND], the metric row [3]; the node at distance m along an axis lies m * PER_NODE further
+    double *mine = chunk0 + PER_NODE * (first + n);
+    constexpr int ON = 3 * NF, OJ = ON + ND;
     // loads, unconditional (see hxk::k_volume)
-    double sx[NV], sy[NV], sz[NV];
-    const ElemFaces ef = elem_faces(nm.ef0, nx, ny, nz);
+    double q[NV], ja[9], gq[3][NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) q[v] = hxk::ldg(Q + v * S, g);
+#pragma unroll
+    for (int c = 0; c < 9; ++c) ja[c] = hxk::ldg(Ja + c * S, g);
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) gq[d][v] = hxk::ldg(U + (d * NV + v) * S, g);
+    const double dl = hxk::ldg(edelta, (unsigned)e);
+    const double jg = hxk::ldg(Jac, g);
+    if (tile + (int)gridDim.x < ntiles) nm = load_map<T>(tmap, tile + gridDim.x, t);   // the next tile's
+    double xs[NV];   // the node's surface integral
+    const ElemFaces ef = elem_faces(ef0, nx, ny, nz);
     if (GAUSS) {
         // surface integral on every node: the face fluxes of all six faces with the node's
         // surface weights, L, R, FR, BK, BOT, T (ScalarWeakIntegrals_StdFace, DGIntegrals.f90:
-        // 214-273), accumulated in sx (sy, sz unused)
+        // 214-273)
         const unsigned xl = ef.s[5] + j + ny * k, xr = ef.s[3] + j + ny * k;
         const unsigned xf = ef.s[0] + i + nx * k, xb = ef.s[1] + i + nx * k;
         const unsigned xo = ef.s[2] + i + nx * j, xt = ef.s[4] + i + nx * j;
@@ -853,13 +880,12 @@ km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, 
             x = x + hxk::ldg(fv, xb) * bb;
             x = x + hxk::ldg(fv, xo) * bo;
             x = x + hxk::ldg(fv, xt) * bt;
-            sx[v] = x;
-            sy[v] = 0.0;
-            sz[v] = 0.0;
+            xs[v] = x;
         }
     } else {
         const unsigned xx = (i == 0 ? ef.s[5] : ef.s[3]) + j + ny * k, xy = (j == 0 ? ef.s[0] : ef.s[1]) + i + nx * k,
                        xz = (k == 0 ? ef.s[2] : ef.s[4]) + i + nx * j;
+        double sx[NV], sy[NV], sz[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const double a = hxk::ldg(fe + v * ES, xx), b = hxk::ldg(fe + v * ES, xy), c = hxk::ldg(fe + v * ES, xz);
@@ -867,66 +893,54 @@ km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, 
             sy[v] = ony ? b : 0.0;
             sz[v] = onz ? c : 0.0;
         }
+#pragma unroll
+        for (int v = 0; v < NV; ++v) xs[v] = ((0.0 + sx[v]) + sy[v]) + sz[v];
     }
-    double q[NV], ja[9], gq[3][NV];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) q[v] = hxk::ldg(Q + v * S, g);
-#pragma unroll
-    for (int c = 0; c < 9; ++c) ja[c] = hxk::ldg(Ja + c * S, g);
-#pragma unroll
-    for (int d = 0; d < 3; ++d)
-#pragma unroll
-        for (int v = 0; v < NV; ++v) gq[d][v] = hxk::ldg(U + (d * NV + v) * S, g);
-    const double dl = hxk::ldg(edelta, (unsigned)e);
-    const double jg = hxk::ldg(Jac, g);
-    if (tile + (int)gridDim.x < ntiles) nm = load_map<T>(tmap, tile + gridDim.x, t);   // the next tile's
+    for (int v = 0; v < NV; ++v) hxk::hold(xs[v]);
+    hxk::sched_fence();
     if (active) {
-        double Fvc[3][NV];
+        double ft[9];   // the viscous tensor (hx::viscous_entry)
         if (!ph.euler) {
-            double vg[12];
+            double vg[12], sh[6], mu, kappa;
             hx::viscous_state(ph, q, gq[0], gq[1], gq[2], vg);
-            double mu, kappa;
             hx::laminar_mu_kappa(ph, q, mu, kappa);
-            if (ph.les) {
+            if (LES) {
                 const double mt = hx::les_mu(ph, dl, q[0], hx::les_factor(ph, q, gq[0], gq[1], gq[2]));
                 mu = mu + mt;
                 kappa = kappa + mt * ph.mu_to_kappa;
             }
             const double ir = 1.0 / q[0];
-            double Fv[NV][3];
-            hx::viscous_flux(mu, kappa, q[1] * ir, q[2] * ir, q[3] * ir, vg, Fv);
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-#pragma unroll
-                for (int v = 0; v < NV; ++v)
-                    Fvc[d][v] = Fv[v][0] * ja[3 * d] + Fv[v][1] * ja[3 * d + 1] + Fv[v][2] * ja[3 * d + 2];
+            hx::stress_shape(vg, sh);
+            hx::viscous_tensor(mu, kappa, q[1] * ir, q[2] * ir, q[3] * ir, sh, vg + 9, ft);
         } else {
 #pragma unroll
-            for (int d = 0; d < 3; ++d)
+            for (int c = 0; c < 9; ++c) ft[c] = 0.0;
+        }
 #pragma unroll
-                for (int v = 0; v < NV; ++v) Fvc[d][v] = 0.0;
+        for (int c = 0; c < 9; ++c) hxk::hold(ft[c]);
+        double pu, pv, pw, pp;
+        hx::euler_primitives(ph, q, pu, pv, pw, pp);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            double fi[NV];
+            if (!SPLIT) hx::euler_contravariant_row(q, pu, pv, pw, pp, &ja[3 * d], fi);
+#pragma unroll
+            for (int v = V0; v < NV; ++v) {
+                const double fv = v == 0 ? 0.0
+                                         : ft[hx::viscous_entry(v, 0)] * ja[3 * d] + ft[hx::viscous_entry(v, 1)] * ja[3 * d + 1] +
+                                               ft[hx::viscous_entry(v, 2)] * ja[3 * d + 2];
+                mine[d * NF + v - V0] = SPLIT ? fv : fi[v] - fv;
+            }
+            hxk::sched_fence();
         }
         if (SPLIT) {
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-#pragma unroll
-                for (int v = 1; v < NV; ++v) sF[(d * NF + v - V0) * ne + n] = Fvc[d][v];
             double a[ND];
             hx::node_data<AVG>(ph, q, a);
 #pragma unroll
-            for (int c = 0; c < ND; ++c) sN[c * ne + n] = a[c];
-        } else {
-            double Fi[3][NV];
-            hx::euler_contravariant(ph, q, ja, Fi);
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-#pragma unroll
-                for (int v = 0; v < NV; ++v) sF[(d * NF + v - V0) * ne + n] = Fi[d][v] - Fvc[d][v];
+            for (int c = 0; c < ND; ++c) mine[ON + c] = a[c];
         }
     }
-    double xs[NV];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) xs[v] = GAUSS ? sx[v] : ((0.0 + sx[v]) + sy[v]) + sz[v];
     double qd[NV], gk[NV], dt0 = 0.0, dt1 = 0.0;
 #pragma unroll
     for (int v = 0; v < NV; ++v) qd[v] = 0.0;
@@ -938,7 +952,7 @@ km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, 
             if (d) __syncthreads();
             if (active) {
 #pragma unroll
-                for (int c = 0; c < 3; ++c) sJ[c * ne + n] = jh[c];
+                for (int c = 0; c < 3; ++c) mine[OJ + c] = jh[c];
             }
         }
         if (SPLIT || d == 0) __syncthreads();
@@ -952,27 +966,29 @@ km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, 
         const int own = d == 0 ? i : (d == 1 ? j : k);
         const int Nd = d == 0 ? Nx : (d == 1 ? Ny : Nz);
         const int stride = d == 0 ? 1 : (d == 1 ? nx : nx * ny);
-        const int base = n - own * stride;
-        const double *hatD = sOp + 64 * Nd, *sharpD = sOp + MAXN1 * 64 + 64 * Nd;
+        const double *line = mine - own * stride * PER_NODE;   // node 0 of this node's line
+        const double *hatD = sOp + 64 * Nd + own * 8, *sharpD = hatD + MAXN1 * 64;
         if (!SPLIT) {
+#pragma unroll(GAUSS ? 2 : 1)
             for (int l = 0; l <= Nd; ++l) {
-                const double hh = hatD[own * 8 + l];
-                const int m = base + l * stride;
+                const double *m = line + l * stride * PER_NODE;
+                const double hh = hatD[l];
 #pragma unroll
-                for (int v = 0; v < NV; ++v) qd[v] = qd[v] + hh * sF[(d * NF + v) * ne + m];
+                for (int v = 0; v < NV; ++v) qd[v] = qd[v] + hh * m[d * NF + v];
             }
         } else {
             double fi[NV], pu, pv, pw, pp;
             hx::euler_primitives(ph, q, pu, pv, pw, pp);
             hx::euler_contravariant_row(q, pu, pv, pw, pp, &ja[3 * d], fi);
+#pragma unroll 1
             for (int l = 0; l <= Nd; ++l) {
-                const double sh = sharpD[own * 8 + l], hh = hatD[own * 8 + l];
-                const int m = base + l * stride;
+                const double sh = sharpD[l], hh = hatD[l];
+                const double *m = line + l * stride * PER_NODE;
                 double a[ND], b[ND], jb[3], fs[NV];
 #pragma unroll
-                for (int c = 0; c < ND; ++c) { a[c] = sN[c * ne + n]; b[c] = sN[c * ne + m]; }
+                for (int c = 0; c < ND; ++c) { a[c] = mine[ON + c]; b[c] = m[ON + c]; }
 #pragma unroll
-                for (int c = 0; c < 3; ++c) jb[c] = sJ[c * ne + m];
+                for (int c = 0; c < 3; ++c) jb[c] = m[OJ + c];
                 if (SYM) {
                     hx::two_point<AVG>(a, jh, b, jb, fs);
                 } else {
@@ -987,7 +1003,7 @@ km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, 
                 qd[0] = qd[0] + sh * (l == own ? fi[0] : fs[0]);
 #pragma unroll
                 for (int v = 1; v < NV; ++v)
-                    qd[v] = qd[v] + sh * (l == own ? fi[v] : fs[v]) + hh * sF[(d * NF + v - V0) * ne + m];
+                    qd[v] = qd[v] + sh * (l == own ? fi[v] : fs[v]) + hh * m[d * NF + v - V0];
             }
         }
     }
