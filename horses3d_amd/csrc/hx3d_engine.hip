@@ -469,6 +469,9 @@ struct hx3d_engine {
     double *dQtr = nullptr, *dQtn = nullptr, *dFvis = nullptr;
     int *dNbx = nullptr;
     hxg::GaussOps gops{};
+    // metric terms once per element (per face) where every node has the same bits (hxk::Metric)
+    int per_elem = 0, per_face = 0;
+    long elem_stride = 0, egeo_stride = 0, fgeo_stride = 0;
     double *dJ = nullptr, *dFgeo = nullptr, *dEgeo = nullptr;
     double *dScal = nullptr, *dPart = nullptr, *dStage = nullptr, *dDtPart = nullptr;
     unsigned long long *dBits = nullptr;
@@ -601,13 +604,21 @@ void refresh_traces(hx3d_engine *eng)
     }
 }
 
+hxk::Metric metric(const hx3d_engine *eng)
+{
+    const long E = eng->elem_stride;
+    if (eng->per_elem)   // behind the planes by node (element_metrics)
+        return hxk::Metric{eng->dJa + 9 * eng->S, eng->dJa + 9 * eng->S + 9 * E, eng->dEgeo, E, eng->egeo_stride, 1, eng->per_face};
+    return hxk::Metric{eng->dJa, eng->dJ, eng->dEgeo, eng->S, eng->egeo_stride, 0, eng->per_face};
+}
+
 template <int N>
 void launch_grad(hx3d_engine *eng, const hxk::DtLimits &dtl, double *curl)
 {
     constexpr int EPB = epb_for(N), ne = (N + 1) * (N + 1) * (N + 1);
     constexpr int TPB = ((EPB * ne + 63) / 64) * 64;
-    hipLaunchKernelGGL((hxk::k_grad<N, EPB>), dim3(elem_grid(eng, EPB)), dim3(TPB), 0, eng->stream, eng->dQ, eng->dJa,
-                       eng->dJ, eng->dNbr, eng->dEgeo, eng->dVisc, curl, eng->K, eng->S, eng->ES, eng->ops, eng->ph, dtl,
+    hipLaunchKernelGGL((hxk::k_grad<N, EPB>), dim3(elem_grid(eng, EPB)), dim3(TPB), 0, eng->stream, eng->dQ, metric(eng),
+                       eng->dNbr, eng->dVisc, curl, eng->K, eng->S, eng->ES, eng->ops, eng->ph, dtl,
                        eng->mc);
 }
 
@@ -618,7 +629,7 @@ void launch_volume_e(hx3d_engine *eng, double a_k, double c_k, int update, const
     constexpr int TPB = ((EPB * ne + 63) / 64) * 64;
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(elem_grid(eng, EPB)), dim3(TPB), 0, eng->stream, eng->dQ, eng->dQn, eng->dVisc,
-                           eng->dEdelta, eng->dEfdelta, eng->dNbx, eng->dEgeo, eng->t2x ? 1 : 0, eng->dJa, eng->dJ, eng->dG, qdot, a_k, c_k,
+                           eng->dEdelta, eng->dEfdelta, eng->dNbx, metric(eng), eng->t2x ? 1 : 0, eng->dG, qdot, a_k, c_k,
                            update, dta, eng->K, eng->S, eng->ES, eng->ops, eng->ph, eng->mc);
     };
     const bool lxf = eng->ph.riemann == HX3D_RIEMANN_LXF, les = eng->ph.les != 0;
@@ -756,7 +767,7 @@ void launch_mvolume(hx3d_engine *eng, double a_k, double c_k, int update, const 
     if (eng->ntiles_s) {
         auto *k = eng->ph.les ? &hxm::km_volume<FORM, GAUSS, true, hxm::TILE_SMALL> : &hxm::km_volume<FORM, GAUSS, false, hxm::TILE_SMALL>;
         hipLaunchKernelGGL(k, dim3(eng->grid_mvol_s), dim3(hxm::TILE_SMALL), mvolume_lds<FORM>(hxm::TILE_SMALL), eng->stream,
-                           eng->dTmap, eng->ntiles_s, eng->dQ, eng->dU, eng->dJa, eng->dJ, eng->dEdelta, eng->dFe,
+                           eng->dTmap, eng->ntiles_s, eng->dQ, eng->dU, metric(eng), eng->dEdelta, eng->dFe,
                            eng->dOpsAll, eng->dG, qdot, a_k, c_k, update, dta, eng->S, eng->ES, eng->ph);
     }
     if (eng->ntiles_b) {
@@ -764,7 +775,7 @@ void launch_mvolume(hx3d_engine *eng, double a_k, double c_k, int update, const 
         if (eng->ntiles_s) db.time = nullptr;
         auto *k = eng->ph.les ? &hxm::km_volume<FORM, GAUSS, true, hxm::TILE> : &hxm::km_volume<FORM, GAUSS, false, hxm::TILE>;
         hipLaunchKernelGGL(k, dim3(eng->grid_mvol_b), dim3(hxm::TILE), mvolume_lds<FORM>(hxm::TILE), eng->stream,
-                           eng->dTmap + eng->map_big, eng->ntiles_b, eng->dQ, eng->dU, eng->dJa, eng->dJ, eng->dEdelta,
+                           eng->dTmap + eng->map_big, eng->ntiles_b, eng->dQ, eng->dU, metric(eng), eng->dEdelta,
                            eng->dFe, eng->dOpsAll, eng->dG, qdot, a_k, c_k, update, db, eng->S, eng->ES, eng->ph);
     }
 }
@@ -778,23 +789,23 @@ void stage_mixed_nodes(hx3d_engine *eng, double a_k, double c_k, int update, con
     hxk::DtLimits lim = dta.lim;
     if (!eng->ph.euler) {
         hipLaunchKernelGGL(hxm::km_face_grad<GAUSS>, dim3(grid_for(eng->nwaves)), dim3(64), 0, eng->stream, eng->dQ,
-                           eng->dFaces, eng->dSched, eng->dFgeo, eng->dOpsAll, eng->dLift, eng->nwaves, eng->S, eng->ES, eng->FSm);
+                           eng->dFaces, eng->dSched, eng->dFgeo, eng->per_face, eng->dOpsAll, eng->dLift, eng->nwaves, eng->S, eng->ES, eng->fgeo_stride);
         // dt partials: the small tiles' blocks first, then the large tiles'
         if (eng->ntiles_s)
             hipLaunchKernelGGL((hxm::km_grad<GAUSS, hxm::TILE_SMALL>), dim3(eng->grid_mgrad_s), dim3(hxm::TILE_SMALL),
                                mgrad_lds(hxm::TILE_SMALL), eng->stream, eng->dTmap, eng->ntiles_s, eng->dQ,
-                               eng->dJa, eng->dJ, eng->dLift, eng->dOpsAll, eng->dU, eng->S, eng->ES, eng->ph, lim, 0);
+                               metric(eng), eng->dLift, eng->dOpsAll, eng->dU, eng->S, eng->ES, eng->ph, lim, 0);
         if (eng->ntiles_b)
             hipLaunchKernelGGL((hxm::km_grad<GAUSS, hxm::TILE>), dim3(eng->grid_mgrad_b), dim3(hxm::TILE),
                                mgrad_lds(hxm::TILE), eng->stream, eng->dTmap + eng->map_big, eng->ntiles_b, eng->dQ,
-                               eng->dJa, eng->dJ, eng->dLift, eng->dOpsAll, eng->dU, eng->S, eng->ES,
+                               metric(eng), eng->dLift, eng->dOpsAll, eng->dU, eng->S, eng->ES,
                                eng->ph, lim, eng->grid_mgrad_s);
     }
     if (ev) (void)hipEventRecord(ev[1], eng->stream);
     auto *face = eng->ph.les ? &hxm::km_face<GAUSS, true> : &hxm::km_face<GAUSS, false>;
     hipLaunchKernelGGL(face, dim3(grid_for(eng->nwaves)), dim3(64), 0, eng->stream, eng->dQ, eng->dU, eng->dFaces,
-                       eng->dSched, eng->dFgeo, eng->dFdelta, eng->dOpsAll, eng->dFe, eng->nwaves, eng->S, eng->ES,
-                       eng->FSm, eng->ph, dta.red);
+                       eng->dSched, eng->dFgeo, eng->per_face, eng->dFdelta, eng->dOpsAll, eng->dFe, eng->nwaves, eng->S, eng->ES,
+                       eng->fgeo_stride, eng->ph, dta.red);
     if (ev) (void)hipEventRecord(ev[2], eng->stream);
     if (GAUSS) launch_mvolume<hxk::FORM_STANDARD, true>(eng, a_k, c_k, update, dta, qdot);
     else if (eng->inviscid != HX3D_INVISCID_SPLIT) launch_mvolume<hxk::FORM_STANDARD>(eng, a_k, c_k, update, dta, qdot);
@@ -1055,6 +1066,24 @@ int set_tiles(hx3d_engine *eng, int policy)
     return HX3D_OK;
 }
 
+// The metric terms once per element, where every node of each element has the same bits (straight
+// elements; a mesh read from a file has metrics that differ in the last bits and keeps them by node):
+// planes of stride eng->elem_stride behind those by node, ja[9*S + c*stride + e], J at c = 9.
+void element_metrics(hx3d_engine *eng, const hx3d_case_desc *d, const std::vector<long> &off, std::vector<double> &ja)
+{
+    const int K = eng->K;
+    for (int e = 0; e < K; ++e)
+        for (long g = off[e] + 1; g < off[e + 1]; ++g)
+            if (std::memcmp(d->Ja + 9 * g, d->Ja + 9 * off[e], 9 * sizeof(double)) || std::memcmp(d->J + g, d->J + off[e], sizeof(double)))
+                return;
+    const long stride = ((K + 63) / 64) * 64, base = ja.size();
+    ja.resize(base + 10 * stride, 1.0);
+    for (int c = 0; c < 10; ++c)
+        for (int e = 0; e < K; ++e) ja[base + c * stride + e] = c < 9 ? d->Ja[9 * off[e] + c] : d->J[off[e]];
+    eng->elem_stride = stride;
+    eng->per_elem = 1;
+}
+
 // Whether a face node's second tangent t2 is n x t1 with vCross's arithmetic (MappedGeometry.f90:745,
 // :807-817), bit for bit.  The reference's geometry and the mesh front end's are at every face node;
 // a descriptor with other tangents keeps them, read by the volume kernel.
@@ -1214,8 +1243,11 @@ int create_mixed(hx3d_engine *eng, const hx3d_case_desc *d)
                 }
         edelta[e] = std::pow(vol / (nx * ny * nz), 1.0 / 3.0);
     }
+    bool constant = true;   // the face geometry, over each face's nodes
+    auto same = [](const double *a, const double *b, int n) { return !std::memcmp(a, b, n * sizeof(double)); };
     for (int f = 0; f < F; ++f) {
         const int Nf0 = shapes[f] & 7, Nf1 = shapes[f] >> 3 & 7;
+        const long q0 = faces[f].foff;
         double surf = 0.0;
         for (int j = 0; j <= Nf1; ++j)
             for (int i = 0; i <= Nf0; ++i) {
@@ -1226,9 +1258,19 @@ int create_mixed(hx3d_engine *eng, const hx3d_case_desc *d)
                     fgeo[(size_t)(6 + c) * fsm + q] = d->fT2[3 * q + c];
                 }
                 fgeo[(size_t)9 * fsm + q] = d->fJac[q];
+                constant = constant && same(d->fNormal + 3 * q, d->fNormal + 3 * q0, 3) && same(d->fT1 + 3 * q, d->fT1 + 3 * q0, 3) &&
+                           same(d->fT2 + 3 * q, d->fT2 + 3 * q0, 3) && same(d->fJac + q, d->fJac + q0, 1);
                 surf += wn[Nf0][i] * wn[Nf1][j] * d->fJac[q];
             }
         fdelta[f] = std::sqrt(surf / ((Nf0 + 1) * (Nf1 + 1)));
+    }
+    eng->per_face = constant ? 1 : 0;
+    eng->fgeo_stride = constant ? F : fsm;
+    if (constant) {
+        std::vector<double> one((size_t)10 * F);
+        for (int c = 0; c < 10; ++c)
+            for (int f = 0; f < F; ++f) one[(size_t)c * F + f] = fgeo[(size_t)c * fsm + faces[f].foff];
+        fgeo.swap(one);
     }
     {
         // the volume kernel keeps three directions of fluxes (+ two-point node data and a metric
@@ -1242,12 +1284,13 @@ int create_mixed(hx3d_engine *eng, const hx3d_case_desc *d)
         if ((long)sizeof(double) * (per_node * hxm::TILE + 2 * hxm::MAXN1 * 64) > maxlds)
             return eng->fail(HX3D_EUNSUPPORTED, "a tile of elements needs more LDS than a block may use");
     }
+    element_metrics(eng, d, off, ja);
     eng->N3h_mixed = N3;
     int rc;
     if ((rc = dalloc(eng, &eng->dQ, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dG, (size_t)NV * S)) ||
-        (rc = dalloc(eng, &eng->dU, (size_t)15 * S)) || (rc = dalloc(eng, &eng->dJa, (size_t)9 * S)) ||
+        (rc = dalloc(eng, &eng->dU, (size_t)15 * S)) || (rc = dalloc(eng, &eng->dJa, ja.size())) ||
         (rc = dalloc(eng, &eng->dWq, (size_t)S)) ||
-        (rc = dalloc(eng, &eng->dJ, (size_t)S)) || (rc = dalloc(eng, &eng->dFgeo, (size_t)10 * fsm)) ||
+        (rc = dalloc(eng, &eng->dJ, (size_t)S)) || (rc = dalloc(eng, &eng->dFgeo, fgeo.size())) ||
         (rc = dalloc(eng, &eng->dFe, (size_t)NV * ES)) || (rc = dalloc(eng, &eng->dLift, (size_t)15 * ES)) ||
         (rc = dalloc(eng, &eng->dQDot, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dEdelta, (size_t)K)) ||
         (rc = dalloc(eng, &eng->dFdelta, (size_t)F)) || (rc = dalloc(eng, &eng->dScal, 4)) ||
@@ -1490,9 +1533,12 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
     };
     eng->t2x = lxf;
     double fr[10][64];
+    bool constant = !eng->gauss;   // the frames, over each face's nodes (the Gauss kernels read them by node)
     for (int f = 0; f < F; ++f) {
         face_frame(f, fr);
         put_frame(f, fr, 0, lxf ? 7 : 4);
+        for (int c = 0; c < (lxf ? 10 : 4) && constant; ++c)
+            for (int x = 1; x < nf && constant; ++x) constant = !std::memcmp(&fr[c][x], &fr[c][0], sizeof(double));
         double surf = 0.0;
         for (int x = 0; x < nf; ++x) surf += wg[x % n1] * wg[x / n1] * fr[3][x];
         // SD.f90:1378, at both elements' slots of the face
@@ -1508,11 +1554,24 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
         }
     for (int c = 0; c < gplanes; ++c)   // the padding past the last face node
         for (long x = (long)K * 6 * nf; x < ES; ++x) egeo[(size_t)c * ES + x] = 0.0;
+    eng->per_face = constant ? 1 : 0;
+    eng->egeo_stride = ES;
+    if (constant) {
+        const long stride = ((6L * K + 63) / 64) * 64;
+        for (int c = 0; c < gplanes; ++c)   // in place: plane c's first nodes lie at or behind their new places
+            for (long x = 0; x < stride; ++x) egeo[(size_t)c * stride + x] = x < 6L * K ? egeo[(size_t)c * ES + x * nf] : 0.0;
+        eng->egeo_stride = stride;
+    }
+    if (!eng->gauss) {
+        std::vector<long> off(K + 1);
+        for (int e = 0; e <= K; ++e) off[e] = (long)e * ne;
+        element_metrics(eng, d, off, ja);
+    }
     // ---- device -------------------------------------------------------------------
     int rc;
     if ((rc = dalloc(eng, &eng->dQ, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dG, (size_t)NV * S)) ||
-        (rc = dalloc(eng, &eng->dJa, (size_t)9 * S)) || (rc = dalloc(eng, &eng->dWq, (size_t)S)) ||
-        (rc = dalloc(eng, &eng->dJ, (size_t)S)) || (rc = dalloc(eng, &eng->dEgeo, (size_t)gplanes * ES)) ||
+        (rc = dalloc(eng, &eng->dJa, ja.size())) || (rc = dalloc(eng, &eng->dWq, (size_t)S)) ||
+        (rc = dalloc(eng, &eng->dJ, (size_t)S)) || (rc = dalloc(eng, &eng->dEgeo, (size_t)gplanes * eng->egeo_stride)) ||
         (rc = dalloc(eng, &eng->dQDot, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dEdelta, (size_t)K)) ||
         (rc = dalloc(eng, &eng->dScal, 4)) || (rc = dalloc(eng, &eng->dPart, (size_t)NV * ((S + 255) / 256 + 1))) ||
         (rc = dalloc(eng, &eng->dDtPart, (size_t)2 * (std::max((long)K, (S + 255) / 256) + 64))) ||
@@ -1537,7 +1596,7 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
     };
     if (!up(eng->dJa, ja.data(), ja.size() * 8) || !up(eng->dJ, jj.data(), jj.size() * 8) ||
         !up(eng->dWq, wq.data(), wq.size() * 8) || !up(eng->dEdelta, edelta.data(), edelta.size() * 8) ||
-        !up(eng->dEgeo, egeo.get(), (size_t)gplanes * ES * 8) || !up(eng->dNbx, nbx.data(), nbx.size() * 4) ||
+        !up(eng->dEgeo, egeo.get(), (size_t)gplanes * eng->egeo_stride * 8) || !up(eng->dNbx, nbx.data(), nbx.size() * 4) ||
         !up(eng->dEfdelta, efdelta.data(), efdelta.size() * 8) ||
         (!eng->gauss && !up(eng->dNbr, nbr.data(), nbr.size() * 4)))
         return bail(eng->fail(HX3D_EDEVICE, "upload failed"));

@@ -413,7 +413,7 @@ __device__ __forceinline__ FaceLane face_lane(const int4 s, int lane)
 template <bool GAUSS>
 __global__ void __launch_bounds__(64)
 km_face_grad(const double *__restrict__ Q, const FaceRec *__restrict__ faces, const int4 *__restrict__ sched,
-             const double *__restrict__ fgeo, const OpsAll *__restrict__ opsp, double *__restrict__ lift, int W,
+             const double *__restrict__ fgeo, int fc, const OpsAll *__restrict__ opsp, double *__restrict__ lift, int W,
              long S, long ES, long FSm)
 {
     // LDS: both sides' Q traces, then one direction's unStar in their place; the mortar
@@ -452,7 +452,7 @@ km_face_grad(const double *__restrict__ Q, const FaceRec *__restrict__ faces, co
     grid_ij(ql, r.Nf0 + 1, i, j);
     const bool on = j <= r.Nf1;
     if (!on) { i = 0; j = 0; }
-    const long fq = f.foff + (on ? ql : 0);
+    const long fq = fc ? (long)fl.f : f.foff + (on ? ql : 0);
     double nrm[3];
     nrm[0] = fgeo[fq];
     nrm[1] = fgeo[FSm + fq];
@@ -508,8 +508,8 @@ km_face_grad(const double *__restrict__ Q, const FaceRec *__restrict__ faces, co
 // ------------------------------------------------------------------------------------
 template <bool GAUSS, int T>
 __global__ void __launch_bounds__(T)
-km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__ Q, const double *__restrict__ Ja,
-        const double *__restrict__ Jac, const double *__restrict__ lift, const OpsAll *__restrict__ opsp,
+km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__ Q, hxk::Metric mt,
+        const double *__restrict__ lift, const OpsAll *__restrict__ opsp,
         double *__restrict__ U, long S, long ES, Phys ph, hxk::DtLimits dtl, int pbase)
 {
     HIP_DYNAMIC_SHARED(double, smem)
@@ -533,8 +533,8 @@ km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__
 #pragma unroll
     for (int v = 0; v < NV; ++v) q[v] = hxk::ldg(Q + v * S, g);
 #pragma unroll
-    for (int c = 0; c < 9; ++c) ja[c] = hxk::ldg(Ja + c * S, g);
-    const double jg = hxk::ldg(Jac, g);
+    for (int c = 0; c < 9; ++c) ja[c] = hxk::ldg(mt.Ja + c * mt.S, mt.node(nm.e, g));
+    const double jg = hxk::ldg(mt.J, mt.node(nm.e, g));
     if (tile + (int)gridDim.x < ntiles) nm = load_map<T>(tmap, tile + gridDim.x, t);   // the next tile's
     const double iJ = 1.0 / jg;   // the same bits as a stored 1/J
     const bool onx = i == 0 || i == Nx, ony = j == 0 || j == Ny, onz = k == 0 || k == Nz;
@@ -645,7 +645,7 @@ km_grad(const NodeMap *__restrict__ tmap, int ntiles, const double *__restrict__
 template <bool GAUSS, bool LES>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
 km_face(const double *__restrict__ Q, const double *__restrict__ U, const FaceRec *__restrict__ faces,
-        const int4 *__restrict__ sched, const double *__restrict__ fgeo, const double *__restrict__ fdelta,
+        const int4 *__restrict__ sched, const double *__restrict__ fgeo, int fc, const double *__restrict__ fdelta,
         const OpsAll *__restrict__ opsp, double *__restrict__ fe, int W, long S, long ES, long FSm, Phys ph,
         hxk::DtReduce dtr)
 {
@@ -693,7 +693,7 @@ km_face(const double *__restrict__ Q, const double *__restrict__ U, const FaceRe
     grid_ij(ql, r.Nf0 + 1, i, j);
     const bool on = j <= r.Nf1;
     if (!on) { i = 0; j = 0; }
-    const long fq = f.foff + (on ? ql : 0);
+    const long fq = fc ? (long)fl.f : f.foff + (on ? ql : 0);
     double nrm[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) nrm[c] = fgeo[c * FSm + fq];
@@ -812,7 +812,7 @@ constexpr int mvolume_per_node()
 template <int FORM, bool GAUSS, bool LES, int T>
 __global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(FORM < 0 && !GAUSS && !LES ? 4 : 2)))
 km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, const double *__restrict__ U,
-          const double *__restrict__ Ja, const double *__restrict__ Jac, const double *__restrict__ edelta,
+          hxk::Metric mt, const double *__restrict__ edelta,
           const double *__restrict__ fe, const OpsAll *__restrict__ opsp, double *__restrict__ G,
           double *__restrict__ qdot_out, double a_k, double c_k, int update, DtArgs dta, long S, long ES,
           Phys ph)
@@ -852,13 +852,13 @@ km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, 
 #pragma unroll
     for (int v = 0; v < NV; ++v) q[v] = hxk::ldg(Q + v * S, g);
 #pragma unroll
-    for (int c = 0; c < 9; ++c) ja[c] = hxk::ldg(Ja + c * S, g);
+    for (int c = 0; c < 9; ++c) ja[c] = hxk::ldg(mt.Ja + c * mt.S, mt.node(e, g));
 #pragma unroll
     for (int d = 0; d < 3; ++d)
 #pragma unroll
         for (int v = 0; v < NV; ++v) gq[d][v] = hxk::ldg(U + (d * NV + v) * S, g);
     const double dl = hxk::ldg(edelta, (unsigned)e);
-    const double jg = hxk::ldg(Jac, g);
+    const double jg = hxk::ldg(mt.J, mt.node(e, g));
     if (tile + (int)gridDim.x < ntiles) nm = load_map<T>(tmap, tile + gridDim.x, t);   // the next tile's
     double xs[NV];   // the node's surface integral
     const ElemFaces ef = elem_faces(ef0, nx, ny, nz);
@@ -906,9 +906,9 @@ km_volume(const NodeMap *__restrict__ tmap, int ntiles, double *__restrict__ Q, 
             hx::viscous_state(ph, q, gq[0], gq[1], gq[2], vg);
             hx::laminar_mu_kappa(ph, q, mu, kappa);
             if (LES) {
-                const double mt = hx::les_mu(ph, dl, q[0], hx::les_factor(ph, q, gq[0], gq[1], gq[2]));
-                mu = mu + mt;
-                kappa = kappa + mt * ph.mu_to_kappa;
+                const double mut = hx::les_mu(ph, dl, q[0], hx::les_factor(ph, q, gq[0], gq[1], gq[2]));
+                mu = mu + mut;
+                kappa = kappa + mut * ph.mu_to_kappa;
             }
             const double ir = 1.0 / q[0];
             hx::stress_shape(vg, sh);

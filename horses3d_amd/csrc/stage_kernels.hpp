@@ -169,7 +169,7 @@ __device__ __forceinline__ unsigned efx(int e, int slot, int a, int b)
 // kernel's faces and nodes read it, and neither forms a viscosity), or with LES what it is formed
 // from (viscous_values).
 //   nbr[x]         2 * (neighbour's node) + (1 if this element is the face's right side)
-//   egeo[c*ES+x]   face normal (c = 0..2) and surface Jacobian |Ja| (c = 3) of the face
+//   mt             metric terms; face frames: normal (c = 0..2) and surface Jacobian |Ja| (c = 3)
 //   visc[c*S+g]    out: the viscous flux tensor or the LES values
 // ------------------------------------------------------------------------------------
 #ifndef HX3D_GRAD_WAVES
@@ -178,6 +178,23 @@ __device__ __forceinline__ unsigned efx(int e, int slot, int a, int b)
 
 // The gradient at node (i, j, k) of the element whose state is sQ[v*ne + m] (LDS), in the
 // reference's order: with u_d = sum_l D(own, l) q(l) along reference direction d,
+// Metric terms of a case of one order: Ja^d_c in planes Ja[c*S + i], J[i], and the face frames
+// face[c*FS + i].  Where they are the same bits at every node of each element (each face), as on boxes of
+// straight elements, they are stored and read once per element (per face): i is the element (the
+// element face) then, else the node.  The wave's loads fall on one line each and the planes
+// stay in the caches: 80 bytes less of 208 per node for the gradient kernel, 80 of 312 and 32..80 of
+// 280 per face node for the volume kernel.  9^3 elements of order 6: k_grad 26.0 -> 24.2 us, k_volume
+// 35.5 -> 32.5; 64 cases of 4^3, order 3: 16.2 -> 14.7 and 25.4 -> 23.0; 20^3, orders 2..7: km_grad 133 ->
+// 121, km_volume 123 -> 109.  By node where they vary (curved elements) there is no other way.
+struct Metric {
+    const double *Ja, *J, *face;
+    long S, FS;
+    int per_elem, per_face;
+    __device__ __forceinline__ unsigned node(int e, unsigned g) const { return per_elem ? (unsigned)e : g; }
+    template <int NF2>
+    __device__ __forceinline__ unsigned face_node(unsigned x) const { return per_face ? x / NF2 : x; }
+};
+
 // gr[c][v] = (sum_d u_d Ja^d_c) / J + gr[c][v] / J, the lifting sums given in gr.  One variable at a
 // time, its results pinned (hold), so that the sums of a variable, not of all five, hold registers
 // (k_volume at N = 4: 255 registers with all in flight).
@@ -243,8 +260,7 @@ __device__ __forceinline__ void les_tensor(const Phys &ph, const double *q, doub
 template <int N, int EPB>
 __global__ void __launch_bounds__(((EPB * (N + 1) * (N + 1) * (N + 1) + 63) / 64) * 64)
 __attribute__((amdgpu_waves_per_eu(HX3D_GRAD_WAVES)))
-k_grad(const double *__restrict__ Q, const double *__restrict__ Ja, const double *__restrict__ Jac,
-       const int *__restrict__ nbr, const double *__restrict__ egeo,
+k_grad(const double *__restrict__ Q, Metric mt, const int *__restrict__ nbr,
        double *__restrict__ visc, double *__restrict__ curl_out, int K, long S, long ES, Ops ops, Phys ph, DtLimits dtl, Multi mc)
 {
     constexpr int n1 = N + 1, nf = n1 * n1, ne = nf * n1;
@@ -275,12 +291,13 @@ k_grad(const double *__restrict__ Q, const double *__restrict__ Ja, const double
 #pragma unroll
     for (int v = 0; v < NV; ++v) q[v] = ldg(Q + v * S, gc);
 #pragma unroll
-    for (int c = 0; c < 9; ++c) ja[c] = ldg(Ja + c * S, gc);
-    const double jg = ldg(Jac, gc);
+    for (int c = 0; c < 9; ++c) ja[c] = ldg(mt.Ja + c * mt.S, mt.node(ec, gc));
+    const double jg = ldg(mt.J, mt.node(ec, gc));
     const double iJ = 1.0 / jg;   // the same bits as a stored 1/J
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-        const double a = ldg(egeo + c * ES, fx), b = ldg(egeo + c * ES, fy), d = ldg(egeo + c * ES, fz);
+        const double a = ldg(mt.face + c * mt.FS, mt.face_node<nf>(fx)), b = ldg(mt.face + c * mt.FS, mt.face_node<nf>(fy)),
+                     d = ldg(mt.face + c * mt.FS, mt.face_node<nf>(fz));
         gx[c] = onx ? a : 0.0;
         gy[c] = ony ? b : 0.0;
         gz[c] = onz ? d : 0.0;
@@ -550,8 +567,7 @@ __global__ void __launch_bounds__(((EPB * (N + 1) * (N + 1) * (N + 1) + 63) / 64
 __attribute__((amdgpu_waves_per_eu(volume_waves(N, FORM))))
 k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__restrict__ visc,
          const double *__restrict__ edelta, const double *__restrict__ efdelta, const int *__restrict__ nbx,
-         const double *__restrict__ egeo, int t2x, const double *__restrict__ Ja,
-         const double *__restrict__ Jac, double *__restrict__ G, double *__restrict__ qdot_out, double a_k, double c_k, int update,
+         Metric mt, int t2x, double *__restrict__ G, double *__restrict__ qdot_out, double a_k, double c_k, int update,
          DtArgs dta, int K, long S, long ES, Ops ops, Phys ph, Multi mc)
 {
     using L = VolumeLds<N, EPB, FORM, LES>;
@@ -614,8 +630,8 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
         sSlot[t] = a == b ? 0 : pair_slot(n1, a < b ? a : b, a < b ? b : a) * NV * nf;
     }
 #pragma unroll
-    for (int c = 0; c < 9; ++c) ja[c] = ldg(Ja + c * S, gc);
-    const double jg = ldg(Jac, gc), dl = LES ? ldg(edelta, (unsigned)ec) : 0.0;
+    for (int c = 0; c < 9; ++c) ja[c] = ldg(mt.Ja + c * mt.S, mt.node(ec, gc));
+    const double jg = ldg(mt.J, mt.node(ec, gc)), dl = LES ? ldg(edelta, (unsigned)ec) : 0.0;
     const double b0 = 1.0 / ops.w[0];
     // What round p's face flux reads from memory; round 0's is asked for before the barrier, to
     // arrive with the element's own data.
@@ -627,8 +643,8 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
 #pragma unroll
         for (int v = 0; v < NV; ++v) qR[v] = ldg(Q + v * S, gn);
 #pragma unroll
-        for (int c = 0; c < 3; ++c) nrm[c] = ldg(egeo + c * ES, x);
-        jac = ldg(egeo + 3 * ES, x);
+        for (int c = 0; c < 3; ++c) nrm[c] = ldg(mt.face + c * mt.FS, mt.face_node<nf>(x));
+        jac = ldg(mt.face + 3 * mt.FS, mt.face_node<nf>(x));
         if (!ph.euler) {
 #pragma unroll
             for (int c = 0; c < NVT; ++c) fn[c] = ldg(visc + c * S, gn);
@@ -636,7 +652,7 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
         if (LES) fd = ldg(efdelta, x / nf);
         if (LXF) {
 #pragma unroll
-            for (int c = 0; c < 3; ++c) t1[c] = ldg(egeo + (4 + c) * ES, x);
+            for (int c = 0; c < 3; ++c) t1[c] = ldg(mt.face + (4 + c) * mt.FS, mt.face_node<nf>(x));
         }
     };
     load_face(0);
@@ -702,9 +718,9 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
                 // bit for bit at every face node (checked on the host), so it is formed here
                 double t2[3];
                 if (!t2x) {
-                    const unsigned x = (unsigned)e0 * NI + it;
+                    const unsigned x = mt.face_node<nf>((unsigned)e0 * NI + it);
 #pragma unroll
-                    for (int c = 0; c < 3; ++c) t2[c] = ldg(egeo + (7 + c) * ES, x);
+                    for (int c = 0; c < 3; ++c) t2[c] = ldg(mt.face + (7 + c) * mt.FS, x);
                 } else {
                     t2[0] = nrm[1] * t1[2] - t1[1] * nrm[2];
                     t2[1] = nrm[2] * t1[0] - t1[2] * nrm[0];
