@@ -617,7 +617,8 @@ void launch_grad(hx3d_engine *eng, const hxk::DtLimits &dtl, double *curl)
 {
     constexpr int EPB = epb_for(N), ne = (N + 1) * (N + 1) * (N + 1);
     constexpr int TPB = ((EPB * ne + 63) / 64) * 64;
-    hipLaunchKernelGGL((hxk::k_grad<N, EPB>), dim3(elem_grid(eng, EPB)), dim3(TPB), 0, eng->stream, eng->dQ, metric(eng),
+    auto *kernel = eng->ph.les ? &hxk::k_grad<N, EPB, true> : &hxk::k_grad<N, EPB, false>;
+    hipLaunchKernelGGL(kernel, dim3(elem_grid(eng, EPB)), dim3(TPB), 0, eng->stream, eng->dQ, metric(eng),
                        eng->dNbr, eng->dVisc, curl, eng->K, eng->S, eng->ES, eng->ops, eng->ph, dtl,
                        eng->mc);
 }
@@ -628,7 +629,8 @@ void launch_volume_e(hx3d_engine *eng, double a_k, double c_k, int update, const
     constexpr int ne = (N + 1) * (N + 1) * (N + 1);
     constexpr int TPB = ((EPB * ne + 63) / 64) * 64;
     auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(elem_grid(eng, EPB)), dim3(TPB), 0, eng->stream, eng->dQ, eng->dQn, eng->dVisc,
+        const size_t lds = sizeof(double) * (eng->ph.les ? hxk::VolumeLds<N, EPB, FORM, true>::SIZE : hxk::VolumeLds<N, EPB, FORM, false>::SIZE);
+        hipLaunchKernelGGL(kernel, dim3(elem_grid(eng, EPB)), dim3(TPB), lds, eng->stream, eng->dQ, eng->dQn, eng->dVisc,
                            eng->dEdelta, eng->dEfdelta, eng->dNbx, metric(eng), eng->t2x ? 1 : 0, eng->dG, qdot, a_k, c_k,
                            update, dta, eng->K, eng->S, eng->ES, eng->ops, eng->ph, eng->mc);
     };

@@ -172,12 +172,15 @@ __device__ __forceinline__ unsigned efx(int e, int slot, int a, int b)
 //   mt             metric terms; face frames: normal (c = 0..2) and surface Jacobian |Ja| (c = 3)
 //   visc[c*S+g]    out: the viscous flux tensor or the LES values
 // ------------------------------------------------------------------------------------
+// Registers: at most 128 (the state is read again after the gradient, LES is a template flag, and
+// order 7 takes its directions one at a time), since a block of six or eight waves finds room beside
+// another only at four waves per SIMD: 9^3 elements of order 6 24.0 -> 19.9 us, of order 7 31.6 -> 25.7 (with
+// LES).  Below that it makes no difference: at 16^3 elements of order 4 the kernel moves 153 MB in 28.4 us, 24^3
+// of order 5 898 MB in 193 us, near the copy rate (6.9 TB/s from the caches, 5 from memory).
 #ifndef HX3D_GRAD_WAVES
 #define HX3D_GRAD_WAVES 1
 #endif
 
-// The gradient at node (i, j, k) of the element whose state is sQ[v*ne + m] (LDS), in the
-// reference's order: with u_d = sum_l D(own, l) q(l) along reference direction d,
 // Metric terms of a case of one order: Ja^d_c in planes Ja[c*S + i], J[i], and the face frames
 // face[c*FS + i].  Where they are the same bits at every node of each element (each face), as on boxes of
 // straight elements, they are stored and read once per element (per face): i is the element (the
@@ -195,6 +198,8 @@ struct Metric {
     __device__ __forceinline__ unsigned face_node(unsigned x) const { return per_face ? x / NF2 : x; }
 };
 
+// The gradient at node (i, j, k) of the element whose state is sQ[v*ne + m] (LDS), in the
+// reference's order: with u_d = sum_l D(own, l) q(l) along reference direction d,
 // gr[c][v] = (sum_d u_d Ja^d_c) / J + gr[c][v] / J, the lifting sums given in gr.  One variable at a
 // time, its results pinned (hold), so that the sums of a variable, not of all five, hold registers
 // (k_volume at N = 4: 255 registers with all in flight).
@@ -203,25 +208,51 @@ __device__ __forceinline__ void element_gradient(const double *sQ, const double 
                                                  const double *ja, double iJ, double (*gr)[NV])
 {
     constexpr int nf = n1 * n1, ne = nf * n1;
-    double dx[n1], dy[n1], dz[n1];
-#pragma unroll
-    for (int l = 0; l < n1; ++l) { dx[l] = sD[i * n1 + l]; dy[l] = sD[j * n1 + l]; dz[l] = sD[k * n1 + l]; }
     const double *lx = sQ + n1 * (j + n1 * k), *ly = sQ + i + nf * k, *lz = sQ + i + n1 * j;
+    if constexpr (n1 < 8) {
+        double dx[n1], dy[n1], dz[n1];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        double u0 = 0.0, u1 = 0.0, u2 = 0.0;
+        for (int l = 0; l < n1; ++l) { dx[l] = sD[i * n1 + l]; dy[l] = sD[j * n1 + l]; dz[l] = sD[k * n1 + l]; }
 #pragma unroll
-        for (int l = 0; l < n1; ++l) {
-            u0 = u0 + lx[v * ne + l] * dx[l];
-            u1 = u1 + ly[v * ne + n1 * l] * dy[l];
-            u2 = u2 + lz[v * ne + nf * l] * dz[l];
+        for (int v = 0; v < NV; ++v) {
+            double u0 = 0.0, u1 = 0.0, u2 = 0.0;
+#pragma unroll
+            for (int l = 0; l < n1; ++l) {
+                u0 = u0 + lx[v * ne + l] * dx[l];
+                u1 = u1 + ly[v * ne + n1 * l] * dy[l];
+                u2 = u2 + lz[v * ne + nf * l] * dz[l];
+            }
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                gr[c][v] = (u0 * ja[c] + u1 * ja[3 + c] + u2 * ja[6 + c]) * iJ + gr[c][v] * iJ;
+                hold(gr[c][v]);
+            }
+            sched_fence();
         }
+    } else {
+        // order 7: a direction at a time, so that one row of the operator holds registers, not three
+        double u[3][NV];
+        auto along = [&](double *ud, const double *line, const double *row, int step) {
+            double w[n1];
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            gr[c][v] = (u0 * ja[c] + u1 * ja[3 + c] + u2 * ja[6 + c]) * iJ + gr[c][v] * iJ;
-            hold(gr[c][v]);
-        }
-        sched_fence();
+            for (int l = 0; l < n1; ++l) w[l] = row[l];
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                ud[v] = 0.0;
+#pragma unroll
+                for (int l = 0; l < n1; ++l) ud[v] = ud[v] + line[v * ne + step * l] * w[l];
+                hold(ud[v]);
+            }
+            sched_fence();
+        };
+        along(u[0], lx, sD + i * n1, 1);
+        along(u[1], ly, sD + j * n1, n1);
+        along(u[2], lz, sD + k * n1, nf);
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+                gr[c][v] = (u[0][v] * ja[c] + u[1][v] * ja[3 + c] + u[2][v] * ja[6 + c]) * iJ + gr[c][v] * iJ;
     }
 }
 
@@ -257,7 +288,7 @@ __device__ __forceinline__ void les_tensor(const Phys &ph, const double *q, doub
     hx::viscous_tensor(mu, kappa, q[1] * ir, q[2] * ir, q[3] * ir, x, x + 6, f);
 }
 
-template <int N, int EPB>
+template <int N, int EPB, bool LES>
 __global__ void __launch_bounds__(((EPB * (N + 1) * (N + 1) * (N + 1) + 63) / 64) * 64)
 __attribute__((amdgpu_waves_per_eu(HX3D_GRAD_WAVES)))
 k_grad(const double *__restrict__ Q, Metric mt, const int *__restrict__ nbr,
@@ -330,9 +361,20 @@ k_grad(const double *__restrict__ Q, Metric mt, const int *__restrict__ nbr,
         lift_face(q, qx, gx, cx & 1 ? -gx[3] : gx[3], b0, gr);
         lift_face(q, qy, gy, cy & 1 ? -gy[3] : gy[3], b0, gr);
         lift_face(q, qz, gz, cz & 1 ? -gz[3] : gz[3], b0, gr);
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+            for (int v = 0; v < NV; ++v) hold(gr[d][v]);
+        sched_fence();
         element_gradient<n1>(&sQ[el][0][0], sD, i, j, k, ja, iJ, gr);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) q[v] = *(const volatile double *)&sQ[el][v][n];   // again: not held through the gradient
         double vg[12], sh[6], mu, kappa, X = 0.0;
-        if (ph.les) X = hx::les_factor(ph, q, gr[0], gr[1], gr[2]);
+        if (LES) {
+            X = hx::les_factor(ph, q, gr[0], gr[1], gr[2]);
+            hold(X);
+            sched_fence();
+        }
         hx::viscous_state(ph, q, gr[0], gr[1], gr[2], vg);
         if (curl_out) {   // |curl u|^2 of the enstrophy monitor
             const double a = vg[5] - vg[7], b = vg[6] - vg[2], c = vg[1] - vg[3];
@@ -340,7 +382,7 @@ k_grad(const double *__restrict__ Q, Metric mt, const int *__restrict__ nbr,
         }
         hx::laminar_mu_kappa(ph, q, mu, kappa);
         hx::stress_shape(vg, sh);
-        if (ph.les) {
+        if (LES) {
 #pragma unroll
             for (int c = 0; c < 6; ++c) stg(visc + c * S, g, sh[c]);
 #pragma unroll
@@ -502,8 +544,12 @@ __host__ __device__ constexpr int pair_slot(int n1, int lo, int hi)
 // The diagonal entry is the node's inviscid contravariant flux.
 // Minimum waves per SIMD asked of the register allocator: 3 for the standard form, and for
 // Kennedy-Gruber and Pirozzoli up to N = 5 (no spills in 168 VGPRs up to N = 4; at N = 5 the
-// few spilled registers cost less than a third wave gains), else no constraint (at N = 6 the
-// forced third wave measured 14% slower than two waves without spills).
+// few spilled registers cost less than a third wave gains), else no constraint.  From N = 6 on a block
+// has six or eight waves, and a second one finds room on a CU only at four waves per SIMD: standard form,
+// 9^3 elements of order 6 with LES 32.4 us at 130 registers, 25.9 at 128; order 7 43.7 and 34.6;
+// Kennedy-Gruber at order 6 54.5 and 53.2 (27 to 43 spills); the other averagings spill more and lost 3 to
+// 5%; at order 7 the split form's LDS admits one block.  The compiler holds to four only where it does not
+// see the block's LDS, so the pool is dynamic.
 #ifndef HX3D_VOL_WAVES
 #define HX3D_VOL_WAVES 3
 #endif
@@ -514,6 +560,8 @@ __host__ __device__ constexpr int pair_slot(int n1, int lo, int hi)
 #endif
 constexpr int volume_waves(int n, int form)
 {
+    if (n >= 6 && form == -1) return 4;
+    if (n == 6 && (form == 2 || form == 3)) return 4;
     return form == -1 ? 3 : (form == 2 || form == 3) && n <= 5 ? HX3D_VOL_WAVES : 1;
 }
 
@@ -577,9 +625,9 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
     constexpr int AVG = SPLIT ? FORM : 0, V0 = SPLIT ? 1 : 0, NP = n1 / 2;
     constexpr bool SYM = hx::two_point_symmetric(AVG);
     constexpr int TPB = ((EPB * ne + 63) / 64) * 64, P = (FACES + TPB - 1) / TPB;
-    __shared__ double pool[L::SIZE];
-    __shared__ double sHat[n1 * n1], sSharp[n1 * n1], sDt;
-    __shared__ int sSlot[n1 * n1];   // pair table offset of (own, l); 0 on the diagonal
+    HIP_DYNAMIC_SHARED(double, pool)   // [L::SIZE]
+    __shared__ double sHat[n1 * n1], sSharp[SPLIT ? n1 * n1 : 1], sDt;
+    __shared__ int sSlot[SPLIT ? n1 * n1 : 1];   // pair table offset of (own, l); 0 on the diagonal
     double *const sQ = pool;                       // [EPB][NV][ne]
     double *const sT = sQ + EPB * NV * ne;         // [EPB][NVT][ne]
     double *const sFb = sT + EPB * NVT * ne;       // [NV][FACES]
@@ -625,9 +673,11 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
     if (update && t < 64) load_dt(dta, cs, t, dtl0, dtl1);
     if (t < n1 * n1) {
         sHat[t] = hop;
-        sSharp[t] = sop;
-        const int a = t / n1, b = t - a * n1;
-        sSlot[t] = a == b ? 0 : pair_slot(n1, a < b ? a : b, a < b ? b : a) * NV * nf;
+        if (SPLIT) {
+            sSharp[t] = sop;
+            const int a = t / n1, b = t - a * n1;
+            sSlot[t] = a == b ? 0 : pair_slot(n1, a < b ? a : b, a < b ? b : a) * NV * nf;
+        }
     }
 #pragma unroll
     for (int c = 0; c < 9; ++c) ja[c] = ldg(mt.Ja + c * mt.S, mt.node(ec, gc));
