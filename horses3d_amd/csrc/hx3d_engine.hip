@@ -61,6 +61,9 @@ namespace {
 
 constexpr int MAXN = 7;
 
+// places of hx3d_engine::hOut: results (0..), the time, then the divergence flags
+constexpr int H_TIME = 8, H_SIZE = 10;
+
 // element face slot 0..5 = EFRONT, EBACK, EBOTTOM, ERIGHT, ETOP, ELEFT
 constexpr int SLOT_AXIS[6] = {1, 1, 2, 0, 2, 0};
 constexpr int SLOT_PLUS[6] = {0, 1, 0, 1, 1, 0};
@@ -141,14 +144,12 @@ __global__ void k_dt_set(unsigned long long *bits, int n, double dt)
 
 // dt = min(convective, viscous) (DGSEMClass.f90:1024-1030); with advance != 0 also
 // time += dt (device scalars: [0] dt, [1] t)
-__global__ void k_dt_finish(const unsigned long long *bits, double *sc, int advance)
+__global__ void k_dt_finish(const unsigned long long *bits, double *out)
 {
     if (threadIdx.x == 0) {
         const double a = __longlong_as_double((long long)bits[0]);
         const double b = __longlong_as_double((long long)bits[1]);
-        const double dt = a < b ? a : b;
-        sc[0] = dt;
-        if (advance) sc[1] += dt;
+        *out = a < b ? a : b;
     }
 }
 
@@ -354,13 +355,32 @@ k_nan(const double *__restrict__ Q, long nodes, long S, int *__restrict__ flag)
 }
 
 // packed (nodes, 5) <-> SoA [5][S]
-__global__ void k_pack_in(const double *__restrict__ in, double *__restrict__ Q, long nodes, long S)
+// A state from outside: packed into Q, with the RK register (the reference allocates G_NS zeroed) and
+// the divergence flags, on both sides, cleared.  hflag: pinned host memory.
+__global__ void __launch_bounds__(256)
+k_set_state(const double *__restrict__ in, double *__restrict__ Q, double *__restrict__ G, long nodes, long S,
+            int *__restrict__ flag, int *__restrict__ hflag, int ncases)
 {
     const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (blockIdx.x == 0)
+        for (int c = threadIdx.x; c < ncases; c += blockDim.x) { flag[c] = 0; hflag[c] = 0; }
     if (g >= nodes) return;
 #pragma unroll
-    for (int v = 0; v < NV; ++v) Q[v * S + g] = in[NV * g + v];
+    for (int v = 0; v < NV; ++v) {
+        Q[v * S + g] = in[NV * g + v];
+        G[v * S + g] = 0.0;
+    }
 }
+// What the host reads once the stream is idle, written to its pinned memory: the divergence flags and
+// the time.  A kernel that stores them costs 3 us on the stream; two copies, one of them to
+// pageable memory, cost 20.
+__global__ void __launch_bounds__(256)
+k_status(const int *__restrict__ flag, int *__restrict__ hflag, int ncases, const double *__restrict__ time, double *__restrict__ htime)
+{
+    for (int c = threadIdx.x; c < ncases; c += blockDim.x) hflag[c] = flag[c];
+    if (threadIdx.x == 0) *htime = *time;
+}
+__global__ void k_set_time(double *time, double t) { *time = t; }
 __global__ void k_pack_out(const double *__restrict__ Q, double *__restrict__ out, long nodes, long S)
 {
     const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -510,6 +530,8 @@ struct hx3d_engine {
     // kernels when a NaN appears.  hFlag: pinned host copy of dFlag[1], refreshed in stream
     // order after each queued step loop (read by hx3d_query once the stream is idle).
     int *hFlag = nullptr;
+    // pinned host memory that finishing kernels write results to (H_* places), hFlag behind it
+    double *hOut = nullptr;
     int device = 0;   // the HIP device the engine was created on
     // several independent cases in one engine (hx3d_engine_create_multi): per-case tables; with
     // one case ncases = 1, mc is all null and dTime = dScal + 1
@@ -744,14 +766,14 @@ DtArgs host_dt(hx3d_engine *eng, double dt)
 }
 
 // Standalone MaxTimeStep of the resident state into dt slot `slot` (bits reset first);
-// k_dt_finish then writes dt to dScal[0].
+// k_dt_finish then writes dt to hOut[0].
 void launch_maxdt_bits(hx3d_engine *eng, double cfl, double dcfl, unsigned long long *bits);
 
 void launch_maxdt(hx3d_engine *eng, double cfl, double dcfl, int slot)
 {
     unsigned long long *b = dt_slot(eng, slot);
     launch_maxdt_bits(eng, cfl, dcfl, b);
-    hipLaunchKernelGGL(k_dt_finish, dim3(1), dim3(64), 0, eng->stream, b, eng->dScal, 0);
+    hipLaunchKernelGGL(k_dt_finish, dim3(1), dim3(64), 0, eng->stream, b, eng->hOut);
 }
 
 // ------------------------------------------------------------------------------------
@@ -845,17 +867,20 @@ void launch_maxdt_bits(hx3d_engine *eng, double cfl, double dcfl, unsigned long 
 int init_flags(hx3d_engine *eng)
 {
     if (!eng->dTime) eng->dTime = eng->dScal + 1;
-    if (hipHostMalloc((void **)&eng->hFlag, sizeof(int) * eng->ncases, hipHostMallocDefault) != hipSuccess)
+    if (hipHostMalloc((void **)&eng->hOut, sizeof(double) * H_SIZE + sizeof(int) * eng->ncases, hipHostMallocDefault) != hipSuccess)
         return eng->fail(HX3D_ENOMEM, "hipHostMalloc failed");
+    eng->hFlag = reinterpret_cast<int *>(eng->hOut + H_SIZE);
+    for (int c = 0; c < H_SIZE; ++c) eng->hOut[c] = 0.0;
     for (int c = 0; c < eng->ncases; ++c) eng->hFlag[c] = 0;
     hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(256), 0, eng->stream, eng->dFlag, 1 + eng->ncases, 0);
     return HX3D_OK;
 }
 
-// hFlag <- dFlag[1] in stream order (read by the host once the stream is idle)
-void queue_flag_readback(hx3d_engine *eng)
+// hFlag <- dFlag[1], hOut[H_TIME] <- the time, in stream order (read by the host once the stream is idle)
+void queue_status(hx3d_engine *eng)
 {
-    (void)hipMemcpyAsync(eng->hFlag, eng->dFlag + 1, sizeof(int) * eng->ncases, hipMemcpyDeviceToHost, eng->stream);
+    hipLaunchKernelGGL(k_status, dim3(1), dim3(256), 0, eng->stream, eng->dFlag + 1, eng->hFlag, eng->ncases, eng->dScal + 1,
+                       eng->hOut + H_TIME);
 }
 
 // After a queued step loop: the divergence flag's read-back, and the time derivative the
@@ -1342,7 +1367,7 @@ void after_steps(hx3d_engine *eng)
 {
     eng->qdot_valid = true;
     if (eng->ctd_after) (void)hx3d_compute_qdot(eng, 0.0, nullptr);
-    queue_flag_readback(eng);
+    queue_status(eng);
 }
 }  // namespace
 
@@ -1718,8 +1743,8 @@ int hx3d_engine_create_multi(const hx3d_case_desc *descs, int ncases, hx3d_engin
     (void)hipFree(eng->dFlag);
     (void)hipFree(eng->dSlots);
     eng->dSlots = nullptr;
-    (void)hipHostFree(eng->hFlag);
-    eng->dBits = nullptr; eng->dFlag = nullptr; eng->hFlag = nullptr;
+    (void)hipHostFree(eng->hOut);
+    eng->dBits = nullptr; eng->dFlag = nullptr; eng->hOut = nullptr;
     eng->ncases = ncases;
     const std::vector<int> ones(ncases, 1);
     if ((rc = dalloc(eng, &eng->dBits, (size_t)2 * DT_SLOTS * ncases)) || (rc = dalloc(eng, &eng->dFlag, (size_t)1 + ncases)) ||
@@ -1774,7 +1799,7 @@ int hx3d_engine_destroy(hx3d_engine *eng)
         if (p) (void)hipFree(p);
     for (auto &e : eng->evpool) (void)hipEventDestroy(e);
     if (eng->step_graph) (void)hipGraphExecDestroy(eng->step_graph);
-    if (eng->hFlag) (void)hipHostFree(eng->hFlag);
+    if (eng->hOut) (void)hipHostFree(eng->hOut);
     if (eng->stream) (void)hipStreamDestroy(eng->stream);
     delete eng;
     return HX3D_OK;
@@ -1784,13 +1809,9 @@ int hx3d_set_state_device(hx3d_engine *eng, const double *Qd)
 {
     if (!eng || !Qd) return HX3D_EINVAL;
     const long nb = (eng->nodes + 255) / 256;
-    hipLaunchKernelGGL(k_pack_in, dim3(nb), dim3(256), 0, eng->stream, Qd, eng->dQ, eng->nodes, eng->S);
+    hipLaunchKernelGGL(k_set_state, dim3(nb), dim3(256), 0, eng->stream, Qd, eng->dQ, eng->dG, eng->nodes, eng->S,
+                       eng->dFlag + 1, eng->hFlag, eng->ncases);
     refresh_traces(eng);   // Gauss nodes: the new state's face traces
-    // a new state restarts the RK register (the reference allocates G_NS zeroed)
-    const long nb2 = (NV * eng->S + 255) / 256;
-    hipLaunchKernelGGL(k_fill, dim3(nb2), dim3(256), 0, eng->stream, eng->dG, (long)NV * eng->S, 0.0);
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(256), 0, eng->stream, eng->dFlag + 1, eng->ncases, 0);
-    queue_flag_readback(eng);
     eng->qdot_valid = false;
     HIPCHK(hipGetLastError());
     return HX3D_OK;
@@ -1919,8 +1940,8 @@ static int finish_steps(hx3d_engine *eng, double *t_inout)
 {
     HIPCHK(hipGetLastError());
     if (!t_inout) return HX3D_OK;
-    HIPCHK(hipMemcpyAsync(t_inout, eng->dScal + 1, sizeof(double), hipMemcpyDeviceToHost, eng->stream));
     HIPCHK(hipStreamSynchronize(eng->stream));
+    *t_inout = eng->hOut[H_TIME];
     if (*eng->hFlag) return eng->fail(HX3D_ENAN, "numerical divergence: a NaN appeared in the state");
     return HX3D_OK;
 }
@@ -1929,7 +1950,7 @@ int hx3d_advance_dt(hx3d_engine *eng, int nsteps, double dt, double *t_inout)
 {
     if (!eng || nsteps < 0 || !(dt > 0.0)) return HX3D_EINVAL;
     if (eng->mc.blocks && t_inout) return eng->fail(HX3D_EINVAL, "several cases: pass no time, read them with hx3d_multi_status");
-    if (t_inout) HIPCHK(hipMemcpyAsync(eng->dScal + 1, t_inout, sizeof(double), hipMemcpyHostToDevice, eng->stream));
+    if (t_inout) hipLaunchKernelGGL(k_set_time, dim3(1), dim3(1), 0, eng->stream, eng->dScal + 1, *t_inout);
     DtArgs a = host_dt(eng, dt);
     a.nan = eng->dFlag + 1;
     for (int s = 0; s < nsteps; ++s)
@@ -1940,6 +1961,7 @@ int hx3d_advance_dt(hx3d_engine *eng, int nsteps, double dt, double *t_inout)
         }
     HIPCHK(hipGetLastError());
     if (nsteps > 0) after_steps(eng);
+    else queue_status(eng);
     return finish_steps(eng, t_inout);
 }
 
@@ -1948,8 +1970,9 @@ int hx3d_max_dt(hx3d_engine *eng, double cfl, double dcfl, double *dt)
     if (!eng || !dt) return HX3D_EINVAL;
     if (eng->mc.blocks) return eng->fail(HX3D_EUNSUPPORTED, "several cases: each case's dt is formed on the device by hx3d_advance");
     launch_maxdt(eng, cfl, dcfl, 3);
-    HIPCHK(hipMemcpyAsync(dt, eng->dScal, sizeof(double), hipMemcpyDeviceToHost, eng->stream));
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(eng->stream));
+    *dt = eng->hOut[0];
     return HX3D_OK;
 }
 
@@ -1957,7 +1980,7 @@ int hx3d_advance(hx3d_engine *eng, int nsteps, double cfl, double dcfl, double *
 {
     if (!eng || nsteps < 0) return HX3D_EINVAL;
     if (eng->mc.blocks && t_inout) return eng->fail(HX3D_EINVAL, "several cases: pass no time, read them with hx3d_multi_status");
-    if (t_inout) HIPCHK(hipMemcpyAsync(eng->dScal + 1, t_inout, sizeof(double), hipMemcpyHostToDevice, eng->stream));
+    if (t_inout) hipLaunchKernelGGL(k_set_time, dim3(1), dim3(1), 0, eng->stream, eng->dScal + 1, *t_inout);
     const size_t nev = eng->timing ? (size_t)12 * nsteps : 0;
     // timing events need no system-scope fence: they are read only through
     // hipEventElapsedTime, and the fence adds its own time to every measured launch
@@ -2064,6 +2087,7 @@ int hx3d_advance(hx3d_engine *eng, int nsteps, double cfl, double dcfl, double *
         eng->ktime[3] = (eng->ktime[0] + eng->ktime[1] + eng->ktime[2]);
     }
     if (nsteps > 0) after_steps(eng);
+    else queue_status(eng);
     return finish_steps(eng, t_inout);
 }
 
@@ -2076,9 +2100,10 @@ int hx3d_residuals(hx3d_engine *eng, double res[5])
     }
     const int nb = (int)((eng->nodes + 255) / 256);
     hipLaunchKernelGGL(k_absmax, dim3(nb), dim3(256), 0, eng->stream, eng->dQDot, eng->nodes, eng->S, eng->dPart);
-    hipLaunchKernelGGL(k_finish_max_block, dim3(1), dim3(256), 0, eng->stream, eng->dPart, nb, eng->dStage);
-    HIPCHK(hipMemcpyAsync(res, eng->dStage, sizeof(double) * NV, hipMemcpyDeviceToHost, eng->stream));
+    hipLaunchKernelGGL(k_finish_max_block, dim3(1), dim3(256), 0, eng->stream, eng->dPart, nb, eng->hOut);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(eng->stream));
+    std::copy(eng->hOut, eng->hOut + NV, res);
     return HX3D_OK;
 }
 
@@ -2113,10 +2138,10 @@ int hx3d_kinetic_energy(hx3d_engine *eng, double *ke)
     if (!eng || !ke) return HX3D_EINVAL;
     const int nb = (int)((eng->nodes + 255) / 256);
     hipLaunchKernelGGL(k_kinetic, dim3(nb), dim3(256), 0, eng->stream, eng->dQ, eng->dJ, eng->dWq, eng->nodes, eng->S, eng->dPart);
-    hipLaunchKernelGGL(k_finish_sum2, dim3(1), dim3(FINISH_TPB), 0, eng->stream, eng->dPart, nb, eng->dStage);
-    double r[2];
-    HIPCHK(hipMemcpyAsync(r, eng->dStage, sizeof(r), hipMemcpyDeviceToHost, eng->stream));
+    hipLaunchKernelGGL(k_finish_sum2, dim3(1), dim3(FINISH_TPB), 0, eng->stream, eng->dPart, nb, eng->hOut);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(eng->stream));
+    const double *r = eng->hOut;
     *ke = r[0] / r[1];
     return HX3D_OK;
 }
@@ -2140,10 +2165,10 @@ int hx3d_volume_monitor(hx3d_engine *eng, int kind, double *value)
     hipLaunchKernelGGL(k_monitor, dim3(nb), dim3(256), 0, eng->stream, kind, eng->dQ, eng->dQDot,
                        eng->mixed ? nullptr : eng->dCurl, eng->dU, eng->dJ, eng->dWq, eng->nodes, eng->S, eng->ph,
                        eng->dPart);
-    hipLaunchKernelGGL(k_finish_sum2, dim3(1), dim3(FINISH_TPB), 0, eng->stream, eng->dPart, nb, eng->dStage);
-    double r[2];
-    HIPCHK(hipMemcpyAsync(r, eng->dStage, sizeof(r), hipMemcpyDeviceToHost, eng->stream));
+    hipLaunchKernelGGL(k_finish_sum2, dim3(1), dim3(FINISH_TPB), 0, eng->stream, eng->dPart, nb, eng->hOut);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(eng->stream));
+    const double *r = eng->hOut;
     *value = (kind == HX3D_MON_ENSTROPHY ? 0.5 * r[0] : r[0]) / r[1];
     return HX3D_OK;
 }
@@ -2182,8 +2207,10 @@ int hx3d_query(hx3d_engine *eng, int *done)
 int hx3d_get_time(hx3d_engine *eng, double *t)
 {
     if (!eng || !t) return HX3D_EINVAL;
-    HIPCHK(hipMemcpyAsync(t, eng->dScal + 1, sizeof(double), hipMemcpyDeviceToHost, eng->stream));
+    queue_status(eng);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(eng->stream));
+    *t = eng->hOut[H_TIME];
     return HX3D_OK;
 }
 
