@@ -161,3 +161,25 @@ def test_constant_metrics_read_once_give_the_same_bits(orders, riemann):
     err = po.normwise_error(out[0][0], ora.qdot(Q0))
     print(orders, riemann, err, flush=True)
     assert err.max() <= TOL
+
+
+@pytest.mark.parametrize("n,N", [(4, 1), (13, 4), (15, 4)])
+def test_host_transfers_through_chunks_are_exact(n, N):
+    """A state smaller than a staging chunk, one of several chunks that reuse the slots (11 MB) and one with a
+    short last chunk (16.9 MB): set, get, a part of it, and the derivative against a copy of it; pageable
+    arrays and the caller's pinned ones."""
+    import torch
+    from horses3d_amd.engine import Engine
+    case = mesh.straight_box(n, N)
+    eng = Engine(case, mach=0.2, reynolds=800.0)
+    base = mesh.taylor_green(case, 0.2)
+    pinned = torch.empty(base.shape, dtype=torch.float64, pin_memory=True).numpy()
+    for k, Q in enumerate((base, mesh.taylor_green(case, 0.2, noise=1e-3, seed=2))):
+        eng.set_state(Q)
+        assert np.array_equal(eng.get_state(), Q)
+        qd = eng.qdot()
+        assert np.array_equal(eng.get_qdot(), qd)
+        pinned[:] = Q
+        eng.set_state(pinned)
+        assert np.array_equal(eng.get_state(), Q) and np.array_equal(eng.qdot(), qd)
+    eng.close()
