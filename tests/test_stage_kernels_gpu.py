@@ -168,12 +168,14 @@ def test_host_transfers_through_chunks_are_exact(n, N):
     """A state smaller than a staging chunk, one of several chunks that reuse the slots (11 MB) and one with a
     short last chunk (16.9 MB): set, get, a part of it, and the derivative against a copy of it; pageable
     arrays and the caller's pinned ones."""
-    import torch
+    import ctypes as C
     from horses3d_amd.engine import Engine
     case = mesh.straight_box(n, N)
     eng = Engine(case, mach=0.2, reynolds=800.0)
     base = mesh.taylor_green(case, 0.2)
-    pinned = torch.empty(base.shape, dtype=torch.float64, pin_memory=True).numpy()
+    hip, p = C.CDLL("libamdhip64.so.7"), C.c_void_p()
+    assert hip.hipHostMalloc(C.byref(p), C.c_size_t(base.nbytes), C.c_uint(0)) == 0
+    pinned = np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_double)), shape=base.shape)
     for k, Q in enumerate((base, mesh.taylor_green(case, 0.2, noise=1e-3, seed=2))):
         eng.set_state(Q)
         assert np.array_equal(eng.get_state(), Q)
@@ -183,3 +185,4 @@ def test_host_transfers_through_chunks_are_exact(n, N):
         eng.set_state(pinned)
         assert np.array_equal(eng.get_state(), Q) and np.array_equal(eng.qdot(), qd)
     eng.close()
+    assert hip.hipHostFree(p) == 0
