@@ -652,17 +652,22 @@ void launch_volume_e(hx3d_engine *eng, double a_k, double c_k, int update, const
 {
     constexpr int ne = (N + 1) * (N + 1) * (N + 1);
     constexpr int TPB = ((EPB * ne + 63) / 64) * 64;
-    auto go = [&](auto kernel) {
-        const size_t lds = sizeof(double) * (eng->ph.les ? hxk::VolumeLds<N, EPB, FORM, true>::SIZE : hxk::VolumeLds<N, EPB, FORM, false>::SIZE);
-        hipLaunchKernelGGL(kernel, dim3(elem_grid(eng, EPB)), dim3(TPB), lds, eng->stream, eng->dQ, eng->dQn, eng->dVisc,
+    auto go = [&](auto lxf, auto vis) {
+        constexpr bool LXF = decltype(lxf)::value;
+        constexpr int VIS = decltype(vis)::value;
+        constexpr size_t lds = sizeof(double) * hxk::VolumeLds<N, EPB, FORM, VIS>::SIZE;
+        hipLaunchKernelGGL((hxk::k_volume<N, EPB, FORM, LXF, VIS>), dim3(elem_grid(eng, EPB)), dim3(TPB), lds, eng->stream,
+                           eng->dQ, eng->dQn, eng->dVisc,
                            eng->dEdelta, eng->dEfdelta, eng->dNbx, metric(eng), eng->t2x ? 1 : 0, eng->dG, qdot, a_k, c_k,
                            update, dta, eng->K, eng->S, eng->ES, eng->ops, eng->ph, eng->mc);
     };
-    const bool lxf = eng->ph.riemann == HX3D_RIEMANN_LXF, les = eng->ph.les != 0;
-    if (lxf && les) go(hxk::k_volume<N, EPB, FORM, true, true>);
-    else if (lxf) go(hxk::k_volume<N, EPB, FORM, true, false>);
-    else if (les) go(hxk::k_volume<N, EPB, FORM, false, true>);
-    else go(hxk::k_volume<N, EPB, FORM, false, false>);
+    auto pick = [&](auto lxf) {
+        if (eng->ph.euler) go(lxf, std::integral_constant<int, hxk::INVISCID>{});
+        else if (eng->ph.les) go(lxf, std::integral_constant<int, hxk::EDDY>{});
+        else go(lxf, std::integral_constant<int, hxk::LAMINAR>{});
+    };
+    if (eng->ph.riemann == HX3D_RIEMANN_LXF) pick(std::true_type{});
+    else pick(std::false_type{});
     if (update) std::swap(eng->dQ, eng->dQn);
 }
 

@@ -580,7 +580,11 @@ __device__ __forceinline__ int face_element_node(int x)
 // values [9 or 11][ne] and the face fluxes [NV] per element face node; then the contravariant fluxes and
 // the direction loop's space.
 constexpr int vol_max(int a, int b) { return a > b ? a : b; }
-template <int N, int EPB, int FORM, bool LES>
+// VIS: the viscous model (INVISCID, LAMINAR, EDDY).  INVISCID: no viscous values, and no viscous fluxes in the
+// split form's direction loop (a quarter of its LDS reads at N = 5: each added an exact zero); 11^3
+// elements of order 5, Ducros, 44.3 -> 40.5 us; 16^3 of order 4, Pirozzoli, 53.6 -> 51.4 us.
+enum { INVISCID = 0, LAMINAR = 1, EDDY = 2 };
+template <int N, int EPB, int FORM, int VIS>
 struct VolumeLds {
     static constexpr int n1 = N + 1, nf = n1 * n1, ne = nf * n1, NI = 6 * nf;
     static constexpr bool SPLIT = FORM >= 0;
@@ -592,9 +596,10 @@ struct VolumeLds {
     static constexpr bool ROW = SPLIT && N == 5 && HX3D_ROW5;
     static constexpr int RN = (ND + 3) * ne, RP = ROW ? 0 : n1 * (n1 - 1) / 2 * NV * nf;
     static constexpr int RSZ = SPLIT ? vol_max(RN, RP) : 0;
-    static constexpr int FSZ = 3 * NF * ne;
+    static constexpr int FSZ = SPLIT && VIS == INVISCID ? 0 : 3 * NF * ne;
+    static constexpr int NVT = VIS == INVISCID ? 0 : viscous_values(VIS == EDDY);
     static constexpr int FACES = EPB * NI;
-    static constexpr int SIZE = vol_max(EPB * (NV + viscous_values(LES)) * ne + NV * FACES, EPB * (FSZ + RSZ));
+    static constexpr int SIZE = vol_max(EPB * (NV + NVT) * ne + NV * FACES, EPB * (FSZ + RSZ));
 };
 
 // What bounds it: bytes first.  Per node 312 B (Q, Ja, J, G, viscous tensor in; G, Q out; 328 B with
@@ -610,7 +615,7 @@ struct VolumeLds {
 // rest.  Forming the gradient again here instead of reading the viscous values measured 76 us.
 // New state to Qn, not in place: the neighbours of later blocks still read Q.
 // LXF: the engine's Riemann solver is Lax-Friedrichs, the one that reads the tangents (Roe does not).
-template <int N, int EPB, int FORM, bool LXF, bool LES>
+template <int N, int EPB, int FORM, bool LXF, int VIS>
 __global__ void __launch_bounds__(((EPB * (N + 1) * (N + 1) * (N + 1) + 63) / 64) * 64)
 __attribute__((amdgpu_waves_per_eu(volume_waves(N, FORM))))
 k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__restrict__ visc,
@@ -618,7 +623,8 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
          Metric mt, int t2x, double *__restrict__ G, double *__restrict__ qdot_out, double a_k, double c_k, int update,
          DtArgs dta, int K, long S, long ES, Ops ops, Phys ph, Multi mc)
 {
-    using L = VolumeLds<N, EPB, FORM, LES>;
+    using L = VolumeLds<N, EPB, FORM, VIS>;
+    constexpr bool LES = VIS == EDDY, EULER = VIS == INVISCID;
     constexpr int NVT = viscous_values(LES);
     constexpr int n1 = L::n1, nf = L::nf, ne = L::ne, NI = L::NI, ND = L::ND, NF = L::NF, FACES = L::FACES;
     constexpr bool SPLIT = L::SPLIT, ROW = L::ROW;
@@ -630,7 +636,7 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
     __shared__ int sSlot[SPLIT ? n1 * n1 : 1];   // pair table offset of (own, l); 0 on the diagonal
     double *const sQ = pool;                       // [EPB][NV][ne]
     double *const sT = sQ + EPB * NV * ne;         // [EPB][NVT][ne]
-    double *const sFb = sT + EPB * NVT * ne;       // [NV][FACES]
+    double *const sFb = sT + EPB * L::NVT * ne;       // [NV][FACES]
     const int lb = xcd_block(blockIdx.x, gridDim.x);
     const int t = threadIdx.x;
     int e0, cnt, cs, idle;
@@ -665,7 +671,7 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
     double q[NV], ja[9], vt[NVT];
 #pragma unroll
     for (int v = 0; v < NV; ++v) q[v] = ldg(Q + v * S, gc);
-    if (!ph.euler) {   // uniform
+    if (!EULER) {   // uniform
 #pragma unroll
         for (int c = 0; c < NVT; ++c) vt[c] = ldg(visc + c * S, gc);
     }
@@ -695,7 +701,7 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
 #pragma unroll
         for (int c = 0; c < 3; ++c) nrm[c] = ldg(mt.face + c * mt.FS, mt.face_node<nf>(x));
         jac = ldg(mt.face + 3 * mt.FS, mt.face_node<nf>(x));
-        if (!ph.euler) {
+        if (!EULER) {
 #pragma unroll
             for (int c = 0; c < NVT; ++c) fn[c] = ldg(visc + c * S, gn);
         }
@@ -709,7 +715,7 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
     if (active) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) sQ[(el * NV + v) * ne + n] = q[v];
-        if (!ph.euler) {
+        if (!EULER) {
 #pragma unroll
             for (int c = 0; c < NVT; ++c) sT[(el * NVT + c) * ne + n] = vt[c];
         }
@@ -728,7 +734,7 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
             double qL[NV], vn[NV];
             const double io = 1.0 / sQ[eo * NV * ne + no], in = 1.0 / qR[0];
             vn[0] = 0.0;
-            if (!ph.euler) {
+            if (!EULER) {
                 // BR1_RiemannSolver (EllipticBR1.f90:816-868): the average of both sides' tensors,
                 // summed in either order with the same bits, and its product with the normal
                 double f[NVF];
@@ -823,7 +829,7 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
         for (int d = 0; d < 3; ++d)
 #pragma unroll
             for (int v = 0; v < NV; ++v) Fvc[d][v] = 0.0;
-        if (!ph.euler) {
+        if (!EULER) {
             // BR1_ComputeInnerFluxes (EllipticBR1.f90:740-814)
             double f[NVF];
 #pragma unroll
@@ -855,7 +861,8 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
     __syncthreads();   // the state and the face values are read: the pool takes the fluxes
     double *const sF = pool + el * (L::FSZ + L::RSZ);   // [3][NF][ne]
     double *const sR = sF + L::FSZ;                     // [RSZ]
-    if (active) {
+    constexpr bool VF = !SPLIT || !EULER;   // the direction loop reads sF
+    if (VF && active) {
 #pragma unroll
         for (int d = 0; d < 3; ++d)
 #pragma unroll
@@ -929,8 +936,10 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
                     }
                     qd[0] = qd[0] + sh * (l == own_i ? fi[0] : tp[0]);
 #pragma unroll
-                    for (int v = 1; v < NV; ++v)
-                        qd[v] = qd[v] + sh * (l == own_i ? fi[v] : tp[v]) + hh * sF[(d * NF + v - V0) * ne + m];
+                    for (int v = 1; v < NV; ++v) {
+                        qd[v] = qd[v] + sh * (l == own_i ? fi[v] : tp[v]);
+                        if (VF) qd[v] = qd[v] + hh * sF[(d * NF + v - V0) * ne + m];
+                    }
                 }
             }
             continue;
@@ -985,8 +994,10 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
                 const int po = sSlot[own_i * n1 + l] + line;
                 qd[0] = qd[0] + sh * (l == own_i ? fi[0] : sR[po]);
 #pragma unroll
-                for (int v = 1; v < NV; ++v)
-                    qd[v] = qd[v] + sh * (l == own_i ? fi[v] : sR[po + v * nf]) + hh * sF[(d * NF + v - V0) * ne + m];
+                for (int v = 1; v < NV; ++v) {
+                    qd[v] = qd[v] + sh * (l == own_i ? fi[v] : sR[po + v * nf]);
+                    if (VF) qd[v] = qd[v] + hh * sF[(d * NF + v - V0) * ne + m];
+                }
             }
         }
     }

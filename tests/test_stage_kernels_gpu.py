@@ -186,3 +186,30 @@ def test_host_transfers_through_chunks_are_exact(n, N):
         assert np.array_equal(eng.get_state(), Q) and np.array_equal(eng.qdot(), qd)
     eng.close()
     assert hip.hipHostFree(p) == 0
+
+
+@pytest.mark.parametrize("riemann", ["roe", "lxf"])
+@pytest.mark.parametrize("N,averaging", [(1, "pirozzoli"), (3, "standard"), (4, "kennedy-gruber"), (5, "ducros"), (6, "morinishi"),
+                                         (7, "pirozzoli"), (2, None), (6, None)])
+def test_euler_volume_kernel_matches_oracle(N, averaging, riemann):
+    """The volume kernel without viscous values, split (with the pair table and, at N = 5, by rows) and
+    standard form: the derivative and a step against the oracle."""
+    from horses3d_amd.engine import Engine
+    case = mesh.periodic_box(3, N, amplitude=0.1, phase_seed=40 + N)
+    Q0 = mesh.taylor_green(case, 0.3, noise=1e-3, seed=N)
+    kw = dict(riemann=riemann, euler=True, inviscid="split-form" if averaging else "standard", averaging=averaging or "standard")
+    ora = po.Oracle(case, po.make_params(0.3, 700.0, **kw))
+    eng = Engine(case, mach=0.3, reynolds=700.0, **kw)
+    eng.set_state(Q0)
+    err = po.normwise_error(eng.qdot(), ora.qdot(Q0))
+    print(N, averaging, riemann, err, flush=True)
+    assert err.max() <= TOL
+    # one step: the increment to the bar, plus four ulp of the state it is added to
+    dt = ora.max_dt(Q0, 0.4, 0.4)
+    assert eng.advance(1, 0.4, 0.4, t=0.0) == pytest.approx(dt, rel=1e-13)
+    Q, G = Q0.copy(), np.zeros_like(Q0)
+    ora.rk3_step(Q, G, 0.0, dt)
+    dq = np.abs(Q - Q0).max(axis=0)
+    floor = 4.0 * np.finfo(float).eps * np.abs(Q).max(axis=0)
+    assert np.all(np.abs(eng.get_state() - Q).max(axis=0) <= TOL * dq + floor)
+    eng.close()
