@@ -1336,8 +1336,9 @@ int create_mixed(hx3d_engine *eng, const hx3d_case_desc *d)
             if (m != n) tset_host(n, m, oa.T[n][m], gauss);
     }
     // geometry, weights, LES filter widths (SD.f90:420, :1378)
-    std::vector<double> ja((size_t)9 * S, 0.0), jj((size_t)S, 1.0), edelta(K), fdelta(F),
-        fgeo((size_t)10 * fsm, 0.0);
+    std::vector<double> ja, jj((size_t)S, 1.0), edelta(K), fdelta(F), fgeo((size_t)10 * fsm, 0.0);
+    ja.reserve((size_t)9 * S + 10 * ((K + 63) / 64) * 64);   // with element_metrics' planes
+    ja.resize((size_t)9 * S, 0.0);
     std::vector<int> eofn((size_t)nodes);
     for (int e = 0; e < K; ++e) {
         const int nx = N3[3 * e] + 1, ny = N3[3 * e + 1] + 1, nz = N3[3 * e + 2] + 1;
@@ -1574,8 +1575,9 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
     if (!offsets_fit(S, ES, FS))
         return bail(eng->fail(HX3D_EUNSUPPORTED, "mesh too large: more than 2^29 - 1 nodes (or face nodes) per array"));
     // geometry SoA, J, 1/J, quadrature weights, LES filter widths, face frames
-    std::vector<double> ja((size_t)9 * S, 0.0), jj((size_t)S, 1.0), wq((size_t)S, 0.0),
-        edelta(K), efdelta((size_t)6 * K);
+    std::vector<double> ja, jj((size_t)S, 1.0), wq((size_t)S, 0.0), edelta(K), efdelta((size_t)6 * K);
+    ja.reserve((size_t)9 * S + 10 * ((K + 63) / 64) * 64);   // with element_metrics' planes
+    ja.resize((size_t)9 * S, 0.0);
     double xg[8], wg[8];
     hxs::nodes_of(eng->gauss, N, xg, wg);
     for (long g = 0; g < nodes; ++g) {
