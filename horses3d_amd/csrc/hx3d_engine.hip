@@ -1075,8 +1075,8 @@ int set_tiles(hx3d_engine *eng, int policy)
         return tiles;
     };
     // one tile size per mesh: small tiles when every element fits (on a 24^3 box with orders on
-    // {2..5}, 5% faster per step than 512-thread tiles), else 512-thread tiles for all (with
-    // orders up to 7, a launch of each size measured 0.6% slower than the large tiles alone)
+    // {2..5}, 1.238 ms per step against 1.242 with 512-thread tiles), else 512-thread tiles for all
+    // (20^3, orders up to 7: 1.220 ms per step, a launch of each size 1.275)
     std::vector<int> small, big;
     for (int e = 0; e < K; ++e) (ne[e] <= hxm::TILE_SMALL ? small : big).push_back(e);
     if (sizes == 1 || (sizes == 0 && !big.empty())) {

@@ -609,7 +609,7 @@ struct VolumeLds {
 // instead of 0.6 Riemann fluxes per node at N = 4, and saves the launch, the 80 B per face node
 // of stored fluxes each way and the second read of both traces.  Measured per stage (k_grad and
 // k_volume; before, with a face kernel between them and the gradients stored): 16^3 x N=4 Pirozzoli
-// 88 us (97), 24^3 x N=5 Kennedy-Gruber + WALE 592 (690), 4^3 x N=3 14 (18), 9^3 x N=6 62 (62).
+// 88 us (97), 24^3 x N=5 Kennedy-Gruber + WALE 592 (690), 4^3 x N=3 14 (18), 9^3 x N=6 46 (62).
 // At 16^3 x N=4 the kernel moves 265 MB in 59 us; without the direction loop it takes 40 us, the
 // rate of a large copy, and the loop's LDS traffic (97 accesses per node and direction) adds the
 // rest.  Forming the gradient again here instead of reading the viscous values measured 76 us.
