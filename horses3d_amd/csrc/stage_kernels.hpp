@@ -4,6 +4,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <climits>
+
 #include "physics.hpp"
 
 namespace hxk {
@@ -139,16 +141,30 @@ __device__ __forceinline__ void block_elements(const Multi &mc, int lb, int K, i
 // Mixed orders (part; null: not this stage): block minima of the convective and viscous limits to
 // part[2*block + 0/1], reduced by the face kernel that follows (DtReduce).  One order (slots; null: not this stage): each block's minima by atomicMin
 // into one of the case's DT_FAN slots, from which every block of the volume kernel that follows
-// takes the minimum.  The minimum of doubles does not depend on the order, and the limits are
-// positive or NaN, whose bit patterns order like the numbers (NaN above +inf, so it is passed over
-// as fmin passes it over).  DT_FAN slots on lines of their own: one slot alone serialises (16k
-// atomics on one address cost 150 us), 32 leave at most a few hundred per line at 24^3 elements.
+// takes the minimum.  The minimum of doubles does not depend on the order; the slots hold keys that
+// order like the numbers, of either sign (order_key: a negative CFL number gives negative limits),
+// and NaN is passed over as fmin passes it over.  DT_FAN slots on lines of their own: one slot alone
+// serialises (16k atomics on one address cost 150 us), 32 leave at most a few hundred per line at 24^3
+// elements.
 struct DtLimits {
     double *part;
     double cfl, dcfl, dcsi;
     unsigned long long *slots;
 };
 constexpr int DT_FAN = 32, DT_LINE = 16;   // slots per case; slot stride in 8-byte words (128 B)
+
+// A double's key, ordered as unsigned whole numbers are: the sign bit set for positive numbers, all bits
+// turned over for negative ones.
+__device__ __forceinline__ unsigned long long order_key(double x)
+{
+    const long long b = __double_as_longlong(fmin(x, INFINITY));   // NaN: +inf
+    return (unsigned long long)(b ^ ((b >> 63) | LLONG_MIN));
+}
+__device__ __forceinline__ double key_value(unsigned long long k)
+{
+    const long long b = (long long)k;
+    return __longlong_as_double(b < 0 ? b ^ LLONG_MIN : ~b);
+}
 
 // Averaging selectors of the templated split-form kernel (RiemannSolvers_NS.f90:229-285)
 enum { AVG_STANDARD = 0, AVG_DUCROS = 1, AVG_KG = 2, AVG_PIROZZOLI = 3, AVG_MORINISHI = 4, FORM_STANDARD = -1 };
@@ -465,8 +481,8 @@ __device__ __forceinline__ void block_min_slot(double a, double b, unsigned long
         const int nw = (blockDim.x + 63) >> 6;
         for (int w = 1; w < nw; ++w) { a = fmin(a, sm[0][w]); b = fmin(b, sm[1][w]); }
         unsigned long long *s = slots + (long)(cs * DT_FAN + lb % DT_FAN) * DT_LINE;
-        atomicMin(s, (unsigned long long)__double_as_longlong(a));
-        atomicMin(s + 1, (unsigned long long)__double_as_longlong(b));
+        atomicMin(s, order_key(a));
+        atomicMin(s + 1, order_key(b));
     }
 }
 
@@ -501,8 +517,8 @@ __device__ __forceinline__ void reduce_dt_partials(const double *part, int n, un
 __device__ __forceinline__ void load_dt(const DtArgs &dta, int cs, int t, double &a, double &b)
 {
     const unsigned long long *s = dta.slots ? dta.slots + (long)(cs * DT_FAN + t % DT_FAN) * DT_LINE : dta.in + 2 * cs;
-    a = bits_to_double(s[0]);
-    b = bits_to_double(s[1]);
+    a = dta.slots ? key_value(s[0]) : bits_to_double(s[0]);
+    b = dta.slots ? key_value(s[1]) : bits_to_double(s[1]);
 }
 __device__ __forceinline__ void reduce_dt(const DtArgs &dta, int cs, bool first, int t, double a, double b, double &sDt)
 {
@@ -519,7 +535,7 @@ __device__ __forceinline__ void reduce_dt(const DtArgs &dta, int cs, bool first,
     }
     if (first && dta.empty && t < DT_FAN) {
         unsigned long long *sl = dta.empty + (long)(cs * DT_FAN + t) * DT_LINE;
-        sl[0] = sl[1] = (unsigned long long)__double_as_longlong(INFINITY);
+        sl[0] = sl[1] = order_key(INFINITY);
     }
 }
 

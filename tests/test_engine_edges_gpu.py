@@ -1,0 +1,64 @@
+"""Edges of the engine's entry points: CFL numbers of either sign."""
+import numpy as np
+import pytest
+
+import pyoracle as po
+from horses3d_amd import mesh, specmesh
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-12   # the parity bar: normwise per variable
+KW = dict(mach=0.3, reynolds=700.0, riemann="roe")
+
+
+def one_step_matches(eng, ora, Q0, cfl, dcfl):
+    """advance() by one step takes max_dt's limit, whatever its sign, and ends where the oracle ends"""
+    dt = eng.max_dt(cfl, dcfl)
+    assert dt == pytest.approx(ora.max_dt(Q0, cfl, dcfl), rel=1e-13) and dt < 0.0
+    assert eng.advance(1, cfl, dcfl, t=0.0) == dt
+    Q, G = Q0.copy(), np.zeros_like(Q0)
+    ora.rk3_step(Q, G, 0.0, dt)
+    dq = np.abs(Q - Q0).max(axis=0)
+    floor = 4.0 * np.finfo(float).eps * np.abs(Q).max(axis=0)   # four ulp of the state the increment is added to
+    assert np.all(np.abs(eng.get_state() - Q).max(axis=0) <= TOL * dq + floor)
+
+
+@pytest.mark.parametrize("kind,cfl,dcfl", [(k, c, d) for k in ("gauss-lobatto", "euler", "gauss", "mixed")
+                                           for c, d in ((-0.1, -0.1), (0.1, -0.1), (-0.1, 0.1))
+                                           if c < 0.0 or k != "euler"])   # Euler: no viscous limit
+def test_negative_cfl_numbers(kind, cfl, dcfl, tmp_path):
+    """A negative CFL number steps backwards with the limit of the smallest value, as max_dt gives it: the
+    minima of the blocks order like the numbers, not like their bits."""
+    from horses3d_amd.engine import Engine, read_specmesh
+    N, euler = 3, kind == "euler"
+    if kind == "gauss":
+        path = str(tmp_path / "box.mesh")
+        specmesh.write_specmesh(path, 3, 0.1, mesh.box_phases(5), bface_order=4)
+        case = read_specmesh(path, N=N, periodic=dict(specmesh.PERIODIC_PAIRS), nodes="gauss")
+        case["fNf"] = np.full((case["F"], 2), N, np.int32)
+        case["foff"] = np.arange(case["F"] + 1, dtype=np.int64) * (N + 1) ** 2
+    elif kind == "mixed":
+        case = mesh.periodic_box_mixed(3, mesh.random_orders(27, 2, 4, 5))
+    else:
+        case = mesh.periodic_box(3, N, amplitude=0.1, phase_seed=5)
+    nodes = "gauss" if kind == "gauss" else "gauss-lobatto"
+    Q0 = mesh.taylor_green(case, 0.3, noise=1e-3, seed=3)
+    ora = po.Oracle(case, po.make_params(0.3, 700.0, riemann="roe", euler=euler, nodes=nodes))
+    eng = Engine(case, euler=euler, nodes=nodes, **KW)
+    eng.set_state(Q0)
+    one_step_matches(eng, ora, Q0, cfl, dcfl)
+    # a zero of either sign is the smallest of these limits: the time stands still
+    eng.set_state(Q0)
+    assert eng.advance(1, -0.0, 0.4, t=0.0) == 0.0
+    # and the next step forwards takes its own limit
+    eng.set_state(Q0)
+    assert eng.advance(1, 0.4, 0.4, t=0.0) == eng_dt(case, Q0, euler, nodes)
+    eng.close()
+
+
+def eng_dt(case, Q0, euler, nodes):
+    from horses3d_amd.engine import Engine
+    e = Engine(case, euler=euler, nodes=nodes, **KW)
+    e.set_state(Q0)
+    dt = e.max_dt(0.4, 0.4)
+    e.close()
+    return dt
