@@ -45,6 +45,7 @@
 #include "mixed_kernels.hpp"
 #include "gauss_kernels.hpp"
 #include "spectral.hpp"
+#include "host_transfer.hpp"
 
 using hx::NV;
 using hx::Phys;
@@ -532,8 +533,7 @@ struct hx3d_engine {
     int *hFlag = nullptr;
     // pinned host memory that finishing kernels write results to (H_* places), hFlag behind it
     double *hOut = nullptr;
-    char *ring = nullptr;   // pinned staging of host transfers (RING_SLOTS chunks), from the first one on
-    hipEvent_t ring_ev[4] = {nullptr, nullptr, nullptr, nullptr};
+    hxt::Ring ring;   // pinned staging of host transfers
     int device = 0;   // the HIP device the engine was created on
     // several independent cases in one engine (hx3d_engine_create_multi): per-case tables; with
     // one case ncases = 1, mc is all null and dTime = dScal + 1
@@ -891,81 +891,14 @@ void queue_status(hx3d_engine *eng)
                        eng->hOut + H_TIME);
 }
 
-// Host arrays move through a ring of pinned chunks, the copy of one chunk by the host overlapping the
-// transfer of the next: 13.7 MB to pageable memory took 759 us with hipMemcpyAsync (18 GB/s), 385 us
-// from it; the link does 55 GB/s from pinned memory and a host core copies 75 GB/s.  Four chunks of
-// 1 MB: the first waits 20 us, and 4 MB stay pinned per engine that moves host arrays.  Memory the
-// runtime knows (the caller's own pinned arrays) goes directly, and so does everything if the ring
-// cannot be had.
-constexpr int RING_SLOTS = 4;
-constexpr size_t RING_CHUNK = 1 << 20;
-
-bool use_ring(hx3d_engine *eng, const void *host)
-{
-    hipPointerAttribute_t at;
-    if (hipPointerGetAttributes(&at, host) != hipSuccess) (void)hipGetLastError();   // unknown: pageable
-    else if (at.type != hipMemoryTypeUnregistered) return false;
-    if (eng->ring) return true;
-    char *p = nullptr;
-    if (hipHostMalloc((void **)&p, RING_SLOTS * RING_CHUNK, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    for (int s = 0; s < RING_SLOTS; ++s)
-        if (!eng->ring_ev[s] && hipEventCreateWithFlags(&eng->ring_ev[s], hipEventDisableTiming) != hipSuccess) {
-            (void)hipGetLastError();
-            (void)hipHostFree(p);
-            return false;
-        }
-    eng->ring = p;
-    return true;
-}
-
-// bytes from the device to the host array dst, in stream order; complete on return
+// Transfers of host arrays on the engine's stream (see hxt)
 hipError_t copy_to_host(hx3d_engine *eng, void *dst, const void *src, size_t bytes)
 {
-    if (!use_ring(eng, dst)) {
-        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, eng->stream);
-        return e != hipSuccess ? e : hipStreamSynchronize(eng->stream);
-    }
-    const size_t n = (bytes + RING_CHUNK - 1) / RING_CHUNK;
-    auto size = [&](size_t c) { return std::min(RING_CHUNK, bytes - c * RING_CHUNK); };
-    for (size_t c = 0; c < n + RING_SLOTS; ++c) {
-        if (c >= RING_SLOTS) {   // chunk c - RING_SLOTS has arrived: out of its slot
-            const size_t b = c - RING_SLOTS;
-            if (b >= n) break;
-            const hipError_t e = hipEventSynchronize(eng->ring_ev[b % RING_SLOTS]);
-            if (e != hipSuccess) return e;
-            std::memcpy((char *)dst + b * RING_CHUNK, eng->ring + (b % RING_SLOTS) * RING_CHUNK, size(b));
-        }
-        if (c < n) {
-            hipError_t e = hipMemcpyAsync(eng->ring + (c % RING_SLOTS) * RING_CHUNK, (const char *)src + c * RING_CHUNK, size(c),
-                                          hipMemcpyDeviceToHost, eng->stream);
-            if (e == hipSuccess) e = hipEventRecord(eng->ring_ev[c % RING_SLOTS], eng->stream);
-            if (e != hipSuccess) return e;
-        }
-    }
-    return hipSuccess;
+    return hxt::copy_to_host(eng->ring, eng->device, eng->stream, dst, src, bytes);
 }
-
-// bytes from the host array src to the device, in stream order; src has been read on return
 hipError_t copy_to_device(hx3d_engine *eng, void *dst, const void *src, size_t bytes)
 {
-    if (!use_ring(eng, src)) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, eng->stream);
-    const size_t n = (bytes + RING_CHUNK - 1) / RING_CHUNK;
-    for (size_t c = 0; c < n; ++c) {
-        const size_t size = std::min(RING_CHUNK, bytes - c * RING_CHUNK);
-        char *slot = eng->ring + (c % RING_SLOTS) * RING_CHUNK;
-        // an earlier transfer of the slot (this call's, or one still queued) has left it
-        hipError_t e = hipEventSynchronize(eng->ring_ev[c % RING_SLOTS]);
-        if (e == hipSuccess) {
-            std::memcpy(slot, (const char *)src + c * RING_CHUNK, size);
-            e = hipMemcpyAsync((char *)dst + c * RING_CHUNK, slot, size, hipMemcpyHostToDevice, eng->stream);
-        }
-        if (e == hipSuccess) e = hipEventRecord(eng->ring_ev[c % RING_SLOTS], eng->stream);
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
+    return hxt::copy_to_device(eng->ring, eng->device, eng->stream, dst, src, bytes);
 }
 
 // After a queued step loop: the divergence flag's read-back, and the time derivative the
@@ -1887,9 +1820,7 @@ int hx3d_engine_destroy(hx3d_engine *eng)
     for (auto &e : eng->evpool) (void)hipEventDestroy(e);
     if (eng->step_graph) (void)hipGraphExecDestroy(eng->step_graph);
     if (eng->hOut) (void)hipHostFree(eng->hOut);
-    if (eng->ring) (void)hipHostFree(eng->ring);
-    for (hipEvent_t e : eng->ring_ev)
-        if (e) (void)hipEventDestroy(e);
+    hxt::destroy_ring(eng->ring);
     if (eng->stream) (void)hipStreamDestroy(eng->stream);
     delete eng;
     return HX3D_OK;

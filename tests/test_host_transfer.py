@@ -1,0 +1,28 @@
+"""The engine's host transfers on a stand-in for the HIP runtime (tests/host/transfer_fake_hip.cpp): exact
+through the ring of pinned chunks whatever the size, and with another device current than the engine's."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "horses3d_amd", "csrc")
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    if shutil.which("g++") is None or not os.path.exists(os.path.join(ROCM, "include", "hip")):
+        pytest.skip("needs g++ and the HIP headers")
+    exe = str(tmp_path_factory.mktemp("host") / "transfer")
+    r = subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROCM, "include"), "-I", CSRC,
+                        os.path.join(HERE, "host", "transfer_fake_hip.cpp"), "-o", exe], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-3000:]
+    return exe
+
+
+@pytest.mark.parametrize("check", ["same device", "another device current"])
+def test_transfers(program, check):
+    r = subprocess.run([program, check], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
