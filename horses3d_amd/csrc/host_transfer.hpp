@@ -56,9 +56,12 @@ inline void destroy_ring(Ring &r)
     r = Ring{};
 }
 
-// bytes from the device to the host array dst, in the order of the stream (of `device`); complete on return
+// bytes from the device to the host array dst, in the order of the stream (of `device`); complete on return.
+// An error that the launches before it left (the kernel that packs src) is this call's result: the
+// look at the pointer, which fails for every pageable array, would take its place.
 inline hipError_t copy_to_host(Ring &r, int device, hipStream_t stream, void *dst, const void *src, size_t bytes)
 {
+    if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     if (!use_ring(r, device, dst)) {
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
         return e != hipSuccess ? e : hipStreamSynchronize(stream);
@@ -84,9 +87,10 @@ inline hipError_t copy_to_host(Ring &r, int device, hipStream_t stream, void *ds
 }
 
 // bytes from the host array src to the device, in the order of the stream; through the ring src has been
-// read on return
+// read on return; earlier errors as in copy_to_host
 inline hipError_t copy_to_device(Ring &r, int device, hipStream_t stream, void *dst, const void *src, size_t bytes)
 {
+    if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     if (!use_ring(r, device, src)) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
     const size_t n = (bytes + RING_CHUNK - 1) / RING_CHUNK;
     for (size_t c = 0; c < n; ++c) {

@@ -97,10 +97,28 @@ static int transfers(int caller, int device)
     return 0;
 }
 
+// a failed launch before a transfer is the transfer's result, with and without a ring in place
+static int failed_launch()
+{
+    ihipStream_t s{0};
+    hxt::Ring r;
+    std::vector<char> a(100), b(100);
+    for (int pass = 0; pass < 2; ++pass) {
+        last = hipErrorLaunchFailure;
+        CHECK(hxt::copy_to_host(r, 0, &s, a.data(), b.data(), a.size()) == hipErrorLaunchFailure);
+        last = hipErrorLaunchFailure;
+        CHECK(hxt::copy_to_device(r, 0, &s, b.data(), a.data(), a.size()) == hipErrorLaunchFailure);
+        CHECK(hxt::copy_to_host(r, 0, &s, a.data(), b.data(), a.size()) == hipSuccess);
+        CHECK(last == hipSuccess);
+    }
+    return 0;
+}
+
 int main(int argc, char **argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "same device") return transfers(0, 0);
     if (what == "another device current") return transfers(1, 0);
+    if (what == "failed launch") return failed_launch();
     return 2;
 }
