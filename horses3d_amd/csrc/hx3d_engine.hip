@@ -1778,7 +1778,7 @@ int hx3d_engine_create_multi(const hx3d_case_desc *descs, int ncases, hx3d_engin
     if (!up(eng->dBlocks, blocks.data(), blocks.size() * sizeof(int4)) || !up(eng->dCC, cc.data(), cc.size() * sizeof(hxk::CaseConst)) ||
         !up(eng->dActive, ones.data(), ones.size() * 4))
         return eng->fail(HX3D_EDEVICE, "upload failed");
-    hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, eng->stream, eng->dTimeM, (long)ncases, 0.0);
+    hipLaunchKernelGGL(k_fill, dim3((ncases + 255) / 256), dim3(256), 0, eng->stream, eng->dTimeM, (long)ncases, 0.0);
     eng->dTime = eng->dTimeM;
     eng->mc = hxk::Multi{eng->dBlocks, eng->dCC, eng->dActive, ncases};
     init_slots(eng, ncases);

@@ -1,4 +1,4 @@
-"""Edges of the engine's entry points: CFL numbers of either sign."""
+"""Edges of the engine's entry points: CFL numbers of either sign, engines of many cases."""
 import numpy as np
 import pytest
 
@@ -62,3 +62,19 @@ def eng_dt(case, Q0, euler, nodes):
     dt = e.max_dt(0.4, 0.4)
     e.close()
     return dt
+
+
+def test_times_of_many_cases_start_at_zero():
+    """An engine of more than 256 cases, created where one that had advanced was before."""
+    from horses3d_amd.engine import MultiEngine
+    box, n = mesh.straight_box(2, 3), 600
+    Q0 = [mesh.taylor_green(box, 0.3)] * n
+    for _ in range(4):
+        eng = MultiEngine([box] * n, KW)
+        times, bad = eng.status()
+        assert not times.any() and not bad.any()
+        eng.set_states(Q0)
+        eng.advance(1, 0.4, 0.4)
+        times, _ = eng.status()
+        assert times[0] > 0.0 and np.all(times == times[0])
+        eng.close()
