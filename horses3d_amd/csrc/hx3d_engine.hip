@@ -1755,8 +1755,6 @@ int hx3d_engine_create_multi(const hx3d_case_desc *descs, int ncases, hx3d_engin
         cc[c].mu_to_kappa = 1.0 / (eng->ph.gm1 * M2 * d.prandtl);
         cc[c].les_c = d.les_c;
     }
-    if ((long)eng->F * nf / 256 + 1 < ncases)
-        return eng->fail(HX3D_EUNSUPPORTED, "too many cases of too few face nodes");
     // per-case replacements of the one-case dt slots, flags and time
     (void)hipStreamSynchronize(eng->stream);
     (void)hipFree(eng->dBits);

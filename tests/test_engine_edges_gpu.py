@@ -78,3 +78,26 @@ def test_times_of_many_cases_start_at_zero():
         times, _ = eng.status()
         assert times[0] > 0.0 and np.all(times == times[0])
         eng.close()
+
+
+@pytest.mark.parametrize("n,N,ncases", [(1, 1, 64), (1, 2, 300), (2, 1, 70)])
+def test_many_small_cases_match_cases_alone(n, N, ncases):
+    """More cases than their face nodes fill blocks of 256 with: each ends where it ends alone."""
+    from horses3d_amd.engine import Engine, MultiEngine
+    box = mesh.periodic_box(n, N, amplitude=0.1, phase_seed=4)
+    assert box["F"] * (N + 1) ** 2 * ncases // 256 + 1 < ncases
+    Q0 = [mesh.taylor_green(box, 0.3, noise=1e-2, seed=c) for c in range(ncases)]
+    phys = [dict(KW, reynolds=200.0 + c) for c in range(ncases)]
+    m = MultiEngine([box] * ncases, phys)
+    m.set_states(Q0)
+    m.advance(3, 0.4, 0.4)
+    times, bad = m.status()
+    got = m.get_states()
+    assert not bad.any()
+    for c in {0, 1, ncases // 2, ncases - 1}:
+        e = Engine(box, **phys[c])
+        e.set_state(Q0[c])
+        assert e.advance(3, 0.4, 0.4, t=0.0) == times[c], c
+        assert np.array_equal(e.get_state(), got[c]), c
+        e.close()
+    m.close()
