@@ -100,7 +100,7 @@ struct CaseConst {
 struct Multi {
     const int4 *blocks;     // per logical block: first element, element count, case, first block of its case
     const CaseConst *cc;    // [cases]
-    const int *active;      // [cases]: 0 = finished, its blocks do no work
+    const int *active;      // [cases]: 0 = finished, its blocks do no work (both copies of its state agree)
     int cases;
 };
 
@@ -113,20 +113,16 @@ __device__ __forceinline__ void case_physics(Phys &ph, const CaseConst &c)
 }
 
 // The elements of logical block lb: first element e0, count cnt (0: nothing to do), case cs,
-// and whether the block is its case's first; idle: the count of a finished case's block, whose
-// cnt is 0.  One case: EPB elements per block.
+// and whether the block is its case's first.  One case: EPB elements per block.
 template <int EPB>
 __device__ __forceinline__ void block_elements(const Multi &mc, int lb, int K, int &e0, int &cnt, int &cs, bool &first,
-                                               int &idle, Phys &ph)
+                                               Phys &ph)
 {
-    idle = 0;
     if (mc.blocks) {
         const int4 b = mc.blocks[lb];
-        const bool on = mc.active[b.z] != 0;
         e0 = b.x;
         cs = b.z;
-        cnt = on ? b.y : 0;
-        idle = on ? 0 : b.y;
+        cnt = mc.active[cs] ? b.y : 0;
         first = b.w != 0;
         case_physics(ph, mc.cc[cs]);
     } else {
@@ -315,9 +311,9 @@ k_grad(const double *__restrict__ Q, Metric mt, const int *__restrict__ nbr,
     __shared__ double sD[n1 * n1];
     const int lb = xcd_block(blockIdx.x, gridDim.x);
     const int t = threadIdx.x;
-    int e0, cnt, cs, idle;
+    int e0, cnt, cs;
     bool first;
-    block_elements<EPB>(mc, lb, K, e0, cnt, cs, first, idle, ph);
+    block_elements<EPB>(mc, lb, K, e0, cnt, cs, first, ph);
     if (cnt == 0) return;   // uniform: a padding block or a finished case
     const int el = t / ne, n = t - el * ne;
     const int e = e0 + el;
@@ -655,19 +651,13 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
     double *const sFb = sT + EPB * L::NVT * ne;       // [NV][FACES]
     const int lb = xcd_block(blockIdx.x, gridDim.x);
     const int t = threadIdx.x;
-    int e0, cnt, cs, idle;
+    int e0, cnt, cs;
     bool first;
     if (SPLIT) ph.averaging = FORM;   // the Lax-Friedrichs flux averages as the volume fluxes do
-    block_elements<EPB>(mc, lb, K, e0, cnt, cs, first, idle, ph);
+    block_elements<EPB>(mc, lb, K, e0, cnt, cs, first, ph);
+    if (cnt == 0) return;   // uniform: a padding block or a finished case
     const int el = t / ne, n = t - el * ne;
     const int e = e0 + el;
-    if (cnt == 0) {   // uniform: a padding block, or a finished case, whose state moves to Qn as it is
-        if (update && el < idle) {
-#pragma unroll
-            for (int v = 0; v < NV; ++v) stg(Qn + v * S, (unsigned)e * ne + n, ldg(Q + v * S, (unsigned)e * ne + n));
-        }
-        return;
-    }
     const bool active = el < cnt;
     const int i = n % n1, j = (n / n1) % n1, k = n / nf;
     const bool onx = i == 0 || i == N, ony = j == 0 || j == N, onz = k == 0 || k == N;

@@ -1,4 +1,7 @@
-"""Edges of the engine's entry points: CFL numbers of either sign, engines of many cases."""
+"""Edges of the engine's entry points: CFL numbers of either sign, engines of many cases and of finished
+ones."""
+import time
+
 import numpy as np
 import pytest
 
@@ -100,4 +103,87 @@ def test_many_small_cases_match_cases_alone(n, N, ncases):
         assert e.advance(3, 0.4, 0.4, t=0.0) == times[c], c
         assert np.array_equal(e.get_state(), got[c]), c
         e.close()
+    m.close()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_finished_cases_keep_their_state(graph):
+    """Cases switched off and on again after odd and even numbers of stages, with states set while one is
+    off: each ends where it ends alone, and a finished one reads back the same after every step."""
+    from horses3d_amd.engine import Engine, MultiEngine
+    boxes = [mesh.periodic_box(n, 3, amplitude=0.1, phase_seed=n) for n in (2, 1, 3)]
+    phys = [dict(KW, reynolds=300.0 + 100.0 * c) for c in range(3)]
+    Q0 = [mesh.taylor_green(b, 0.3, noise=1e-2, seed=c) for c, b in enumerate(boxes)]
+    alone = [Engine(b, **p) for b, p in zip(boxes, phys)]
+    m = MultiEngine(boxes, phys)
+    m.set_step_graph(graph)
+    on = [True] * 3
+
+    def states(qs):
+        m.set_states(qs)
+        for e, q in zip(alone, qs):
+            e.set_state(q)
+
+    def switch(c, to):
+        m.set_active(c, to)
+        on[c] = to
+
+    def steps(n):
+        m.advance(n, 0.4, 0.4)
+        for c, e in enumerate(alone):
+            if on[c]:
+                e.advance(n, 0.4, 0.4)
+        got = m.get_states()
+        for c, e in enumerate(alone):
+            assert np.array_equal(got[c], e.get_state()), c
+
+    states(Q0)
+    steps(1)
+    switch(1, False)
+    steps(1)
+    steps(2)
+    switch(0, False)
+    switch(0, False)                 # again: nothing changes
+    steps(5)
+    switch(1, True)
+    steps(1)
+    states([q[::-1].copy() for q in Q0])   # while case 0 is off
+    steps(3)
+    switch(0, True)
+    steps(2)
+    switch(0, False)
+    switch(2, False)
+    m.rk3_step(0.0, 1e-4)
+    alone[1].rk3_step(0.0, 1e-4)
+    steps(0)
+    m.close()
+    for e in alone:
+        e.close()
+
+
+def test_finished_cases_cost_no_memory_traffic():
+    """Sixteen cases of 12^3 elements of order 4: a step with all of them finished takes what its launches
+    take (33 us, 0.026 of a step with all of them on); carrying the states along from copy to copy took 241
+    us (0.19)."""
+    from horses3d_amd.engine import MultiEngine
+    box = mesh.straight_box(12, 4)
+    m = MultiEngine([box] * 16, KW)
+    m.set_states([mesh.taylor_green(box, 0.3)] * 16)
+
+    def per_step():
+        best = np.inf
+        for _ in range(7):
+            m.synchronize()
+            t0 = time.perf_counter()
+            m.advance(20, 0.4, 0.4)
+            m.synchronize()
+            best = min(best, (time.perf_counter() - t0) / 20)
+        return best
+
+    on = per_step()
+    for c in range(16):
+        m.set_active(c, False)
+    off = per_step()
+    print("step with all on %.1f us, with all finished %.1f us" % (1e6 * on, 1e6 * off), flush=True)
+    assert off < 0.06 * on
     m.close()
