@@ -1475,6 +1475,9 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
 
     const int K = eng->K, n1 = eng->n1, nf = eng->nf, ne = eng->ne, F = eng->F;
     const long S = eng->S, nodes = eng->nodes, FS = eng->FS, ES = eng->ES;
+    // before the tables, whose entries (up to 2 ES) are 32-bit
+    if (!offsets_fit(S, ES, FS))
+        return bail(eng->fail(HX3D_EUNSUPPORTED, "mesh too large: more than 2^29 - 1 nodes (or face nodes) per array"));
     // ---- host tables --------------------------------------------------------------
     auto node_of = [&](int e, int slot, int a, int b) -> long {
         int idx[3];
@@ -1519,8 +1522,6 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
     }
     for (size_t x = 0; x < nbx.size(); ++x)
         if (nbx[x] < 0) return bail(eng->fail(HX3D_EINVAL, "an element face node has no neighbour"));
-    if (!offsets_fit(S, ES, FS))
-        return bail(eng->fail(HX3D_EUNSUPPORTED, "mesh too large: more than 2^29 - 1 nodes (or face nodes) per array"));
     // geometry SoA, J, 1/J, quadrature weights, LES filter widths, face frames
     std::vector<double> ja, jj((size_t)S, 1.0), wq((size_t)S, 0.0), edelta(K), efdelta((size_t)6 * K);
     ja.reserve((size_t)9 * S + 10 * ((K + 63) / 64) * 64);   // with element_metrics' planes

@@ -1,5 +1,5 @@
 """Edges of the engine's entry points: CFL numbers of either sign, engines of many cases and of finished
-ones."""
+ones, meshes beyond the 32-bit offsets."""
 import time
 
 import numpy as np
@@ -187,3 +187,15 @@ def test_finished_cases_cost_no_memory_traffic():
     print("step with all on %.1f us, with all finished %.1f us" % (1e6 * on, 1e6 * off), flush=True)
     assert off < 0.06 * on
     m.close()
+
+
+def test_mesh_beyond_the_offsets_is_refused_by_its_size():
+    """2^29 element face nodes and more: refused as too large before any table is built, whose 32-bit
+    entries would wrap (the tables and geometry here are untouched zeros)."""
+    from horses3d_amd.engine import Engine
+    K = 2 ** 29 // 24 + 1   # order 1
+    case = dict(K=K, F=3 * K, N=np.ones((K, 3), np.int32), J=np.zeros(8 * K), Ja=np.zeros((8 * K, 9)))
+    for name, shape in (("faceID", (K, 6)), ("faceSide", (K, 6)), ("fElem", (3 * K, 2)), ("fESide", (3 * K, 2)), ("fRot", 3 * K)):
+        case[name] = np.zeros(shape, np.int32)
+    with pytest.raises(Exception, match="mesh too large"):
+        Engine(case, **KW)
