@@ -19,9 +19,13 @@ struct Phys {
     int riemann, averaging, les, euler;
 };
 
-// a / b with y = 1 / b in hand, the bits of the division: q = a y, the exact remainder a - b q by a
-// fused multiply-add, and one correction (Markstein, IBM J. Res. Dev. 34(1), 1990).  Three
-// instructions instead of the division's eleven, for the many quotients by one density.
+// a / b with y = 1 / b in hand: q = a y, the remainder a - b q by a fused multiply-add, and one correction
+// (Markstein, IBM J. Res. Dev. 34(1), 1990).  Three instructions instead of the division's eleven, for
+// the many quotients by one density.  The bits of the division for finite a and b with 1/b and a/b normal
+// and |a| >= 2^-968: tested, not proven (the proof wants q within one ulp, a y is within one and a half;
+// 3.7e9 pairs, 7e8 of them the quotients nearest to the middle between two doubles, show no difference).
+// Elsewhere: -0/b gives +0; an infinite a or b and a b that is zero or subnormal give NaN, where the
+// division may give infinity or zero: a state with such values has diverged and becomes NaN a little sooner.
 HX_HD double quot(double a, double b, double y)
 {
     const double q = a * y;
