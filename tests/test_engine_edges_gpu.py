@@ -1,5 +1,5 @@
 """Edges of the engine's entry points: CFL numbers of either sign, engines of many cases and of finished
-ones, meshes beyond the 32-bit offsets."""
+ones, meshes beyond the 32-bit offsets, what an Euler engine holds."""
 import time
 
 import numpy as np
@@ -25,20 +25,27 @@ def one_step_matches(eng, ora, Q0, cfl, dcfl):
     assert np.all(np.abs(eng.get_state() - Q).max(axis=0) <= TOL * dq + floor)
 
 
+def gauss_box(n, N, tmp_path):
+    """An n^3 curvilinear box from the front end on Gauss nodes, with the oracle's face tables."""
+    from horses3d_amd.engine import read_specmesh
+    path = str(tmp_path / "box.mesh")
+    specmesh.write_specmesh(path, n, 0.1, mesh.box_phases(5), bface_order=N + 1)
+    case = read_specmesh(path, N=N, periodic=dict(specmesh.PERIODIC_PAIRS), nodes="gauss")
+    case["fNf"] = np.full((case["F"], 2), N, np.int32)
+    case["foff"] = np.arange(case["F"] + 1, dtype=np.int64) * (N + 1) ** 2
+    return case
+
+
 @pytest.mark.parametrize("kind,cfl,dcfl", [(k, c, d) for k in ("gauss-lobatto", "euler", "gauss", "mixed")
                                            for c, d in ((-0.1, -0.1), (0.1, -0.1), (-0.1, 0.1))
                                            if c < 0.0 or k != "euler"])   # Euler: no viscous limit
 def test_negative_cfl_numbers(kind, cfl, dcfl, tmp_path):
     """A negative CFL number steps backwards with the limit of the smallest value, as max_dt gives it: the
     minima of the blocks order like the numbers, not like their bits."""
-    from horses3d_amd.engine import Engine, read_specmesh
+    from horses3d_amd.engine import Engine
     N, euler = 3, kind == "euler"
     if kind == "gauss":
-        path = str(tmp_path / "box.mesh")
-        specmesh.write_specmesh(path, 3, 0.1, mesh.box_phases(5), bface_order=4)
-        case = read_specmesh(path, N=N, periodic=dict(specmesh.PERIODIC_PAIRS), nodes="gauss")
-        case["fNf"] = np.full((case["F"], 2), N, np.int32)
-        case["foff"] = np.arange(case["F"] + 1, dtype=np.int64) * (N + 1) ** 2
+        case = gauss_box(3, N, tmp_path)
     elif kind == "mixed":
         case = mesh.periodic_box_mixed(3, mesh.random_orders(27, 2, 4, 5))
     else:
@@ -199,3 +206,28 @@ def test_mesh_beyond_the_offsets_is_refused_by_its_size():
         case[name] = np.zeros(shape, np.int32)
     with pytest.raises(Exception, match="mesh too large"):
         Engine(case, **KW)
+
+
+@pytest.mark.parametrize("nodes", ["gauss-lobatto", "gauss"])
+def test_euler_engine_holds_no_viscous_arrays(nodes, tmp_path):
+    """An Euler engine's memory is that of a Navier-Stokes one without nine viscous values and |curl u|^2 a
+    node (Gauss nodes: and nine values an element face node); every call works on it."""
+    from horses3d_amd.engine import Engine
+    n, N = 4, 3
+    case = gauss_box(n, N, tmp_path) if nodes == "gauss" else mesh.periodic_box(n, N, amplitude=0.1, phase_seed=5)
+    ns, eu = (Engine(case, euler=e, nodes=nodes, **KW) for e in (False, True))
+    held = 10 * n ** 3 * (N + 1) ** 3 + (9 * 6 * n ** 3 * (N + 1) ** 2 if nodes == "gauss" else 0)
+    assert ns.device_bytes() - eu.device_bytes() == 8 * held
+    Q0 = mesh.taylor_green(case, 0.3)
+    eu.set_state(Q0)
+    eu.advance(2, 0.4, 0.4, t=0.0)
+    for kind in ("kinetic energy", "kinetic energy rate", "mean velocity", "internal energy", "entropy", "math entropy"):
+        assert np.isfinite(eu.volume_monitor(kind)), kind
+    with pytest.raises(Exception, match="enstrophy"):
+        eu.volume_monitor("enstrophy")
+    assert np.all(np.isfinite(eu.residuals())) and np.all(np.isfinite(eu.qdot()))
+    ora = po.Oracle(case, po.make_params(0.3, 700.0, riemann="roe", euler=True, nodes=nodes))
+    eu.set_state(Q0)
+    assert po.normwise_error(eu.qdot(), ora.qdot(Q0)).max() <= TOL
+    ns.close()
+    eu.close()
