@@ -512,9 +512,7 @@ struct hx3d_engine {
     bool mixed = false;
     bool t2x = false;     // uniform orders: the volume kernel forms t2 = n x t1 (see tangent2_is_cross)
     bool gauss = false;   // Gauss nodes (one order: hxg kernels; per-element orders: the mixed path's)
-    long FSm = 0;
     int *dN3 = nullptr, *dEofn = nullptr;
-    long *dOff = nullptr;
     hxm::FaceRec *dFaces = nullptr;
     int4 *dSched = nullptr;   // the face kernels' waves (hxm::face_lane): one face, or two of one shape
     int nwaves = 0;
@@ -529,9 +527,6 @@ struct hx3d_engine {
     long map_big = 0;
     int grid_mgrad_s = 0, grid_mgrad_b = 0, grid_mvol_s = 0, grid_mvol_b = 0;
     std::vector<int> N3h_mixed;   // [3K] element orders (host copy for re-tiling)
-    // side streams for the element-bucket launches (the buckets touch disjoint elements, so
-    // they run side by side), forked from and joined back to the engine stream with events
-    bool capturing = false;   // a step graph is being captured
     std::vector<int> N3h;   // element orders (Nx, Ny, Nz), host copy for solution files
     double mach = 0;
     bool qdot_valid = false, timing = false;
@@ -619,7 +614,6 @@ int elem_grid(const hx3d_engine *eng, int epb)
     if (eng->mc.blocks) return grid_for(eng->nblocks_multi);
     return grid_for((eng->K + epb - 1) / epb);
 }
-int grad_grid(const hx3d_engine *eng) { return elem_grid(eng, eng->gauss ? 1 : epb_for(eng->N)); }
 
 // Gauss nodes, one order: the Q traces of the resident state, after it is set from outside
 template <int N>
@@ -657,7 +651,7 @@ void launch_grad(hx3d_engine *eng, const hxk::DtLimits &dtl, double *curl)
     constexpr int TPB = ((EPB * ne + 63) / 64) * 64;
     auto *kernel = eng->ph.les ? &hxk::k_grad<N, EPB, true> : &hxk::k_grad<N, EPB, false>;
     hipLaunchKernelGGL(kernel, dim3(elem_grid(eng, EPB)), dim3(TPB), 0, eng->stream, eng->dQ, metric(eng),
-                       eng->dNbr, eng->dVisc, curl, eng->K, eng->S, eng->ES, eng->ops, eng->ph, dtl,
+                       eng->dNbr, eng->dVisc, curl, eng->K, eng->S, eng->ops, eng->ph, dtl,
                        eng->mc);
 }
 
@@ -673,7 +667,7 @@ void launch_volume_e(hx3d_engine *eng, double a_k, double c_k, int update, const
         hipLaunchKernelGGL((hxk::k_volume<N, EPB, FORM, LXF, VIS>), dim3(elem_grid(eng, EPB)), dim3(TPB), lds, eng->stream,
                            eng->dQ, eng->dQn, eng->dVisc,
                            eng->dEdelta, eng->dEfdelta, eng->dNbx, metric(eng), eng->t2x ? 1 : 0, eng->dG, qdot, a_k, c_k,
-                           update, dta, eng->K, eng->S, eng->ES, eng->ops, eng->ph, eng->mc);
+                           update, dta, eng->K, eng->S, eng->ops, eng->ph, eng->mc);
     };
     auto pick = [&](auto lxf) {
         if (eng->ph.euler) go(lxf, std::integral_constant<int, hxk::INVISCID>{});
@@ -1253,7 +1247,6 @@ int create_mixed(hx3d_engine *eng, const hx3d_case_desc *d)
         r.foff = (int)fsm;
         fsm += (long)(Nf0 + 1) * (Nf1 + 1);
     }
-    eng->FSm = fsm;
     const std::vector<int4> sched = face_waves(shapes);
     eng->nwaves = (int)sched.size();
     // operators of every order
@@ -1357,7 +1350,7 @@ int create_mixed(hx3d_engine *eng, const hx3d_case_desc *d)
         (rc = dalloc(eng, &eng->dDtPart, (size_t)2 * (std::max((long)K, (S + 255) / 256) + 64))) ||
         (rc = dalloc(eng, &eng->dStage, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dBits, 2 * DT_SLOTS)) ||
         (rc = dalloc(eng, &eng->dFlag, 2)) || (rc = dalloc(eng, &eng->dN3, N3.size())) ||
-        (rc = dalloc(eng, &eng->dOff, off.size())) || (rc = dalloc(eng, &eng->dEofn, eofn.size())) ||
+        (rc = dalloc(eng, &eng->dEofn, eofn.size())) ||
         (rc = dalloc(eng, &eng->dFaces, faces.size())) || (rc = dalloc(eng, &eng->dSched, sched.size())) ||
         (rc = dalloc(eng, &eng->dOpsAll, 1)))
         return rc;
@@ -1370,7 +1363,6 @@ int create_mixed(hx3d_engine *eng, const hx3d_case_desc *d)
         !up(eng->dJ, jj.data(), jj.size() * 8) || !up(eng->dFgeo, fgeo.data(), fgeo.size() * 8) ||
         !up(eng->dWq, wq.data(), wq.size() * 8) || !up(eng->dEdelta, edelta.data(), edelta.size() * 8) ||
         !up(eng->dFdelta, fdelta.data(), fdelta.size() * 8) || !up(eng->dN3, N3.data(), N3.size() * 4) ||
-        !up(eng->dOff, off.data(), off.size() * 8) ||
         !up(eng->dEofn, eofn.data(), eofn.size() * 4) ||
         !up(eng->dFaces, faces.data(), faces.size() * sizeof(hxm::FaceRec)) ||
         !up(eng->dSched, sched.data(), sched.size() * sizeof(int4)) || !up(eng->dOpsAll, &oa, sizeof(oa)))
@@ -1833,7 +1825,7 @@ int hx3d_engine_destroy(hx3d_engine *eng)
     void *ptrs[] = {eng->dQ, eng->dG, eng->dJa, eng->dJ, eng->dFgeo, eng->dEgeo, eng->dFe,
                     eng->dQDot, eng->dEdelta, eng->dFdelta, eng->dWq, eng->dScal, eng->dPart, eng->dStage,
                     eng->dBits, eng->dNbr, eng->dFlag, eng->dN3,
-                    eng->dEofn, eng->dOff, eng->dFaces, eng->dSched, eng->dOpsAll, eng->dU, eng->dLift, eng->dDtPart, eng->dTmap,
+                    eng->dEofn, eng->dFaces, eng->dSched, eng->dOpsAll, eng->dU, eng->dLift, eng->dDtPart, eng->dTmap,
                     eng->dBlocks, eng->dCC, eng->dActive, eng->dTimeM,
                     eng->dQtr, eng->dQtn, eng->dFvis, eng->dNbx, eng->dQn, eng->dVisc, eng->dCurl, eng->dEfdelta, eng->dSlots};
     for (void *p : ptrs)
@@ -2036,7 +2028,7 @@ int hx3d_advance(hx3d_engine *eng, int nsteps, double cfl, double dcfl, double *
     // copies of the state: ev, when given, holds 12 events for the step.
     auto issue_step = [eng, cfl, dcfl](hipEvent_t *ev, double *qdot) {
         unsigned long long *slot = dt_slot(eng, 0);
-        int nparts;
+        int nparts = eng->mixed ? eng->grid_mgrad_s + eng->grid_mgrad_b : 0;   // of the gradient kernel (mixed orders)
         if (eng->ph.euler) {
             const long nb = (eng->nodes + 255) / 256;
             if (eng->mixed)
@@ -2048,8 +2040,6 @@ int hx3d_advance(hx3d_engine *eng, int nsteps, double cfl, double dcfl, double *
                                    eng->nodes, eng->S, eng->dcsi, cfl, dcfl, eng->ph, eng->dDtPart,
                                    two_launch(eng) ? eng->dSlots : nullptr);
             nparts = (int)nb;
-        } else {
-            nparts = eng->mixed ? eng->grid_mgrad_s + eng->grid_mgrad_b : grad_grid(eng);
         }
         for (int k = 0; k < 3; ++k) {
             DtArgs a{};
@@ -2085,10 +2075,8 @@ int hx3d_advance(hx3d_engine *eng, int nsteps, double cfl, double dcfl, double *
             }
             hipGraph_t g = nullptr;
             HIPCHK(hipStreamBeginCapture(eng->stream, hipStreamCaptureModeThreadLocal));
-            eng->capturing = true;
             eng->graph_Q = current_copy(eng);
             for (int s = 0; s < per; ++s) issue_step(nullptr, nullptr);
-            eng->capturing = false;
             const hipError_t ce = hipStreamEndCapture(eng->stream, &g);
             if (ce != hipSuccess || !g) return eng->fail(HX3D_EDEVICE, std::string("step capture: ") + hipGetErrorString(ce));
             const hipError_t ie = hipGraphInstantiate(&eng->step_graph, g, nullptr, nullptr, 0);

@@ -98,12 +98,12 @@ HX_HD void euler_contravariant(const Phys &ph, const double q[NV], const double 
             out[d][c] = F[c][0] * ja[3 * d] + F[c][1] * ja[3 * d + 1] + F[c][2] * ja[3 * d + 2];
 }
 
-// navierstokes/Physics_NS.f90:246-304 ViscousFlux_STATE (beta = 0), split in two halves:
+// navierstokes/Physics_NS.f90:246-304 ViscousFlux_STATE (beta = 0), split in parts:
 //   viscous_state   the velocity gradients u_x, u_y, u_z and grad T it forms from Q and the
 //                   lifted state gradients: vg[0..2] = u_x, vg[3..5] = u_y, vg[6..8] = u_z,
 //                   vg[9..11] = grad T;
-//   viscous_flux    the stress / heat-flux tail F[v][c] from mu, kappa, the velocity and vg, itself
-//                   the viscous_tensor of the stress_shape.
+//   viscous_tensor  the stress / heat-flux tail F[v][c] from mu, kappa, the velocity, the stress_shape
+//                   of vg and grad T.
 // Together they perform the reference's operations in its order.
 HX_HD void viscous_state(const Phys &ph, const double q[NV], const double gx[NV], const double gy[NV],
                          const double gz[NV], double vg[12])
@@ -151,20 +151,6 @@ HX_HD void viscous_tensor(double mu, double kappa, double u, double v, double w,
 constexpr int viscous_entry(int v, int c)
 {
     return v == 4 ? 6 + c : v == 1 ? c : v == 2 ? (c == 0 ? 1 : 2 + c) : (c == 0 ? 2 : 3 + c);
-}
-
-HX_HD void viscous_flux(double mu, double kappa, double u, double v, double w, const double vg[12],
-                        double F[NV][3])
-{
-    double s[6], f[9];
-    stress_shape(vg, s);
-    viscous_tensor(mu, kappa, u, v, w, s, vg + 9, f);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        F[0][c] = 0.0;
-#pragma unroll
-        for (int q = 1; q < NV; ++q) F[q][c] = f[viscous_entry(q, c)];
-    }
 }
 
 // common/LESModels.f90:256-307 Smagorinsky and :358-~440 WALE eddy viscosity (no wall model),

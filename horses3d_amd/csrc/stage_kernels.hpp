@@ -304,7 +304,7 @@ template <int N, int EPB, bool LES>
 __global__ void __launch_bounds__(((EPB * (N + 1) * (N + 1) * (N + 1) + 63) / 64) * 64)
 __attribute__((amdgpu_waves_per_eu(HX3D_GRAD_WAVES)))
 k_grad(const double *__restrict__ Q, Metric mt, const int *__restrict__ nbr,
-       double *__restrict__ visc, double *__restrict__ curl_out, int K, long S, long ES, Ops ops, Phys ph, DtLimits dtl, Multi mc)
+       double *__restrict__ visc, double *__restrict__ curl_out, int K, long S, Ops ops, Phys ph, DtLimits dtl, Multi mc)
 {
     constexpr int n1 = N + 1, nf = n1 * n1, ne = nf * n1;
     __shared__ double sQ[EPB][NV][ne];
@@ -633,7 +633,7 @@ __attribute__((amdgpu_waves_per_eu(volume_waves(N, FORM))))
 k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__restrict__ visc,
          const double *__restrict__ edelta, const double *__restrict__ efdelta, const int *__restrict__ nbx,
          Metric mt, int t2x, double *__restrict__ G, double *__restrict__ qdot_out, double a_k, double c_k, int update,
-         DtArgs dta, int K, long S, long ES, Ops ops, Phys ph, Multi mc)
+         DtArgs dta, int K, long S, Ops ops, Phys ph, Multi mc)
 {
     using L = VolumeLds<N, EPB, FORM, VIS>;
     constexpr bool LES = VIS == EDDY, EULER = VIS == INVISCID;
