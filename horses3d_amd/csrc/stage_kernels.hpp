@@ -184,14 +184,11 @@ __device__ __forceinline__ unsigned efx(int e, int slot, int a, int b)
 //   mt             metric terms; face frames: normal (c = 0..2) and surface Jacobian |Ja| (c = 3)
 //   visc[c*S+g]    out: the viscous flux tensor or the LES values
 // ------------------------------------------------------------------------------------
-// Registers: at most 128 (the state is read again after the gradient, LES is a template flag, and
-// order 7 takes its directions one at a time), since a block of six or eight waves finds room beside
-// another only at four waves per SIMD: 9^3 elements of order 6 24.0 -> 19.9 us, of order 7 31.6 -> 25.7 (with
+// Registers: at most 128, which the attribute holds it to (114 to 124 are taken: the state is read again
+// after the gradient, LES is a template flag, and order 7 takes its directions one at a time), since a
+// block of six or eight waves finds room beside another only at four waves per SIMD: 9^3 elements of order 6 24.0 -> 19.9 us, of order 7 31.6 -> 25.7 (with
 // LES).  Below that it makes no difference: at 16^3 elements of order 4 the kernel moves 153 MB in 28.4 us, 24^3
 // of order 5 898 MB in 193 us, near the copy rate (6.9 TB/s from the caches, 5 from memory).
-#ifndef HX3D_GRAD_WAVES
-#define HX3D_GRAD_WAVES 1
-#endif
 
 // Metric terms of a case of one order: Ja^d_c in planes Ja[c*S + i], J[i], and the face frames
 // face[c*FS + i].  Where they are the same bits at every node of each element (each face), as on boxes of
@@ -302,7 +299,7 @@ __device__ __forceinline__ void les_tensor(const Phys &ph, const double *q, doub
 
 template <int N, int EPB, bool LES>
 __global__ void __launch_bounds__(((EPB * (N + 1) * (N + 1) * (N + 1) + 63) / 64) * 64)
-__attribute__((amdgpu_waves_per_eu(HX3D_GRAD_WAVES)))
+__attribute__((amdgpu_waves_per_eu(4)))
 k_grad(const double *__restrict__ Q, Metric mt, const int *__restrict__ nbr,
        double *__restrict__ visc, double *__restrict__ curl_out, int K, long S, Ops ops, Phys ph, DtLimits dtl, Multi mc)
 {
