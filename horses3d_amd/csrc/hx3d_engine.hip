@@ -1471,27 +1471,27 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
     if (!offsets_fit(S, ES, FS))
         return bail(eng->fail(HX3D_EUNSUPPORTED, "mesh too large: more than 2^29 - 1 nodes (or face nodes) per array"));
     // ---- host tables --------------------------------------------------------------
-    auto node_of = [&](int e, int slot, int a, int b) -> long {
-        int idx[3];
-        idx[SLOT_AXIS[slot]] = SLOT_PLUS[slot] ? N : 0;
-        idx[SLOT_U[slot]] = a;
-        idx[SLOT_V[slot]] = b;
-        return (long)e * ne + idx[0] + n1 * (idx[1] + n1 * idx[2]);
-    };
-    // per element face node x = (6e + slot) nf + a + (N+1) b: nbr[x] = 2 * (neighbour's node) and
-    // nbx[x] = 2 * (neighbour's element face node), each + 1 on the face's right side; per face, the
-    // right side's element face nodes in the left side's order (permuted by the rotation)
-    std::vector<int> nbr(eng->gauss ? 0 : (size_t)K * 6 * nf), nbx((size_t)K * 6 * nf, -1);
-    auto right_nodes = [&](int f, long *xR, long *gR) {
-        const int eR = d->fElem[2 * f + 1], sR = d->fESide[2 * f + 1] - 1, rot = d->fRot[f];
-        for (int j = 0; j <= N; ++j)
-            for (int i = 0; i <= N; ++i) {
-                int ii, jj;
-                left_to_right(i, j, N, N, rot, ii, jj);
-                xR[i + n1 * j] = ((long)eR * 6 + sR) * nf + ii + n1 * jj;
-                if (gR) gR[i + n1 * j] = node_of(eR, sR, ii, jj);
+    // face node x = a + (N+1) b of a slot as the element's node, and, under each rotation, the right side's
+    // face node that meets the left side's node x
+    int slot_node[6][64], turned[8][64];
+    for (int b = 0; b <= N; ++b)
+        for (int a = 0; a <= N; ++a) {
+            for (int slot = 0; slot < 6; ++slot) {
+                int idx[3];
+                idx[SLOT_AXIS[slot]] = SLOT_PLUS[slot] ? N : 0;
+                idx[SLOT_U[slot]] = a;
+                idx[SLOT_V[slot]] = b;
+                slot_node[slot][a + n1 * b] = idx[0] + n1 * (idx[1] + n1 * idx[2]);
             }
-    };
+            for (int rot = 0; rot < 8; ++rot) {
+                int ii, jj;
+                left_to_right(a, b, N, N, rot, ii, jj);
+                turned[rot][a + n1 * b] = ii + n1 * jj;
+            }
+        }
+    // per element face node x = (6e + slot) nf + a + (N+1) b: nbr[x] = 2 * (neighbour's node) and
+    // nbx[x] = 2 * (neighbour's element face node), each + 1 on the face's right side
+    std::vector<int> nbr(eng->gauss ? 0 : (size_t)K * 6 * nf), nbx((size_t)K * 6 * nf, -1);
     for (int f = 0; f < F; ++f) {
         const int eL = d->fElem[2 * f], eR = d->fElem[2 * f + 1];
         const int sL = d->fESide[2 * f] - 1, sR = d->fESide[2 * f + 1] - 1, rot = d->fRot[f];
@@ -1500,15 +1500,14 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
         if (d->faceID[6 * eL + sL] != f || d->faceSide[6 * eL + sL] != 1 || d->faceID[6 * eR + sR] != f ||
             d->faceSide[6 * eR + sR] != 2)
             return bail(eng->fail(HX3D_EINVAL, "face " + std::to_string(f) + ": inconsistent with element faceID/faceSide"));
-        long xR[64], gR[64];
-        right_nodes(f, xR, gR);
-        const long xL0 = ((long)eL * 6 + sL) * nf;
+        const long xL0 = ((long)eL * 6 + sL) * nf, xR0 = ((long)eR * 6 + sR) * nf, gL0 = (long)eL * ne, gR0 = (long)eR * ne;
         for (int x = 0; x < nf; ++x) {
-            nbx[xL0 + x] = (int)(2 * xR[x]);
-            nbx[xR[x]] = (int)(2 * (xL0 + x) + 1);
+            const int y = turned[rot][x];
+            nbx[xL0 + x] = (int)(2 * (xR0 + y));
+            nbx[xR0 + y] = (int)(2 * (xL0 + x) + 1);
             if (!eng->gauss) {
-                nbr[xL0 + x] = (int)(2 * gR[x]);
-                nbr[xR[x]] = (int)(2 * node_of(eL, sL, x % n1, x / n1) + 1);
+                nbr[xL0 + x] = (int)(2 * (gR0 + slot_node[sR][y]));
+                nbr[xR0 + y] = (int)(2 * (gL0 + slot_node[sL][x]) + 1);
             }
         }
     }
@@ -1553,7 +1552,7 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
                 for (int c = 0; c < 3; ++c) { nr[c] = d->fNormal[3 * q + c]; t1[c] = d->fT1[3 * q + c]; t2[c] = d->fT2[3 * q + c]; }
                 jac = d->fJac[q];
             } else {
-                const long g = node_of(eL, sL, x % n1, x / n1);
+                const long g = (long)eL * ne + slot_node[sL][x];
                 for (int c = 0; c < 3; ++c) nr[c] = sg * d->Ja[9 * g + 3 * dax + c];
                 jac = std::sqrt(nr[0] * nr[0] + nr[1] * nr[1] + nr[2] * nr[2]);
                 for (int c = 0; c < 3; ++c) nr[c] /= jac;
@@ -1572,20 +1571,29 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
             if (lxf && eng->t2x) eng->t2x = tangent2_is_cross(nr, t1, t2);
         }
     };
+    // The planes in arrays of their own (pages touched as they are filled): n and |Ja|, t1, t2.  Together
+    // they pass the 32 MB up to which the allocator keeps freed pages on meshes where each alone does not:
+    // 16^3 elements of order 4 faulted 34 MB in again at every creation, 24.5 against 22.3 ms.
+    std::unique_ptr<double[]> eplanes[3] = {std::unique_ptr<double[]>(new double[(size_t)4 * ES]),
+                                            std::unique_ptr<double[]>(lxf ? new double[(size_t)3 * ES] : nullptr), nullptr};
+    auto plane = [&](int c, long stride) {
+        const int part = c < 4 ? 0 : c < 7 ? 1 : 2;
+        return eplanes[part].get() + (c - (part ? 3 * part + 1 : 0)) * stride;
+    };
     // planes c0..c1-1 of a face's frame to both sides, a run of nodes at a time
-    std::unique_ptr<double[]> egeo(new double[(size_t)(lxf ? 10 : 4) * ES]);   // pages touched as planes are filled
     auto put_frame = [&](int f, const double (*fr)[64], int c0, int c1) {
-        long xR[64];
-        right_nodes(f, xR, nullptr);
-        const long xL0 = ((long)d->fElem[2 * f] * 6 + d->fESide[2 * f] - 1) * nf;
+        const long xL0 = ((long)d->fElem[2 * f] * 6 + d->fESide[2 * f] - 1) * nf,
+                   xR0 = ((long)d->fElem[2 * f + 1] * 6 + d->fESide[2 * f + 1] - 1) * nf;
+        const int *y = turned[d->fRot[f]];
         for (int c = c0; c < c1; ++c) {
-            double *eg = egeo.get() + (size_t)c * ES;
+            double *eg = plane(c, ES);
             for (int x = 0; x < nf; ++x) eg[xL0 + x] = fr[c][x];
-            for (int x = 0; x < nf; ++x) eg[xR[x]] = fr[c][x];
+            for (int x = 0; x < nf; ++x) eg[xR0 + y[x]] = fr[c][x];
         }
     };
     eng->t2x = lxf;
-    double fr[10][64];
+    double fr[10][64], wf[64];
+    for (int x = 0; x < nf; ++x) wf[x] = wg[x % n1] * wg[x / n1];
     bool constant = !eng->gauss;   // the frames, over each face's nodes (the Gauss kernels read them by node)
     for (int f = 0; f < F; ++f) {
         face_frame(f, fr);
@@ -1593,26 +1601,28 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
         for (int c = 0; c < (lxf ? 10 : 4) && constant; ++c)
             for (int x = 1; x < nf && constant; ++x) constant = !std::memcmp(&fr[c][x], &fr[c][0], sizeof(double));
         double surf = 0.0;
-        for (int x = 0; x < nf; ++x) surf += wg[x % n1] * wg[x / n1] * fr[3][x];
+        for (int x = 0; x < nf; ++x) surf += wf[x] * fr[3][x];
         // SD.f90:1378, at both elements' slots of the face
         const double fd = std::sqrt(surf / nf);
         efdelta[6 * (long)d->fElem[2 * f] + d->fESide[2 * f] - 1] = fd;
         efdelta[6 * (long)d->fElem[2 * f + 1] + d->fESide[2 * f + 1] - 1] = fd;
     }
     const int gplanes = !lxf ? 4 : eng->t2x ? 7 : 10;
-    if (gplanes == 10)
+    if (gplanes == 10) {
+        eplanes[2].reset(new double[(size_t)3 * ES]);
         for (int f = 0; f < F; ++f) {
             face_frame(f, fr);
             put_frame(f, fr, 7, 10);
         }
+    }
     for (int c = 0; c < gplanes; ++c)   // the padding past the last face node
-        for (long x = (long)K * 6 * nf; x < ES; ++x) egeo[(size_t)c * ES + x] = 0.0;
+        std::fill(plane(c, ES) + (long)K * 6 * nf, plane(c, ES) + ES, 0.0);
     eng->per_face = constant ? 1 : 0;
     eng->egeo_stride = ES;
     if (constant) {
         const long stride = ((6L * K + 63) / 64) * 64;
         for (int c = 0; c < gplanes; ++c)   // in place: plane c's first nodes lie at or behind their new places
-            for (long x = 0; x < stride; ++x) egeo[(size_t)c * stride + x] = x < 6L * K ? egeo[(size_t)c * ES + x * nf] : 0.0;
+            for (long x = 0; x < stride; ++x) plane(c, stride)[x] = x < 6L * K ? plane(c, ES)[x * nf] : 0.0;
         eng->egeo_stride = stride;
     }
     if (!eng->gauss) {
@@ -1648,7 +1658,10 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
     };
     if (!up(eng->dJa, ja.data(), ja.size() * 8) || !up(eng->dJ, jj.data(), jj.size() * 8) ||
         !up(eng->dWq, wq.data(), wq.size() * 8) || !up(eng->dEdelta, edelta.data(), edelta.size() * 8) ||
-        !up(eng->dEgeo, egeo.get(), (size_t)gplanes * eng->egeo_stride * 8) || !up(eng->dNbx, nbx.data(), nbx.size() * 4) ||
+        !up(eng->dEgeo, eplanes[0].get(), (size_t)4 * eng->egeo_stride * 8) ||
+        (gplanes > 4 && !up(eng->dEgeo + 4 * eng->egeo_stride, eplanes[1].get(), (size_t)3 * eng->egeo_stride * 8)) ||
+        (gplanes > 7 && !up(eng->dEgeo + 7 * eng->egeo_stride, eplanes[2].get(), (size_t)3 * eng->egeo_stride * 8)) ||
+        !up(eng->dNbx, nbx.data(), nbx.size() * 4) ||
         !up(eng->dEfdelta, efdelta.data(), efdelta.size() * 8) ||
         (!eng->gauss && !up(eng->dNbr, nbr.data(), nbr.size() * 4)))
         return bail(eng->fail(HX3D_EDEVICE, "upload failed"));

@@ -1,5 +1,6 @@
 """Edges of the engine's entry points: CFL numbers of either sign, engines of many cases and of finished
-ones, meshes beyond the 32-bit offsets, what an Euler engine holds."""
+ones, meshes beyond the 32-bit offsets, what an Euler engine holds and what creation costs."""
+import resource
 import time
 
 import numpy as np
@@ -231,3 +232,20 @@ def test_euler_engine_holds_no_viscous_arrays(nodes, tmp_path):
     assert po.normwise_error(eu.qdot(), ora.qdot(Q0)).max() <= TOL
     ns.close()
     eu.close()
+
+
+def test_repeated_creation_reuses_its_host_pages():
+    """16^3 elements of order 4: the face tangents of a Lax-Friedrichs engine (15 MB) cost no page faults of
+    their own when engines are created one after another (in one array with the normals, past the size of
+    which the allocator keeps pages, they cost 8400 on top of 9000)."""
+    from horses3d_amd.engine import Engine
+    case = mesh.periodic_box(16, 4, amplitude=0.1, phase_seed=1)
+    faults = {}
+    for _ in range(4):
+        for riemann in ("roe", "lxf"):
+            before = resource.getrusage(resource.RUSAGE_SELF).ru_minflt
+            e = Engine(case, mach=0.3, reynolds=700.0, riemann=riemann)
+            faults[riemann] = resource.getrusage(resource.RUSAGE_SELF).ru_minflt - before
+            e.close()
+    print(faults, flush=True)
+    assert faults["lxf"] < 1.3 * faults["roe"] + 500
