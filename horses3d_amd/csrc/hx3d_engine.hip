@@ -586,9 +586,8 @@ int alloc_slots(hx3d_engine *eng, int ncases)
 void init_slots(hx3d_engine *eng, int ncases)
 {
     const long n = (long)ncases * hxk::DT_FAN * hxk::DT_LINE;
-    // the key of +inf (hxk::order_key) has the bits of -inf
     hipLaunchKernelGGL(k_fill, dim3((n + 255) / 256), dim3(256), 0, eng->stream, reinterpret_cast<double *>(eng->dSlots), n,
-                       (double)-INFINITY);
+                       (double)INFINITY);
 }
 
 // The stage kernels address every array plane through a 32-bit byte offset (hxk::ldg), and the
