@@ -357,11 +357,10 @@ k_nan(const double *__restrict__ Q, long nodes, long S, int *__restrict__ flag)
 
 // packed (nodes, 5) <-> SoA [5][S]
 // A state from outside: packed into Q, with the RK register (the reference allocates G_NS zeroed) and
-// the divergence flags, on both sides, cleared.  hflag: pinned host memory.  Qn: the state's second copy
-// where a case is finished (see hx3d_multi_set_active), else null.
+// the divergence flags, on both sides, cleared.  hflag: pinned host memory.
 __global__ void __launch_bounds__(256)
-k_set_state(const double *__restrict__ in, double *__restrict__ Q, double *__restrict__ Qn, double *__restrict__ G, long nodes,
-            long S, int *__restrict__ flag, int *__restrict__ hflag, int ncases)
+k_set_state(const double *__restrict__ in, double *__restrict__ Q, double *__restrict__ G, long nodes, long S,
+            int *__restrict__ flag, int *__restrict__ hflag, int ncases)
 {
     const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (blockIdx.x == 0)
@@ -369,9 +368,7 @@ k_set_state(const double *__restrict__ in, double *__restrict__ Q, double *__res
     if (g >= nodes) return;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-        const double x = in[NV * g + v];
-        Q[v * S + g] = x;
-        if (Qn) Qn[v * S + g] = x;
+        Q[v * S + g] = in[NV * g + v];
         G[v * S + g] = 0.0;
     }
 }
@@ -1855,9 +1852,10 @@ int hx3d_set_state_device(hx3d_engine *eng, const double *Qd)
 {
     if (!eng || !Qd) return HX3D_EINVAL;
     const long nb = (eng->nodes + 255) / 256;
-    const bool both = std::find(eng->finished.begin(), eng->finished.end(), 1) != eng->finished.end();
-    hipLaunchKernelGGL(k_set_state, dim3(nb), dim3(256), 0, eng->stream, Qd, eng->dQ, both ? eng->dQn : nullptr, eng->dG,
-                       eng->nodes, eng->S, eng->dFlag + 1, eng->hFlag, eng->ncases);
+    hipLaunchKernelGGL(k_set_state, dim3(nb), dim3(256), 0, eng->stream, Qd, eng->dQ, eng->dG, eng->nodes, eng->S,
+                       eng->dFlag + 1, eng->hFlag, eng->ncases);
+    if (std::find(eng->finished.begin(), eng->finished.end(), 1) != eng->finished.end())   // see hx3d_multi_set_active
+        hipLaunchKernelGGL(k_copy_state, dim3(nb), dim3(256), 0, eng->stream, eng->dQ, eng->dQn, eng->nodes, eng->S);
     refresh_traces(eng);   // Gauss nodes: the new state's face traces
     eng->qdot_valid = false;
     HIPCHK(hipGetLastError());

@@ -118,9 +118,10 @@ __device__ __forceinline__ void block_elements(const Multi &mc, int lb, int K, i
 {
     if (mc.blocks) {
         const int4 b = mc.blocks[lb];
+        const bool on = mc.active[b.z] != 0;
         e0 = b.x;
         cs = b.z;
-        cnt = mc.active[cs] ? b.y : 0;
+        cnt = on ? b.y : 0;
         first = b.w != 0;
         case_physics(ph, mc.cc[cs]);
     } else {
@@ -648,9 +649,9 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
     bool first;
     if (SPLIT) ph.averaging = FORM;   // the Lax-Friedrichs flux averages as the volume fluxes do
     block_elements<EPB>(mc, lb, K, e0, cnt, cs, first, ph);
-    if (cnt == 0) return;   // uniform: a padding block or a finished case
     const int el = t / ne, n = t - el * ne;
     const int e = e0 + el;
+    if (cnt == 0) return;   // uniform: a padding block or a finished case
     const bool active = el < cnt;
     const int i = n % n1, j = (n / n1) % n1, k = n / nf;
     const bool onx = i == 0 || i == N, ony = j == 0 || j == N, onz = k == 0 || k == N;
