@@ -8,12 +8,14 @@
 
 namespace hxt {
 
-// Host arrays move through a ring of pinned chunks, the copy of one chunk by the host overlapping the
-// transfer of the next: 13.7 MB to pageable memory took 759 us with hipMemcpyAsync (18 GB/s), 385 us
-// from it; the link does 55 GB/s from pinned memory and a host core copies 75 GB/s.  Four chunks of
-// 1 MB: the first waits 20 us, and 4 MB stay pinned per engine that moves host arrays.  Memory the
+// Results leave for host arrays through a ring of pinned chunks, the copy of one chunk by the host
+// overlapping the transfer of the next: 13.7 MB to pageable memory took 759 us with hipMemcpyAsync (18
+// GB/s); the link does 55 GB/s to pinned memory and a host core copies 75 GB/s.  hx3d_get_state into an
+// array that is kept: 13.7 MB 0.88 -> 0.57 ms, 20.5 MB 1.30 -> 0.85, 320 MB 18.8 -> 12.7.  Four chunks of
+// 1 MB: the first waits 20 us, and 4 MB stay pinned per engine that reads host arrays back.  Memory the
 // runtime knows (the caller's own pinned arrays) goes directly, and so does everything if the ring
-// cannot be had.
+// cannot be had.  The other way the runtime's own staging is as good (36 GB/s), and setting a state through the
+// ring measured slower: 8.6 MB 0.27 -> 0.32 ms, 20.5 MB 0.74 -> 0.82, 320 MB 11.5 -> 12.1.
 constexpr int RING_SLOTS = 4;
 constexpr size_t RING_CHUNK = 1 << 20;
 
@@ -22,7 +24,7 @@ struct Ring {
     hipEvent_t ev[RING_SLOTS] = {};
 };
 
-// Whether a transfer of `host` takes the ring, which is made if need be.  Its events must belong to the
+// Whether a transfer to `host` takes the ring, which is made if need be.  Its events must belong to the
 // stream's device (hipEventRecord refuses others), so that device is made current for it: the caller
 // may have another one.
 inline bool use_ring(Ring &r, int device, const void *host)
@@ -82,28 +84,6 @@ inline hipError_t copy_to_host(Ring &r, int device, hipStream_t stream, void *ds
             if (e == hipSuccess) e = hipEventRecord(r.ev[c % RING_SLOTS], stream);
             if (e != hipSuccess) return e;
         }
-    }
-    return hipSuccess;
-}
-
-// bytes from the host array src to the device, in the order of the stream; through the ring src has been
-// read on return; earlier errors as in copy_to_host
-inline hipError_t copy_to_device(Ring &r, int device, hipStream_t stream, void *dst, const void *src, size_t bytes)
-{
-    if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-    if (!use_ring(r, device, src)) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
-    const size_t n = (bytes + RING_CHUNK - 1) / RING_CHUNK;
-    for (size_t c = 0; c < n; ++c) {
-        const size_t size = std::min(RING_CHUNK, bytes - c * RING_CHUNK);
-        char *slot = r.mem + (c % RING_SLOTS) * RING_CHUNK;
-        // an earlier transfer of the slot (this call's, or one still queued) has left it
-        hipError_t e = hipEventSynchronize(r.ev[c % RING_SLOTS]);
-        if (e == hipSuccess) {
-            std::memcpy(slot, (const char *)src + c * RING_CHUNK, size);
-            e = hipMemcpyAsync((char *)dst + c * RING_CHUNK, slot, size, hipMemcpyHostToDevice, stream);
-        }
-        if (e == hipSuccess) e = hipEventRecord(r.ev[c % RING_SLOTS], stream);
-        if (e != hipSuccess) return e;
     }
     return hipSuccess;
 }

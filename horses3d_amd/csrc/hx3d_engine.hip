@@ -894,14 +894,10 @@ void queue_status(hx3d_engine *eng)
                        eng->hOut + H_TIME);
 }
 
-// Transfers of host arrays on the engine's stream (see hxt)
+// From the device to a host array on the engine's stream (see hxt); complete on return
 hipError_t copy_to_host(hx3d_engine *eng, void *dst, const void *src, size_t bytes)
 {
     return hxt::copy_to_host(eng->ring, eng->device, eng->stream, dst, src, bytes);
-}
-hipError_t copy_to_device(hx3d_engine *eng, void *dst, const void *src, size_t bytes)
-{
-    return hxt::copy_to_device(eng->ring, eng->device, eng->stream, dst, src, bytes);
 }
 
 // After a queued step loop: the divergence flag's read-back, and the time derivative the
@@ -1885,7 +1881,7 @@ int hx3d_get_state_nodes(hx3d_engine *eng, long first, long count, double *Qh)
 int hx3d_set_state(hx3d_engine *eng, const double *Qh)
 {
     if (!eng || !Qh) return HX3D_EINVAL;
-    HIPCHK(copy_to_device(eng, eng->dStage, Qh, sizeof(double) * NV * eng->nodes));
+    HIPCHK(hipMemcpyAsync(eng->dStage, Qh, sizeof(double) * NV * eng->nodes, hipMemcpyHostToDevice, eng->stream));
     int rc = hx3d_set_state_device(eng, eng->dStage);
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(eng->stream));

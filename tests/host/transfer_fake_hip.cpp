@@ -75,7 +75,7 @@ static std::vector<char> bytes(size_t n, unsigned seed)
     return v;
 }
 
-// both ways, twice through one ring, with another device current than the engine's
+// twice through one ring, with another device current than the engine's
 static int transfers(int caller, int device)
 {
     ihipStream_t s{device};
@@ -83,12 +83,10 @@ static int transfers(int caller, int device)
     for (int pass = 0; pass < 2; ++pass)
         for (size_t n : SIZES) {
             current = caller;
-            const std::vector<char> host = bytes(n, (unsigned)n + pass);
-            std::vector<char> src = host, dev(n), back(n);
-            CHECK(hxt::copy_to_device(r, device, &s, dev.data(), src.data(), n) == hipSuccess);
-            std::fill(src.begin(), src.end(), 0);   // read on return
-            CHECK(hxt::copy_to_host(r, device, &s, back.data(), dev.data(), n) == hipSuccess);
-            CHECK(back == host);
+            const std::vector<char> dev = bytes(n, (unsigned)n + pass);
+            std::vector<char> host(n);
+            CHECK(hxt::copy_to_host(r, device, &s, host.data(), dev.data(), n) == hipSuccess);
+            CHECK(host == dev);
             CHECK(current == caller);
         }
     CHECK(pinned == 1 && events == hxt::RING_SLOTS);
@@ -106,8 +104,6 @@ static int failed_launch()
     for (int pass = 0; pass < 2; ++pass) {
         last = hipErrorLaunchFailure;
         CHECK(hxt::copy_to_host(r, 0, &s, a.data(), b.data(), a.size()) == hipErrorLaunchFailure);
-        last = hipErrorLaunchFailure;
-        CHECK(hxt::copy_to_device(r, 0, &s, b.data(), a.data(), a.size()) == hipErrorLaunchFailure);
         CHECK(hxt::copy_to_host(r, 0, &s, a.data(), b.data(), a.size()) == hipSuccess);
         CHECK(last == hipSuccess);
     }

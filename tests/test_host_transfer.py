@@ -1,4 +1,4 @@
-"""The engine's host transfers on a stand-in for the HIP runtime (tests/host/transfer_fake_hip.cpp): exact
+"""The engine's transfers to host arrays on a stand-in for the HIP runtime (tests/host/transfer_fake_hip.cpp): exact
 through the ring of pinned chunks whatever the size, and with another device current than the engine's;
 a launch that failed before a transfer is reported by it."""
 import os
