@@ -1633,13 +1633,15 @@ int hx3d_engine_create(const hx3d_case_desc *d, hx3d_engine **out)
         (rc = dalloc(eng, &eng->dStage, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dBits, 2 * DT_SLOTS)) ||
         (rc = dalloc(eng, &eng->dFlag, 2)) || (rc = dalloc(eng, &eng->dNbx, nbx.size())))
         return bail(rc);
-    if ((rc = dalloc(eng, &eng->dEfdelta, efdelta.size())) || (rc = alloc_slots(eng, 1))) return bail(rc);
     if (!eng->ph.euler &&   // the viscous arrays: no kernel of an Euler case reads or writes them
         ((rc = dalloc(eng, &eng->dVisc, (size_t)(eng->gauss ? hxk::NVF : hxk::viscous_values(eng->ph.les)) * S)) ||
-         (rc = dalloc(eng, &eng->dCurl, (size_t)S)) || (eng->gauss && (rc = dalloc(eng, &eng->dFvis, (size_t)hxk::NVF * ES)))))
+         (rc = dalloc(eng, &eng->dCurl, (size_t)S))))
         return bail(rc);
+    if ((rc = dalloc(eng, &eng->dEfdelta, efdelta.size())) || (rc = alloc_slots(eng, 1))) return bail(rc);
     if (eng->gauss) {
-        if ((rc = dalloc(eng, &eng->dQtr, (size_t)NV * ES)) || (rc = dalloc(eng, &eng->dQtn, (size_t)NV * ES))) return bail(rc);
+        if ((rc = dalloc(eng, &eng->dQtr, (size_t)NV * ES)) || (rc = dalloc(eng, &eng->dQtn, (size_t)NV * ES)) ||
+            (!eng->ph.euler && (rc = dalloc(eng, &eng->dFvis, (size_t)hxk::NVF * ES))))
+            return bail(rc);
     } else if ((rc = dalloc(eng, &eng->dQn, (size_t)NV * S)) || (rc = dalloc(eng, &eng->dNbr, nbr.size()))) {
         return bail(rc);
     }

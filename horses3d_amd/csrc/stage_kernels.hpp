@@ -37,6 +37,17 @@ __device__ __forceinline__ void hold(double &x)
 #endif
 }
 
+// A kernel argument wanted in scalar registers at this point
+template <class T>
+__device__ __forceinline__ void wanted(T x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : : "s"(x));
+#else
+    (void)x;
+#endif
+}
+
 // Element i of an array through its (wave-uniform) base and a 32-bit offset: the access takes
 // the base from scalar registers and one 32-bit vector offset, with no 64-bit address
 // arithmetic per access.  Every array plane the kernels index holds fewer than 2^29 elements
@@ -647,6 +658,20 @@ k_volume(const double *__restrict__ Q, double *__restrict__ Qn, const double *__
     const int t = threadIdx.x;
     int e0, cnt, cs;
     bool first;
+    if (N <= 3) {
+        // one wave per block: the first loads' addresses ahead of the early return, with the scalar loads
+        // before it (15^3 x N=2: 13.03 -> 12.60 us).  Larger blocks hide that wait behind one another, and
+        // the registers spill (9^3 x N=6 with LES: 10% slower).
+        wanted(Q);
+        wanted(nbx);
+        wanted(visc);
+        wanted(mt.Ja);
+        wanted(mt.face);
+        wanted(K);
+        wanted(S);
+        wanted(mt.S);
+        wanted(mt.FS);
+    }
     if (SPLIT) ph.averaging = FORM;   // the Lax-Friedrichs flux averages as the volume fluxes do
     block_elements<EPB>(mc, lb, K, e0, cnt, cs, first, ph);
     const int el = t / ne, n = t - el * ne;
