@@ -700,17 +700,15 @@ void launch_volume(hx3d_engine *eng, double a_k, double c_k, int update, const D
 bool two_launch(const hx3d_engine *eng) { return !eng->mixed; }
 double *current_copy(const hx3d_engine *eng) { return eng->gauss ? eng->dQtr : eng->dQ; }
 
-// One stage on the engine stream.  ev: NULL, or 4 events recorded around the launches
-// (timing only); like a failed launch, a failed record surfaces through hipGetLastError, which
+// One stage on the engine stream.  ev: NULL, or 4 events recorded around the launches (timing
+// only; two launches take no ev[2]); like a failed launch, a failed record surfaces through hipGetLastError, which
 // the calling entry point checks after its launches.
 template <int N>
 void stage_n(hx3d_engine *eng, double a_k, double c_k, int update, const DtArgs &dta, double *qdot,
              hipEvent_t *ev)
 {
-    auto face_events = [&]() {   // no face kernel of its own
-        if (!ev) return;
-        (void)hipEventRecord(ev[1], eng->stream);
-        (void)hipEventRecord(ev[2], eng->stream);
+    auto mid_event = [&]() {   // no face kernel of its own, and no event for one
+        if (ev) (void)hipEventRecord(ev[1], eng->stream);
     };
     if (eng->gauss) {
         // Gauss nodes: traces in element-face order (hxg)
@@ -722,7 +720,7 @@ void stage_n(hx3d_engine *eng, double a_k, double c_k, int update, const DtArgs 
                                eng->dJ, eng->dNbx, eng->dEgeo, eng->dEdelta, eng->dEfdelta, eng->dVisc, eng->dFvis,
                                qdot ? eng->dCurl : nullptr, eng->K, eng->S, eng->ES, eng->ops, eng->gops, eng->ph,
                                dta.lim);
-        face_events();
+        mid_event();
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(nb), dim3(TPB), 0, eng->stream, eng->dQ, eng->dQtr, eng->dQtn, eng->dVisc,
                                eng->dFvis, eng->dNbx, eng->dEgeo, eng->t2x ? 1 : 0, eng->dJa, eng->dJ, eng->dG, qdot, a_k,
@@ -736,7 +734,7 @@ void stage_n(hx3d_engine *eng, double a_k, double c_k, int update, const DtArgs 
     }
     if (ev) (void)hipEventRecord(ev[0], eng->stream);
     if (!eng->ph.euler) launch_grad<N>(eng, dta.lim, qdot ? eng->dCurl : nullptr);
-    face_events();
+    mid_event();
     launch_volume<N>(eng, a_k, c_k, update, dta, qdot);
     if (ev) (void)hipEventRecord(ev[3], eng->stream);
 }
@@ -2112,11 +2110,16 @@ int hx3d_advance(hx3d_engine *eng, int nsteps, double cfl, double dcfl, double *
         HIPCHK(hipStreamSynchronize(eng->stream));
         double acc[3] = {0, 0, 0};
         for (size_t x = 0; x < (size_t)3 * nsteps; ++x) {
-            for (int kk = 0; kk < 3; ++kk) {
+            hipEvent_t *const ev = &eng->evpool[4 * x];
+            auto add = [&](int kk, int from, int to) {
                 float ms = 0.f;
-                HIPCHK(hipEventElapsedTime(&ms, eng->evpool[4 * x + kk], eng->evpool[4 * x + kk + 1]));
+                const hipError_t e = hipEventElapsedTime(&ms, ev[from], ev[to]);
                 acc[kk] += ms;
-            }
+                return e;
+            };
+            HIPCHK(add(0, 0, 1));
+            if (!two_launch(eng)) HIPCHK(add(1, 1, 2));
+            HIPCHK(add(2, two_launch(eng) ? 1 : 2, 3));
         }
         for (int x = 0; x < 3; ++x) eng->ktime[x] = acc[x] / (3.0 * nsteps);
         eng->ktime[3] = (eng->ktime[0] + eng->ktime[1] + eng->ktime[2]);

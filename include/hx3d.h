@@ -217,9 +217,9 @@ int hx3d_set_tiling(hx3d_engine *eng, int policy);
 int hx3d_get_tiling(const hx3d_engine *eng, int *policy, int *ntiles);
 /* Average duration (ms) per launch of each stage kernel over the last hx3d_advance call,
  * measured with HIP events on the engine stream when timing was enabled with
- * hx3d_set_timing(eng, 1): out[0..2] = gradient+lifting, face flux (no launch of its own with
- * Gauss-Lobatto nodes of one order: the volume kernel forms the face fluxes), volume+surface+RK;
- * out[3] = their sum (one stage). */
+ * hx3d_set_timing(eng, 1): out[0..2] = gradient+lifting, face flux (0 for cases of one order, either
+ * node type: the volume kernel forms the face fluxes), volume+surface+RK; out[3] = their sum (one
+ * stage). */
 int hx3d_set_timing(hx3d_engine *eng, int on);
 int hx3d_kernel_times(hx3d_engine *eng, double out_ms[4]);
 

@@ -1,5 +1,6 @@
 """Edges of the engine's entry points: CFL numbers of either sign, engines of many cases and of finished
-ones, meshes beyond the 32-bit offsets, what an Euler engine holds and what creation costs."""
+ones, meshes beyond the 32-bit offsets, what an Euler engine holds, what creation costs and
+what the kernel times count."""
 import resource
 import time
 
@@ -249,3 +250,20 @@ def test_repeated_creation_reuses_its_host_pages():
             e.close()
     print(faults, flush=True)
     assert faults["lxf"] < 1.3 * faults["roe"] + 500
+
+
+@pytest.mark.parametrize("kind", ["gauss-lobatto", "gauss", "mixed"])
+def test_kernel_times_count_launches(kind, tmp_path):
+    """A case of one order has no face kernel, and none is timed (two events with nothing between them are
+    4 us apart); mixed orders have one."""
+    from horses3d_amd.engine import Engine
+    case = {"gauss": lambda: gauss_box(3, 3, tmp_path), "mixed": lambda: mesh.periodic_box_mixed(3, mesh.random_orders(27, 2, 4, 5)),
+            "gauss-lobatto": lambda: mesh.periodic_box(3, 3, amplitude=0.1, phase_seed=5)}[kind]()
+    eng = Engine(case, nodes="gauss" if kind == "gauss" else "gauss-lobatto", **KW)
+    eng.set_state(mesh.taylor_green(case, 0.3))
+    eng.set_timing(True)
+    eng.advance(3, 0.4, 0.4, t=0.0)
+    grad, face, volume, stage = eng.kernel_times()
+    assert grad > 0.0 and volume > 0.0 and stage == grad + face + volume
+    assert (face > 0.0) == (kind == "mixed")
+    eng.close()
