@@ -12,12 +12,14 @@ namespace hxt {
 // overlapping the transfer of the next: 13.7 MB to pageable memory took 759 us with hipMemcpyAsync (18
 // GB/s); the link does 55 GB/s to pinned memory and a host core copies 75 GB/s.  hx3d_get_state into an
 // array that is kept: 13.7 MB 0.88 -> 0.57 ms, 20.5 MB 1.30 -> 0.85, 320 MB 18.8 -> 12.7.  Four chunks of
-// 1 MB: the first waits 20 us, and 4 MB stay pinned per engine that reads host arrays back.  Memory the
+// 1 MB: the first waits 20 us, and 4 MB stay pinned per engine that reads such arrays back.  Memory the
 // runtime knows (the caller's own pinned arrays) goes directly, and so does everything if the ring
 // cannot be had.  The other way the runtime's own staging is as good (36 GB/s), and setting a state through the
 // ring measured slower: 8.6 MB 0.27 -> 0.32 ms, 20.5 MB 0.74 -> 0.82, 320 MB 11.5 -> 12.1.
+// From RING_MIN bytes on: hx3d_get_state of 0.16 MB 29 us directly and 35 through the ring (67 the first time, which
+// makes it), 0.88 MB 57 and 63 (87), 1.9 MB 116 and 101 (130), 2.6 MB 163 and 131 (160).
 constexpr int RING_SLOTS = 4;
-constexpr size_t RING_CHUNK = 1 << 20;
+constexpr size_t RING_CHUNK = 1 << 20, RING_MIN = 2 << 20;
 
 struct Ring {
     char *mem = nullptr;   // RING_SLOTS chunks, from the first transfer on
@@ -64,7 +66,7 @@ inline void destroy_ring(Ring &r)
 inline hipError_t copy_to_host(Ring &r, int device, hipStream_t stream, void *dst, const void *src, size_t bytes)
 {
     if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-    if (!use_ring(r, device, dst)) {
+    if (bytes < RING_MIN || !use_ring(r, device, dst)) {
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream);
         return e != hipSuccess ? e : hipStreamSynchronize(stream);
     }

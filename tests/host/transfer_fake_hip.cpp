@@ -64,9 +64,9 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipSt
 
 #define CHECK(x) do { if (!(x)) { std::printf("line %d: %s\n", __LINE__, #x); return 1; } } while (0)
 
-// sizes below, at and past the chunks and the slots
-static const size_t SIZES[] = {1, hxt::RING_CHUNK - 1, hxt::RING_CHUNK, hxt::RING_CHUNK + 1, 4 * hxt::RING_CHUNK,
-                               4 * hxt::RING_CHUNK + 7, 11 * hxt::RING_CHUNK - 3};
+// sizes below, at and past the ring's least, the chunks and the slots
+static const size_t SIZES[] = {1, hxt::RING_MIN - 1, hxt::RING_MIN, hxt::RING_MIN + 1, 3 * hxt::RING_CHUNK - 1,
+                               4 * hxt::RING_CHUNK, 4 * hxt::RING_CHUNK + 7, 11 * hxt::RING_CHUNK - 3};
 
 static std::vector<char> bytes(size_t n, unsigned seed)
 {
@@ -95,12 +95,26 @@ static int transfers(int caller, int device)
     return 0;
 }
 
-// a failed launch before a transfer is the transfer's result, with and without a ring in place
-static int failed_launch()
+// results below the ring's least make none
+static int small_results()
 {
     ihipStream_t s{0};
     hxt::Ring r;
-    std::vector<char> a(100), b(100);
+    for (size_t n : {(size_t)1, hxt::RING_MIN - 1}) {
+        const std::vector<char> dev = bytes(n, (unsigned)n);
+        std::vector<char> host(n);
+        CHECK(hxt::copy_to_host(r, 0, &s, host.data(), dev.data(), n) == hipSuccess);
+        CHECK(host == dev && pinned == 0 && events == 0);
+    }
+    return 0;
+}
+
+// a failed launch before a transfer is the transfer's result, with and without a ring in place
+static int failed_launch(size_t n)
+{
+    ihipStream_t s{0};
+    hxt::Ring r;
+    std::vector<char> a(n), b(n);
     for (int pass = 0; pass < 2; ++pass) {
         last = hipErrorLaunchFailure;
         CHECK(hxt::copy_to_host(r, 0, &s, a.data(), b.data(), a.size()) == hipErrorLaunchFailure);
@@ -115,6 +129,7 @@ int main(int argc, char **argv)
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "same device") return transfers(0, 0);
     if (what == "another device current") return transfers(1, 0);
-    if (what == "failed launch") return failed_launch();
+    if (what == "small results") return small_results();
+    if (what == "failed launch") return failed_launch(100) || failed_launch(hxt::RING_MIN);
     return 2;
 }

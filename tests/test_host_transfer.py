@@ -1,6 +1,6 @@
 """The engine's transfers to host arrays on a stand-in for the HIP runtime (tests/host/transfer_fake_hip.cpp): exact
 through the ring of pinned chunks whatever the size, and with another device current than the engine's;
-a launch that failed before a transfer is reported by it."""
+small results make no ring; a launch that failed before a transfer is reported by it."""
 import os
 import shutil
 import subprocess
@@ -23,7 +23,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["same device", "another device current", "failed launch"])
+@pytest.mark.parametrize("check", ["same device", "another device current", "small results", "failed launch"])
 def test_transfers(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
