@@ -8,12 +8,12 @@
 //   km_face_grad  one wave per face (or two small faces of one shape, see face_lane): both Q
 //                 traces to the face order, BR1 unStar there,
 //                 projected back onto each side's element face (lift[15][ES]);
-//   km_grad       element tiles: local gradient + lifting -> grad Q (15 values);
+//   km_grad       element tiles: local gradient + lifting -> grad Q (15 values); in a step's
+//                 first stage, the dt limits;
 //   km_face       as km_face_grad: Q and grad Q traces to the face order, Riemann + BR1
 //                 fluxes there, projected back (right side negated) and scaled by the
 //                 receiving element's surface weight -> fe[5][ES];
-//   km_volume     element tiles: volume integral, surface integral, 1/J, RK update and
-//                 the next step's dt limits.
+//   km_volume     element tiles: volume integral, surface integral, 1/J and RK update.
 // The element kernels are persistent: one launch per stage sweeps every element, each block
 // taking tiles (elements packed into at most 512 nodes, one thread per node) in turn, each
 // thread reading what it works on from the tiles' node map.
@@ -500,8 +500,9 @@ km_face_grad(const double *__restrict__ Q, const FaceRec *__restrict__ faces, co
 // km_grad: local gradient (HexElement_ComputeLocalGradient, HexElementClass.f90:427-531) and
 // BR1 lifting (BR1_GradientFaceLoop, EllipticBR1.f90:531-569, with the weights b of
 // VectorWeakIntegrals_StdFace): grad Q at every node, U[(5d + v)*S + g].
-// Bound by memory: 256 bytes a node and 120 an element face node (515 MB on 20^3 elements of orders
-// 2..7, 154.9 -> 133.3 us, 3.9 TB/s).  What keeps the registers under 128 and two large tiles on a CU:
+// Bound by memory: 176 bytes a node (256 where the metrics are by node) and 120 an element face node; 440 MB
+// on 20^3 elements of orders 2..7, 3.8 TB/s, 115 us (154.9 before what follows and before the metrics were
+// read once per element).  What keeps the registers under 128 and two large tiles on a CU:
 // the nodes of a tile lie together in LDS (one address per node with constant offsets, instead of one
 // per value; the odd stride keeps a line's nodes in distinct banks), derivative loops that are
 // not unrolled, and the lifting a direction at a time.  10^3 Gauss elements of orders 2..5: 29.6 -> 13.3 us.
@@ -795,12 +796,14 @@ km_face(const double *__restrict__ Q, const double *__restrict__ U, const FaceRe
 // state formed from grad Q (ViscousFlux_STATE), and MaxTimeStep's 1/|x_1 - x_0| per direction.
 // LDS (dynamic): hatD and sharpD of every order [2][MAXN1][64], then each node's fluxes and data
 // together (see km_grad).
-// Bound by memory: 376 bytes a node and 40 an element face node (558 MB on 20^3 elements of orders
-// 2..7, standard form, 158.3 -> 123.3 us, 4.5 TB/s).  That takes two large tiles per CU (four waves per SIMD,
+// Bound by memory: 296 bytes a node (376 where the metrics are by node) and 40 an element face node; 493 MB
+// on 20^3 elements of orders 2..7, standard form, 5.0 TB/s, 99 us (158.3 before what follows and before the
+// metrics were read once per element).  That takes two large tiles per CU (four waves per SIMD,
 // 128 registers): the surface integral is summed as its loads arrive, the fluxes go to LDS a direction
-// at a time.  The split form's LDS admits one large tile, and Gauss nodes, with six faces' loads in
+// at a time.  The split form's LDS admits one large tile.  Gauss nodes, with six faces' loads in
 // flight per node, are faster with the registers (10^3 elements of orders 2..5: 12.7 us against 18.5 at
-// four waves).
+// four waves), and so is LES, which takes 164 of them (20^3, orders 2..7, Smagorinsky 113.8 us against 117.6,
+// WALE 118.1 against 157.1; 20^3 of order 3 but for one element 38.6 against 42.8 and 39.4 against 58.9).
 // ------------------------------------------------------------------------------------
 template <int FORM>
 constexpr int mvolume_per_node()

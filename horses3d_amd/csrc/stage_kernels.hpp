@@ -145,9 +145,9 @@ __device__ __forceinline__ void block_elements(const Multi &mc, int lb, int K, i
 
 // MaxTimeStep of the state a stage starts from, accumulated by the stage's gradient kernel.
 // Mixed orders (part; null: not this stage): block minima of the convective and viscous limits to
-// part[2*block + 0/1], reduced by the face kernel that follows (DtReduce).  One order (slots; null: not this stage): each block's minima by atomicMin
-// into one of the case's DT_FAN slots, from which every block of the volume kernel that follows
-// takes the minimum.  The minimum of doubles does not depend on the order; limits of either sign (those
+// part[2*block + 0/1], reduced by the face kernel that follows (DtReduce).  One order (slots; null: not
+// this stage): each block's minima by atomics into one of the case's DT_FAN slots, from which every block
+// of the volume kernel that follows takes the minimum.  The minimum of doubles does not depend on the order; limits of either sign (those
 // of a negative CFL number are negative) take their places like the numbers (slot_min), and NaN is
 // passed over as fmin passes it over.  DT_FAN slots on lines of their own: one slot alone
 // serialises (16k atomics on one address cost 150 us), 32 leave at most a few hundred per line at 24^3
@@ -195,8 +195,8 @@ __device__ __forceinline__ unsigned efx(int e, int slot, int a, int b)
 // Registers: at most 128, which the attribute holds it to (114 to 124 are taken: the state is read again
 // after the gradient, LES is a template flag, and order 7 takes its directions one at a time), since a
 // block of six or eight waves finds room beside another only at four waves per SIMD: 9^3 elements of order 6 24.0 -> 19.9 us, of order 7 31.6 -> 25.7 (with
-// LES).  Below that it makes no difference: at 16^3 elements of order 4 the kernel moves 153 MB in 28.4 us, 24^3
-// of order 5 898 MB in 193 us, near the copy rate (6.9 TB/s from the caches, 5 from memory).
+// LES).  Below that it makes no difference: at 16^3 elements of order 4 the kernel moves 135 MB in 25.7 us, 24^3
+// of order 5 with LES 795 MB in 194 us, 0.76 and 0.82 of the copy rate (6.9 TB/s from the caches, 5 from memory).
 
 // Metric terms of a case of one order: Ja^d_c in planes Ja[c*S + i], J[i], and the face frames
 // face[c*FS + i].  Where they are the same bits at every node of each element (each face), as on boxes of
@@ -626,9 +626,9 @@ struct VolumeLds {
 // instead of 0.6 Riemann fluxes per node at N = 4, and saves the launch, the 80 B per face node
 // of stored fluxes each way and the second read of both traces.  Measured per stage (k_grad and
 // k_volume; before, with a face kernel between them and the gradients stored): 16^3 x N=4 Pirozzoli
-// 88 us (97), 24^3 x N=5 Kennedy-Gruber + WALE 592 (690), 4^3 x N=3 14 (18), 9^3 x N=6 46 (62).
-// At 16^3 x N=4 the kernel moves 265 MB in 59 us; without the direction loop it takes 40 us, the
-// rate of a large copy, and the loop's LDS traffic (97 accesses per node and direction) adds the
+// 81 us (91), 24^3 x N=5 Kennedy-Gruber + WALE 587 (701), 4^3 x N=3 13 (18), 9^3 x N=6 44 (62).
+// At 16^3 x N=4 the kernel moves 241 MB in 55 us.  Without the direction loop it took 40 us where it took 59
+// with it, the rate of a large copy; the loop's LDS traffic (97 accesses per node and direction) adds the
 // rest.  Forming the gradient again here instead of reading the viscous values measured 76 us.
 // New state to Qn, not in place: the neighbours of later blocks still read Q.
 // LXF: the engine's Riemann solver is Lax-Friedrichs, the one that reads the tangents (Roe does not).
